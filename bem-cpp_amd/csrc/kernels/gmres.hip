@@ -41,26 +41,44 @@ namespace {
 constexpr int GS_ROWS = 256;  // rows per partial sum of the Gram-Schmidt products
 
 // P[(i * nchunk + chunk) * ncol + j] = sum over the chunk's rows k of
-// conj(V_i[k][j]) w[k][j]; grid (nchunk, m), one column per thread.
+// conj(V_i[k][j]) w[k][j]; grid (nchunk, m).  A workgroup takes min(ncol, 256)
+// columns side by side and the chunk's rows in 256 / columns lanes, summed in
+// lane order (one thread per column left all but ncol of the 256 idle, a
+// serial chain of 256 loads each: 101 us at n = 4608 with 16 columns).
 __global__ __launch_bounds__(256) void k_gs_partial(int n, int ncol, const double* __restrict__ Vr,
                                                     const double* __restrict__ Vi, long vstride,
                                                     const double* __restrict__ wr, const double* __restrict__ wi,
                                                     double* __restrict__ Pr, double* __restrict__ Pi, int nchunk) {
+    __shared__ double red[2][256];
     const int chunk = blockIdx.x, i = blockIdx.y;
     const int k0 = chunk * GS_ROWS, k1 = min(n, k0 + GS_ROWS);
     const double* vr = Vr + (long)i * vstride;
     const double* vi = Vi + (long)i * vstride;
-    for (int j = threadIdx.x; j < ncol; j += blockDim.x) {
+    const int cw = min(ncol, 256), lanes = 256 / cw, tx = threadIdx.x % cw, ty = threadIdx.x / cw;
+    for (int c0 = 0; c0 < ncol; c0 += cw) {
+        const int j = c0 + tx;
         double sr = 0.0, si = 0.0;
-        for (int k = k0; k < k1; k++) {
-            const long o = (long)k * ncol + j;
-            const double a = vr[o], b = vi[o], c = wr[o], d = wi[o];
-            sr += a * c + b * d;  // conj(a + ib) (c + id)
-            si += a * d - b * c;
+        if (ty < lanes && j < ncol)
+#pragma unroll 4
+            for (int k = k0 + ty; k < k1; k += lanes) {
+                const long o = (long)k * ncol + j;
+                const double a = vr[o], b = vi[o], c = wr[o], d = wi[o];
+                sr += a * c + b * d;  // conj(a + ib) (c + id)
+                si += a * d - b * c;
+            }
+        red[0][threadIdx.x] = sr;
+        red[1][threadIdx.x] = si;
+        __syncthreads();
+        if (ty == 0 && j < ncol) {
+            for (int l = 1; l < lanes; l++) {
+                sr += red[0][l * cw + tx];
+                si += red[1][l * cw + tx];
+            }
+            const long p = ((long)i * nchunk + chunk) * ncol + j;
+            Pr[p] = sr;
+            Pi[p] = si;
         }
-        const long p = ((long)i * nchunk + chunk) * ncol + j;
-        Pr[p] = sr;
-        Pi[p] = si;
+        __syncthreads();
     }
 }
 

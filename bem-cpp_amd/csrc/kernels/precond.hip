@@ -10,17 +10,17 @@
 //   k_bj_gather  copies rows/columns {rwg_j, N + rwg_j : j in the extended
 //                block} of the FP64 Z into a zero-padded n2max x n2max slot
 //                per block (one launch for all blocks);
-//   k_bj_inv     inverts every block in its own workgroup by Gauss-Jordan
-//                elimination with the reference's pivoting: at step k the
-//                pivot is the first row of largest |a_ik| (precond.cu:842-851),
-//                rows k and p are swapped, a pivot below 1e-30 in magnitude
-//                is replaced by 1e-15 (precond.cu:858-859); the row swaps
-//                become column swaps of the inverse at the end;
+//   k_bj_panel, k_bj_inner, k_bj_rows, k_bj_update
+//                invert every block in place by blocked Gauss-Jordan
+//                elimination with the reference's pivoting (the largest
+//                |a_ik| of the rows not used yet, precond.cu:842-851; a pivot
+//                below 1e-30 in magnitude is replaced by 1e-15,
+//                precond.cu:858-859);
 //   apply        gathers each block's extended part of r into a padded slot,
-//                multiplies all slots by their inverses in one batched
-//                FP64 complex GEMM on the matrix cores, and scatters only the
-//                block's own unknowns (restricted additive Schwarz; without
-//                overlap plain block-Jacobi).
+//                multiplies the slots by their inverses on the matrix cores
+//                (k_bj_mult), and scatters only the block's own unknowns
+//                (restricted additive Schwarz; without overlap plain
+//                block-Jacobi).
 // The inverse gives the same M^{-1} r as the reference's LU solve up to
 // rounding, at three times the factorisation work, and turns the apply into
 // one matrix-core product instead of sequential substitutions.
@@ -63,141 +63,420 @@ __global__ __launch_bounds__(256) void k_bj_gather(BjView v, int N, int ld, cons
     }
 }
 
-// In-place Gauss-Jordan inverse of the n2 x n2 block at (Ar, Ai) (row-major,
-// leading dimension ld), one workgroup per block (1024 threads: one column
-// each for blocks up to 1024 unknowns, and enough waves per CU to cover the
-// memory latency of the row sweeps); F is an n2-entry column scratch per
-// block, piv the row interchanges.
-constexpr int BJ_INV_THREADS = 1024;
-__global__ __launch_bounds__(BJ_INV_THREADS) void k_bj_inv(BjView v, int ld, double* __restrict__ Ar, double* __restrict__ Ai,
-                                                double* __restrict__ Fr, double* __restrict__ Fi,
-                                                int* __restrict__ piv) {
-    __shared__ double red_v[BJ_INV_THREADS];
-    __shared__ int red_i[BJ_INV_THREADS];
-    const int b = blockIdx.x, t = threadIdx.x;
+// ---------------------------------------------------------------------------
+// Inverse of every block by blocked Gauss-Jordan elimination in place, all
+// blocks in each launch.  Rows are not interchanged: column k takes its pivot
+// among the rows not used yet and remembers it in prow[k].  With slot k then
+// holding the column of b_{prow[k]}, the result M at the end gives
+//   x_k = sum_j M[prow_k][j] b_{prow_j},
+// so the apply gathers r and scatters the result through prow and no row or
+// column is ever moved.  For a set K of columns whose panel G (all rows of
+// the columns K after their elimination) is known, every other column c is
+//   a_ic <- (i in prow_K ? 0 : a_ic) + sum_{k in K} G_ik a_{prow_k, c}:
+// an outer panel of 64 columns is eliminated in four inner panels of 16
+// (k_bj_panel, then k_bj_inner for the other 48 columns of the panel), then
+// the rest of the matrix takes one rank-64 product (k_bj_rows, k_bj_update).
+//
+// What bounds it: the panels' serial chain of pivot steps (98 us per 16
+// columns at 1107 unknowns, blocks side by side), then the rank-64 FP64
+// products (175 us each).  26 blocks of up to 1107 unknowns: 15 ms, where one
+// workgroup sweeping its whole block from memory at every pivot step (the
+// earlier form) took 1600 ms, n2^2 complex values moved per step.
+// ---------------------------------------------------------------------------
+constexpr int BJ_W = 16;   // inner panel
+constexpr int BJ_O = 64;   // outer panel
+constexpr int BJ_T = 512;  // threads of k_bj_panel (256 threads with twice the rows each measured the same)
+constexpr int BJ_MAXR = 3; // rows per thread it can hold in registers (64 registers each)
+
+// 32-bit order-preserving key of |z|^2 (20 mantissa bits); 0: no candidate.
+__device__ __forceinline__ unsigned bj_key(double r, double i) {
+    const double m = r * r + i * i;
+    return m >= 0.0 ? (unsigned)((unsigned long long)__double_as_longlong(m) >> 32) + 1u : 1u;
+}
+extern "C" __device__ unsigned __ockl_wfred_max_u32(unsigned);
+
+// Elimination of columns c0 .. c0+15 of every block, one workgroup each.
+// RPT > 0: the panel's rows in registers, rows t + BJ_T r, r < RPT (n2 <= RPT
+// BJ_T); RPT == 0: the panel stays in memory (any n2).  step[row] is the
+// column a row is the pivot of (-1: none yet).  The pivot is the largest |a|
+// (to 2^-20; ties: the lowest row of the lowest thread) of the unused rows; a
+// pivot below 1e-30 in modulus is replaced by 1e-15 (precond.cu:842-859).
+// At the end the pivot rows' entries in the outer panel's 64 columns (from k0)
+// go to Bin (16 x 64 per plane and block).
+template <int RPT>
+__global__ __launch_bounds__(BJ_T) void k_bj_panel(BjView v, int ld, int c0, int k0, double* __restrict__ Ar,
+                                                   double* __restrict__ Ai, int* __restrict__ step,
+                                                   int* __restrict__ prow, double* __restrict__ Bin) {
+    constexpr int NW = BJ_T / 64, R = RPT > 0 ? RPT : 1;
+    __shared__ unsigned long long kb[NW];
+    __shared__ double row_r[BJ_W], row_i[BJ_W];
+    __shared__ int prows[BJ_W];
+    const int b = blockIdx.x, t = threadIdx.x, wave = t >> 6;
     const int n2 = 2 * v.Be[b];
-    double* ar = Ar + (long)b * ld * ld;
-    double* ai = Ai + (long)b * ld * ld;
-    double* fr = Fr + (long)b * ld;
-    double* fi = Fi + (long)b * ld;
-    int* pv = piv + v.poff[b];
-    for (int k = 0; k < n2; k++) {
-        // pivot: first row of largest modulus in column k, rows k..n2-1
-        double best = -1.0;
-        int bi = k;
-        for (int i = k + t; i < n2; i += BJ_INV_THREADS) {
-            const double m = hypot(ar[(long)i * ld + k], ai[(long)i * ld + k]);
-            if (m > best) {
-                best = m;
-                bi = i;
+    if (c0 >= n2) return;
+    const int w = min(BJ_W, n2 - c0);
+    double* ar = Ar + (long)b * ld * ld + c0;
+    double* ai = Ai + (long)b * ld * ld + c0;
+    int* st = step + (long)b * ld;
+    double xr[R][BJ_W], xi[R][BJ_W];
+    int used[R];
+    if constexpr (RPT > 0) {
+#pragma unroll
+        for (int q = 0; q < R; q++) {
+            const int i = t + BJ_T * q;
+            used[q] = i < n2 ? st[i] : 0;
+#pragma unroll
+            for (int c = 0; c < BJ_W; c++) {
+                xr[q][c] = i < n2 ? ar[(long)i * ld + c] : 0.0;  // columns beyond n2 are zero (ld is a multiple of 64)
+                xi[q][c] = i < n2 ? ai[(long)i * ld + c] : 0.0;
             }
         }
-        red_v[t] = best;
-        red_i[t] = bi;
-        __syncthreads();
-        for (int s = BJ_INV_THREADS / 2; s > 0; s >>= 1) {
-            if (t < s) {
-                const double o = red_v[t + s];
-                const int oi = red_i[t + s];
-                if (o > red_v[t] || (o == red_v[t] && oi < red_i[t])) {
-                    red_v[t] = o;
-                    red_i[t] = oi;
+    }
+#pragma unroll
+    for (int j = 0; j < BJ_W; j++) {
+        if (j < w) {  // the same for the whole workgroup; a break would keep the loop from unrolling
+        unsigned key = 0;
+        int best = 0x7fffffff;
+        if constexpr (RPT > 0) {
+#pragma unroll
+            for (int q = 0; q < R; q++) {
+                const unsigned k = used[q] < 0 ? bj_key(xr[q][j], xi[q][j]) : 0u;
+                if (k > key) {
+                    key = k;
+                    best = t + BJ_T * q;
                 }
             }
-            __syncthreads();
-        }
-        const int p = red_i[0];
-        if (t == 0) pv[k] = p;
-        if (p != k)
-            for (int j = t; j < n2; j += BJ_INV_THREADS) {
-                const long a = (long)k * ld + j, c = (long)p * ld + j;
-                const double xr = ar[a], xi = ai[a];
-                ar[a] = ar[c];
-                ai[a] = ai[c];
-                ar[c] = xr;
-                ai[c] = xi;
+        } else {
+            for (int i = t; i < n2; i += BJ_T) {
+                const unsigned k = st[i] < 0 ? bj_key(ar[(long)i * ld + j], ai[(long)i * ld + j]) : 0u;
+                if (k > key) {
+                    key = k;
+                    best = i;
+                }
             }
+        }
+        const unsigned wk = __ockl_wfred_max_u32(key);
+        const int lane = __ffsll((long long)__ballot(key == wk)) - 1;
+        if ((t & 63) == lane) kb[wave] = ((unsigned long long)wk << 32) | (0xffffffffu - (unsigned)best);
         __syncthreads();
-        double dr = ar[(long)k * ld + k], di = ai[(long)k * ld + k];
+        unsigned long long kbest = kb[0];
+#pragma unroll
+        for (int q = 1; q < NW; q++) kbest = max(kbest, kb[q]);
+        const int p = (int)(0xffffffffu - (unsigned)kbest);  // some row is unused: n2 pivots over n2 steps
+        if (p % BJ_T == t) {
+            if constexpr (RPT > 0) {
+#pragma unroll
+                for (int q = 0; q < R; q++)
+                    if (p == t + BJ_T * q) {
+                        used[q] = c0 + j;
+#pragma unroll
+                        for (int c = 0; c < BJ_W; c++) {
+                            row_r[c] = xr[q][c];
+                            row_i[c] = xi[q][c];
+                        }
+                    }
+            } else {
+                for (int c = 0; c < BJ_W; c++) {
+                    row_r[c] = ar[(long)p * ld + c];
+                    row_i[c] = ai[(long)p * ld + c];
+                }
+            }
+            st[p] = c0 + j;
+            prows[j] = p;
+        }
+        __syncthreads();
+        double dr = row_r[j], di = row_i[j];
         if (hypot(dr, di) < 1e-30) {
             dr = 1e-15;
             di = 0.0;
         }
-        const double d2 = dr * dr + di * di, qr = dr / d2, qi = -di / d2;  // 1 / pivot
-        // column k (the multipliers) into the scratch
-        for (int i = t; i < n2; i += BJ_INV_THREADS) {
-            fr[i] = ar[(long)i * ld + k];
-            fi[i] = ai[(long)i * ld + k];
-        }
-        __syncthreads();
-        // row k scaled by 1 / pivot; its column-k entry becomes 1 / pivot
-        for (int j = t; j < n2; j += BJ_INV_THREADS) {
-            const long o = (long)k * ld + j;
-            if (j == k) {
-                ar[o] = qr;
-                ai[o] = qi;
-            } else {
-                const double xr = ar[o], xi = ai[o];
-                ar[o] = xr * qr - xi * qi;
-                ai[o] = xr * qi + xi * qr;
+        const double inv = 1.0 / (dr * dr + di * di), qr = dr * inv, qi = -di * inv;  // 1 / pivot
+        // row i: a_ic -= g u_c (c != j), a_ij = -g, g = a_ij / pivot; the pivot
+        // row: a_pc = u_c / pivot, a_pj = 1 / pivot
+        auto eliminate = [&](int i, double (&yr)[BJ_W], double (&yi)[BJ_W]) {
+            const bool piv = i == p;
+            const double fr = yr[j], fi = yi[j];
+            const double gr = piv ? -qr : fr * qr - fi * qi, gi = piv ? -qi : fr * qi + fi * qr;
+#pragma unroll
+            for (int c = 0; c < BJ_W; c++) {
+                if (c == j) continue;
+                const double ur = row_r[c], ui = row_i[c];
+                const double br = piv ? 0.0 : yr[c], bi = piv ? 0.0 : yi[c];
+                yr[c] = br - (gr * ur - gi * ui);
+                yi[c] = bi - (gr * ui + gi * ur);
             }
-        }
-        __syncthreads();
-        // every other row: a_ij -= f_i a_kj (j != k), a_ik = -f_i / pivot
-        for (int j = t; j < n2; j += BJ_INV_THREADS) {
-            const double ur = ar[(long)k * ld + j], ui = ai[(long)k * ld + j];
-#pragma unroll 4
-            for (int i = 0; i < n2; i++) {
-                if (i == k) continue;
-                const long o = (long)i * ld + j;
-                const double gr = fr[i], gi = fi[i];
-                if (j == k) {
-                    ar[o] = -(gr * ur - gi * ui);
-                    ai[o] = -(gr * ui + gi * ur);
-                } else {
-                    ar[o] -= gr * ur - gi * ui;
-                    ai[o] -= gr * ui + gi * ur;
+            yr[j] = -gr;
+            yi[j] = -gi;
+        };
+        if constexpr (RPT > 0) {
+#pragma unroll
+            for (int q = 0; q < R; q++) eliminate(t + BJ_T * q, xr[q], xi[q]);
+        } else {
+            for (int i = t; i < n2; i += BJ_T) {
+#pragma unroll
+                for (int c = 0; c < BJ_W; c++) {
+                    xr[0][c] = ar[(long)i * ld + c];
+                    xi[0][c] = ai[(long)i * ld + c];
+                }
+                eliminate(i, xr[0], xi[0]);
+#pragma unroll
+                for (int c = 0; c < BJ_W; c++) {
+                    ar[(long)i * ld + c] = xr[0][c];
+                    ai[(long)i * ld + c] = xi[0][c];
                 }
             }
         }
-        __syncthreads();
+        __syncthreads();  // the row and the keys are read before the next step writes them
+        }
     }
-    // row interchanges of the elimination = column interchanges of the inverse, in reverse
-    for (int k = n2 - 1; k >= 0; k--) {
-        const int p = pv[k];
-        if (p != k)
-            for (int i = t; i < n2; i += BJ_INV_THREADS) {
-                const long a = (long)i * ld + k, c = (long)i * ld + p;
-                const double xr = ar[a], xi = ai[a];
-                ar[a] = ar[c];
-                ai[a] = ai[c];
-                ar[c] = xr;
-                ai[c] = xi;
+    if constexpr (RPT > 0) {
+#pragma unroll
+        for (int q = 0; q < R; q++) {
+            const int i = t + BJ_T * q;
+            if (i >= n2) continue;
+#pragma unroll
+            for (int c = 0; c < BJ_W; c++) {
+                ar[(long)i * ld + c] = xr[q][c];
+                ai[(long)i * ld + c] = xi[q][c];
             }
-        __syncthreads();
+        }
+    }
+    if (t < w) prow[v.poff[b] + c0 + t] = prows[t];
+    if (!Bin) return;
+    double* br = Bin + (long)b * 2 * BJ_W * BJ_O;
+    double* bi = br + BJ_W * BJ_O;
+    const int off = k0 - c0;  // the outer panel's first column relative to c0
+    for (int e = t; e < BJ_W * BJ_O; e += BJ_T) {
+        const int k = e / BJ_O, c = e % BJ_O;
+        const bool in = k < w && !(c + off >= 0 && c + off < BJ_W);  // the panel's own columns are not used
+        br[e] = in ? ar[(long)prows[k] * ld + off + c] : 0.0;
+        bi[e] = in ? ai[(long)prows[k] * ld + off + c] : 0.0;
     }
 }
 
-// Slot b of S (ld x ncol per plane) = the extended block of r (rows beyond
-// 2 Be stay zero); one workgroup per block.
+// The other columns of the outer panel [k0, k0 + 64) after the inner panel at
+// c0: 32 rows per workgroup (blockIdx.y), one column and 8 rows per thread, G
+// and the pivot rows from LDS.
+__global__ __launch_bounds__(256) void k_bj_inner(BjView v, int ld, int c0, int k0, double* __restrict__ Ar,
+                                                  double* __restrict__ Ai, const int* __restrict__ step,
+                                                  const double* __restrict__ Bin) {
+    __shared__ double gr[32][BJ_W + 1], gi[32][BJ_W + 1], ur[BJ_W][BJ_O], ui[BJ_W][BJ_O];
+    const int b = blockIdx.x, t = threadIdx.x, i0 = blockIdx.y * 32;
+    const int n2 = 2 * v.Be[b];
+    if (c0 >= n2 || i0 >= n2) return;
+    double* ar = Ar + (long)b * ld * ld;
+    double* ai = Ai + (long)b * ld * ld;
+    const double* br = Bin + (long)b * 2 * BJ_W * BJ_O;
+    for (int e = t; e < BJ_W * BJ_O; e += 256) {
+        ur[e / BJ_O][e % BJ_O] = br[e];
+        ui[e / BJ_O][e % BJ_O] = br[BJ_W * BJ_O + e];
+    }
+    for (int e = t; e < 32 * BJ_W; e += 256) {
+        const int i = e / BJ_W, k = e % BJ_W;
+        const bool in = i0 + i < n2;
+        gr[i][k] = in ? ar[(long)(i0 + i) * ld + c0 + k] : 0.0;
+        gi[i][k] = in ? ai[(long)(i0 + i) * ld + c0 + k] : 0.0;
+    }
+    __syncthreads();
+    const int c = k0 + t % BJ_O;
+    if (c >= c0 && c < c0 + BJ_W) return;
+    if (c >= n2) return;
+    for (int r = t / BJ_O; r < 32; r += 256 / BJ_O) {
+        const int i = i0 + r;
+        if (i >= n2) break;
+        const int s = step[(long)b * ld + i];
+        const long o = (long)i * ld + c;
+        double sr = 0.0, si = 0.0;
+        if (!(s >= c0 && s < c0 + BJ_W)) {
+            sr = ar[o];
+            si = ai[o];
+        }
+#pragma unroll
+        for (int k = 0; k < BJ_W; k++) {
+            const double pr = ur[k][t % BJ_O], pi = ui[k][t % BJ_O];
+            sr += gr[r][k] * pr - gi[r][k] * pi;
+            si += gr[r][k] * pi + gi[r][k] * pr;
+        }
+        ar[o] = sr;
+        ai[o] = si;
+    }
+}
+
+// The outer panel's pivot rows before its rank-64 product: Bo (64 x ld per
+// plane and block), rows beyond n2 zero.
+__global__ __launch_bounds__(256) void k_bj_rows(BjView v, int ld, int k0, const double* __restrict__ Ar,
+                                                 const double* __restrict__ Ai, const int* __restrict__ prow,
+                                                 double* __restrict__ Bo) {
+    const int b = blockIdx.x, k = blockIdx.y;
+    const int n2 = 2 * v.Be[b];
+    if (k0 >= n2) return;
+    const bool in = k0 + k < n2;
+    const long src = (long)b * ld * ld + (in ? (long)prow[v.poff[b] + k0 + k] * ld : 0);
+    double* br = Bo + (long)b * 2 * BJ_O * ld + (long)k * ld;
+    double* bi = br + (long)BJ_O * ld;
+    for (int c = threadIdx.x; c < ld; c += 256) {
+        br[c] = in ? Ar[src + c] : 0.0;
+        bi[c] = in ? Ai[src + c] : 0.0;
+    }
+}
+
+// The columns outside the outer panel [k0, k0 + 64): 64 x 64 tiles
+// (workgroup = block + nb (tile column + nt tile row)), each of the four waves a 32 x 32 sub-tile.  The operands go straight from memory to
+// the registers of v_mfma_f64_16x16x4f64 (K is only 64 and the tiles' rows are
+// shared through the caches): lane (r, g) holds G[row r][4g + s] and
+// Bo[4g + s][col r] for product s = 0..3 of a 16-wide piece of K.  Tiles
+// beyond a block's own size end at once.
+__global__ __launch_bounds__(256) void k_bj_update(BjView v, int nb, int ld, int k0, int nt,
+                                                   double* __restrict__ Ar, double* __restrict__ Ai,
+                                                   const int* __restrict__ step, const double* __restrict__ Bo) {
+    const int b = blockIdx.x % nb, tile = blockIdx.x / nb, tm = tile / nt, tn = tile % nt;
+    const int n2 = 2 * v.Be[b];
+    if (k0 >= n2 || tm * 64 >= n2 || tn * 64 >= n2 || tn * 64 == k0) return;
+    double* ar = Ar + (long)b * ld * ld;
+    double* ai = Ai + (long)b * ld * ld;
+    const double* br = Bo + (long)b * 2 * BJ_O * ld;
+    const double* bi = br + (long)BJ_O * ld;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+    const int m0 = tm * 64 + (wave >> 1) * 32, n0 = tn * 64 + (wave & 1) * 32;
+    v4d acc[2][2][2];
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) acc[p][i][j] = v4d{};
+#pragma unroll
+    for (int kk = 0; kk < BJ_O; kk += 16) {
+        double a[2][2][4], u[2][2][4];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const long oa = (long)(m0 + 16 * i + r) * ld + k0 + kk + 4 * g;
+            load_row4<double>(ar + oa, a[0][i]);
+            load_row4<double>(ai + oa, a[1][i]);
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const long ob = (long)(kk + 4 * g + s) * ld + n0 + 16 * i + r;
+                u[0][i][s] = br[ob];
+                u[1][i][s] = bi[ob];
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    acc[0][i][j] = mfma16x16x4(a[0][i][s], u[0][j][s], acc[0][i][j]);
+                    acc[0][i][j] = mfma16x16x4(a[1][i][s], -u[1][j][s], acc[0][i][j]);
+                    acc[1][i][j] = mfma16x16x4(a[0][i][s], u[1][j][s], acc[1][i][j]);
+                    acc[1][i][j] = mfma16x16x4(a[1][i][s], u[0][j][s], acc[1][i][j]);
+                }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int row = m0 + 16 * i + g + 4 * q;
+            if (row >= n2) continue;
+            const int s = step[(long)b * ld + row];
+            const bool clear = s >= k0 && s < k0 + BJ_O;
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const long o = (long)row * ld + n0 + 16 * j + r;
+                ar[o] = (clear ? 0.0 : ar[o]) + acc[0][i][j][q];
+                ai[o] = (clear ? 0.0 : ai[o]) + acc[1][i][j][q];
+            }
+        }
+}
+
+// Slot b of S (ld x ncol per plane) = the extended block of r in pivot order
+// (row k: r at row prow[k] of the block; rows beyond 2 Be stay zero); rows
+// blockIdx.y, blockIdx.y + gridDim.y, ... of a block per workgroup.
 __global__ __launch_bounds__(256) void k_bj_gather_vec(BjView v, int N, int ld, int ncol,
-                                                       const double* __restrict__ Rr, const double* __restrict__ Ri,
-                                                       double* __restrict__ Sr, double* __restrict__ Si) {
+                                                       const int* __restrict__ prow, const double* __restrict__ Rr,
+                                                       const double* __restrict__ Ri, double* __restrict__ Sr,
+                                                       double* __restrict__ Si) {
     const int b = blockIdx.x;
     const int Be = v.Be[b], n2 = 2 * Be;
     const int* rwg = v.rwg + v.roff[b];
+    const int* pr = prow + v.poff[b];
     double* sr = Sr + (long)b * ld * ncol;
     double* si = Si + (long)b * ld * ncol;
-    for (long e = threadIdx.x; e < (long)n2 * ncol; e += blockDim.x) {
+    for (long e = (long)blockIdx.y * 256 + threadIdx.x; e < (long)ld * ncol; e += 256L * gridDim.y) {
         const int p = (int)(e / ncol), j = (int)(e % ncol);
-        const long g = (long)bj_row(rwg, Be, N, p) * ncol + j;
-        sr[e] = Rr[g];
-        si[e] = Ri[g];
+        const long g = p < n2 ? (long)bj_row(rwg, Be, N, pr[p]) * ncol + j : 0;
+        sr[e] = p < n2 ? Rr[g] : 0.0;
+        si[e] = p < n2 ? Ri[g] : 0.0;
     }
 }
 
-// z at the block's own unknowns = rows {0..B-1, Be..Be+B-1} of slot b of Y.
-__global__ __launch_bounds__(256) void k_bj_scatter(BjView v, int N, int ld, int ncol, const double* __restrict__ Yr,
+// Y_b = M_b S_b for every block (rows in the storage order of M): one 16 x
+// (16 NT) tile per workgroup (blockIdx.x = block + nb row tile, columns
+// blockIdx.y), the four waves each a quarter of K in 16-wide pieces straight
+// from memory, summed through LDS in wave order.  Bound by reading M once per
+// 16 NT columns; a tile beyond the block's own size ends at once and K stops
+// there (16 columns, the blocks above: 90 us; the batched 64 x 64 tile product
+// over the padded slots took 527 us).
+template <int NT>
+__global__ __launch_bounds__(256) void k_bj_mult(BjView v, int nb, int ld, int ncol,
+                                                 const double* __restrict__ Ar, const double* __restrict__ Ai,
+                                                  const double* __restrict__ Sr,
+                                                 const double* __restrict__ Si, double* __restrict__ Yr,
+                                                 double* __restrict__ Yi) {
+    __shared__ double red[4][2][16][17];
+    const int b = blockIdx.x % nb, m0 = blockIdx.x / nb * 16, n0 = blockIdx.y * 16 * NT;
+    const int n2 = 2 * v.Be[b];
+    if (m0 >= n2) return;
+    const double* ar = Ar + (long)b * ld * ld;
+    const double* ai = Ai + (long)b * ld * ld;
+    const double* sr = Sr + (long)b * ld * ncol;
+    const double* si = Si + (long)b * ld * ncol;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+    v4d acc[2][NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++) acc[0][j] = acc[1][j] = v4d{};
+    for (int kk = wave * 16; kk < n2; kk += 64) {  // rows and columns up to ld (a multiple of 64) are zero beyond n2
+        double a[2][4], u[NT][2][4];
+        const long oa = (long)(m0 + r) * ld + kk + 4 * g;
+        load_row4<double>(ar + oa, a[0]);
+        load_row4<double>(ai + oa, a[1]);
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const long ob = (long)(kk + 4 * g + s) * ncol + n0 + 16 * j + r;
+                u[j][0][s] = sr[ob];
+                u[j][1][s] = si[ob];
+            }
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                acc[0][j] = mfma16x16x4(a[0][s], u[j][0][s], acc[0][j]);
+                acc[0][j] = mfma16x16x4(a[1][s], -u[j][1][s], acc[0][j]);
+                acc[1][j] = mfma16x16x4(a[0][s], u[j][1][s], acc[1][j]);
+                acc[1][j] = mfma16x16x4(a[1][s], u[j][0][s], acc[1][j]);
+            }
+    }
+    const int row = threadIdx.x / 16, col = threadIdx.x % 16;
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        if (j) __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            red[wave][0][g + 4 * q][r] = acc[0][j][q];
+            red[wave][1][g + 4 * q][r] = acc[1][j][q];
+        }
+        __syncthreads();
+        const long o = (long)b * ld * ncol + (long)(m0 + row) * ncol + n0 + 16 * j + col;
+        Yr[o] = ((red[0][0][row][col] + red[1][0][row][col]) + red[2][0][row][col]) + red[3][0][row][col];
+        Yi[o] = ((red[0][1][row][col] + red[1][1][row][col]) + red[2][1][row][col]) + red[3][1][row][col];
+    }
+}
+
+// z at the block's own unknowns k in {0..B-1, Be..Be+B-1} = row prow[k] of slot b of Y.
+__global__ __launch_bounds__(256) void k_bj_scatter(BjView v, int N, int ld, int ncol,
+                                                    const int* __restrict__ prow, const double* __restrict__ Yr,
                                                     const double* __restrict__ Yi, double* __restrict__ Zr,
                                                     double* __restrict__ Zi) {
     const int b = blockIdx.x;
@@ -205,12 +484,13 @@ __global__ __launch_bounds__(256) void k_bj_scatter(BjView v, int N, int ld, int
     const int* rwg = v.rwg + v.roff[b];
     const double* yr = Yr + (long)b * ld * ncol;
     const double* yi = Yi + (long)b * ld * ncol;
-    for (long e = threadIdx.x; e < 2L * B * ncol; e += blockDim.x) {
+    const int* pr = prow + v.poff[b];
+    for (long e = (long)blockIdx.y * 256 + threadIdx.x; e < 2L * B * ncol; e += 256L * gridDim.y) {
         const int q = (int)(e / ncol), j = (int)(e % ncol);
         const int p = q < B ? q : Be + (q - B);
         const long g = (long)bj_row(rwg, Be, N, p) * ncol + j;
-        Zr[g] = yr[(long)p * ncol + j];
-        Zi[g] = yi[(long)p * ncol + j];
+        Zr[g] = yr[(long)pr[p] * ncol + j];
+        Zi[g] = yi[(long)pr[p] * ncol + j];
     }
 }
 
@@ -285,13 +565,19 @@ int bj_build_launch(bem_ctx* c, double radius_mult, int max_block_rwg, int overl
         bj_free(c);
         return bem_fail(c, BEM_ERR_NOMEM, "block_jacobi: inverses (" + std::to_string(nb * slot * 16) + " bytes)");
     }
-    void* scr = nullptr;  // the Gauss-Jordan column scratch
-    if (int e = ctx_scratch(c, 2 * (size_t)nb * ld * sizeof(double), &scr)) {
+    // scratch of the elimination: pivot rows of an inner and of an outer panel,
+    // and per row the column it is the pivot of
+    // (none where one panel holds every block)
+    const size_t nbin = n2max > BJ_W ? 2 * (size_t)nb * BJ_W * BJ_O : 0;
+    const size_t nbo = n2max > BJ_O ? 2 * (size_t)nb * BJ_O * ld : 0;
+    void* scr = nullptr;
+    if (int e = ctx_scratch(c, (nbin + nbo) * sizeof(double) + (size_t)nb * ld * sizeof(int), &scr)) {
         bj_free(c);
         return e;
     }
-    double* Fr = static_cast<double*>(scr);
-    double* Fi = Fr + (size_t)nb * ld;
+    double* Bin = static_cast<double*>(scr);
+    double* Bo = Bin + nbin;
+    int* step = reinterpret_cast<int*>(Bo + nbo);
     J.nb = nb;
     J.n2max = n2max;
     J.ld = ld;
@@ -305,7 +591,26 @@ int bj_build_launch(bem_ctx* c, double radius_mult, int max_block_rwg, int overl
     BEM_HIP(c, hipMemsetAsync(J.Ai, 0, nb * slot * sizeof(double), s));
     hipLaunchKernelGGL(k_bj_gather, dim3(nb, 64), dim3(256), 0, s, v, N, ld, c->Zr, c->Zi, (long)c->npad, J.Ar,
                        J.Ai);
-    hipLaunchKernelGGL(k_bj_inv, dim3(nb), dim3(BJ_INV_THREADS), 0, s, v, ld, J.Ar, J.Ai, Fr, Fi, J.piv);
+    BEM_HIP(c, hipMemsetAsync(step, 0xff, (size_t)nb * ld * sizeof(int), s));
+    // rows per thread of the panel kernel: in registers up to BJ_MAXR BJ_T
+    // rows, from memory beyond
+    const int rpt = (n2max + BJ_T - 1) / BJ_T, nt = ld / 64;
+    for (int k0 = 0; k0 < n2max; k0 += BJ_O) {
+        for (int c0 = k0; c0 < std::min(n2max, k0 + BJ_O); c0 += BJ_W) {
+            auto panel = rpt == 1 ? k_bj_panel<1> : rpt == 2 ? k_bj_panel<2> : rpt <= BJ_MAXR ? k_bj_panel<3>
+                                                                                                 : k_bj_panel<0>;
+            hipLaunchKernelGGL(panel, dim3(nb), dim3(BJ_T), 0, s, v, ld, c0, k0, J.Ar, J.Ai, step, J.piv,
+                               nbin ? Bin : nullptr);
+            if (nbin)
+                hipLaunchKernelGGL(k_bj_inner, dim3(nb, (n2max + 31) / 32), dim3(256), 0, s, v, ld, c0, k0, J.Ar,
+                                   J.Ai, (const int*)step, (const double*)Bin);
+        }
+        if (n2max <= BJ_O) break;
+        hipLaunchKernelGGL(k_bj_rows, dim3(nb, BJ_O), dim3(256), 0, s, v, ld, k0, (const double*)J.Ar,
+                           (const double*)J.Ai, (const int*)J.piv, Bo);
+        hipLaunchKernelGGL(k_bj_update, dim3(nb * nt * nt), dim3(256), 0, s, v, nb, ld, k0, nt, J.Ar, J.Ai,
+                           (const int*)step, (const double*)Bo);
+    }
     BEM_HIP(c, hipGetLastError());
     BEM_HIP(c, hipStreamSynchronize(s));
     J.valid = true;
@@ -328,12 +633,22 @@ int bj_apply(bem_ctx* c, const double* Rr, const double* Ri, double* Zr, double*
     double* Yi = Yr + vs;
     hipStream_t s = c->stream;
     const BjView v{J.B, J.Be, J.rwg, J.roff, J.poff};
-    BEM_HIP(c, hipMemsetAsync(Sr, 0, 2 * vs * sizeof(double), s));  // padding rows stay zero
-    hipLaunchKernelGGL(k_bj_gather_vec, dim3(nb), dim3(256), 0, s, v, J.N, ld, ncol, Rr, Ri, Sr, Si);
-    // Y_b = inv_b S_b for every block: one batched FP64 complex GEMM (64 x 64 tile)
-    cgemm_any<double>(1, s, ld, ncol, ld, J.Ar, J.Ai, ld, Sr, Si, ncol, Yr, Yi, ncol, 1, nb, (long)ld * ld,
-                      (long)ld * ncol, (long)ld * ncol);
-    hipLaunchKernelGGL(k_bj_scatter, dim3(nb), dim3(256), 0, s, v, J.N, ld, ncol, Yr, Yi, Zr, Zi);
+    const unsigned gy = (unsigned)std::min<long>(64, ((long)ld * ncol + 1023) / 1024);
+    hipLaunchKernelGGL(k_bj_gather_vec, dim3(nb, gy), dim3(256), 0, s, v, J.N, ld, ncol, (const int*)J.piv, Rr, Ri,
+                       Sr, Si);
+    const int tiles = ncol / 16;  // ldr is a multiple of 16
+    const unsigned mt = (unsigned)((J.n2max + 15) / 16);
+    if (tiles % 4 == 0)
+        hipLaunchKernelGGL(k_bj_mult<4>, dim3(nb * mt, tiles / 4), dim3(256), 0, s, v, nb, ld, ncol, (const double*)J.Ar,
+                           (const double*)J.Ai, (const double*)Sr, (const double*)Si, Yr, Yi);
+    else if (tiles % 2 == 0)
+        hipLaunchKernelGGL(k_bj_mult<2>, dim3(nb * mt, tiles / 2), dim3(256), 0, s, v, nb, ld, ncol, (const double*)J.Ar,
+                           (const double*)J.Ai, (const double*)Sr, (const double*)Si, Yr, Yi);
+    else
+        hipLaunchKernelGGL(k_bj_mult<1>, dim3(nb * mt, tiles), dim3(256), 0, s, v, nb, ld, ncol, (const double*)J.Ar,
+                           (const double*)J.Ai, (const double*)Sr, (const double*)Si, Yr, Yi);
+    hipLaunchKernelGGL(k_bj_scatter, dim3(nb, gy), dim3(256), 0, s, v, J.N, ld, ncol, (const int*)J.piv, Yr, Yi, Zr,
+                       Zi);
     const long from = (long)c->n * ncol, count = (long)c->npad * ncol;
     if (count > from)
         hipLaunchKernelGGL(k_copy_tail, dim3((unsigned)((count - from + 255) / 256)), dim3(256), 0, s, from, count,
