@@ -950,8 +950,9 @@ int bem_farfield(bem_ctx* c, const double* cJ, const double* cM, const double* r
     // coefficient planes (n_calls x N each for J and M), directions, output
     const size_t nc = (size_t)n_calls * N;
     const size_t bytes = (4 * nc + (size_t)n_orient * ndir * 3 + (size_t)n_calls * ndir * 6) * sizeof(double);
+    const size_t at = (bytes + 255) / 256 * 256;  // the far-field work area follows
     void* s = nullptr;
-    if (int rc = ctx_scratch(c, bytes, &s)) return rc;
+    if (int rc = ctx_scratch(c, at + ff_work_bytes(c, n_calls, n_orient, ndir), &s)) return rc;
     double* d = static_cast<double*>(s);
     std::vector<double> h(4 * nc);
     for (size_t i = 0; i < nc; i++) {
@@ -965,7 +966,8 @@ int bem_farfield(bem_ctx* c, const double* cJ, const double* cM, const double* r
     BEM_HIP(c, hipMemcpy(drh, rh, (size_t)n_orient * ndir * 3 * sizeof(double), hipMemcpyHostToDevice));
     double* dfv = drh + (size_t)n_orient * ndir * 3;
     EventTimer tm(c);
-    if (int rc = ff_launch(c, d, d + nc, d + 2 * nc, d + 3 * nc, N, drh, kr, ki, eta, n_calls, n_orient, ndir, dfv))
+    if (int rc = ff_launch(c, d, d + nc, d + 2 * nc, d + 3 * nc, N, drh, rh, kr, ki, eta, n_calls, n_orient, ndir, dfv,
+                           static_cast<char*>(s) + at))
         return rc;
     c->t_ms[4] = tm.stop();
     BEM_HIP(c, hipMemcpy(Fv, dfv, (size_t)n_calls * ndir * 6 * sizeof(double), hipMemcpyDeviceToHost));

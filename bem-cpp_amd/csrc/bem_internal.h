@@ -236,9 +236,13 @@ int gmres_solve_launch(bem_ctx* c, int nrhs, double tol, int restart, int max_it
 int lu_solve_launch(bem_ctx* c, int nrhs, double ir_tol, int ir_max, int* iters, double* res0, double* res,
                     double* t_solve_ms, double* t_ir_ms);
 int rhs_launch(bem_ctx* c, double kr, double ki, double eta, const double* khat, const double* E0, int nrhs);
+// Far field of n_calls device coefficient sets into dFv; work holds
+// ff_work_bytes (16-byte aligned); drh and rh: the directions on the device and
+// on the host.
+size_t ff_work_bytes(const bem_ctx* c, int n_calls, int n_orient, int ndir);
 int ff_launch(bem_ctx* c, const double* dJr, const double* dJi, const double* dMr, const double* dMi, int ldc,
-              const double* drh, double kr, double ki, double eta, int n_calls, int n_orient, int ndir,
-              double* dFv);
+              const double* drh, const double* rh, double kr, double ki, double eta, int n_calls, int n_orient,
+              int ndir, double* dFv, void* work);
 // bem_farfield without device allocation: all staging in the library's static
 // per-GPU array of kNoAllocBytes (farfield.hip); ff_noalloc_init fetches its
 // device address into c->noalloc_ptr (once per context, device current).

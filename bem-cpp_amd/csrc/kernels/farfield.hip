@@ -12,17 +12,19 @@
 // solution is first folded into a current density per triangle point
 // (k_current: J_x = jw_x sum_a c_a (x - p_a) coef[n(a)], likewise M_x; 3x fewer
 // points), and the phase e^{-ik r.x} of a point is shared by both polarisations
-// of an orientation.  k_ff_partial stages a chunk of points in LDS and lets
-// every thread of the block (one direction each) sweep it: the point data is
-// read once per orientation, not once per direction.  Partial sums over point
-// chunks are combined in a fixed order by k_ff_final (deterministic).
+// of an orientation.  In k_ff_partial a lane is a direction and a wave sweeps a
+// chunk of points; partial sums over the chunks are combined in a fixed order
+// by k_ff_final (deterministic).
+#include <algorithm>
+#include <cmath>
+
 #include "../bem_internal.h"
 
 namespace {
 
 constexpr double kPi = 3.14159265358979323846;
-constexpr int kChunk = 1024;  // points per k_ff_partial block
-constexpr int kTile = 64;     // points per LDS tile
+constexpr int kMaxChunk = 1024;  // points per partial sum
+constexpr int kMinChunk = 64;
 
 // ---------------------------------------------------------------------------
 // RHS: B[n][j] = sum_halves sum_q f.E0_j e^{ik k_j.r} jw, B[N+n][j] likewise with
@@ -122,62 +124,109 @@ __global__ __launch_bounds__(256) void k_current(int T, int Nq, int n_calls, con
     for (int e = 0; e < 12; e++) out[e] = v[e];
 }
 
+// sin and cos in FP64 for |x| < kBigPhase: reduction to [-pi/4, pi/4] by
+// quarter turns (pi/2 in two parts; the fma products are exact, so the reduced
+// argument is good to its last place as long as the quotient is exact), Taylor
+// series to x^17 and x^16 (truncation < 1e-18 and < 3e-18).
+constexpr double kBigPhase = 3.5e13;
+__device__ __forceinline__ void sincos64(double x, double& sn, double& cs) {
+    const double q = rint(x * 0.63661977236758134308);
+    double r = fma(q, -1.57079632679489655800, x);
+    r = fma(q, -6.12323399573676603587e-17, r);
+    const double z = r * r;
+    double s = fma(z, 1.0 / 355687428096000.0, -1.0 / 1307674368000.0);
+    s = fma(z, s, 1.0 / 6227020800.0);
+    s = fma(z, s, -1.0 / 39916800.0);
+    s = fma(z, s, 1.0 / 362880.0);
+    s = fma(z, s, -1.0 / 5040.0);
+    s = fma(z, s, 1.0 / 120.0);
+    s = fma(z, s, -1.0 / 6.0);
+    s = fma(z * r, s, r);
+    double c = fma(z, 1.0 / 20922789888000.0, -1.0 / 87178291200.0);
+    c = fma(z, c, 1.0 / 479001600.0);
+    c = fma(z, c, -1.0 / 3628800.0);
+    c = fma(z, c, 1.0 / 40320.0);
+    c = fma(z, c, -1.0 / 720.0);
+    c = fma(z, c, 1.0 / 24.0);
+    c = fma(z, c, -0.5);
+    c = fma(z, c, 1.0);
+    const int iq = (int)fma(-4.0, rint(0.25 * q), q);  // q mod 4, in -2 .. 2
+    const double sv = (iq & 1) ? c : s, cv = (iq & 1) ? s : c;
+    sn = (iq & 2) ? -sv : sv;
+    cs = ((iq + 1) & 2) ? -cv : cv;
+}
+
 // ---------------------------------------------------------------------------
-// Partial far-field sums.  Block (o, chunk): thread d accumulates, over the
-// chunk's points, e^{-ik rhat_{o,d}.x} times the currents of calls 2o, 2o+1.
-// part[((o * nchunk + chunk) * ndir + d) * 24 + ...].
+// Partial far-field sums: part[((o nchunk + chunk) ndir + d) 24 + 12 call + 2 k
+// + {re, im}] = sum over the chunk's points x of e^{-ik rhat_{o,d}.x} times
+// component k of the currents of call 2o + call.
+// One wave per (o, chunk, group of 64 directions), one direction per lane.  A
+// point's coordinates and currents are the same for the whole wave, so they
+// come through the scalar cache into scalar registers, which the FMAs read
+// directly: no LDS and no barrier.  Bound by FP64 VALU issue: 48 FMAs and ~45
+// instructions of phase per direction and point.  Staging the points in LDS
+// instead (224 bytes read per point and wave) with the library's sincos and one
+// workgroup per 1024 points took 2.75 ms for 64 orientations x 181 directions
+// x 43008 points and 510 us for 1 x 181 x 8960; the products on
+// v_mfma_f64_16x16x4f64, which has no higher rate than the VALU, 2.28 ms; this
+// form 1.90 ms and 43 us.
+// BIG: phases of kBigPhase and more take the library's sincos (whose general
+// reduction would cost every call 60 registers).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_ff_partial(long P, int n_calls, int ndir, const double4* __restrict__ qp,
-                                                    const double* __restrict__ cur, const double* __restrict__ rh,
-                                                    double kr, double ki, double* __restrict__ part) {
-    __shared__ double4 sx[kTile];
-    __shared__ double sc[kTile][24];
-    const int o = blockIdx.x, chunk = blockIdx.y, nchunk = gridDim.y;
-    const long x0 = (long)chunk * kChunk, x1 = min(P, x0 + kChunk);
-    const int c0 = 2 * o, ncall = min(2, n_calls - c0);
-    for (int d0 = 0; d0 < ndir; d0 += 256) {
-        const int d = d0 + threadIdx.x;
-        double rx = 0, ry = 0, rz = 0;
-        if (d < ndir) {
-            const double* r = rh + ((long)o * ndir + d) * 3;
-            rx = r[0]; ry = r[1]; rz = r[2];
-        }
-        double acc[24];
-        for (int e = 0; e < 24; e++) acc[e] = 0.0;
-        for (long xt = x0; xt < x1; xt += kTile) {
-            const int nt = (int)min((long)kTile, x1 - xt);
-            __syncthreads();
-            for (int e = threadIdx.x; e < nt * 24; e += 256) {
-                const int p = e / 24, k = e % 24;
-                const int call = k / 12;
-                sc[p][k] = call < ncall ? cur[((long)(c0 + call) * P + xt + p) * 12 + (k % 12)] : 0.0;
-            }
-            for (int p = threadIdx.x; p < nt; p += 256) sx[p] = qp[xt + p];
-            __syncthreads();
-            if (d < ndir) {
-                for (int p = 0; p < nt; p++) {
-                    const double rd = rx * sx[p].x + ry * sx[p].y + rz * sx[p].z;
-                    double sn, cs;
-                    sincos(kr * rd, &sn, &cs);
-                    double pr = cs, pi = -sn;  // e^{-ik rd}
-                    if (ki != 0.0) {
-                        const double ea = exp(ki * rd);
-                        pr *= ea;
-                        pi *= ea;
-                    }
+template <bool LOSSY, bool BIG>
+__global__ __launch_bounds__(256, (LOSSY ? 4 : 5)) void k_ff_partial(long P, int n_orient, int n_calls, int ndir, int nchunk, int chunk,
+                                                    const double4* __restrict__ qp, const double* __restrict__ cur,
+                                                    const double* __restrict__ rh, double kr, double ki,
+                                                    double* __restrict__ part) {
+    const int ngrp = (ndir + 63) / 64;
+    const int unit = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+    const int grp = unit % ngrp;
+    const long oc = unit / ngrp;  // o nchunk + chunk
+    const int o = (int)(oc / nchunk);
+    if (o >= n_orient) return;
+    const long x0 = (oc % nchunk) * (long)chunk;
+    const int nx = (int)min((long)chunk, P - x0);
+    const int d = grp * 64 + (threadIdx.x & 63);
+    const double* r = rh + ((long)o * ndir + min(d, ndir - 1)) * 3;
+    const double rx = r[0], ry = r[1], rz = r[2];
+    // the currents of both calls; with one call its values stand in for the other's, whose sums nobody reads
+    const double* __restrict__ c0 = cur + ((long)(2 * o) * P + x0) * 12;
+    const double* __restrict__ c1 = 2 * o + 1 < n_calls ? c0 + P * 12 : c0;
+    const double4* __restrict__ qx = qp + x0;
+    double acc[24];
 #pragma unroll
-                    for (int k = 0; k < 12; k++) {
-                        const double ar = sc[p][2 * k], ai = sc[p][2 * k + 1];
-                        acc[2 * k] = fma(pr, ar, fma(-pi, ai, acc[2 * k]));
-                        acc[2 * k + 1] = fma(pr, ai, fma(pi, ar, acc[2 * k + 1]));
-                    }
-                }
-            }
+    for (int e = 0; e < 24; e++) acc[e] = 0.0;
+    for (int p = 0; p < nx; p++) {
+        const double4 X = qx[p];
+        double a[24];
+#pragma unroll
+        for (int e = 0; e < 12; e++) {
+            a[e] = c0[p * 12 + e];
+            a[12 + e] = c1[p * 12 + e];
         }
-        if (d < ndir) {
-            double* out = part + (((long)o * nchunk + chunk) * ndir + d) * 24;
-            for (int e = 0; e < 24; e++) out[e] = acc[e];
+        const double rd = rx * X.x + ry * X.y + rz * X.z;
+        double sn, cs;
+        if (BIG)
+            sincos(kr * rd, &sn, &cs);
+        else
+            sincos64(kr * rd, sn, cs);
+        double pr = cs, pi = -sn;  // e^{-ik rd}
+        if (LOSSY) {
+            const double ea = exp(ki * rd);
+            pr *= ea;
+            pi *= ea;
         }
+#pragma unroll
+        for (int k = 0; k < 12; k++) {
+            const double ar = a[2 * k], ai = a[2 * k + 1];
+            acc[2 * k] = fma(pr, ar, fma(-pi, ai, acc[2 * k]));
+            acc[2 * k + 1] = fma(pr, ai, fma(pi, ar, acc[2 * k + 1]));
+        }
+    }
+    if (d < ndir) {
+        double* out = part + (oc * ndir + d) * 24;
+#pragma unroll
+        for (int e = 0; e < 24; e += 2) *reinterpret_cast<double2*>(out + e) = make_double2(acc[e], acc[e + 1]);
     }
 }
 
@@ -197,29 +246,35 @@ __device__ __forceinline__ void far_vector(const double* j, const double* m, con
 }
 
 // Sums the partials of (o, d) in chunk order and writes Fv[c][d][3] complex
-// for the calls of orientation o.
-__global__ __launch_bounds__(256) void k_ff_final(int n_orient, int n_calls, int ndir, int nchunk,
+// for the calls of orientation o: 24 threads, one per partial value, and then
+// one thread per call for each of the workgroup's 8 (o, d).
+__global__ __launch_bounds__(192) void k_ff_final(int n_orient, int n_calls, int ndir, int nchunk,
                                                   const double* __restrict__ part, const double* __restrict__ rh,
                                                   double kr, double ki, double eta, double* __restrict__ Fv) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= n_orient * ndir) return;
-    const int o = idx / ndir, d = idx % ndir;
-    double s[24];
-    for (int e = 0; e < 24; e++) s[e] = 0.0;
-    for (int ch = 0; ch < nchunk; ch++) {
-        const double* p = part + (((long)o * nchunk + ch) * ndir + d) * 24;
-        for (int e = 0; e < 24; e++) s[e] += p[e];
+    __shared__ double sum[8][24];
+    const int u = threadIdx.x / 24, e = threadIdx.x % 24;
+    const long od = (long)blockIdx.x * 8 + u, total = (long)n_orient * ndir;
+    if (od < total) {
+        const int o = (int)(od / ndir), d = (int)(od % ndir);
+        const double* p = part + ((long)o * nchunk * ndir + d) * 24 + e;
+        double s = 0.0;
+#pragma unroll 4
+        for (int ch = 0; ch < nchunk; ch++) s += p[(long)ch * ndir * 24];
+        sum[u][e] = s;
     }
-    const double* r0 = rh + ((long)o * ndir + d) * 3;
+    __syncthreads();
+    if (threadIdx.x >= 16) return;
+    const int w = threadIdx.x / 2, call = threadIdx.x % 2;
+    const long id = (long)blockIdx.x * 8 + w;
+    if (id >= total) return;
+    const int c = 2 * (int)(id / ndir) + call, d = (int)(id % ndir);
+    if (c >= n_calls) return;
+    const double* r0 = rh + id * 3;
     const double r[3] = {r0[0], r0[1], r0[2]};
-    for (int call = 0; call < 2; call++) {
-        const int c = 2 * o + call;
-        if (c >= n_calls) break;
-        double F[6];
-        far_vector(s + 12 * call, s + 12 * call + 6, r, kr, ki, eta, F);
-        double* out = Fv + ((long)c * ndir + d) * 6;
-        for (int e = 0; e < 6; e++) out[e] = F[e];
-    }
+    double F[6];
+    far_vector(sum[w] + 12 * call, sum[w] + 12 * call + 6, r, kr, ki, eta, F);
+    double* out = Fv + ((long)c * ndir + d) * 6;
+    for (int k = 0; k < 6; k++) out[k] = F[k];
 }
 
 // Amplitudes and Mueller matrix per (orientation, angle), main.cpp:809-842 and
@@ -301,24 +356,47 @@ __global__ __launch_bounds__(256) void k_mueller_avg(int n_orient, int ntheta, c
     M[idx] = s;
 }
 
-// Far field of n_calls coefficient sets at the given directions into dFv.
+// Points per partial sum: 4096 waves where there is work for them (four per
+// SIMD), within [kMinChunk, kMaxChunk].
+int ff_chunk(long P, int n_orient, int ndir) {
+    const long ngrp = (ndir + 63) / 64;
+    const long want = (P * n_orient * ngrp + 4095) / 4096;
+    return (int)std::min<long>(kMaxChunk, std::max<long>(kMinChunk, (want + 15) / 16 * 16));
+}
+
+// Whether a phase kr rhat.x may reach kBigPhase (rh: the directions on the host).
+bool ff_big(const bem_ctx* c, double kr, const double* rh, long nd) {
+    double x2 = 0.0, r2 = 0.0;
+    for (const Vec3& v : c->mesh.verts) x2 = std::max(x2, v.x * v.x + v.y * v.y + v.z * v.z);
+    for (long i = 0; i < nd; i++)
+        r2 = std::max(r2, rh[3 * i] * rh[3 * i] + rh[3 * i + 1] * rh[3 * i + 1] + rh[3 * i + 2] * rh[3 * i + 2]);
+    return !(std::fabs(kr) * std::sqrt(x2) * std::sqrt(r2) < 0.5 * kBigPhase);
+}
+
+// Far field of n_calls coefficient sets at the given directions (drh on the
+// device, rh the same on the host) into dFv.
 int farfield_core(bem_ctx* c, const double* Jr, const double* Ji, const double* Mr, const double* Mi, long sc, long sn,
-                  const double* drh, double kr, double ki, double eta, int n_calls, int n_orient, int ndir,
-                  double* dFv, char* work) {
+                  const double* drh, const double* rh, double kr, double ki, double eta, int n_calls, int n_orient,
+                  int ndir, int chunk, double* dFv, char* work) {
     const DevMesh& d = c->dm;
     const long P = (long)d.T * d.Nq;
-    const int nchunk = (int)((P + kChunk - 1) / kChunk);
+    const int nchunk = (int)((P + chunk - 1) / chunk);
     double* cur = reinterpret_cast<double*>(work);
     double* part = cur + P * n_calls * 12;
     hipStream_t s = c->stream;
     hipLaunchKernelGGL(k_current, dim3((unsigned)((P * n_calls + 255) / 256)), dim3(256), 0, s, d.T, d.Nq, n_calls,
                        d.qp, d.hc, d.hp, d.hrwg, Jr, Ji, Mr, Mi, sc, sn, cur);
     const int kt = kt_mark(c, KS_FARFIELD);
-    hipLaunchKernelGGL(k_ff_partial, dim3(n_orient, nchunk), dim3(256), 0, s, P, n_calls, ndir, d.qp, cur, drh, kr,
-                       ki, part);
+    const long units = (long)n_orient * nchunk * ((ndir + 63) / 64);
+    auto partial = ff_big(c, kr, rh, (long)n_orient * ndir) ? k_ff_partial<true, true>
+                   : ki != 0.0                              ? k_ff_partial<true, false>
+                                                            : k_ff_partial<false, false>;
+    hipLaunchKernelGGL(partial, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, P, n_orient, n_calls, ndir,
+                       nchunk, chunk, d.qp, cur, drh, kr, ki, part);
     kt_close(c, kt, (double)n_orient * ndir * P * (8.0 * 12.0), (double)n_orient * P * (4.0 + 24.0) * 8.0);
-    hipLaunchKernelGGL(k_ff_final, dim3((n_orient * ndir + 255) / 256), dim3(256), 0, s, n_orient, n_calls, ndir,
-                       nchunk, part, drh, kr, ki, eta, dFv);
+    const long nod = (long)n_orient * ndir;
+    hipLaunchKernelGGL(k_ff_final, dim3((unsigned)((nod + 7) / 8)), dim3(192), 0, s, n_orient, n_calls, ndir, nchunk,
+                       part, drh, kr, ki, eta, dFv);
     return 0;
 }
 
@@ -567,9 +645,9 @@ __global__ __launch_bounds__(256) void k_current_adj(int N, int Nq, int n_calls,
     gi[(long)(N + n) * ldr + c] = M[1];
 }
 
-size_t farfield_scratch_bytes(const DevMesh& d, int n_calls, int n_orient, int ndir) {
+size_t farfield_scratch_bytes(const DevMesh& d, int n_calls, int n_orient, int ndir, int chunk) {
     const long P = (long)d.T * d.Nq;
-    const int nchunk = (int)((P + kChunk - 1) / kChunk);
+    const int nchunk = (int)((P + chunk - 1) / chunk);
     return (size_t)(P * n_calls * 12 + (long)n_orient * nchunk * ndir * 24) * sizeof(double);
 }
 
@@ -654,7 +732,13 @@ int ff_noalloc_launch(bem_ctx* c, const double* cJ, const double* cM, const doub
     const size_t bc = up((size_t)n_calls * N * 2 * sizeof(double));       // one interleaved coefficient set
     const size_t br = up((size_t)n_orient * ndir * 3 * sizeof(double));    // directions
     const size_t bf = up((size_t)n_calls * ndir * 6 * sizeof(double));     // result
-    const size_t bw = up(farfield_scratch_bytes(c->dm, n_calls, n_orient, ndir));  // currents, partial sums
+    // currents, partial sums: the largest chunk where the preferred one does not fit
+    int chunk = ff_chunk((long)c->dm.T * c->dm.Nq, n_orient, ndir);
+    size_t bw = up(farfield_scratch_bytes(c->dm, n_calls, n_orient, ndir, chunk));
+    if (2 * bc + br + bf + bw > kNoAllocBytes) {
+        chunk = kMaxChunk;
+        bw = up(farfield_scratch_bytes(c->dm, n_calls, n_orient, ndir, chunk));
+    }
     const size_t need = 2 * bc + br + bf + bw;
     if (need > kNoAllocBytes)
         return bem_fail(c, BEM_ERR_ARG, "farfield_noalloc: the call needs " + std::to_string(need) +
@@ -671,25 +755,25 @@ int ff_noalloc_launch(bem_ctx* c, const double* cJ, const double* cM, const doub
     BEM_HIP(c, hipMemcpyAsync(dM, cM, (size_t)n_calls * N * 2 * sizeof(double), hipMemcpyHostToDevice, s));
     BEM_HIP(c, hipMemcpyAsync(drh, rh, (size_t)n_orient * ndir * 3 * sizeof(double), hipMemcpyHostToDevice, s));
     // the coefficients stay interleaved: call c, RWG n at 2 (c N + n) (+1 imaginary)
-    farfield_core(c, dJ, dJ + 1, dM, dM + 1, 2L * N, 2L, drh, kr, ki, eta, n_calls, n_orient, ndir, dFv, work);
+    farfield_core(c, dJ, dJ + 1, dM, dM + 1, 2L * N, 2L, drh, rh, kr, ki, eta, n_calls, n_orient, ndir, chunk, dFv,
+                  work);
     BEM_HIP(c, hipGetLastError());
     BEM_HIP(c, hipMemcpyAsync(Fv, dFv, (size_t)n_calls * ndir * 6 * sizeof(double), hipMemcpyDeviceToHost, s));
     BEM_HIP(c, hipStreamSynchronize(s));
     return 0;
 }
 
+size_t ff_work_bytes(const bem_ctx* c, int n_calls, int n_orient, int ndir) {
+    return farfield_scratch_bytes(c->dm, n_calls, n_orient, ndir,
+                                  ff_chunk((long)c->dm.T * c->dm.Nq, n_orient, ndir));
+}
+
 int ff_launch(bem_ctx* c, const double* dJr, const double* dJi, const double* dMr, const double* dMi, int ldc,
-              const double* drh, double kr, double ki, double eta, int n_calls, int n_orient, int ndir,
-              double* dFv) {
-    // uploaded coefficients live in the scratch area already; allocate the
-    // far-field work area separately
-    const size_t bytes = farfield_scratch_bytes(c->dm, n_calls, n_orient, ndir);
-    char* w = nullptr;
-    if (hipMalloc(&w, bytes) != hipSuccess) return bem_fail(c, BEM_ERR_NOMEM, "farfield: work area");
-    farfield_core(c, dJr, dJi, dMr, dMi, (long)ldc, 1, drh, kr, ki, eta, n_calls, n_orient, ndir, dFv, w);
-    const hipError_t e = hipStreamSynchronize(c->stream);
-    (void)hipFree(w);
-    if (e != hipSuccess) return bem_fail(c, BEM_ERR_HIP, std::string("farfield: ") + hipGetErrorString(e));
+              const double* drh, const double* rh, double kr, double ki, double eta, int n_calls, int n_orient,
+              int ndir, double* dFv, void* work) {
+    farfield_core(c, dJr, dJi, dMr, dMi, (long)ldc, 1, drh, rh, kr, ki, eta, n_calls, n_orient, ndir,
+                  ff_chunk((long)c->dm.T * c->dm.Nq, n_orient, ndir), dFv, static_cast<char*>(work));
+    BEM_HIP(c, hipGetLastError());
     return 0;
 }
 
@@ -729,7 +813,8 @@ int mueller_launch(bem_ctx* c, double kr, double ki, double eta, const double* R
     const size_t fvb = (size_t)n_calls * ntheta * 6 * sizeof(double);
     const size_t mob = (size_t)n_orient * 16 * ntheta * sizeof(double);
     const size_t small = rh.size() * 8 + geo.size() * 8 + (size_t)n_orient * 8 + 16 * (size_t)ntheta * 8;
-    const size_t bytes = farfield_scratch_bytes(c->dm, n_calls, n_orient, ntheta) + fvb + mob + small + 1024;
+    const int chunk = ff_chunk((long)c->dm.T * c->dm.Nq, n_orient, ntheta);
+    const size_t bytes = farfield_scratch_bytes(c->dm, n_calls, n_orient, ntheta, chunk) + fvb + mob + small + 1024;
     void* scr = nullptr;
     if (int rc = ctx_scratch(c, bytes, &scr)) return rc;
     char* p = static_cast<char*>(scr);
@@ -740,6 +825,7 @@ int mueller_launch(bem_ctx* c, double kr, double ki, double eta, const double* R
     double* dw = dgeo + geo.size();
     double* dM = dw + n_orient;
     char* work = reinterpret_cast<char*>(dM + 16 * (size_t)ntheta);
+    work += (256 - reinterpret_cast<uintptr_t>(work) % 256) % 256;
     hipStream_t s = c->stream;
     BEM_HIP(c, hipMemcpyAsync(drh, rh.data(), rh.size() * 8, hipMemcpyHostToDevice, s));
     BEM_HIP(c, hipMemcpyAsync(dgeo, geo.data(), geo.size() * 8, hipMemcpyHostToDevice, s));
@@ -747,8 +833,8 @@ int mueller_launch(bem_ctx* c, double kr, double ki, double eta, const double* R
     // device solution: column c is call c; J rows 0..N-1, M rows N..2N-1
     const int N = c->rwg.N;
     const long ld = c->ldr;
-    farfield_core(c, c->Xr, c->Xi, c->Xr + (long)N * ld, c->Xi + (long)N * ld, 1, ld, drh, kr, ki, eta, n_calls,
-                  n_orient, ntheta, dFv, work);
+    farfield_core(c, c->Xr, c->Xi, c->Xr + (long)N * ld, c->Xi + (long)N * ld, 1, ld, drh, rh.data(), kr, ki, eta, n_calls,
+                  n_orient, ntheta, chunk, dFv, work);
     hipLaunchKernelGGL(k_mueller, dim3((n_orient * ntheta + 255) / 256), dim3(256), 0, s, n_orient, ntheta, dFv, dgeo,
                        kr, ki, mirror, dMo);
     hipLaunchKernelGGL(k_mueller_avg, dim3((16 * ntheta + 255) / 256), dim3(256), 0, s, n_orient, ntheta, dMo, dw, dM);
@@ -766,17 +852,17 @@ int ff_adjoint_launch(bem_ctx* c, const double* dL_dM, double* gr, double* gi, d
     build_dirs(c->last_RT.data(), n_orient, c->last_theta.data(), ntheta, rh, geo);
     const DevMesh& d = c->dm;
     const long P = (long)d.T * d.Nq;
-    const int nchunk = (int)((P + 255) / 256);
+    const int nchunk = (int)((P + 255) / 256), chunk = ff_chunk(P, n_orient, ntheta);
     const size_t nfv = (size_t)n_calls * ntheta * 6, ncoef = (size_t)n_orient * ntheta * 24;
     const size_t nacur = (size_t)n_calls * P * 12, nsmall = rh.size() + geo.size() + (size_t)n_orient +
                                                            16 * (size_t)ntheta + (size_t)n_orient * ntheta +
                                                            (size_t)n_orient * nchunk;
-    const size_t bytes = farfield_scratch_bytes(d, n_calls, n_orient, ntheta) +
+    const size_t bytes = farfield_scratch_bytes(d, n_calls, n_orient, ntheta, chunk) +
                          (nfv + ncoef + nacur + nsmall + 64) * sizeof(double);
     char* base = nullptr;
     if (hipMalloc(&base, bytes) != hipSuccess) return bem_fail(c, BEM_ERR_NOMEM, "far-field adjoint: work area");
     double* work = reinterpret_cast<double*>(base);  // cur + partials of farfield_core first
-    double* dFv = work + farfield_scratch_bytes(d, n_calls, n_orient, ntheta) / sizeof(double);
+    double* dFv = work + farfield_scratch_bytes(d, n_calls, n_orient, ntheta, chunk) / sizeof(double);
     double* dcoef = dFv + nfv;
     double* dacur = dcoef + ncoef;
     double* drh = dacur + nacur;
@@ -802,8 +888,8 @@ int ff_adjoint_launch(bem_ctx* c, const double* dL_dM, double* gr, double* gi, d
         const int N = c->rwg.N;
         const long ld = c->ldr;
         // forward far field again (currents in `work`, field in dFv)
-        farfield_core(c, c->Xr, c->Xi, c->Xr + (long)N * ld, c->Xi + (long)N * ld, 1, ld, drh, kr, ki, eta, n_calls,
-                      n_orient, ntheta, dFv, reinterpret_cast<char*>(work));
+        farfield_core(c, c->Xr, c->Xi, c->Xr + (long)N * ld, c->Xi + (long)N * ld, 1, ld, drh, rh.data(), kr, ki, eta, n_calls,
+                      n_orient, ntheta, chunk, dFv, reinterpret_cast<char*>(work));
         hipLaunchKernelGGL(k_mueller_bwd, dim3((n_orient * ntheta + 255) / 256), dim3(256), 0, s, n_orient, ntheta,
                            dFv, dgeo, dG, dw, kr, ki, eta, c->last_mirror, dcoef, dexpl);
         hipLaunchKernelGGL(k_ff_adj, dim3(n_orient, nchunk), dim3(256), 0, s, P, n_calls, ntheta, d.qp, work, dcoef,
