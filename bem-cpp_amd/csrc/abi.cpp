@@ -33,7 +33,6 @@ int ctx_scratch(bem_ctx* c, size_t bytes, void** out) {
 void kt_resolve(bem_ctx* c) {
     KernelTimer& k = c->kt;
     if (k.pending.empty()) return;
-    (void)hipStreamSynchronize(c->stream3);
     (void)hipStreamSynchronize(c->stream2);
     (void)hipStreamSynchronize(c->stream);
     for (KernelTimer::Rec& r : k.pending) {
@@ -213,19 +212,16 @@ bem_ctx* bem_create(int device) {
     c->device = device;
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
         hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking) != hipSuccess ||
-        hipStreamCreateWithFlags(&c->stream3, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&c->ev[0]) != hipSuccess || hipEventCreate(&c->ev[1]) != hipSuccess ||
         hipEventCreateWithFlags(&c->lu_ev[0], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->lu_ev[1], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->lu_ev[2], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->lu_ev[3], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->lu_ev[4], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->lu_ev[5], hipEventDisableTiming) != hipSuccess) {
+        hipEventCreateWithFlags(&c->lu_ev[3], hipEventDisableTiming) != hipSuccess) {
         for (hipEvent_t e : {c->ev[0], c->ev[1]})
             if (e) (void)hipEventDestroy(e);
         for (hipEvent_t e : c->lu_ev)
             if (e) (void)hipEventDestroy(e);
-        for (hipStream_t s : {c->stream, c->stream2, c->stream3})
+        for (hipStream_t s : {c->stream, c->stream2})
             if (s) (void)hipStreamDestroy(s);
         delete c;
         return nullptr;
@@ -240,7 +236,6 @@ bem_ctx* bem_create(int device) {
 void bem_destroy(bem_ctx* c) {
     if (!c) return;
     (void)hipSetDevice(c->device);
-    (void)hipStreamSynchronize(c->stream3);
     (void)hipStreamSynchronize(c->stream2);
     (void)hipStreamSynchronize(c->stream);
     free_mesh(c);
@@ -253,7 +248,6 @@ void bem_destroy(bem_ctx* c) {
     (void)hipEventDestroy(c->ev[1]);
     for (hipEvent_t e : c->lu_ev) (void)hipEventDestroy(e);
     (void)hipStreamDestroy(c->stream2);
-    (void)hipStreamDestroy(c->stream3);
     (void)hipStreamDestroy(c->stream);
     delete c;
 }

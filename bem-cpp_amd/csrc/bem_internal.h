@@ -134,12 +134,11 @@ struct bem_ctx {
     KernelTimer kt;
     hipStream_t stream = nullptr;
     hipStream_t stream2 = nullptr;  // panel stream of the look-ahead factorisation
-    hipStream_t stream3 = nullptr;  // updates inside an outer panel off its critical path
     // factorisation stream layout (see factor() in kernels/lu.hip): 0 one
     // stream, 1 panel + update streams on all CUs
     int lu_streams = -1;            // -1: not chosen yet
     hipEvent_t ev[2] = {nullptr, nullptr};
-    hipEvent_t lu_ev[6] = {};  // cross-stream ordering inside the factorisation
+    hipEvent_t lu_ev[4] = {};  // cross-stream ordering inside the factorisation
     std::string err;
 
     // mesh and basis (host copies)

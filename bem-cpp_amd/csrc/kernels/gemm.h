@@ -427,8 +427,8 @@ inline int gemm_choose(const bem_ctx* c, int M, int N) {
 // No LDS and no barrier: every wave owns one 16 x 16 tile of C over the whole
 // K and issues all of its operand loads before the first MFMA (A as 16-byte
 // pieces of its row, B as single values of its column).  For the products on
-// the factorisation's panel chain (the rank-32 updates of a panel step, the
-// L11^{-1} doubling), which run beside the trailing update: there a kernel
+// the factorisation's panel chain (the L11^{-1} doubling), which run beside the
+// trailing update: there a kernel
 // that stages operands through LDS with a barrier per slice slows down about
 // three times.  The MFMA takes the B fragment first, so each lane ends with
 // four consecutive columns of one row of C.  Batched over blockIdx.y with
@@ -532,10 +532,8 @@ inline void cgemm_rd(hipStream_t s, int M, int N, int K, const float* Ar, const 
 
 // Launch flags of cgemm_ctx: GEMM_HEADROOM caps the grid as
 // gemm_headroom_cap does (an update running beside the panel stream);
-// GEMM_PANEL marks a product of the panel stream's critical path: the plan's
-// panel configuration at raised issue priority; GEMM_UPDATE: an LU trailing
-// update (its own kernel symbol and timing class).
-constexpr int GEMM_HEADROOM = 1, GEMM_PANEL = 2, GEMM_UPDATE = 4;
+// GEMM_UPDATE: an LU trailing update (its own kernel symbol and timing class).
+constexpr int GEMM_HEADROOM = 1, GEMM_UPDATE = 4;
 
 // GEMM with optional per-launch timing, on stream s (default: the context
 // stream), tile configuration from the context's plan.  Counted work: 3M
@@ -549,17 +547,9 @@ inline void cgemm_ctx(bem_ctx* c, int M, int N, int K, const T* Ar, const T* Ai,
     const bool upd = flags & GEMM_UPDATE;
     const int k = kt_mark(c, sizeof(T) == 4 ? (upd ? KS_UPDATE32 : KS_GEMM32) : (upd ? KS_UPDATE64 : KS_GEMM64), s);
     const GemmPlan& plan = c->gemm_plan[sizeof(T) == 4 ? 0 : 1];
-    const int cfg = (flags & GEMM_PANEL) ? plan.panel : gemm_choose<T>(c, M, N);
+    const int cfg = gemm_choose<T>(c, M, N);
     const long cap = (flags & GEMM_HEADROOM) ? gemm_headroom_cap(plan, cfg) : 0;
-    if (flags & GEMM_PANEL) mode |= GEMM_MODE_URGENT;
-    bool done = false;
-    if constexpr (sizeof(T) == 4) {
-        if ((flags & GEMM_PANEL) && cgemm_rd_fits(M, N, K, Ar, Ai, lda, Cr, Ci, ldc)) {
-            cgemm_rd(s, M, N, K, Ar, Ai, lda, Br, Bi, ldb, Cr, Ci, ldc, mode);
-            done = true;
-        }
-    }
-    if (!done) cgemm_any<T>(cfg, s, M, N, K, Ar, Ai, lda, Br, Bi, ldb, Cr, Ci, ldc, mode, 1, 0, 0, 0, cap, upd ? 1 : 0);
+    cgemm_any<T>(cfg, s, M, N, K, Ar, Ai, lda, Br, Bi, ldb, Cr, Ci, ldc, mode, 1, 0, 0, 0, cap, upd ? 1 : 0);
     const double mnk = (double)M * N * K;
     const double bytes = 2.0 * sizeof(T) * ((double)M * K + (double)K * N + (mode == 1 ? 1.0 : 2.0) * M * N);
     kt_close(c, k, (sizeof(T) == 4 ? 6.0 : 8.0) * mnk, bytes);

@@ -7,18 +7,20 @@
 // The pivots differ from cuSOLVER's; the solution does not.
 //
 // Right-looking two-level blocking on the padded matrix (npad = 256 k):
-//   outer panel of NB = 256 columns, factored in 8 inner steps of PB = 32:
+//   outer panel of NB = 256 columns, factored in 8 inner steps of PB = 32, two
+//   launches each:
 //     1. pivot selection for the 32 columns over all remaining rows by a
 //        tournament (communication-avoiding "TSLU": Grigori, Demmel & Xiang,
-//        SIAM J. Matrix Anal. Appl. 32 (2011)), in one launch: 256-row chunks
-//        each choose 32 candidate rows by partial pivoting in LDS; the last
-//        block of every group of 8 to finish (integer arrival counter) merges
-//        the group's candidates, up to the root, whose pivot order becomes
-//        LAPACK-style swaps ipiv[j0 .. j0+31].  No block ever waits.
-//     2. the swaps are applied to whole rows (all columns)
-//     3. the 32 x 32 diagonal block is factored without further pivoting,
-//        L21 = A21 U11^{-1} row by row, U12 of the rest of the outer panel
-//     4. rank-32 update of the rest of the outer panel on the matrix cores
+//        SIAM J. Matrix Anal. Appl. 32 (2011)): sets of 256 rows (512 where that
+//        saves a level) each choose 32 candidate rows by partial pivoting in
+//        registers; the last block of every group of sets to finish (integer
+//        arrival counter) merges the group's candidates, up to the root, whose
+//        pivot order becomes LAPACK-style swaps ipiv[j0 .. j0+31] and the
+//        factored 32 x 32 diagonal block.  No block ever waits.
+//     2. (k_step) the swaps in the panel, L21 = A21 U11^{-1}, U12 = L11^{-1} A12
+//        and the rank-32 update of the next 32 columns on the matrix cores; the
+//        update of the panel's other columns rides in the next tournament's
+//        launch
 //   then L11^{-1} of the 256 x 256 diagonal block (by doubling: eight 32 x 32
 //   inverses in LDS, then three levels of batched GEMMs), U12 = L11^{-1} A12
 //   and the rank-256 trailing update A22 -= L21 U12 as matrix-core GEMMs
@@ -36,21 +38,6 @@ namespace {
 
 constexpr int NB = 256;  // outer panel width = solve block size
 constexpr int PB = 32;   // inner panel width (pivot block)
-
-// Tournament block: CH rows, one per thread, so a merge takes CH / PB
-// candidate sets.  256 threads: larger blocks need fewer tree levels but pay
-// more per elimination step (measured slower at 512), and at about 150
-// registers the FP32 block still fits beside the trailing-update GEMM on a CU.
-template <typename T>
-struct Tslu;
-template <>
-struct Tslu<float> {
-    static constexpr int CH = 256;
-};
-template <>
-struct Tslu<double> {
-    static constexpr int CH = 256;
-};
 
 template <typename T>
 __device__ __forceinline__ T mag2(T r, T i) {
@@ -97,209 +84,486 @@ __device__ __forceinline__ void store_row(T* __restrict__ p, const T (&x)[PB]) {
 __device__ __forceinline__ float recip(float d) { return __builtin_amdgcn_rcpf(d); }
 __device__ __forceinline__ double recip(double d) { return 1.0 / d; }
 
-// Wave-wide maximum of an unsigned value (DPP reduction of the device library).
-extern "C" __device__ unsigned __ockl_wfred_max_u32(unsigned);
-
-// Order-preserving 32-bit key of a non-negative magnitude; 0 is reserved for
-// "no candidate".  Doubles keep their sign, exponent and 20 leading mantissa
-// bits: rows closer than 2^-20 in magnitude tie and the lower one wins.
-__device__ __forceinline__ unsigned mag_key(float m) { return __float_as_uint(m) + 1u; }
-__device__ __forceinline__ unsigned mag_key(double m) {
-    return (unsigned)((unsigned long long)__double_as_longlong(m) >> 32) + 1u;
+// Order-preserving 32-bit key of a non-negative magnitude, with the row in its
+// low bits (r of R rows per thread, then the lane; ties: lowest), so the wave's
+// maximum names its row; 0 is "no candidate".  That leaves 17 mantissa bits of a
+// float and 14 of a double (one less for two rows per thread): rows closer than
+// that in magnitude tie.  (The sign of a NaN is masked.)
+__device__ __forceinline__ unsigned mag_bits(float m) { return __float_as_uint(m); }
+__device__ __forceinline__ unsigned mag_bits(double m) {
+    return (unsigned)((unsigned long long)__double_as_longlong(m) >> 32);
+}
+template <int R, typename T>
+__device__ __forceinline__ unsigned mag_key(T m, int r, int lane) {
+    static_assert(R <= 2, "one bit for the row");
+    constexpr unsigned low = 64 * R;  // values of the row part
+    return (mag_bits(m) & 0x7fffffffu & ~(low - 1)) + low + 64 * (R - 1 - r) + (unsigned)(63 - lane);
 }
 
-// Exchange area of the register-resident elimination for NW waves.  A step
-// takes two barriers: the waves' best keys first, then only the winning
-// row.  (Every wave writing its candidate row before one barrier costs NW
-// times the LDS writes, which serialise on the CU's LDS and cost more than
-// the second barrier.)  Writes of a step happen after the previous step's
-// last barrier and its reads before the next step's first, so one buffer
-// suffices.
-template <typename T, int NW>
+// Maximum over the wave, in a scalar register (DPP within rows of 16, then
+// across the rows).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned max_dpp(unsigned v) {
+    return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ unsigned wave_max(unsigned v) {
+    v = max_dpp<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8
+    v = max_dpp<0x112, 0xf>(v);
+    v = max_dpp<0x114, 0xf>(v);
+    v = max_dpp<0x118, 0xf>(v);
+    v = max_dpp<0x142, 0xa>(v);  // row_bcast 15, 31
+    v = max_dpp<0x143, 0xc>(v);
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// v of lane l (l the same for the whole wave) as a scalar.
+__device__ __forceinline__ float from_lane(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ double from_lane(double v, int l) {
+    const long long u = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)u, l), hi = __builtin_amdgcn_readlane((int)(u >> 32), l);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+constexpr int EW = 4;  // columns of an elimination window
+
+// Columns EW .. PB-1 to the front, columns 0 .. EW-1 to the end.
+template <typename T>
+__device__ __forceinline__ void rotate_row(T (&x)[PB]) {
+    T h[EW];
+#pragma unroll
+    for (int c = 0; c < EW; c++) h[c] = x[c];
+#pragma unroll
+    for (int c = 0; c < PB - EW; c++) x[c] = x[c + EW];
+#pragma unroll
+    for (int c = 0; c < EW; c++) x[PB - EW + c] = h[c];
+}
+
+// Exchange area of the register-resident elimination (4 waves).
+template <typename T>
 struct ElimLds {
-    alignas(16) T row[2 * PB];  // the pivot row (columns > the step): real parts, then imaginary
-    T rp[2];                    // 1 / the pivot element
-    unsigned long long kb[NW];  // best key of each wave (high word) and ~its thread (low word)
-    int oid[PB], osrc[PB];      // chosen rows in pivot order
+    alignas(16) T win[2][4][2][EW];   // [step parity][wave][plane]: the wave's best row, window columns
+    alignas(16) unsigned key[2][4];   // its key
+    alignas(16) T raw[EW][2][PB];     // the window's pivot rows before the window's updates right of it
+    alignas(16) T u[4][EW][2][PB];    // the same as rows of U, one copy per wave
+    alignas(16) int oid[PB];          // chosen rows in pivot order
+    int osrc[PB];
+    alignas(16) int sw[2][PB];        // root_swaps
     int last;
     int zmin;  // first zero pivot of the root (1-based)
 };
 
-// Partial pivoting over the block's rows, one row per thread in registers
-// (rows t >= nrows take no part; nrows >= PB), with implicit row
-// interchanges: rows stay with their thread and a chosen row is only marked.
-// Step jc: the largest |x_jc|^2 among the rows not chosen yet (by mag_key;
-// ties: lower thread) becomes pivot jc, and the remaining rows are eliminated
-// (multiplier stored in x_jc).  An all-zero column chooses the lowest open
-// row and eliminates nothing.
-// Afterwards the thread of pivot r holds row r of L11 \ U11 and returns r
-// (-1 for rows not chosen); oid/osrc list the chosen rows in pivot order.
-template <typename T, int NW>
-__device__ __forceinline__ int elim_rows(ElimLds<T, NW>& L, T (&xr)[PB], T (&xi)[PB], int id, int src, int nrows) {
-    const int t = threadIdx.x, wave = t >> 6;
-    const bool valid = t < nrows;
-    int mine = -1;
+// Partial pivoting over the block's rows, R rows per thread in registers (row
+// t + 256 r; rows at nrows and beyond take no part; nrows >= PB), with
+// implicit row interchanges: rows stay with their thread and a chosen row is
+// only marked.  Step jc: the largest |x_jc|^2 among the rows not chosen yet (by
+// mag_key; ties: lowest r, wave, lane) becomes pivot jc, and the remaining rows
+// are eliminated (multiplier stored in x_jc).  An all-zero column chooses the
+// lowest open row and eliminates nothing.
+// Afterwards mine[r] is the pivot number of row r (its thread holds that row of
+// L11 \ U11), -1 for rows not chosen; oid/osrc list the chosen rows in pivot
+// order.
+//
+// The chain of 32 steps is bound by the exchange between the waves and by
+// instruction fetch, so:
+// - a step has one exchange: every wave's best row goes to LDS with its key
+//   before one barrier, but only the columns of the current window of EW, which
+//   is also all that is updated within the window.  The columns right of it take
+//   the window's EW pivots at once: their rows go to LDS, each wave solves them
+//   against the window's unit triangle, one column per lane, and updates its
+//   rows.  Per element the operations and their order are those of the
+//   column-by-column elimination.
+// - the windows are a loop, not unrolled code: the row registers rotate by EW
+//   columns after each window, so the window is always columns 0 .. EW-1 of the
+//   registers and the eighth rotation brings every column home.  (Unrolled, the
+//   32 steps are 40 KB of code per call site.)
+// 3840 rows: 72.7 us before, 58.7 now (with the root's parallel swaps and sets
+// of 512 rows); one level of 256 rows 27.7 and 24.5.
+template <typename T, int R>
+__device__ __forceinline__ void elim_rows(ElimLds<T>& L, T (&xr)[R][PB], T (&xi)[R][PB], const int (&id)[R],
+                                          const int (&src)[R], int nrows, int (&mine)[R]) {
+    using V = typename Vec16<T>::type;
+    constexpr int E = 16 / sizeof(T);
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    bool valid[R];
 #pragma unroll
-    for (int jc = 0; jc < PB; jc++) {
-        const bool open = valid && mine < 0;
-        const unsigned key = open ? mag_key(mag2(xr[jc], xi[jc])) : 0u;
-        const unsigned wk = __ockl_wfred_max_u32(key);
-        const int p = wave * 64 + __ffsll((long long)__ballot(key == wk)) - 1;  // ties: lowest thread
-        if (t == p) L.kb[wave] = ((unsigned long long)wk << 32) | (0xffffffffu - (unsigned)p);
-        __syncthreads();
-        // largest key, ties to the lowest thread: one maximum over the packed words
-        unsigned long long kbest = L.kb[0];
+    for (int r = 0; r < R; r++) {
+        valid[r] = t + 256 * r < nrows;
+        mine[r] = -1;
+    }
+#pragma unroll 1
+    for (int w = 0; w < PB / EW; w++) {
+        const int s = w * EW, ng = PB / EW - 1 - w;  // first column; groups of EW columns right of the window
+        T lr[R][EW], li[R][EW];  // the window's multipliers (0: row not eliminated)
 #pragma unroll
-        for (int w = 1; w < NW; w++) kbest = max(kbest, L.kb[w]);
-        const unsigned best = (unsigned)(kbest >> 32);
-        const int pp = (int)(0xffffffffu - (unsigned)kbest);
-        if (t == pp) {
-            mine = jc;
-            // 16-byte stores from the aligned piece holding column jc + 1
-            using V = typename Vec16<T>::type;
-            constexpr int E = 16 / sizeof(T);
+        for (int q = 0; q < EW; q++) {
+            const int par = q & 1;
+            unsigned key = 0u;
+            int rb = 0;
 #pragma unroll
-            for (int q = 0; q < PB / E; q++)
-                if (q * E + E - 1 > jc) {
-                    V a, d;
-                    __builtin_memcpy(&a, &xr[q * E], 16);
-                    __builtin_memcpy(&d, &xi[q * E], 16);
-                    *reinterpret_cast<V*>(L.row + q * E) = a;
-                    *reinterpret_cast<V*>(L.row + PB + q * E) = d;
-                }
-            // reciprocal of the pivot (the rows scale by it, as zgetf2 does)
-            const T d = xr[jc] * xr[jc] + xi[jc] * xi[jc];
-            const T inv = d > T(0) ? recip(d) : T(0);
-            L.rp[0] = xr[jc] * inv;
-            L.rp[1] = -xi[jc] * inv;
-        }
-        __syncthreads();
-        // branch-free update: rows that are not eliminated use multiplier 0
-        // (keeps one copy of the row in registers across the step)
-        const bool upd = open && best > 1u && t != pp;
-        const T qr = L.rp[0], qi = L.rp[1];
-        const T lr = upd ? xr[jc] * qr - xi[jc] * qi : T(0);
-        const T li = upd ? xr[jc] * qi + xi[jc] * qr : T(0);
-        xr[jc] = upd ? lr : xr[jc];
-        xi[jc] = upd ? li : xi[jc];
-        // x_c -= l u_c as four fused multiply-adds per element, the pivot row
-        // read in 16-byte pieces from the aligned piece holding column jc + 1
-        const T nlr = -lr, nli = -li;
-        constexpr int E = 16 / sizeof(T);
-#pragma unroll
-        for (int q = 0; q < PB / E; q++)
-            if (q * E + E - 1 > jc) {
-                T ur[E], ui[E];
-                const typename Vec16<T>::type a = *reinterpret_cast<const typename Vec16<T>::type*>(L.row + q * E);
-                const typename Vec16<T>::type d = *reinterpret_cast<const typename Vec16<T>::type*>(L.row + PB + q * E);
-                __builtin_memcpy(ur, &a, 16);
-                __builtin_memcpy(ui, &d, 16);
-#pragma unroll
-                for (int e = 0; e < E; e++) {
-                    const int c = q * E + e;
-                    if (c > jc) {
-                        xr[c] = fmadd(nlr, ur[e], xr[c]);
-                        xr[c] = fmadd(li, ui[e], xr[c]);
-                        xi[c] = fmadd(nlr, ui[e], xi[c]);
-                        xi[c] = fmadd(nli, ur[e], xi[c]);
-                    }
+            for (int r = 0; r < R; r++) {
+                const unsigned k = valid[r] && mine[r] < 0 ? mag_key<R>(mag2(xr[r][q], xi[r][q]), r, lane) : 0u;
+                if (k > key) {
+                    key = k;
+                    rb = r;
                 }
             }
+            const unsigned wk = wave_max(key);
+            T wr[EW], wi[EW];
+#pragma unroll
+            for (int c = 0; c < EW; c++) {
+                wr[c] = xr[0][c];
+                wi[c] = xi[0][c];
+#pragma unroll
+                for (int r = 1; r < R; r++) {
+                    wr[c] = rb == r ? xr[r][c] : wr[c];
+                    wi[c] = rb == r ? xi[r][c] : wi[c];
+                }
+            }
+            if (key == wk) {  // one lane, or a wave without candidates
+#pragma unroll
+                for (int c = 0; c < EW; c += E)
+                    if (c + E - 1 >= q) {
+                        V a, d;
+                        __builtin_memcpy(&a, &wr[c], 16);
+                        __builtin_memcpy(&d, &wi[c], 16);
+                        *reinterpret_cast<V*>(&L.win[par][wave][0][c]) = a;
+                        *reinterpret_cast<V*>(&L.win[par][wave][1][c]) = d;
+                    }
+                L.key[par][wave] = wk;
+            }
+            __syncthreads();
+            // lane l reads wave l % 4's entry; the maximum over four lanes then
+            // names the wave whose window the scalar registers take (one LDS
+            // latency instead of the keys' and then the window's)
+            const unsigned kw = L.key[par][lane & 3] | 63u;  // without the lane: ties go to the lower wave
+            T cr[EW], ci[EW];
+#pragma unroll
+            for (int c = 0; c < EW; c += E)
+                if (c + E - 1 >= q) {
+                    const V a = *reinterpret_cast<const V*>(&L.win[par][lane & 3][0][c]);
+                    const V d = *reinterpret_cast<const V*>(&L.win[par][lane & 3][1][c]);
+                    __builtin_memcpy(&cr[c], &a, 16);
+                    __builtin_memcpy(&ci[c], &d, 16);
+                }
+            unsigned best = max_dpp<0xb1, 0xf>(kw);  // quad_perm [1, 0, 3, 2], then [2, 3, 0, 1]
+            best = max_dpp<0x4e, 0xf>(best);
+            const int wv = __ffsll((long long)__ballot(kw == best)) - 1;
+            T ur[EW], ui[EW];
+#pragma unroll
+            for (int c = q; c < EW; c++) {
+                ur[c] = from_lane(cr[c], wv);
+                ui[c] = from_lane(ci[c], wv);
+            }
+            const bool won = wave == wv && key == wk;
+            // reciprocal of the pivot (the rows scale by it, as zgetf2 does)
+            const T d = ur[q] * ur[q] + ui[q] * ui[q];
+            const T inv = d > T(0) ? recip(d) : T(0);
+            const T qr = ur[q] * inv, qi = -ui[q] * inv;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                if (won && rb == r) mine[r] = s + q;
+                // branch-free update: rows that are not eliminated use multiplier 0
+                const bool upd = valid[r] && mine[r] < 0 && d > T(0);
+                const T a = xr[r][q] * qr - xi[r][q] * qi, b = xr[r][q] * qi + xi[r][q] * qr;
+                lr[r][q] = upd ? a : T(0);
+                li[r][q] = upd ? b : T(0);
+                xr[r][q] = upd ? a : xr[r][q];
+                xi[r][q] = upd ? b : xi[r][q];
+                const T nlr = -lr[r][q], nli = -li[r][q];
+#pragma unroll
+                for (int c = q + 1; c < EW; c++) {
+                    xr[r][c] = fmadd(nlr, ur[c], xr[r][c]);
+                    xr[r][c] = fmadd(li[r][q], ui[c], xr[r][c]);
+                    xi[r][c] = fmadd(nlr, ui[c], xi[r][c]);
+                    xi[r][c] = fmadd(nli, ur[c], xi[r][c]);
+                }
+            }
+        }
+        if (ng > 0) {
+            // the window's pivot rows (window columns final, the others without
+            // the window's updates)
+#pragma unroll
+            for (int r = 0; r < R; r++)
+                if (mine[r] >= s) {
+#pragma unroll
+                    for (int g = 0; g < PB / EW; g++)
+                        if (g <= ng) {
+#pragma unroll
+                            for (int c = g * EW; c < (g + 1) * EW; c += E) {
+                                V a, d;
+                                __builtin_memcpy(&a, &xr[r][c], 16);
+                                __builtin_memcpy(&d, &xi[r][c], 16);
+                                *reinterpret_cast<V*>(&L.raw[mine[r] - s][0][c]) = a;
+                                *reinterpret_cast<V*>(&L.raw[mine[r] - s][1][c]) = d;
+                            }
+                        }
+                }
+            __syncthreads();
+            if (lane < ng * EW) {
+                T vr[EW], vi[EW];
+#pragma unroll
+                for (int q = 0; q < EW; q++) {
+                    vr[q] = L.raw[q][0][EW + lane];
+                    vi[q] = L.raw[q][1][EW + lane];
+                }
+#pragma unroll
+                for (int q = 0; q < EW; q++) {
+#pragma unroll
+                    for (int k = 0; k < q; k++) {
+                        const T mr = L.raw[q][0][k], mi = L.raw[q][1][k];
+                        vr[q] = fmadd(-mr, vr[k], vr[q]);
+                        vr[q] = fmadd(mi, vi[k], vr[q]);
+                        vi[q] = fmadd(-mr, vi[k], vi[q]);
+                        vi[q] = fmadd(-mi, vr[k], vi[q]);
+                    }
+                    L.u[wave][q][0][EW + lane] = vr[q];
+                    L.u[wave][q][1][EW + lane] = vi[q];
+                }
+            }
+            __builtin_amdgcn_wave_barrier();  // the wave's own copy: LDS operations of a wave stay in order
+            // the scheduling barriers keep the reads of later columns from being
+            // hoisted (they would not fit in the registers)
+#pragma unroll
+            for (int g = 1; g < PB / EW; g++)
+                if (g <= ng) {
+#pragma unroll
+                    for (int c0 = g * EW; c0 < (g + 1) * EW; c0 += E) {
+                        T ur[EW][E], ui[EW][E];
+#pragma unroll
+                        for (int q = 0; q < EW; q++) {
+                            const V a = *reinterpret_cast<const V*>(&L.u[wave][q][0][c0]);
+                            const V d = *reinterpret_cast<const V*>(&L.u[wave][q][1][c0]);
+                            __builtin_memcpy(ur[q], &a, 16);
+                            __builtin_memcpy(ui[q], &d, 16);
+                        }
+#pragma unroll
+                        for (int q = 0; q < EW; q++)
+#pragma unroll
+                            for (int r = 0; r < R; r++) {
+                                const T nlr = -lr[r][q], nli = -li[r][q];
+#pragma unroll
+                                for (int e = 0; e < E; e++) {
+                                    const int c = c0 + e;
+                                    xr[r][c] = fmadd(nlr, ur[q][e], xr[r][c]);
+                                    xr[r][c] = fmadd(li[r][q], ui[q][e], xr[r][c]);
+                                    xi[r][c] = fmadd(nlr, ui[q][e], xi[r][c]);
+                                    xi[r][c] = fmadd(nli, ur[q][e], xi[r][c]);
+                                }
+                            }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            rotate_row(xr[r]);
+            rotate_row(xi[r]);
+        }
     }
-    if (mine >= 0) {
-        L.oid[mine] = id;
-        L.osrc[mine] = src;
-    }
+#pragma unroll
+    for (int r = 0; r < R; r++)
+        if (mine[r] >= 0) {
+            L.oid[mine[r]] = id[r];
+            L.osrc[mine[r]] = src[r];
+        }
     __syncthreads();
-    return mine;
 }
 
 // Root of the tournament, one wave: pivot order -> LAPACK-style swaps
 // ipiv[j0 .. j0+31], and their net effect on the touched rows as a list of
 // (destination, source) row pairs: pl[0] = count, pl[1 + 2k] = destination,
-// pl[2 + 2k] = source.  Lane l tracks one touched row (<= 64 rows).
-__device__ void root_swaps(const int* __restrict__ oid, int j0, int* __restrict__ ipiv, int* __restrict__ pl) {
-    const int lane = threadIdx.x;  // wave 0
-    // pos: lane c < PB holds the current location of the c-th chosen row
-    int pos = lane < PB ? oid[lane] : -1;
-    int rows = -1, cont = -1, nt = 0;
-    for (int c = 0; c < PB; c++) {
-        const int x = j0 + c;
-        const int y = __builtin_amdgcn_readlane(pos, c);
-        if (lane == 0) ipiv[x] = y;
-        if (lane > c && pos == x) pos = y;  // the row at x moves to y
-        if (y == x) continue;
-        // net permutation of the touched rows
-        unsigned long long m = __ballot(rows == x);
-        int ix;
-        if (m == 0ull) {
-            ix = nt++;
-            if (lane == ix) rows = cont = x;
-        } else {
-            ix = __ffsll((long long)m) - 1;
-        }
-        m = __ballot(rows == y);
-        int iy;
-        if (m == 0ull) {
-            iy = nt++;
-            if (lane == iy) rows = cont = y;
-        } else {
-            iy = __ffsll((long long)m) - 1;
-        }
-        const int cx = __builtin_amdgcn_readlane(cont, ix), cy = __builtin_amdgcn_readlane(cont, iy);
-        if (lane == ix) cont = cy;
-        if (lane == iy) cont = cx;
+// pl[2 + 2k] = source (at most 2 PB pairs).
+// Step c swaps row j0 + c with the row y_c where the c-th chosen row is by
+// then.  A row moves only when its slot is swapped: chosen row o_c stays put
+// unless it started in a slot k < c, whose content went to y_k, and so on, so y_c
+// is the end of the chain v <- o_{slot of v} while v is in a slot below c.  The
+// content of slot c at step c is the row j0 + c unless an earlier step put its
+// own content there; the last such step's content, and so on (cont below).
+// Row j0 + c ends as o_c, and a row y outside the slots as the content of the
+// last step that swaps with it.  All lanes follow their chains side by side
+// (the 32 swaps one after the other took 13 500 cycles, 5.5 us of each
+// tournament).
+__device__ void root_swaps(const int* __restrict__ oid, int* __restrict__ y, int* __restrict__ lastw, int j0,
+                           int* __restrict__ ipiv, int* __restrict__ pl) {
+    const int lane = threadIdx.x, c = lane & (PB - 1);  // both halves of the wave hold step c
+    const int o = oid[c];
+    int v = o;
+    while (v - j0 < c && v >= j0) v = oid[v - j0];
+    if (lane < PB) {
+        y[c] = v;
+        ipiv[j0 + c] = v;
     }
-    const bool moved = lane < nt && cont != rows;
+    __builtin_amdgcn_wave_barrier();
+    int lw = -1;        // the last step below c that puts its content into slot c
+    bool final = true;  // no later step swaps with the same row
+#pragma unroll
+    for (int k = 0; k < PB; k++) {
+        const int yk = y[k];
+        if (k < c && yk == j0 + c) lw = k;
+        if (k > c && yk == v) final = false;
+    }
+    if (lane < PB) lastw[c] = lw;
+    __builtin_amdgcn_wave_barrier();
+    int cont = c;
+    for (int k = lw; k >= 0; k = lastw[k]) cont = k;
+    // lanes below PB: the slots; the others: the rows outside them
+    const int dst = lane < PB ? j0 + c : v, from = lane < PB ? o : j0 + cont;
+    const bool moved = lane < PB ? dst != from : v >= j0 + PB && final;
     const unsigned long long mm = __ballot(moved);
     const int k = __popcll(mm & ((1ull << lane) - 1ull));
     if (moved) {
-        pl[1 + 2 * k] = rows;
-        pl[2 + 2 * k] = cont;
+        pl[1 + 2 * k] = dst;
+        pl[2 + 2 * k] = from;
     }
     if (lane == 0) pl[0] = __popcll(mm);
 }
 
+// What the columns of the panel beyond the next 32 still need from the step at
+// columns jp: the rank-32 update of the columns [c0, c0 + ncol), rows from jp +
+// 32 on (16 x 16 tiles, four per workgroup), and U12 of the next 32 columns put
+// in place (one workgroup).  It rides in the launch of the next tournament,
+// whose few workgroups leave the device idle, instead of on a stream of its own
+// with an event each way.
+struct FarUpdate {
+    int jp, c0, ncol, blocks;  // blocks: workgroups of the launch that do this
+};
+
+// One 16 x 16 tile of C -= L21 U12 per wave with K = 32, operands straight from
+// memory to the matrix cores, every load issued before the first product.
+template <typename T>
+__device__ __forceinline__ void far_update(T* __restrict__ Ar, T* __restrict__ Ai, long ld, int n, FarUpdate f,
+                                           int block, const T* __restrict__ Ur, const T* __restrict__ Ui) {
+    if (block == f.blocks - 1) {
+        for (int e = threadIdx.x; e < PB * PB; e += 256) {
+            const long o = (long)(f.jp + e / PB) * ld + f.jp + PB + e % PB;
+            Ar[o] = Ur[e];
+            Ai[o] = Ui[e];
+        }
+        return;
+    }
+    const int i0 = f.jp + PB, nct = f.ncol / 16, ntiles = (n - i0) / 16 * nct;
+    const int tile = block * 4 + (threadIdx.x >> 6);
+    if (tile >= ntiles) return;
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int m0 = i0 + tile / nct * 16, n0 = f.c0 + tile % nct * 16;
+    T a0[2][4], a1[2][4], b0[2][4], b1[2][4];
+    const long oa = (long)(m0 + r) * ld + f.jp + 4 * g;
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        load_row4<T>(Ar + oa + 16 * q, a0[q]);
+        load_row4<T>(Ai + oa + 16 * q, a1[q]);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const long ob = (long)(f.jp + 16 * q + 4 * g + e) * ld + n0 + r;
+            b0[q][e] = Ar[ob];
+            b1[q][e] = Ai[ob];
+        }
+    }
+    if constexpr (sizeof(T) == 4) {
+        const long oc = (long)(m0 + r) * ld + n0 + 4 * g;
+        const v4f cr = *reinterpret_cast<const v4f*>(Ar + oc), ci = *reinterpret_cast<const v4f*>(Ai + oc);
+        __builtin_amdgcn_sched_barrier(0);
+        v4f t1 = v4f{0.f, 0.f, 0.f, 0.f}, t2 = t1, t3 = t1;
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                t1 = mfma16x16x4(b0[q][e], a0[q][e], t1);
+                t2 = mfma16x16x4(b1[q][e], a1[q][e], t2);
+                t3 = mfma16x16x4(b0[q][e] + b1[q][e], a0[q][e] + a1[q][e], t3);
+            }
+        *reinterpret_cast<v4f*>(Ar + oc) = cr - (t1 - t2);
+        *reinterpret_cast<v4f*>(Ai + oc) = ci - (t3 - t1 - t2);
+    } else {
+        const long oc = (long)(m0 + g) * ld + n0 + r;
+        v4d cr, ci, re{}, im{};
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            cr[q] = Ar[oc + 4 * q * ld];
+            ci[q] = Ai[oc + 4 * q * ld];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                re = mfma16x16x4(a0[q][e], b0[q][e], re);
+                re = mfma16x16x4(a1[q][e], -b1[q][e], re);
+                im = mfma16x16x4(a0[q][e], b1[q][e], im);
+                im = mfma16x16x4(a1[q][e], b0[q][e], im);
+            }
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            Ar[oc + 4 * q * ld] = cr[q] - re[q];
+            Ai[oc + 4 * q * ld] = ci[q] - im[q];
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
-// Pivot tournament for columns j0..j0+31 over rows j0..n-1, one launch.
+// Pivot tournament for columns j0..j0+31 over rows j0..n-1, one launch; row i
+// of the columns at S + i lds.  Sets of CH = 256 R rows (R per thread) choose 32
+// candidates each, groups of G = CH / 32 sets merge.
 // Candidate sets of level L live at set index off[L] + i; a set is 32 ids and
 // the 32 x 32 original values per plane.  cnt: one arrival counter per group
 // per level (zero on entry; reset by the merging block).  The root writes
 // ipiv, the row-pair list pl, the factored diagonal block d11 (32 x 32 per
-// plane) and the first zero pivot into *info.
+// plane) and the first zero pivot into *info.  The last f.blocks workgroups do
+// the previous step's far update instead (A, U; other columns than S's).
 // ---------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(Tslu<T>::CH) void k_tslu(const T* __restrict__ Ar, const T* __restrict__ Ai, long ld,
-                                                      int j0, int n, int* __restrict__ cid, T* __restrict__ cvr,
-                                                      T* __restrict__ cvi, int* __restrict__ cnt,
-                                                      int* __restrict__ ipiv, int* __restrict__ pl,
-                                                      T* __restrict__ d11r, T* __restrict__ d11i,
-                                                      int* __restrict__ info) {
+template <typename T, int R>
+__global__ __launch_bounds__(256) void k_tslu(const T* __restrict__ Sr, const T* __restrict__ Si, long lds, int j0,
+                                              int n, int* __restrict__ cid, T* __restrict__ cvr, T* __restrict__ cvi,
+                                              int* __restrict__ cnt, int* __restrict__ ipiv, int* __restrict__ pl,
+                                              T* __restrict__ d11r, T* __restrict__ d11i, int* __restrict__ info,
+                                              T* __restrict__ Ar, T* __restrict__ Ai, long ld, FarUpdate f,
+                                              const T* __restrict__ Ur, const T* __restrict__ Ui) {
     __builtin_amdgcn_s_setprio(3);  // latency-bound: win issue slots over co-resident GEMM waves
-    constexpr int CH = Tslu<T>::CH, G = CH / PB;
-    __shared__ ElimLds<T, CH / 64> L;
+    constexpr int CH = 256 * R, G = CH / PB;
+    if (blockIdx.x >= gridDim.x - f.blocks) {
+        far_update<T>(Ar, Ai, ld, n, f, blockIdx.x - (gridDim.x - f.blocks), Ur, Ui);
+        return;
+    }
+    __shared__ ElimLds<T> L;
     const int t = threadIdx.x;
     // level 0: rows j0 + b*CH .. (n - j0 is a multiple of PB, so every set is full)
     const int r0 = j0 + blockIdx.x * CH;
     int nrows = min(CH, n - r0);
-    T xr[PB], xi[PB];
-    if (t < nrows) {
-        load_row(Ar + (long)(r0 + t) * ld + j0, xr);
-        load_row(Ai + (long)(r0 + t) * ld + j0, xi);
+    T xr[R][PB], xi[R][PB];
+    int id[R], src[R], mine[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int i = t + 256 * r;
+        id[r] = src[r] = r0 + i;
+        if (i < nrows) {
+            load_row(Sr + (long)(r0 + i) * lds, xr[r]);
+            load_row(Si + (long)(r0 + i) * lds, xi[r]);
+        }
     }
-    int mine = elim_rows(L, xr, xi, r0 + t, r0 + t, nrows);
     int level_sets = (n - j0 + CH - 1) / CH;  // sets at this level
     int set = blockIdx.x, off = 0, cnt_off = 0;
     bool from_matrix = true;
-    while (level_sets > 1) {
+    for (;;) {
+        if (R > 1 && nrows <= 256) {  // a merge that needs one row per thread
+#pragma unroll
+            for (int r = 1; r < R; r++) mine[r] = -1;
+            elim_rows<T, 1>(L, reinterpret_cast<T(&)[1][PB]>(xr), reinterpret_cast<T(&)[1][PB]>(xi),
+                            reinterpret_cast<const int(&)[1]>(id), reinterpret_cast<const int(&)[1]>(src), nrows,
+                            reinterpret_cast<int(&)[1]>(mine));
+        } else {
+            elim_rows<T, R>(L, xr, xi, id, src, nrows, mine);
+        }
+        if (level_sets <= 1) break;
         // candidate set = original values of the chosen rows
-        for (int e = t; e < PB * PB; e += CH) {
+        for (int e = t; e < PB * PB; e += 256) {
             const int r = e / PB, c = e % PB;
             const long o = ((long)(off + set) * PB + r) * PB + c;
             if (from_matrix) {
-                const long g = (long)L.osrc[r] * ld + j0 + c;
-                cvr[o] = Ar[g];
-                cvi[o] = Ai[g];
+                const long g = (long)L.osrc[r] * lds + c;
+                cvr[o] = Sr[g];
+                cvi[o] = Si[g];
             } else {
                 const long g = (long)L.osrc[r] * PB + c;
                 cvr[o] = cvr[g];
@@ -322,13 +586,17 @@ __global__ __launch_bounds__(Tslu<T>::CH) void k_tslu(const T* __restrict__ Ar, 
         __threadfence();
         const int s0 = off + grp * G;
         nrows = gsize * PB;
-        int id = -1;
-        if (t < nrows) {
-            load_row(cvr + ((long)s0 * PB + t) * PB, xr);
-            load_row(cvi + ((long)s0 * PB + t) * PB, xi);
-            id = cid[s0 * PB + t];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int i = t + 256 * r;
+            id[r] = -1;
+            src[r] = s0 * PB + i;
+            if (i < nrows) {
+                load_row(cvr + ((long)s0 * PB + i) * PB, xr[r]);
+                load_row(cvi + ((long)s0 * PB + i) * PB, xi[r]);
+                id[r] = cid[s0 * PB + i];
+            }
         }
-        mine = elim_rows(L, xr, xi, id, s0 * PB + t, nrows);
         from_matrix = false;
         cnt_off += (level_sets + G - 1) / G;
         off += level_sets;
@@ -338,21 +606,32 @@ __global__ __launch_bounds__(Tslu<T>::CH) void k_tslu(const T* __restrict__ Ar, 
     // root: the factored diagonal block, swaps, row-pair list, zero pivot
     if (t == 0) L.zmin = 0x7fffffff;
     __syncthreads();
-    if (mine >= 0) {
-        store_row(d11r + mine * PB, xr);
-        store_row(d11i + mine * PB, xi);
-        T dr = T(0), di = T(0);
 #pragma unroll
-        for (int c = 0; c < PB; c++)
-            if (c == mine) {
-                dr = xr[c];
-                di = xi[c];
-            }
-        if (dr == T(0) && di == T(0)) atomicMin(&L.zmin, j0 + mine + 1);
-    }
+    for (int r = 0; r < R; r++)
+        if (mine[r] >= 0) {
+            store_row(d11r + mine[r] * PB, xr[r]);
+            store_row(d11i + mine[r] * PB, xi[r]);
+            T dr = T(0), di = T(0);
+#pragma unroll
+            for (int c = 0; c < PB; c++)
+                if (c == mine[r]) {
+                    dr = xr[r][c];
+                    di = xi[r][c];
+                }
+            if (dr == T(0) && di == T(0)) atomicMin(&L.zmin, j0 + mine[r] + 1);
+        }
     __syncthreads();
     if (t == 0 && L.zmin != 0x7fffffff && *info == 0) *info = L.zmin;
-    if (t < 64) root_swaps(L.oid, j0, ipiv, pl);
+    if (t < 64) root_swaps(L.oid, L.sw[0], L.sw[1], j0, ipiv, pl);
+}
+
+constexpr int kWideSetRows = 4096;
+
+// Levels of the tournament over m rows with sets of 256 r rows.
+int tslu_levels(int m, int r) {
+    int l = 1;
+    for (int sets = (m + 256 * r - 1) / (256 * r); sets > 1; sets = (sets + 8 * r - 1) / (8 * r)) l++;
+    return l;
 }
 
 // Applies nl row-pair lists in order (list l at pl + l * PLS, each the net
@@ -403,117 +682,327 @@ __global__ __launch_bounds__(256) void k_laswp(T* __restrict__ Ar, T* __restrict
     }
 }
 
-// Panel step after the swaps, with the factored 32 x 32 diagonal block d11
-// from the tournament.  Block 0 writes d11 in place and forms U12 = L11^{-1}
-// A12 for the nright columns right of the block (one column per thread);
-// blocks >= 1 form L21 = A21 U11^{-1} for 256 rows each (one row per thread).
-// Both substitutions run right-looking with the vector in registers and the
-// triangle streamed from LDS in 16-byte chunks of one row (U) or one column
-// (L, stored transposed), which keeps the kernel near 100 registers so it can
-// share CUs with the trailing-update GEMM.  A zero pivot leaves its column
-// unscaled.
-template <typename T>
-__global__ __launch_bounds__(256) void k_panel(T* __restrict__ Ar, T* __restrict__ Ai, long ld, int j0, int nrows,
-                                               int nright, const T* __restrict__ d11r,
-                                               const T* __restrict__ d11i) {
-    __builtin_amdgcn_s_setprio(3);
+// Triangular solves of the panel steps: a row x of 32 is spread over the four
+// lanes of a quad, lane j holding x[4 k + j] in x[k] (cyclic, so the work stays
+// even to the last column).  The triangle lies in LDS as M[l][j][k] = M_l,4k+j
+// with zeros at and left of the diagonal, so a lane reads its part of row l in
+// 16-byte pieces and needs no mask.
+constexpr int QK = PB / 4;  // elements of a row per lane
+__device__ __forceinline__ int tri_index(int l, int c) { return l * PB + (c & 3) * QK + c / 4; }
+
+// Lane JL's value of each quad.
+template <int JL>
+__device__ __forceinline__ float quad_bcast(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), JL * 0x55, 0xf, 0xf, false));
+}
+template <int JL>
+__device__ __forceinline__ double quad_bcast(double v) {
+    const long long u = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)u, JL * 0x55, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), JL * 0x55, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+template <typename T, int L>
+__device__ __forceinline__ void solve_step(T (&xr)[QK], T (&xi)[QK], const T* mr, const T* mi, bool scale,
+                                           const T* rr, const T* ri) {
     using V = typename Vec16<T>::type;
-    constexpr int E = 16 / sizeof(T);
-    __shared__ __align__(16) T ur[PB][PB], ui[PB][PB];  // U11 (rows)
-    __shared__ __align__(16) T lr[PB][PB], li[PB][PB];  // L11 transposed: lr[l][r] = L[r][l]
-    __shared__ T rr[PB], ri[PB];
-    const int t = threadIdx.x;
-    for (int e = t; e < PB * PB; e += 256) {
-        const int r = e / PB, c = e % PB;
-        ur[r][c] = d11r[e];
-        ui[r][c] = d11i[e];
-        lr[c][r] = d11r[e];
-        li[c][r] = d11i[e];
+    constexpr int E = 16 / sizeof(T), K0 = L / 4, JL = L % 4;
+    const int j = threadIdx.x & 3;
+    if (scale) {
+        const T a = xr[K0], b = xi[K0], sr = rr[L], si = ri[L];
+        xr[K0] = j == JL ? a * sr - b * si : a;
+        xi[K0] = j == JL ? a * si + b * sr : b;
     }
-    if (t < PB) {
-        const T a = d11r[t * PB + t], b = d11i[t * PB + t];
-        if (a == T(0) && b == T(0)) {
-            rr[t] = T(1);
-            ri[t] = T(0);
-        } else {
-            cdiv(T(1), T(0), a, b, rr[t], ri[t]);
+    if constexpr (L < PB - 1) {
+        const T lr = quad_bcast<JL>(xr[K0]), li = quad_bcast<JL>(xi[K0]);
+#pragma unroll
+        for (int k0 = K0 / E * E; k0 < QK; k0 += E) {
+            T ur[E], ui[E];
+            const V a = *reinterpret_cast<const V*>(mr + L * PB + j * QK + k0);
+            const V d = *reinterpret_cast<const V*>(mi + L * PB + j * QK + k0);
+            __builtin_memcpy(ur, &a, 16);
+            __builtin_memcpy(ui, &d, 16);
+#pragma unroll
+            for (int e = 0; e < E; e++) {
+                const int k = k0 + e;
+                if (k < K0) continue;
+                xr[k] = fmadd(-lr, ur[e], xr[k]);
+                xr[k] = fmadd(li, ui[e], xr[k]);
+                xi[k] = fmadd(-lr, ui[e], xi[k]);
+                xi[k] = fmadd(-li, ur[e], xi[k]);
+            }
+        }
+        solve_step<T, L + 1>(xr, xi, mr, mi, scale, rr, ri);
+    }
+}
+
+// Solves x M = x in place for the upper triangle M: x_l is scaled by the
+// reciprocal (rr, ri)[l] of the diagonal when `scale` (else unit diagonal), then
+// x_c -= x_l M_lc for c > l (four fused multiply-adds per element).
+template <typename T>
+__device__ __forceinline__ void solve_tri(T (&xr)[QK], T (&xi)[QK], const T* mr, const T* mi, bool scale, const T* rr,
+                                          const T* ri) {
+    solve_step<T, 0>(xr, xi, mr, mi, scale, rr, ri);
+}
+
+// The 32 columns from c on: the row pairs of a step's list pl (np of them)
+// interchanged in place, one workgroup for all rows, and with u12 the rows j0 ..
+// j0+31 replaced by U12 = L11^{-1} A12 (L11 transposed at lr, li; top: the rows
+// they come from).  Every source is in registers before the first store.
+template <typename T>
+__device__ __forceinline__ void swap_strip(T* __restrict__ Ar, T* __restrict__ Ai, long ld, int j0, int c, bool u12,
+                                           const int* __restrict__ pl, int np, const int* top, const T* lr,
+                                           const T* li) {
+    constexpr int RG = 256 / PB, PER = 2 * PB / RG;  // row groups; pairs per thread
+    const int t = threadIdx.x, tx = t % PB, ty = t / PB, i = t / 4, j = t & 3;
+    T vr[PER], vi[PER], xr[QK], xi[QK];
+    int dst[PER];
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+        const int k = ty + RG * u;
+        dst[u] = -1;
+        if (k < np) {
+            dst[u] = pl[1 + 2 * k];
+            const long o = (long)pl[2 + 2 * k] * ld + c + tx;
+            vr[u] = Ar[o];
+            vi[u] = Ai[o];
+        }
+    }
+    const bool solve = u12 && t < 4 * PB;  // a column per quad of lanes
+    if (solve) {
+#pragma unroll
+        for (int k = 0; k < QK; k++) {
+            const long o = (long)top[4 * k + j] * ld + c + i;
+            xr[k] = Ar[o];
+            xi[k] = Ai[o];
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PER; u++)
+        if (dst[u] >= (u12 ? j0 + PB : 0)) {
+            const long o = (long)dst[u] * ld + c + tx;
+            Ar[o] = vr[u];
+            Ai[o] = vi[u];
+        }
+    if (solve) {
+        solve_tri<T>(xr, xi, lr, li, false, lr, li);
+#pragma unroll
+        for (int k = 0; k < QK; k++) {
+            const long o = (long)(j0 + 4 * k + j) * ld + c + i;
+            Ar[o] = xr[k];
+            Ai[o] = xi[k];
+        }
+    }
+}
+
+// Panel step after the tournament of columns J = j0..j0+31, for 32 rows per
+// workgroup (rows from j0 + 32 on): the step's row interchanges, L21 = A21
+// U11^{-1}, and for the next 32 columns J' (with_next) U12 = L11^{-1} A12 and the
+// rank-32 update, all that the next tournament waits for.
+//
+// Nothing is interchanged in place: a row is read from where the step's
+// row-pair list pl says it comes from.  The columns J are read from S (row i at
+// S + 32 i, a compact copy) and L21 goes to the matrix; the columns J' are read
+// from the matrix and go, updated, to the compact copy D that the next
+// tournament and step read.  U12 of J' goes to U (32 x 32), not over the rows
+// other workgroups still read.  The other columns of the panel follow on
+// another stream.
+//
+// Waves 0 and 1 form L21 (one row per quad of lanes), waves 2 and 3 U12 (one
+// column per quad) at the same time, then each wave multiplies one 16 x 16 tile
+// on the matrix cores (3M in FP32, as the products of the other columns).
+// Latency-bound: the loads that depend on nothing are issued first, and the
+// quads cut the substitution's chain to a quarter of the multiply-adds of a
+// whole row per lane (3840 rows: 10 us for what three launches of 7, 14 and 5 us
+// did).  It needs few enough registers and little
+// enough LDS to start beside the trailing update as soon as one of its
+// workgroups ends.  A zero pivot leaves its column unscaled.
+template <typename T>
+__global__ __launch_bounds__(256) void k_step(T* __restrict__ Ar, T* __restrict__ Ai, long ld,
+                                              const T* __restrict__ Sr, const T* __restrict__ Si, int k0, int j0,
+                                              int n, int with_next, const int* __restrict__ pl,
+                                              const T* __restrict__ d11r, const T* __restrict__ d11i,
+                                              T* __restrict__ Dr, T* __restrict__ Di, T* __restrict__ Ur,
+                                              T* __restrict__ Ui) {
+    __builtin_amdgcn_s_setprio(3);
+    constexpr int SL = PB + 4;  // row stride of L21 and U12 in LDS
+    __shared__ __align__(16) T ur[PB * PB], ui[PB * PB], lr[PB * PB], li[PB * PB];  // U11; L11 transposed
+    __shared__ __align__(16) T pr[PB * SL], pi[PB * SL], vr[PB * SL], vi[PB * SL];  // L21, U12
+    __shared__ T rr[PB], ri[PB];
+    __shared__ int map[PB], top[PB];  // source rows of this workgroup's rows and of rows j0 .. j0+31
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int nrow = max(1, (n - j0 - PB) / PB), strip = (int)blockIdx.x - nrow;  // strip >= 0: other columns
+    const int r0 = j0 + PB + blockIdx.x * PB;
+    const int np = pl[0];
+    int2 pair = make_int2(-1, -1);
+    if (t < 2 * PB) pair = make_int2(pl[1 + 2 * t], pl[2 + 2 * t]);  // beyond np: not used
+    T da[4], db[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        da[u] = d11r[t + 256 * u];
+        db[u] = d11i[t + 256 * u];
+    }
+    if (t < PB)
+        map[t] = min(r0 + t, n - 1);
+    else if (t < 2 * PB)
+        top[t - PB] = j0 + t - PB;
+    __syncthreads();
+    if (t < np) {  // np <= 2 PB
+        if (pair.x < j0 + PB)
+            top[pair.x - j0] = pair.y;
+        else if (strip < 0 && pair.x >= r0 && pair.x < r0 + PB)
+            map[pair.x - r0] = pair.y;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int e = t + 256 * u, r = e / PB, c = e % PB;
+        const T a = da[u], b = db[u];
+        ur[tri_index(r, c)] = c > r ? a : T(0);
+        ui[tri_index(r, c)] = c > r ? b : T(0);
+        lr[tri_index(c, r)] = r > c ? a : T(0);
+        li[tri_index(c, r)] = r > c ? b : T(0);
+        if (r == c) {
+            if (a == T(0) && b == T(0)) {
+                rr[r] = T(1);
+                ri[r] = T(0);
+            } else {
+                cdiv(T(1), T(0), a, b, rr[r], ri[r]);
+            }
+        }
+        if (blockIdx.x == 0) {
+            Ar[(long)(j0 + r) * ld + j0 + c] = a;
+            Ai[(long)(j0 + r) * ld + j0 + c] = b;
         }
     }
     __syncthreads();
-    // x_c -= s * M[l][c] for c > l (four fused multiply-adds per element),
-    // row l of M streamed from LDS
-    auto eliminate = [&](T (&xr)[PB], T (&xi)[PB], const T (*mr)[PB], const T (*mi)[PB], int l, T sr, T si) {
-        const V* vr = reinterpret_cast<const V*>(&mr[l][0]);
-        const V* vi = reinterpret_cast<const V*>(&mi[l][0]);
-        const T nsr = -sr, nsi = -si;
-#pragma unroll
-        for (int q = 0; q < PB / E; q++) {
-            if (q * E + E - 1 <= l) continue;
-            T a[E], b[E];
-            const V x = vr[q], y = vi[q];
-            __builtin_memcpy(a, &x, 16);
-            __builtin_memcpy(b, &y, 16);
-#pragma unroll
-            for (int e = 0; e < E; e++) {
-                const int c = q * E + e;
-                if (c > l) {
-                    xr[c] = fmadd(nsr, a[e], xr[c]);
-                    xr[c] = fmadd(si, b[e], xr[c]);
-                    xi[c] = fmadd(nsr, b[e], xi[c]);
-                    xi[c] = fmadd(nsi, a[e], xi[c]);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-    if (blockIdx.x == 0) {
-        for (int e = t; e < PB * PB; e += 256) {
-            const int r = e / PB, c = e % PB;
-            Ar[(long)(j0 + r) * ld + j0 + c] = ur[r][c];
-            Ai[(long)(j0 + r) * ld + j0 + c] = ui[r][c];
-        }
-        // Row r of the strip at a block-uniform address, the column as a
-        // 32-bit offset; the store addresses are formed anew after the
-        // substitution (the empty asm hides the offset from common-
-        // subexpression elimination), else the 64 per-thread 64-bit load
-        // addresses stay live across it (222 instead of ~100 registers).
-        T* __restrict__ sr0 = Ar + (long)j0 * ld + j0 + PB;
-        T* __restrict__ si0 = Ai + (long)j0 * ld + j0 + PB;
-        for (int c = t; c < nright; c += 256) {
-            T xr[PB], xi[PB];
-#pragma unroll
-            for (int r = 0; r < PB; r++) {
-                xr[r] = (sr0 + r * ld)[(unsigned)c];
-                xi[r] = (si0 + r * ld)[(unsigned)c];
-            }
-#pragma clang loop unroll(full)
-            for (int l = 0; l < PB - 1; l++) eliminate(xr, xi, lr, li, l, xr[l], xi[l]);  // unit lower
-            unsigned cs = (unsigned)c;
-            asm volatile("" : "+v"(cs));
-#pragma unroll
-            for (int r = 0; r < PB; r++) {
-                (sr0 + r * ld)[cs] = xr[r];
-                (si0 + r * ld)[cs] = xi[r];
-            }
-        }
+    if (strip >= 0) {
+        const int nleft = (j0 - k0) / PB;
+        const bool left = strip < nleft;
+        swap_strip<T>(Ar, Ai, ld, j0, left ? k0 + strip * PB : j0 + 2 * PB + (strip - nleft) * PB, !left, pl, np, top,
+                      lr, li);
         return;
     }
-    const int row = j0 + PB + (blockIdx.x - 1) * 256 + t;
-    if (row >= j0 + nrows) return;
-    T xr[PB], xi[PB];
-    T* pr = Ar + (long)row * ld + j0;
-    T* pi = Ai + (long)row * ld + j0;
-    load_row(pr, xr);
-    load_row(pi, xi);
-#pragma clang loop unroll(full)  // a partial unroll indexes the row registers at run time
-    for (int l = 0; l < PB; l++) {
-        const T a = xr[l], b = xi[l];
-        xr[l] = a * rr[l] - b * ri[l];  // x_l / U[l][l]
-        xi[l] = a * ri[l] + b * rr[l];
-        if (l < PB - 1) eliminate(xr, xi, ur, ui, l, xr[l], xi[l]);
+    const bool rows = wave < 2;
+    const int i = (wave & 1) * 16 + lane / 4, j = lane & 3;  // row of L21 or column of U12; part of it
+    const int r16 = lane & 15, g = lane >> 4, m0 = (wave >> 1) * 16, n0 = (wave & 1) * 16;
+    const bool inside = r0 < n;  // n - r0 is a multiple of 32
+    T xr[QK], xi[QK];
+    if (rows) {
+        const long o = (long)map[i] * PB + j;
+#pragma unroll
+        for (int k = 0; k < QK; k++) {
+            xr[k] = Sr[o + 4 * k];
+            xi[k] = Si[o + 4 * k];
+        }
+    } else if (with_next) {
+#pragma unroll
+        for (int k = 0; k < QK; k++) {
+            const long o = (long)top[4 * k + j] * ld + j0 + PB + i;
+            xr[k] = Ar[o];
+            xi[k] = Ai[o];
+        }
     }
-    store_row(pr, xr);
-    store_row(pi, xi);
+    // this wave's 16 x 16 tile of J' before the update: FP32 row m0 + r16,
+    // columns n0 + 4 g .. + 3; FP64 rows m0 + g + 4 q, column n0 + r16
+    typedef typename std::conditional<sizeof(T) == 4, v4f, v4d>::type acc_t;
+    acc_t cr{}, ci{};
+    if (with_next) {
+        if constexpr (sizeof(T) == 4) {
+            const long o = (long)map[m0 + r16] * ld + j0 + PB + n0 + 4 * g;
+            cr = *reinterpret_cast<const v4f*>(Ar + o);
+            ci = *reinterpret_cast<const v4f*>(Ai + o);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const long o = (long)map[m0 + g + 4 * q] * ld + j0 + PB + n0 + r16;
+                cr[q] = Ar[o];
+                ci[q] = Ai[o];
+            }
+        }
+    }
+    if (rows || with_next) solve_tri<T>(xr, xi, rows ? ur : lr, rows ? ui : li, rows, rr, ri);
+    if (rows) {
+        if (inside) {
+            const long o = (long)(r0 + i) * ld + j0 + j;
+#pragma unroll
+            for (int k = 0; k < QK; k++) {
+                Ar[o + 4 * k] = xr[k];
+                Ai[o + 4 * k] = xi[k];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < QK; k++) {
+            pr[i * SL + 4 * k + j] = xr[k];
+            pi[i * SL + 4 * k + j] = xi[k];
+        }
+    } else if (with_next) {
+#pragma unroll
+        for (int k = 0; k < QK; k++) {
+            vr[(4 * k + j) * SL + i] = xr[k];
+            vi[(4 * k + j) * SL + i] = xi[k];
+            if (blockIdx.x == 0) {
+                Ur[(4 * k + j) * PB + i] = xr[k];
+                Ui[(4 * k + j) * PB + i] = xi[k];
+            }
+        }
+    }
+    if (!with_next || !inside) return;
+    __syncthreads();
+    if constexpr (sizeof(T) == 4) {
+        v4f t1 = v4f{0.f, 0.f, 0.f, 0.f}, t2 = t1, t3 = t1;
+#pragma unroll
+        for (int q = 0; q < PB / 16; q++) {
+            const v4f a0 = *reinterpret_cast<const v4f*>(pr + (m0 + r16) * SL + 16 * q + 4 * g);
+            const v4f a1 = *reinterpret_cast<const v4f*>(pi + (m0 + r16) * SL + 16 * q + 4 * g);
+            const v4f a2 = a0 + a1;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int o = (16 * q + 4 * g + e) * SL + n0 + r16;
+                const float b0 = vr[o], b1 = vi[o];
+                t1 = mfma16x16x4(b0, a0[e], t1);
+                t2 = mfma16x16x4(b1, a1[e], t2);
+                t3 = mfma16x16x4(b0 + b1, a2[e], t3);
+            }
+        }
+        const long o = (long)(r0 + m0 + r16) * PB + n0 + 4 * g;
+        *reinterpret_cast<v4f*>(Dr + o) = cr - (t1 - t2);
+        *reinterpret_cast<v4f*>(Di + o) = ci - (t3 - t1 - t2);
+    } else {
+        v4d re{}, im{};
+#pragma unroll
+        for (int q = 0; q < PB / 4; q++) {
+            const int k = 4 * q + g;
+            const T a0 = pr[(m0 + r16) * SL + k], a1 = pi[(m0 + r16) * SL + k];
+            const T b0 = vr[k * SL + n0 + r16], b1 = vi[k * SL + n0 + r16];
+            re = mfma16x16x4(a0, b0, re);
+            re = mfma16x16x4(a1, -b1, re);
+            im = mfma16x16x4(a0, b1, im);
+            im = mfma16x16x4(a1, b0, im);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const long o = (long)(r0 + m0 + g + 4 * q) * PB + n0 + r16;
+            Dr[o] = cr[q] - re[q];
+            Di[o] = ci[q] - im[q];
+        }
+    }
+}
+
+// The first 32 columns of an outer panel, rows [k0, n), into the compact copy D
+// (row i at D + 32 i).
+template <typename T>
+__global__ __launch_bounds__(256) void k_compact(const T* __restrict__ Ar, const T* __restrict__ Ai, long ld, int k0,
+                                                 int n, T* __restrict__ Dr, T* __restrict__ Di) {
+    using V = typename Vec16<T>::type;
+    constexpr int E = 16 / sizeof(T), W = PB / E;
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    const int i = k0 + e / W, q = (e % W) * E;
+    if (i >= n) return;
+    *reinterpret_cast<V*>(Dr + (long)i * PB + q) = *reinterpret_cast<const V*>(Ar + (long)i * ld + k0 + q);
+    *reinterpret_cast<V*>(Di + (long)i * PB + q) = *reinterpret_cast<const V*>(Ai + (long)i * ld + k0 + q);
 }
 
 template <typename T>
@@ -561,7 +1050,9 @@ struct LuWork {
     int* cid;        // candidate row ids
     T *cvr, *cvi;    // candidate values
     int* pl;         // row-pair lists of the 8 steps of an outer panel (PLS ints each), two sets
-    T *d11r, *d11i;  // factored 32 x 32 diagonal block
+    T* d11;          // factored 32 x 32 diagonal block (2 planes), two sets by step parity
+    T *cpr, *cpi;    // compact copies (n x 32 per plane) of the columns being factored, two sets by step parity
+    T *sur, *sui;    // U12 of the next 32 columns (32 x 32)
     T *ubr, *ubi;    // 256 x n U12 buffer
     T *utr, *uti;    // n x 256 transpose of U12 (FP32 trailing update)
     T *tr, *ti;      // 128 x 128 product of the L11^{-1} doubling
@@ -624,51 +1115,53 @@ void invert_lower_doubling(hipStream_t s, const T* Fr, const T* Fi, long ldf, T*
 }
 
 // Factors the outer panel of columns k0 .. k0+NB-1 (rows k0 .. n-1) on stream
-// s: 8 steps of tournament, swaps within the panel's columns, L21/U12 of the
-// step and the rank-32 update of the panel's remaining columns.  The swaps of
-// step j are kept as row-pair list j for the columns outside the panel.
-// Look-ahead inside the panel: the rank-32 update of the next 32 columns
-// stays on s (the next tournament needs them); the update of the columns
-// beyond runs on stream ss and is joined before the next step's swaps, so
-// every column still receives its updates in step order.
+// s: 8 steps of 32 columns, two launches each.  k_step finishes the step's own
+// columns, the next 32 and the swaps of the others; the rank-32 update of the
+// columns beyond the next 32 rides in the launch of the next tournament, which
+// does not need them.  (With that update and the other columns' swaps on a third
+// stream, behind an event each way, and the next 32 columns' swaps, panel solve
+// and update as three launches a step took 115 us at 3840 rows; now 75.)  The
+// swaps of step j are kept as row-pair list j for the columns outside the panel.
+// The FP32 tournament takes sets of 512 rows where they save a level: a set costs
+// 29 us of elimination instead of 19 for 256 rows, a level of merges ~23 (3840
+// rows: 58.7 against 73.1 us, 12288 rows, which save none: 91.9 against 80.6).
+// Up to kWideSetRows only: with two rows per thread the kernel does not start
+// beside the trailing update until a whole CU is free.  In FP64 two rows per
+// thread do not fit the registers.
 template <typename T>
-void factor_panel(bem_ctx* c, hipStream_t s, hipStream_t ss, T* Ar, T* Ai, int k0, const LuWork<T>& w) {
+void factor_panel(bem_ctx* c, hipStream_t s, T* Ar, T* Ai, int k0, const LuWork<T>& w) {
     const int n = c->npad;
-    const long ld = n;
-    hipEvent_t e_step = c->lu_ev[4], e_rest = c->lu_ev[5];
-    bool rest_pending = false;
-    for (int j0 = k0; j0 < k0 + NB; j0 += PB) {
-        const int m = n - j0;
-        const int nsets = (m + Tslu<T>::CH - 1) / Tslu<T>::CH;
+    const long ld = n, cp = (long)n * PB;
+    const int k1 = k0 + NB, first = ((n - k0) * (PB * (int)sizeof(T) / 16) + 255) / 256;
+    int kt = kt_mark(c, KS_OTHER, s);
+    hipLaunchKernelGGL(k_compact<T>, dim3(first), dim3(256), 0, s, Ar, Ai, ld, k0, n, w.cpr, w.cpi);
+    kt_close(c, kt, 0.0, 4.0 * sizeof(T) * (double)(n - k0) * PB);
+    FarUpdate far{0, 0, 0, 0};
+    for (int j0 = k0; j0 < k1; j0 += PB) {
+        const int m = n - j0, par = ((j0 - k0) / PB) & 1;
+        T *Sr = w.cpr + par * cp, *Si = w.cpi + par * cp;
+        T *Dr = w.cpr + (par ^ 1) * cp, *Di = w.cpi + (par ^ 1) * cp;
+        T *d11r = w.d11 + par * 2 * PB * PB, *d11i = d11r + PB * PB;
         int* pl = panel_lists(w, k0) + ((j0 - k0) / PB) * PLS;
-        int kt = kt_mark(c, KS_TSLU, s);
-        hipLaunchKernelGGL(k_tslu<T>, dim3(nsets), dim3(Tslu<T>::CH), 0, s, Ar, Ai, ld, j0, n, w.cid, w.cvr, w.cvi, w.cnt,
-                           c->ipiv, pl, w.d11r, w.d11i, w.info);
-        kt_close(c, kt, 0.0, 2.0 * sizeof(T) * (double)m * PB);
-        if (rest_pending) {  // the previous step's update of the far columns
-            (void)hipStreamWaitEvent(s, e_rest, 0);
-            rest_pending = false;
-        }
-        launch_laswp<T>(c, s, Ar, Ai, ld, k0, k0 + NB, 0, 0, pl, 1);
-        const int nright = k0 + NB - (j0 + PB);
-        const int nblk = 1 + (m - PB + 255) / 256;
-        kt = kt_mark(c, KS_PANEL, s);
-        hipLaunchKernelGGL(k_panel<T>, dim3(nblk), dim3(256), 0, s, Ar, Ai, ld, j0, m, nright, w.d11r, w.d11i);
-        kt_close(c, kt, 4.0 * (double)m * PB * PB, 4.0 * sizeof(T) * (double)m * PB);
-        if (nright > 0) {
-            const long o21 = (long)(j0 + PB) * ld + j0, o12 = (long)j0 * ld + j0 + PB;
-            const long o22 = (long)(j0 + PB) * ld + j0 + PB;
-            if (nright > PB) {
-                (void)hipEventRecord(e_step, s);  // L21 and U12 of this step are in place
-                (void)hipStreamWaitEvent(ss, e_step, 0);
-                cgemm_ctx<T>(c, m - PB, nright - PB, PB, Ar + o21, Ai + o21, ld, Ar + o12 + PB, Ai + o12 + PB, ld,
-                             Ar + o22 + PB, Ai + o22 + PB, ld, 0, ss, GEMM_PANEL);
-                (void)hipEventRecord(e_rest, ss);
-                rest_pending = true;
+        kt = kt_mark(c, KS_TSLU, s);
+        auto tslu = k_tslu<T, 1>;
+        int set = 256;
+        if constexpr (sizeof(T) == 4)
+            if (m <= kWideSetRows && tslu_levels(m, 2) < tslu_levels(m, 1)) {
+                tslu = k_tslu<T, 2>;
+                set = 512;
             }
-            cgemm_ctx<T>(c, m - PB, PB, PB, Ar + o21, Ai + o21, ld, Ar + o12, Ai + o12, ld, Ar + o22, Ai + o22, ld, 0,
-                         s, GEMM_PANEL);
-        }
+        hipLaunchKernelGGL(tslu, dim3((m + set - 1) / set + far.blocks), dim3(256), 0, s, Sr, Si, (long)PB, j0, n,
+                           w.cid, w.cvr, w.cvi, w.cnt, c->ipiv, pl, d11r, d11i, w.info, Ar, Ai, ld, far, w.sur, w.sui);
+        kt_close(c, kt, (sizeof(T) == 4 ? 6.0 : 8.0) * far.ncol * (double)m * PB,
+                 2.0 * sizeof(T) * (double)m * (PB + 2 * far.ncol));
+        const int next = j0 + PB < k1, others = NB / PB - 1 - next;
+        kt = kt_mark(c, KS_PANEL, s);
+        hipLaunchKernelGGL(k_step<T>, dim3(std::max(1, (m - PB) / PB) + others), dim3(256), 0, s, Ar, Ai, ld, Sr, Si,
+                           k0, j0, n, next, pl, d11r, d11i, Dr, Di, w.sur, w.sui);
+        kt_close(c, kt, (next ? 10.0 : 4.0) * (double)m * PB * PB, (next ? 8.0 : 4.0) * sizeof(T) * (double)m * PB);
+        const int c0 = std::min(k1, j0 + 2 * PB), ncol = k1 - c0;  // columns beyond the next 32
+        far = FarUpdate{j0, c0, ncol, next ? ((m - PB) / 16 * (ncol / 16) + 3) / 4 + 1 : 0};
     }
 }
 
@@ -733,13 +1226,13 @@ template <typename T>
 void factor(bem_ctx* c, T* Ar, T* Ai, T* Lir, T* Lii, T* Uir, T* Uii, const LuWork<T>& w) {
     const int n = c->npad, nb = n / NB;
     const long ld = n;
-    hipStream_t us = c->stream, ps = c->stream2, ss = c->stream3;
-    if (c->lu_streams == 0) ps = ss = us;
+    hipStream_t us = c->stream, ps = c->stream2;
+    if (c->lu_streams == 0) ps = us;
     hipEvent_t e_panel = c->lu_ev[0], e_next = c->lu_ev[1], e_start = c->lu_ev[2], e_linv = c->lu_ev[3];
     (void)hipEventRecord(e_start, c->stream);  // the matrix and work buffers are ready
     (void)hipStreamWaitEvent(ps, e_start, 0);
     if (us != c->stream) (void)hipStreamWaitEvent(us, e_start, 0);
-    factor_panel<T>(c, ps, ss, Ar, Ai, 0, w);
+    factor_panel<T>(c, ps, Ar, Ai, 0, w);
     for (int K = 0; K < nb; K++) {
         const int k0 = K * NB;
         const int nr = n - (k0 + NB);
@@ -770,7 +1263,7 @@ void factor(bem_ctx* c, T* Ar, T* Ai, T* Lir, T* Lii, T* Uir, T* Uii, const LuWo
         launch_laswp<T>(c, us, Ar, Ai, ld, 0, k0, k0 + 2 * NB, n, panel_lists(w, k0), NB / PB);
         if (nr > NB)
             update_columns<T>(c, us, Ar, Ai, Lir, Lii, k0, k0 + 2 * NB, nr - NB, w, ps != us && c->gemm_plan[sizeof(T) == 4 ? 0 : 1].cap > 0);
-        factor_panel<T>(c, ps, ss, Ar, Ai, k0 + NB, w);
+        factor_panel<T>(c, ps, Ar, Ai, k0 + NB, w);
     }
     // U^{-1} of all diagonal blocks in one launch (FP32; the FP64 solves
     // substitute with the diagonal blocks themselves)
@@ -809,13 +1302,13 @@ int factor_prec(bem_ctx* c, T* Ar, T* Ai, void*& inv, size_t& inv_bytes) {
     T* Uir = with_inv ? Lii + (size_t)n * NB : nullptr;
     T* Uii = with_inv ? Uir + (size_t)n * NB : nullptr;
     // work: info, counters, row-pair list, candidate ids, candidate values,
-    // diagonal block, U12 buffer
-    const int nsets0 = (n + Tslu<T>::CH - 1) / Tslu<T>::CH;
+    // diagonal blocks, compact columns, U12 buffers
+    const int nsets0 = (n + 255) / 256;
     const size_t ncnt = 2 * (size_t)nsets0 + 64;
     const size_t nint = 64 + ncnt + 2 * (NB / PB) * PLS + 2 * (size_t)nsets0 * PB;
     const size_t bytes = nint * sizeof(int) + 256 + 4 * (size_t)nsets0 * PB * PB * sizeof(T) +
-                         2 * (size_t)PB * PB * sizeof(T) + 4 * (size_t)NB * n * sizeof(T) +
-                         2 * (size_t)(NB / 2) * (NB / 2) * sizeof(T) + 256;
+                         6 * (size_t)PB * PB * sizeof(T) + 4 * (size_t)NB * n * sizeof(T) +
+                         2 * (size_t)(NB / 2) * (NB / 2) * sizeof(T) + 4 * (size_t)PB * n * sizeof(T) + 256;
     void* scr = nullptr;
     if (int rc = ctx_scratch(c, bytes, &scr)) return rc;
     LuWork<T> w;
@@ -827,9 +1320,12 @@ int factor_prec(bem_ctx* c, T* Ar, T* Ai, void*& inv, size_t& inv_bytes) {
     p += (256 - reinterpret_cast<uintptr_t>(p) % 256) % 256;
     w.cvr = reinterpret_cast<T*>(p);
     w.cvi = w.cvr + 2 * (size_t)nsets0 * PB * PB;
-    w.d11r = w.cvi + 2 * (size_t)nsets0 * PB * PB;
-    w.d11i = w.d11r + PB * PB;
-    w.ubr = w.d11i + PB * PB;
+    w.d11 = w.cvi + 2 * (size_t)nsets0 * PB * PB;
+    w.sur = w.d11 + 4 * PB * PB;
+    w.sui = w.sur + PB * PB;
+    w.cpr = w.sui + PB * PB;
+    w.cpi = w.cpr + 2 * (size_t)PB * n;
+    w.ubr = w.cpi + 2 * (size_t)PB * n;
     w.ubi = w.ubr + (size_t)NB * n;
     w.utr = w.ubi + (size_t)NB * n;
     w.uti = w.utr + (size_t)NB * n;
