@@ -137,6 +137,7 @@ struct bem_ctx {
     // factorisation stream layout (see factor() in kernels/lu.hip): 0 one
     // stream, 1 panel + update streams on all CUs
     int lu_streams = -1;            // -1: not chosen yet
+    bool lu_streams_checked = false;  // the two streams run side by side (or nothing better was found)
     hipEvent_t ev[2] = {nullptr, nullptr};
     hipEvent_t lu_ev[4] = {};  // cross-stream ordering inside the factorisation
     std::string err;
@@ -266,8 +267,9 @@ int gemm_set_plan(bem_ctx* c, int prec, int large, int skinny, long cap);
 void gemm_cache_store(bem_ctx* c, bool f32);
 // Fills cus and occ of the plan of one precision from the device (no timing).
 void gemm_plan_occupancy(bem_ctx* c, bool f32);
-// Chooses the factorisation stream layout (environment BEM_LU_STREAMS,
-// BEM_LU_PANEL_CUS) and creates the CU-masked streams it needs.
+// Chooses the factorisation stream layout (environment BEM_LU_STREAMS) and, once
+// a system is large enough to gain, a panel stream that runs beside the context
+// stream.
 int lu_setup_streams(bem_ctx* c);
 // One copy kernel of n16 16-byte vectors between two fresh device buffers.
 int device_copy_launch(bem_ctx* c, size_t n16);

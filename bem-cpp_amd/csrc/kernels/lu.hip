@@ -1340,13 +1340,66 @@ int factor_prec(bem_ctx* c, T* Ar, T* Ai, void*& inv, size_t& inv_bytes) {
 
 }  // namespace
 
+namespace {
+
+// Notes the time at its start and end in at[0], at[1] and lasts `ticks` of the
+// constant clock (bounded besides by the number of looks at it).
+__global__ void k_interval(long long ticks, long long* at) {
+    const long long t0 = wall_clock64();
+    long long t1 = t0;
+    for (int i = 0; i < 100000 && t1 - t0 < ticks; i++) {
+        __builtin_amdgcn_s_sleep(8);
+        t1 = wall_clock64();
+    }
+    at[0] = t0;
+    at[1] = t1;
+}
+
+// Whether kernels of the two streams run side by side.
+bool streams_overlap(hipStream_t a, hipStream_t b, long long* at, long long ticks) {
+    long long h[4] = {0, 0, 0, 0};
+    for (int warm = 1; warm >= 0; warm--) {  // a stream's first launch can take long
+        hipLaunchKernelGGL(k_interval, dim3(1), dim3(1), 0, a, warm ? 0 : ticks, at);
+        hipLaunchKernelGGL(k_interval, dim3(1), dim3(1), 0, b, warm ? 0 : ticks, at + 2);
+        if (hipStreamSynchronize(a) != hipSuccess || hipStreamSynchronize(b) != hipSuccess) return true;
+    }
+    if (hipMemcpy(h, at, sizeof(h), hipMemcpyDeviceToHost) != hipSuccess) return true;
+    return h[0] < h[3] && h[2] < h[1];
+}
+
+}  // namespace
+
+// The panel stream has to run beside the context stream.  The runtime spreads a
+// process's streams over a few hardware queues (four by default) by their load,
+// and two streams of one queue run one after the other: a second context's pair
+// can end on one (the factorisation at n = 18432 then takes 176 instead of 141
+// ms).  So the first factorisation large enough to gain looks whether the two
+// overlap (~0.1 ms) and otherwise takes another panel stream.
 int lu_setup_streams(bem_ctx* c) {
-    if (c->lu_streams >= 0) return 0;
     // (A layout with the panel stream on CUs reserved by a CU mask ended in a
     // host-side crash in its first run, cause not established; it was removed.)
-    const char* e1 = std::getenv("BEM_LU_STREAMS");
-    const int mode = e1 ? std::atoi(e1) : 1;
-    c->lu_streams = mode == 0 ? 0 : 1;
+    if (c->lu_streams < 0) {
+        const char* e1 = std::getenv("BEM_LU_STREAMS");
+        c->lu_streams = e1 && std::atoi(e1) == 0 ? 0 : 1;
+    }
+    constexpr int kOverlapMinN = 2048, kTries = 4;
+    if (c->lu_streams == 0 || c->lu_streams_checked || c->npad < kOverlapMinN) return 0;
+    c->lu_streams_checked = true;
+    void* scr = nullptr;
+    if (int rc = ctx_scratch(c, 4 * sizeof(long long), &scr)) return rc;
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c->device) != hipSuccess || khz <= 0) return 0;
+    const long long ticks = khz / 25;  // 40 us
+    hipStream_t tried[kTries] = {};
+    for (int i = 0; i < kTries && !streams_overlap(c->stream, c->stream2, static_cast<long long*>(scr), ticks); i++) {
+        hipStream_t other = nullptr;
+        if (hipStreamCreateWithFlags(&other, hipStreamNonBlocking) != hipSuccess) break;
+        tried[i] = c->stream2;  // kept until the end: its queue stays the more loaded one
+        c->stream2 = other;
+    }
+    for (hipStream_t s : tried)
+        if (s) (void)hipStreamDestroy(s);
+    (void)hipGetLastError();
     return 0;
 }
 
