@@ -215,8 +215,7 @@ bem_ctx* bem_create(int device) {
         hipEventCreate(&c->ev[0]) != hipSuccess || hipEventCreate(&c->ev[1]) != hipSuccess ||
         hipEventCreateWithFlags(&c->lu_ev[0], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->lu_ev[1], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->lu_ev[2], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->lu_ev[3], hipEventDisableTiming) != hipSuccess) {
+        hipEventCreateWithFlags(&c->lu_ev[2], hipEventDisableTiming) != hipSuccess) {
         for (hipEvent_t e : {c->ev[0], c->ev[1]})
             if (e) (void)hipEventDestroy(e);
         for (hipEvent_t e : c->lu_ev)

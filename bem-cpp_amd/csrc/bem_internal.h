@@ -97,7 +97,7 @@ struct KernelTimer {
 struct GemmPlan {
     static constexpr int kMaxCfgs = 5;
     int large = 0, skinny = 2;
-    int panel = 3;                           // products of the panel stream (smallest LDS footprint)
+    int panel = 3;                           // kept for saved plans: no product asks for it any more
     int nt = 0;                              // FP32 trailing update: configuration of k_cupdate_nt
     long fill = 512;
     bool tuned = false;
@@ -139,7 +139,7 @@ struct bem_ctx {
     int lu_streams = -1;            // -1: not chosen yet
     bool lu_streams_checked = false;  // the two streams run side by side (or nothing better was found)
     hipEvent_t ev[2] = {nullptr, nullptr};
-    hipEvent_t lu_ev[4] = {};  // cross-stream ordering inside the factorisation
+    hipEvent_t lu_ev[3] = {};  // cross-stream ordering inside the factorisation
     std::string err;
 
     // mesh and basis (host copies)

@@ -56,6 +56,10 @@ struct Vec16<double> {
     using type = double2;
 };
 
+// The same as a native vector (arrays of it stay in registers).
+template <typename T>
+using Nat16 = T __attribute__((ext_vector_type(16 / sizeof(T))));
+
 // PB consecutive values at p (16-byte aligned) <-> registers.
 template <typename T>
 __device__ __forceinline__ void load_row(const T* __restrict__ p, T (&x)[PB]) {
@@ -634,53 +638,7 @@ int tslu_levels(int m, int r) {
     return l;
 }
 
-// Applies nl row-pair lists in order (list l at pl + l * PLS, each the net
-// effect of one panel step's swaps, at most 2 PB pairs) to the columns
-// [ca, cb) and [cc, cd).  A block owns 32 columns and 8 row groups; each
-// thread reads the sources of its pairs of a list into registers (all loads
-// in flight together), the block synchronises, and the thread writes them to
-// the destinations, so every source is read before any destination of the
-// list is written.  No LDS, so the kernel fits beside a running GEMM.
 constexpr int PLS = 256;  // ints per row-pair list
-constexpr int LASWP_COLS = 32;
-template <typename T>
-__global__ __launch_bounds__(256) void k_laswp(T* __restrict__ Ar, T* __restrict__ Ai, long ld, int ca, int cb, int cc,
-                                               int cd, const int* __restrict__ pl, int nl) {
-    __builtin_amdgcn_s_setprio(3);
-    constexpr int RG = 256 / LASWP_COLS;  // row groups
-    constexpr int PER = 2 * PB / RG;      // pairs per thread and list
-    const int tx = threadIdx.x % LASWP_COLS, ty = threadIdx.x / LASWP_COLS;
-    const int v = blockIdx.x * LASWP_COLS + tx;  // virtual column over both ranges
-    const int w1 = cb - ca;
-    const int c = v < w1 ? ca + v : cc + (v - w1);
-    const bool ok = v < w1 + (cd - cc);
-    for (int l = 0; l < nl; l++) {
-        const int* q = pl + l * PLS;
-        const int np = q[0];
-        if (np == 0) continue;
-        T vr[PER], vi[PER];
-#pragma unroll
-        for (int u = 0; u < PER; u++) {
-            const int k = ty + RG * u;
-            if (ok && k < np) {
-                const long o = (long)q[2 + 2 * k] * ld + c;
-                vr[u] = Ar[o];
-                vi[u] = Ai[o];
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < PER; u++) {
-            const int k = ty + RG * u;
-            if (ok && k < np) {
-                const long o = (long)q[1 + 2 * k] * ld + c;
-                Ar[o] = vr[u];
-                Ai[o] = vi[u];
-            }
-        }
-        __syncthreads();
-    }
-}
 
 // Triangular solves of the panel steps: a row x of 32 is spread over the four
 // lanes of a quad, lane j holding x[4 k + j] in x[k] (cyclic, so the work stays
@@ -757,17 +715,19 @@ __device__ __forceinline__ void swap_strip(T* __restrict__ Ar, T* __restrict__ A
     constexpr int RG = 256 / PB, PER = 2 * PB / RG;  // row groups; pairs per thread
     const int t = threadIdx.x, tx = t % PB, ty = t / PB, i = t / 4, j = t & 3;
     T vr[PER], vi[PER], xr[QK], xi[QK];
-    int dst[PER];
+    int dst[PER], src[PER];  // unconditional loads stay in flight together
 #pragma unroll
     for (int u = 0; u < PER; u++) {
-        const int k = ty + RG * u;
-        dst[u] = -1;
-        if (k < np) {
-            dst[u] = pl[1 + 2 * k];
-            const long o = (long)pl[2 + 2 * k] * ld + c + tx;
-            vr[u] = Ar[o];
-            vi[u] = Ai[o];
-        }
+        dst[u] = pl[1 + 2 * (ty + RG * u)];
+        src[u] = pl[2 + 2 * (ty + RG * u)];
+    }
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+        const bool in = ty + RG * u < np;
+        dst[u] = in ? dst[u] : -1;
+        const long o = (long)(in ? src[u] : j0) * ld + c + tx;
+        vr[u] = Ar[o];
+        vi[u] = Ai[o];
     }
     const bool solve = u12 && t < 4 * PB;  // a column per quad of lanes
     if (solve) {
@@ -798,6 +758,58 @@ __device__ __forceinline__ void swap_strip(T* __restrict__ Ar, T* __restrict__ A
     }
 }
 
+// The net effect of an outer panel's row interchanges: net[i] (i < NB) is the
+// row that ends in row k0 + i, net[NB] the number of (destination, source) pairs
+// that follow for the rows below the panel's top NB (at most NB of them).
+constexpr int NETS = 3 * NB + 64;  // ints per net list
+
+// Composes the NB / PB row-pair lists of a panel (list l at pl + l PLS, applied in
+// order) into net: the last list with a row as destination names its source, whose
+// content before that list is followed through the earlier lists.  One workgroup.
+__device__ void compose_lists(const int* __restrict__ pl, int k0, int* __restrict__ net, int2 (*list)[2 * PB],
+                              int* top, int* count) {
+    constexpr int NL = NB / PB;
+    const int t = threadIdx.x;
+    int np[NL];
+#pragma unroll
+    for (int l = 0; l < NL; l++) np[l] = pl[l * PLS];
+#pragma unroll
+    for (int u = 0; u < NL * 2 * PB / 256; u++) {
+        const int e = t + 256 * u, l = e / (2 * PB), k = e % (2 * PB);
+        list[l][k] = make_int2(pl[l * PLS + 1 + 2 * k], pl[l * PLS + 2 + 2 * k]);  // beyond np: not used
+    }
+    top[t] = k0 + t;
+    if (t == 0) *count = 0;
+    __syncthreads();
+#pragma unroll 1
+    for (int u = 0; u < NL * 2 * PB / 256; u++) {
+        const int e = t + 256 * u, l = __builtin_amdgcn_readfirstlane(e / (2 * PB)), k = e % (2 * PB);
+        if (k >= np[l]) continue;
+        const int2 p = list[l][k];
+        bool last = true;
+        for (int m = l + 1; m < NL; m++)
+            for (int q = 0; q < np[m]; q++) last = last && list[m][q].x != p.x;
+        if (!last) continue;
+        int src = p.y;
+        for (int m = l - 1; m >= 0; m--) {
+            int from = src;
+            for (int q = 0; q < np[m]; q++)
+                if (list[m][q].x == src) from = list[m][q].y;
+            src = from;
+        }
+        if (p.x < k0 + NB) {
+            top[p.x - k0] = src;
+        } else if (src != p.x) {
+            const int i = atomicAdd(count, 1);
+            net[NB + 1 + 2 * i] = p.x;
+            net[NB + 2 + 2 * i] = src;
+        }
+    }
+    __syncthreads();
+    net[t] = top[t];
+    if (t == 0) net[NB] = *count;
+}
+
 // Panel step after the tournament of columns J = j0..j0+31, for 32 rows per
 // workgroup (rows from j0 + 32 on): the step's row interchanges, L21 = A21
 // U11^{-1}, and for the next 32 columns J' (with_next) U12 = L11^{-1} A12 and the
@@ -826,7 +838,7 @@ __global__ __launch_bounds__(256) void k_step(T* __restrict__ Ar, T* __restrict_
                                               int n, int with_next, const int* __restrict__ pl,
                                               const T* __restrict__ d11r, const T* __restrict__ d11i,
                                               T* __restrict__ Dr, T* __restrict__ Di, T* __restrict__ Ur,
-                                              T* __restrict__ Ui) {
+                                              T* __restrict__ Ui, int* __restrict__ net) {
     __builtin_amdgcn_s_setprio(3);
     constexpr int SL = PB + 4;  // row stride of L21 and U12 in LDS
     __shared__ __align__(16) T ur[PB * PB], ui[PB * PB], lr[PB * PB], li[PB * PB];  // U11; L11 transposed
@@ -836,6 +848,11 @@ __global__ __launch_bounds__(256) void k_step(T* __restrict__ Ar, T* __restrict_
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int nrow = max(1, (n - j0 - PB) / PB), strip = (int)blockIdx.x - nrow;  // strip >= 0: other columns
     const int r0 = j0 + PB + blockIdx.x * PB;
+    if (strip == NB / PB - 1 && !with_next) {  // beside the panel's last step
+        compose_lists(pl - (NB / PB - 1) * PLS, k0, net, reinterpret_cast<int2(*)[2 * PB]>(ur),
+                      reinterpret_cast<int*>(ui), map);
+        return;
+    }
     const int np = pl[0];
     int2 pair = make_int2(-1, -1);
     if (t < 2 * PB) pair = make_int2(pl[1 + 2 * t], pl[2 + 2 * t]);  // beyond np: not used
@@ -1005,41 +1022,371 @@ __global__ __launch_bounds__(256) void k_compact(const T* __restrict__ Ar, const
     *reinterpret_cast<V*>(Di + (long)i * PB + q) = *reinterpret_cast<const V*>(Ai + (long)i * ld + k0 + q);
 }
 
+// A panel's row interchanges (net, see compose_lists) in place in the columns
+// c0, c0 + 16, ...: 16 columns per workgroup, every source read before the first
+// store.
 template <typename T>
-__global__ __launch_bounds__(256) void k_copy_rows(int rows, int cols, const T* __restrict__ Sr,
-                                                   const T* __restrict__ Si, long lds, T* __restrict__ Dr,
-                                                   T* __restrict__ Di, long ldd) {
-    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (long)rows * cols) return;
-    const int r = (int)(idx / cols), c = (int)(idx % cols);
-    Dr[(long)r * ldd + c] = Sr[(long)r * lds + c];
-    Di[(long)r * ldd + c] = Si[(long)r * lds + c];
-}
-
-// U12 (NB x nc in the work buffer, ld lds) into the matrix rows (ld ldd) and
-// its transpose Ut (nc x NB, ld NB) for the FP32 trailing update, whose
-// operands are both k-contiguous (gemm_nt.h).  32 x 32 tiles through LDS;
-// grid (nc / 32, NB / 32).
-__global__ __launch_bounds__(256) void k_u12_out(const float* __restrict__ Sr, const float* __restrict__ Si, long lds,
-                                                 float* __restrict__ Dr, float* __restrict__ Di, long ldd,
-                                                 float* __restrict__ Utr, float* __restrict__ Uti) {
-    __shared__ float tr[32][33], ti[32][33];
-    const int c0 = blockIdx.x * 32, k0 = blockIdx.y * 32;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-#pragma unroll
-    for (int r = ty; r < 32; r += 8) {
-        const float vr = Sr[(long)(k0 + r) * lds + c0 + tx], vi = Si[(long)(k0 + r) * lds + c0 + tx];
-        Dr[(long)(k0 + r) * ldd + c0 + tx] = vr;
-        Di[(long)(k0 + r) * ldd + c0 + tx] = vi;
-        tr[r][tx] = vr;
-        ti[r][tx] = vi;
+__global__ __launch_bounds__(256) void k_swap_net(T* __restrict__ Ar, T* __restrict__ Ai, long ld, int k0, int c0,
+                                                  const int* __restrict__ net) {
+    using V = Nat16<T>;
+    constexpr int E = 16 / sizeof(T), W = 16 / E;  // 16-byte pieces per row
+    const int t = threadIdx.x;
+    const long c = c0 + 16 * (long)blockIdx.x;
+    int dst[2], src[2];
+    dst[0] = k0 + t;
+    src[0] = net[t];
+    dst[1] = src[1] = 0;
+    if (t < net[NB]) {
+        dst[1] = net[NB + 1 + 2 * t];
+        src[1] = net[NB + 2 + 2 * t];
     }
+    V vr[2][W], vi[2][W];
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+        if (dst[u] != src[u])
+#pragma unroll
+            for (int k = 0; k < W; k++) {
+                vr[u][k] = *reinterpret_cast<const V*>(Ar + (long)src[u] * ld + c + k * E);
+                vi[u][k] = *reinterpret_cast<const V*>(Ai + (long)src[u] * ld + c + k * E);
+            }
+    __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
 #pragma unroll
-    for (int r = ty; r < 32; r += 8) {
-        Utr[(long)(c0 + r) * NB + k0 + tx] = tr[tx][r];
-        Uti[(long)(c0 + r) * NB + k0 + tx] = ti[tx][r];
+    for (int u = 0; u < 2; u++)
+        if (dst[u] != src[u])
+#pragma unroll
+            for (int k = 0; k < W; k++) {
+                *reinterpret_cast<V*>(Ar + (long)dst[u] * ld + c + k * E) = vr[u][k];
+                *reinterpret_cast<V*>(Ai + (long)dst[u] * ld + c + k * E) = vi[u][k];
+            }
+}
+
+// Columns right of outer panel k0, 16 per workgroup (c0, c0 + 16, ...): the
+// panel's row interchanges (net) and U12 = L11^{-1} A12 (256 x 16), by blocked
+// substitution with L11 itself.  U12 goes to the matrix and, for the FP32
+// trailing update, transposed to Ut (row = column c0 + i, ld NB).
+//
+// The strip stays in registers as the accumulators of 16 x 16 matrix-core tiles,
+// wave w holding the 32-row block w.  Step j: wave j solves its block against the
+// 32 x 32 unit triangle (quads of lanes per column, the block through LDS), one
+// barrier, then every later wave subtracts L_wj X_j from its block.  What does not
+// depend on X is loaded ahead: a wave's triangle at the start (to LDS one step
+// before its turn), the rows of L before the barrier.
+//
+// Latency-bound for the next panel's 256 columns (16 workgroups), which the
+// next panel waits for.  Before, those took eight row-pair lists one after the
+// other (15 us), the explicit inverse of L11 (seven launches, 67 us), a product
+// (15 us) and a transposing copy (5 us); now one launch of 37 us (FP64, before
+// by substitution in 62 us behind the lists: 51).
+template <typename T>
+__global__ __launch_bounds__(512) void k_u12_strip(T* __restrict__ Ar, T* __restrict__ Ai, long ld, int k0, int c0,
+                                                   const int* __restrict__ net, T* __restrict__ Utr,
+                                                   T* __restrict__ Uti) {
+    __builtin_amdgcn_s_setprio(3);
+    using V = Nat16<T>;
+    constexpr int E = 16 / sizeof(T), W = 16 / E, NJ = NB / PB, XS = 16 + E;  // XS: row stride of a block in LDS
+    __shared__ __align__(16) T tri[2][2][PB * PB];  // [step parity][plane]: the triangle, transposed
+    __shared__ __align__(16) T xb[2][2][PB * XS];   // [step parity][plane]: block j, then X_j
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int r16 = lane & 15, g = lane >> 4;
+    const long c = c0 + 16 * (long)blockIdx.x;
+    typedef typename std::conditional<sizeof(T) == 4, v4f, v4d>::type acc_t;
+    // tile i: rows 32 wave + 16 i + .. of the panel.  FP32: row r16, columns 4 g ..
+    // + 3; FP64: rows g + 4 q, column r16
+    acc_t cr[2], ci[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int row = PB * wave + 16 * i;
+        if constexpr (sizeof(T) == 4) {
+            const long o = (long)net[row + r16] * ld + c + 4 * g;
+            cr[i] = *reinterpret_cast<const v4f*>(Ar + o);
+            ci[i] = *reinterpret_cast<const v4f*>(Ai + o);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const long o = (long)net[row + g + 4 * q] * ld + c + r16;
+                cr[i][q] = Ar[o];
+                ci[i][q] = Ai[o];
+            }
+        }
     }
+    // the rows below the panel: half a row per thread
+    int dst = -1;
+    V vr[W / 2], vi[W / 2];
+    const long half = c + (t & 1) * 8;
+    if (t / 2 < net[NB]) {
+        dst = net[NB + 1 + t / 2 * 2];
+        const long o = (long)net[NB + 2 + t / 2 * 2] * ld + half;
+#pragma unroll
+        for (int k = 0; k < W / 2; k++) {
+            vr[k] = *reinterpret_cast<const V*>(Ar + o + k * E);
+            vi[k] = *reinterpret_cast<const V*>(Ai + o + k * E);
+        }
+    }
+    T ta[PB * PB / 64], tb[PB * PB / 64];  // this wave's triangle
+    {
+        const T* lr = Ar + (long)(k0 + PB * wave) * (ld + 1);
+        const T* li = Ai + (long)(k0 + PB * wave) * (ld + 1);
+#pragma unroll
+        for (int u = 0; u < PB * PB / 64; u++) {
+            const int e = lane + 64 * u;
+            ta[u] = lr[(long)(e / PB) * ld + e % PB];
+            tb[u] = li[(long)(e / PB) * ld + e % PB];
+        }
+    }
+    auto put_tri = [&](int par) {
+#pragma unroll
+        for (int u = 0; u < PB * PB / 64; u++) {
+            const int e = lane + 64 * u, r = e / PB, q = e % PB;
+            tri[par][0][tri_index(q, r)] = q < r ? ta[u] : T(0);
+            tri[par][1][tri_index(q, r)] = q < r ? tb[u] : T(0);
+        }
+    };
+    if (wave == 0) put_tri(0);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();  // every source has been read
+    if (dst >= 0) {
+#pragma unroll
+        for (int k = 0; k < W / 2; k++) {
+            *reinterpret_cast<V*>(Ar + (long)dst * ld + half + k * E) = vr[k];
+            *reinterpret_cast<V*>(Ai + (long)dst * ld + half + k * E) = vi[k];
+        }
+    }
+#pragma unroll 1
+    for (int j = 0; j < NJ; j++) {
+        const int par = j & 1;
+        T(*x)[PB * XS] = xb[par];
+        T la[2][2][4], lb[2][2][4];  // element k = 16 q + 4 g + e of row r16 of the wave's tiles
+        if (wave > j) {
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    const long o = (long)(k0 + PB * wave + 16 * i + r16) * ld + k0 + PB * j + 16 * q + 4 * g;
+                    load_row4<T>(Ar + o, la[i][q]);
+                    load_row4<T>(Ai + o, lb[i][q]);
+                }
+            if (wave == j + 1) put_tri(par ^ 1);
+        } else if (wave == j) {
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                if constexpr (sizeof(T) == 4) {
+                    *reinterpret_cast<v4f*>(&x[0][(16 * i + r16) * XS + 4 * g]) = cr[i];
+                    *reinterpret_cast<v4f*>(&x[1][(16 * i + r16) * XS + 4 * g]) = ci[i];
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        x[0][(16 * i + g + 4 * q) * XS + r16] = cr[i][q];
+                        x[1][(16 * i + g + 4 * q) * XS + r16] = ci[i][q];
+                    }
+                }
+            }
+            __builtin_amdgcn_wave_barrier();  // the wave's own data: its LDS operations stay in order
+            T yr[QK], yi[QK];
+#pragma unroll
+            for (int k = 0; k < QK; k++) {
+                yr[k] = x[0][(4 * k + (lane & 3)) * XS + lane / 4];
+                yi[k] = x[1][(4 * k + (lane & 3)) * XS + lane / 4];
+            }
+            solve_tri<T>(yr, yi, tri[par][0], tri[par][1], false, yr, yi);
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int k = 0; k < QK; k++) {
+                x[0][(4 * k + (lane & 3)) * XS + lane / 4] = yr[k];
+                x[1][(4 * k + (lane & 3)) * XS + lane / 4] = yi[k];
+            }
+        }
+        __syncthreads();
+        if (wave > j) {
+            if constexpr (sizeof(T) == 4) {
+                v4f t1[2], t2[2], t3[2];
+#pragma unroll
+                for (int i = 0; i < 2; i++) t1[i] = t2[i] = t3[i] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int q = 0; q < 2; q++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int o = (16 * q + 4 * g + e) * XS + r16;
+                        const float b0 = x[0][o], b1 = x[1][o], b2 = b0 + b1;
+#pragma unroll
+                        for (int i = 0; i < 2; i++) {
+                            t1[i] = mfma16x16x4(b0, la[i][q][e], t1[i]);
+                            t2[i] = mfma16x16x4(b1, lb[i][q][e], t2[i]);
+                            t3[i] = mfma16x16x4(b2, la[i][q][e] + lb[i][q][e], t3[i]);
+                        }
+                    }
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    cr[i] -= t1[i] - t2[i];
+                    ci[i] -= t3[i] - t1[i] - t2[i];
+                }
+            } else {
+                v4d re[2], im[2];
+#pragma unroll
+                for (int i = 0; i < 2; i++) re[i] = im[i] = v4d{};
+#pragma unroll
+                for (int q = 0; q < 2; q++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int o = (16 * q + 4 * g + e) * XS + r16;
+                        const T b0 = x[0][o], b1 = x[1][o];
+#pragma unroll
+                        for (int i = 0; i < 2; i++) {
+                            re[i] = mfma16x16x4(la[i][q][e], b0, re[i]);
+                            re[i] = mfma16x16x4(lb[i][q][e], -b1, re[i]);
+                            im[i] = mfma16x16x4(la[i][q][e], b1, im[i]);
+                            im[i] = mfma16x16x4(lb[i][q][e], b0, im[i]);
+                        }
+                    }
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    cr[i] -= re[i];
+                    ci[i] -= im[i];
+                }
+            }
+        } else {  // the waves that are done: X_j to the matrix by rows and to Ut by columns
+            for (int e = t; e < PB * 16; e += (j + 1) * 64) {
+                const int r = e / 16, q = e % 16;
+                const long o = (long)(k0 + PB * j + r) * ld + c + q;
+                Ar[o] = x[0][r * XS + q];
+                Ai[o] = x[1][r * XS + q];
+                if constexpr (sizeof(T) == 4) {
+                    const int n = e / PB, k = e % PB;
+                    const long u = (16 * (long)blockIdx.x + n) * NB + PB * j + k;
+                    Utr[u] = x[0][k * XS + n];
+                    Uti[u] = x[1][k * XS + n];
+                }
+            }
+        }
+    }
+}
+
+// Inverses of the 32 x 32 diagonal triangles of every 256 x 256 diagonal block
+// (block p at F + p NB (ldf + 1)) into the diagonals of the zeroed blocks Li, Ui
+// (block p at p NB NB, ld NB): blockIdx.x = triangle, blockIdx.y = 0 unit lower, 1
+// upper.  One wave each, the triangle staged in LDS, lane j forms column j by
+// substitution in registers.
+template <typename T>
+__global__ __launch_bounds__(64) void k_inv_tri32(const T* __restrict__ Fr, const T* __restrict__ Fi, long ldf,
+                                                  T* __restrict__ Lr, T* __restrict__ Li, T* __restrict__ Ur,
+                                                  T* __restrict__ Ui) {
+    __shared__ T sr[PB][PB + 1], si[PB][PB + 1];
+    const int lane = threadIdx.x, p = blockIdx.x / (NB / PB), d = blockIdx.x % (NB / PB);
+    const long f = (long)(p * NB + d * PB) * (ldf + 1), o = (long)p * NB * NB + (long)d * PB * (NB + 1);
+#pragma unroll
+    for (int u = 0; u < PB * PB / 64; u++) {
+        const int e = lane + 64 * u, r = e / PB, q = e % PB;
+        sr[r][q] = Fr[f + r * ldf + q];
+        si[r][q] = Fi[f + r * ldf + q];
+    }
+    __syncthreads();
+    const int j = lane & (PB - 1);
+    T xr[PB], xi[PB];
+    const bool lower = blockIdx.y == 0;
+#pragma unroll
+    for (int v = 0; v < PB; v++) {  // lower: rows 0, 1, ..; upper: rows 31, 30, ..
+        // x_i = delta_ij - sum_k t_ik x_k over the rows k done before
+        const int i = v, iu = PB - 1 - v;
+        const int row = lower ? i : iu;
+        T ar = row == j ? T(1) : T(0), ai = T(0);
+#pragma unroll
+        for (int w = 0; w < v; w++) {
+            const int k = lower ? w : PB - 1 - w;
+            const T a = sr[row][k], b = si[row][k];
+            ar = fmadd(-a, xr[w], ar);
+            ar = fmadd(b, xi[w], ar);
+            ai = fmadd(-a, xi[w], ai);
+            ai = fmadd(-b, xr[w], ai);
+        }
+        if (!lower) {
+            T qr, qi;
+            cdiv(ar, ai, sr[row][row], si[row][row], qr, qi);
+            ar = qr;
+            ai = qi;
+        }
+        xr[v] = ar;
+        xi[v] = ai;
+    }
+    if (lane >= PB) return;
+    T* outr = lower ? Lr : Ur;
+    T* outi = lower ? Li : Ui;
+#pragma unroll
+    for (int v = 0; v < PB; v++) {
+        const int row = lower ? v : PB - 1 - v;
+        outr[o + (long)row * NB + j] = xr[v];
+        outi[o + (long)row * NB + j] = xi[v];
+    }
+}
+
+// One product of the doubling of the block inverses: every pair of h x h diagonal
+// inverses (h = 16 KQ) of every 256 x 256 block is joined,
+//   lower [X11 0; X21 X22]  with X21 = -X22 (L21 X11),
+//   upper [X11 X12; 0 X22]  with X12 = -X11 (U12 X22)
+// (blockIdx.z = 0, 1; blockIdx.y = pair of all blocks; stage 0: W = the inner
+// product, 1: the outer one).  FP32 in the 3M form, no LDS and no barrier: a
+// wave owns one 16 x 16 tile over the whole K and issues every operand load before
+// the first product.
+template <int KQ>
+__global__ __launch_bounds__(256) void k_tri_join(int stage, const float* __restrict__ Fr,
+                                                  const float* __restrict__ Fi, long ldf, float* Lr, float* Li,
+                                                  float* Ur, float* Ui, float* Wr, float* Wi) {
+    constexpr int h = 16 * KQ, pairs = NB / (2 * h), nt = h / 16;
+    const int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (tile >= nt * nt) return;
+    const bool lower = blockIdx.z == 0;
+    const int p = blockIdx.y / pairs, d = (blockIdx.y % pairs) * 2 * h;
+    const long fo = (long)(p * NB + d) * (ldf + 1), xo = (long)p * NB * NB + (long)d * (NB + 1);
+    const long wo = ((long)blockIdx.z * gridDim.y + blockIdx.y) * h * h;
+    float* Xr = lower ? Lr : Ur;
+    float* Xi = lower ? Li : Ui;
+    const long x11 = xo, x22 = xo + (long)h * (NB + 1), x21 = xo + (long)h * NB, x12 = xo + h;
+    const float *ar, *ai, *br, *bi;
+    float *cr, *ci;
+    long lda, ldb, ldc;
+    if (stage == 0) {
+        const long f = lower ? fo + (long)h * ldf : fo + h;
+        const long b = lower ? x11 : x22;
+        ar = Fr + f, ai = Fi + f, lda = ldf;
+        br = Xr + b, bi = Xi + b, ldb = NB;
+        cr = Wr + wo, ci = Wi + wo, ldc = h;
+    } else {
+        const long a = lower ? x22 : x11, o = lower ? x21 : x12;
+        ar = Xr + a, ai = Xi + a, lda = NB;
+        br = Wr + wo, bi = Wi + wo, ldb = h;
+        cr = Xr + o, ci = Xi + o, ldc = NB;
+    }
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int m0 = tile / nt * 16, n0 = tile % nt * 16;
+    v4f a0[KQ], a1[KQ];
+    float b0[KQ][4], b1[KQ][4];
+    const long oa = (long)(m0 + r) * lda + 4 * g;
+#pragma unroll
+    for (int q = 0; q < KQ; q++) {
+        a0[q] = *reinterpret_cast<const v4f*>(ar + oa + 16 * q);
+        a1[q] = *reinterpret_cast<const v4f*>(ai + oa + 16 * q);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const long ob = (long)(16 * q + 4 * g + e) * ldb + n0 + r;
+            b0[q][e] = br[ob];
+            b1[q][e] = bi[ob];
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    v4f t1 = v4f{0.f, 0.f, 0.f, 0.f}, t2 = t1, t3 = t1;
+#pragma unroll
+    for (int q = 0; q < KQ; q++) {
+        const v4f a2 = a0[q] + a1[q];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            t1 = mfma16x16x4(b0[q][e], a0[q][e], t1);
+            t2 = mfma16x16x4(b1[q][e], a1[q][e], t2);
+            t3 = mfma16x16x4(b0[q][e] + b1[q][e], a2[e], t3);
+        }
+    }
+    const v4f pr = t1 - t2, pi = t3 - t1 - t2;
+    const long oc = (long)(m0 + r) * ldc + n0 + 4 * g;
+    *reinterpret_cast<v4f*>(cr + oc) = stage == 0 ? pr : -pr;
+    *reinterpret_cast<v4f*>(ci + oc) = stage == 0 ? pi : -pi;
 }
 
 // Work buffers of one factorisation (device).
@@ -1053,65 +1400,33 @@ struct LuWork {
     T* d11;          // factored 32 x 32 diagonal block (2 planes), two sets by step parity
     T *cpr, *cpi;    // compact copies (n x 32 per plane) of the columns being factored, two sets by step parity
     T *sur, *sui;    // U12 of the next 32 columns (32 x 32)
-    T *ubr, *ubi;    // 256 x n U12 buffer
-    T *utr, *uti;    // n x 256 transpose of U12 (FP32 trailing update)
-    T *tr, *ti;      // 128 x 128 product of the L11^{-1} doubling
+    T *utr, *uti;    // n x 256 transpose of U12 (FP32 trailing update), then the products of the inverses
+    int* net;        // net row interchanges of an outer panel, two sets
 };
 
-// The row-pair lists of outer panel k0.  Two sets, by panel parity: the
-// update stream applies panel K's swaps to the far columns while the
-// tournaments of panel K+1 already write theirs.
+// The net row interchanges of outer panel k0.  Two sets, by panel parity: the
+// update stream applies panel K's while panel K+1 composes its own.
 template <typename T>
-int* panel_lists(const LuWork<T>& w, int k0) {
-    return w.pl + ((k0 / NB) & 1) * (NB / PB) * PLS;
+int* panel_net(const LuWork<T>& w, int k0) {
+    return w.net + ((k0 / NB) & 1) * NETS;
 }
 
-template <typename T>
-void launch_laswp(bem_ctx* c, hipStream_t s, T* Ar, T* Ai, long ld, int ca, int cb, int cc, int cd, const int* pl,
-                  int nl) {
-    const int ncols = (cb - ca) + (cd - cc);
-    if (ncols <= 0) return;
-    const int kt = kt_mark(c, KS_LASWP, s);
-    hipLaunchKernelGGL(k_laswp<T>, dim3((ncols + LASWP_COLS - 1) / LASWP_COLS), dim3(256), 0, s, Ar, Ai, ld, ca, cb,
-                       cc, cd, pl, nl);
-    kt_close(c, kt, 0.0, 2.0 * 2.0 * sizeof(T) * (double)ncols * 2 * PB * nl);
-}
-
-// L11^{-1} of the NB x NB unit lower triangle at F (ld ldf) into I (ld NB) by
-// doubling.  The inverses of the eight 32 x 32 diagonal blocks come from one
-// launch (one wave per block, k_inv_lower32); then for s = 32, 64, 128 every pair of s x s
-// diagonal blocks is joined,
-//     [X11 0; X21 X22] with X21 = -X22 (L21 X11),
-// as two batched GEMMs (all pairs of a level in one launch each, on the 32 x 32
-// tile: many blocks, little LDS, since they run beside the trailing update).  The blocks
-// above the diagonal are not written: the caller keeps them zero.  Seven
-// launches with short dependency chains replace one 256-step substitution.
-template <typename T>
-void invert_lower_doubling(hipStream_t s, const T* Fr, const T* Fi, long ldf, T* Ir, T* Ii, const LuWork<T>& w) {
-    constexpr int D = 32;
-    hipLaunchKernelGGL(k_inv_lower32<T>, dim3(NB / D), dim3(64), 0, s, Fr, Fi, ldf, (long)D * (ldf + 1), Ir, Ii,
-                       (long)NB, (long)D * (NB + 1));
-    for (int h = D; h < NB; h *= 2) {
-        const int pairs = NB / (2 * h);
-        const long sf = 2L * h * (ldf + 1), si = 2L * h * (NB + 1), st = (long)h * h;
-        const long f21 = (long)h * ldf, i21 = (long)h * NB, i22 = (long)h * (NB + 1);
-        // T = L21 X11, then X21 = -X22 T
-        if constexpr (sizeof(T) == 4) {  // register-direct short-K products (no LDS, no barrier)
-            if (cgemm_rd_fits(h, h, h, Fr + f21, Fi + f21, ldf, w.tr, w.ti, h, sf, st) &&
-                cgemm_rd_fits(h, h, h, Ir + i22, Ii + i22, NB, Ir + i21, Ii + i21, NB, si, si)) {
-                cgemm_rd(s, h, h, h, Fr + f21, Fi + f21, ldf, Ir, Ii, NB, w.tr, w.ti, h, 1 | GEMM_MODE_URGENT, pairs,
-                         sf, si, st);
-                cgemm_rd(s, h, h, h, Ir + i22, Ii + i22, NB, w.tr, w.ti, h, Ir + i21, Ii + i21, NB,
-                         3 | GEMM_MODE_URGENT, pairs, si, st, si);
-                continue;
-            }
-        }
-        cgemm_any<T>(kGemmSmall, s, h, h, h, Fr + f21, Fi + f21, ldf, Ir, Ii, NB, w.tr, w.ti, h, 1 | GEMM_MODE_URGENT,
-                     pairs, sf, si, st);
-        cgemm_any<T>(kGemmSmall, s, h, h, h, Ir + i22, Ii + i22, NB, w.tr, w.ti, h, Ir + i21, Ii + i21, NB,
-                     3 | GEMM_MODE_URGENT, pairs, si, st,
-                     si);
-    }
+// L^{-1} and U^{-1} of the NB x NB diagonal blocks of the FP32 factors at F into
+// the blocks at L and U (zeroed), all blocks in each launch: the 32 x 32 diagonal
+// triangles by substitution, then joined in pairs three times.  For the solves;
+// the factorisation itself does not use them.
+void invert_blocks(hipStream_t s, int nb, const float* Fr, const float* Fi, long ldf, float* Lr, float* Li, float* Ur,
+                   float* Ui, float* Wr, float* Wi) {
+    hipLaunchKernelGGL(k_inv_tri32<float>, dim3(nb * (NB / PB), 2), dim3(64), 0, s, Fr, Fi, ldf, Lr, Li, Ur, Ui);
+    for (int stage = 0; stage < 2; stage++)
+        hipLaunchKernelGGL(k_tri_join<2>, dim3(1, 4 * nb, 2), dim3(256), 0, s, stage, Fr, Fi, ldf, Lr, Li, Ur, Ui, Wr,
+                           Wi);
+    for (int stage = 0; stage < 2; stage++)
+        hipLaunchKernelGGL(k_tri_join<4>, dim3(4, 2 * nb, 2), dim3(256), 0, s, stage, Fr, Fi, ldf, Lr, Li, Ur, Ui, Wr,
+                           Wi);
+    for (int stage = 0; stage < 2; stage++)
+        hipLaunchKernelGGL(k_tri_join<8>, dim3(16, nb, 2), dim3(256), 0, s, stage, Fr, Fi, ldf, Lr, Li, Ur, Ui, Wr,
+                           Wi);
 }
 
 // Factors the outer panel of columns k0 .. k0+NB-1 (rows k0 .. n-1) on stream
@@ -1121,7 +1436,7 @@ void invert_lower_doubling(hipStream_t s, const T* Fr, const T* Fi, long ldf, T*
 // does not need them.  (With that update and the other columns' swaps on a third
 // stream, behind an event each way, and the next 32 columns' swaps, panel solve
 // and update as three launches a step took 115 us at 3840 rows; now 75.)  The
-// swaps of step j are kept as row-pair list j for the columns outside the panel.
+// swaps of the steps end as one net list for the columns outside the panel.
 // The FP32 tournament takes sets of 512 rows where they save a level: a set costs
 // 29 us of elimination instead of 19 for 256 rows, a level of merges ~23 (3840
 // rows: 58.7 against 73.1 us, 12288 rows, which save none: 91.9 against 80.6).
@@ -1142,7 +1457,7 @@ void factor_panel(bem_ctx* c, hipStream_t s, T* Ar, T* Ai, int k0, const LuWork<
         T *Sr = w.cpr + par * cp, *Si = w.cpi + par * cp;
         T *Dr = w.cpr + (par ^ 1) * cp, *Di = w.cpi + (par ^ 1) * cp;
         T *d11r = w.d11 + par * 2 * PB * PB, *d11i = d11r + PB * PB;
-        int* pl = panel_lists(w, k0) + ((j0 - k0) / PB) * PLS;
+        int* pl = w.pl + ((j0 - k0) / PB) * PLS;
         kt = kt_mark(c, KS_TSLU, s);
         auto tslu = k_tslu<T, 1>;
         int set = 256;
@@ -1157,45 +1472,35 @@ void factor_panel(bem_ctx* c, hipStream_t s, T* Ar, T* Ai, int k0, const LuWork<
                  2.0 * sizeof(T) * (double)m * (PB + 2 * far.ncol));
         const int next = j0 + PB < k1, others = NB / PB - 1 - next;
         kt = kt_mark(c, KS_PANEL, s);
-        hipLaunchKernelGGL(k_step<T>, dim3(std::max(1, (m - PB) / PB) + others), dim3(256), 0, s, Ar, Ai, ld, Sr, Si,
-                           k0, j0, n, next, pl, d11r, d11i, Dr, Di, w.sur, w.sui);
+        hipLaunchKernelGGL(k_step<T>, dim3(std::max(1, (m - PB) / PB) + others + !next), dim3(256), 0, s, Ar, Ai, ld,
+                           Sr, Si, k0, j0, n, next, pl, d11r, d11i, Dr, Di, w.sur, w.sui, panel_net(w, k0));
         kt_close(c, kt, (next ? 10.0 : 4.0) * (double)m * PB * PB, (next ? 8.0 : 4.0) * sizeof(T) * (double)m * PB);
         const int c0 = std::min(k1, j0 + 2 * PB), ncol = k1 - c0;  // columns beyond the next 32
         far = FarUpdate{j0, c0, ncol, next ? ((m - PB) / 16 * (ncol / 16) + 3) / 4 + 1 : 0};
     }
 }
 
-// U12 = L11^{-1} A12 and A22 -= L21 U12 for the columns [c0, c0 + nc) right
-// of outer panel k0, on stream us; U12 goes through the work buffer.  FP32:
-// U12 as a GEMM with the explicit L11^{-1} (Lir, Lii); FP64: by substitution
-// with L11 itself (k_trsm_rhs), the backward-stable form of Zgetrf's TRSM.
+// The swaps of outer panel k0, U12 = L11^{-1} A12 and A22 -= L21 U12 for the
+// columns [c0, c0 + nc) right of the panel, on stream us.
 template <typename T>
-void update_columns(bem_ctx* c, hipStream_t us, T* Ar, T* Ai, const T* Lir, const T* Lii, int k0, int c0, int nc,
-                    const LuWork<T>& w, bool headroom) {
+void update_columns(bem_ctx* c, hipStream_t us, T* Ar, T* Ai, int k0, int c0, int nc, const LuWork<T>& w,
+                    bool headroom) {
     const int n = c->npad;
     const long ld = n;
     const int nr = n - (k0 + NB);
-    const long io = (long)(k0 / NB) * NB * NB;
     const long o12 = (long)k0 * ld + c0, o21 = (long)(k0 + NB) * ld + k0, o22 = (long)(k0 + NB) * ld + c0;
-    T* ubr = w.ubr + (c0 - (k0 + NB));
-    T* ubi = w.ubi + (c0 - (k0 + NB));
-    if constexpr (sizeof(T) == 8) {
-        const long o11 = (long)k0 * ld + k0;
-        const int kt = kt_mark(c, KS_TRSM, us);
-        trsm_rhs<T>(us, true, Ar + o11, Ai + o11, ld, Ar + o12, Ai + o12, ld, ubr, ubi, ld, nc);
-        kt_close(c, kt, 4.0 * (double)NB * NB * nc, 2.0 * sizeof(T) * ((double)NB * NB + 2.0 * NB * nc));
-    } else {
-        cgemm_ctx<T>(c, NB, nc, NB, Lir + io, Lii + io, NB, Ar + o12, Ai + o12, ld, ubr, ubi, ld, 1, us);
-        // FP32: the trailing update on the k-contiguous kernel (U12 transposed
-        // beside its copy into the matrix), when the shape fits it
+    T *utr = nullptr, *uti = nullptr;
+    if constexpr (sizeof(T) == 4) {
+        utr = w.utr + (long)(c0 - (k0 + NB)) * NB;
+        uti = w.uti + (long)(c0 - (k0 + NB)) * NB;
+    }
+    int kt = kt_mark(c, KS_TRSM, us);
+    hipLaunchKernelGGL(k_u12_strip<T>, dim3(nc / 16), dim3(512), 0, us, Ar, Ai, ld, k0, c0, panel_net(w, k0), utr, uti);
+    kt_close(c, kt, 4.0 * (double)NB * NB * nc, (sizeof(T) == 4 ? 8.0 : 6.0) * sizeof(T) * (double)NB * nc);
+    if constexpr (sizeof(T) == 4) {
+        // FP32: the trailing update on the k-contiguous kernel, when the shape fits it
         const GemmPlan& plan = c->gemm_plan[0];
-        float* utr = w.utr + (long)(c0 - (k0 + NB)) * NB;
-        float* uti = w.uti + (long)(c0 - (k0 + NB)) * NB;
         if (cupdate_nt_fits(plan.nt, nr, nc, NB, Ar + o21, Ai + o21, ld, utr, uti, NB, Ar + o22, Ai + o22, ld)) {
-            int kt = kt_mark(c, KS_OTHER, us);
-            hipLaunchKernelGGL(k_u12_out, dim3((unsigned)(nc / 32), NB / 32), dim3(256), 0, us, ubr, ubi, ld,
-                               Ar + o12, Ai + o12, ld, utr, uti);
-            kt_close(c, kt, 0.0, 6.0 * sizeof(T) * (double)NB * nc);
             kt = kt_mark(c, KS_UPDATE32, us);
             cupdate_nt(plan.nt, us, nr, nc, NB, Ar + o21, Ai + o21, ld, utr, uti, NB, Ar + o22, Ai + o22, ld,
                        headroom ? gemm_headroom_cap(plan, plan.large) : 0);
@@ -1204,22 +1509,17 @@ void update_columns(bem_ctx* c, hipStream_t us, T* Ar, T* Ai, const T* Lir, cons
             return;
         }
     }
-    cgemm_ctx<T>(c, nr, nc, NB, Ar + o21, Ai + o21, ld, ubr, ubi, ld, Ar + o22, Ai + o22, ld, 0, us,
+    cgemm_ctx<T>(c, nr, nc, NB, Ar + o21, Ai + o21, ld, Ar + o12, Ai + o12, ld, Ar + o22, Ai + o22, ld, 0, us,
                  GEMM_UPDATE | (headroom ? GEMM_HEADROOM : 0));
-    const int kt = kt_mark(c, KS_OTHER, us);
-    hipLaunchKernelGGL(k_copy_rows<T>, dim3((unsigned)(((long)NB * nc + 255) / 256)), dim3(256), 0, us, NB, nc, ubr,
-                       ubi, ld, Ar + o12, Ai + o12, ld);
-    kt_close(c, kt, 0.0, 4.0 * sizeof(T) * (double)NB * nc);
 }
 
 // Blocked right-looking factorisation of the padded npad x npad matrix with
 // look-ahead of depth one: outer panel K+1 is factored on the panel stream
 // while the trailing update of panel K runs on the update stream.  Panel K+1
 // only touches its own columns; its swaps reach the other columns on the
-// update stream.  After panel K, the critical path to panel K+1 is: swaps in
-// the columns of panel K+1 (update stream) beside L11^{-1} (panel stream),
-// then U12 and the update of those 256 columns; the swaps and the update of
-// all other columns follow on the update stream while panel K+1 is factored.
+// update stream.  After panel K, the critical path to panel K+1 is the swaps, U12
+// and the update of those 256 columns; the swaps and the update of all other
+// columns follow on the update stream while panel K+1 is factored.
 // Stream layout (c->lu_streams): 0 = everything on the context stream (no
 // overlap); 1 = panel stream and context stream over all CUs.
 template <typename T>
@@ -1228,53 +1528,43 @@ void factor(bem_ctx* c, T* Ar, T* Ai, T* Lir, T* Lii, T* Uir, T* Uii, const LuWo
     const long ld = n;
     hipStream_t us = c->stream, ps = c->stream2;
     if (c->lu_streams == 0) ps = us;
-    hipEvent_t e_panel = c->lu_ev[0], e_next = c->lu_ev[1], e_start = c->lu_ev[2], e_linv = c->lu_ev[3];
-    (void)hipEventRecord(e_start, c->stream);  // the matrix and work buffers are ready
+    hipEvent_t e_panel = c->lu_ev[0], e_next = c->lu_ev[1], e_start = c->lu_ev[2];
+    (void)hipEventRecord(e_start, us);  // the matrix and work buffers are ready
     (void)hipStreamWaitEvent(ps, e_start, 0);
-    if (us != c->stream) (void)hipStreamWaitEvent(us, e_start, 0);
+    auto swap_left = [&](int k0) {
+        if (k0 == 0) return;
+        const int kt = kt_mark(c, KS_LASWP, us);
+        hipLaunchKernelGGL(k_swap_net<T>, dim3(k0 / 16), dim3(256), 0, us, Ar, Ai, ld, k0, 0, panel_net(w, k0));
+        kt_close(c, kt, 0.0, 4.0 * sizeof(T) * (double)k0 * 2 * NB);
+    };
     factor_panel<T>(c, ps, Ar, Ai, 0, w);
     for (int K = 0; K < nb; K++) {
         const int k0 = K * NB;
         const int nr = n - (k0 + NB);
-        const long o11 = (long)k0 * ld + k0;
-        const long io = (long)K * NB * NB;
         (void)hipEventRecord(e_panel, ps);
-        if constexpr (sizeof(T) == 4) {  // FP64 solves with L11 by substitution instead
-            const int kt = kt_mark(c, KS_TRSM, ps);
-            invert_lower_doubling<T>(ps, Ar + o11, Ai + o11, ld, Lir + io, Lii + io, w);
-            kt_close(c, kt, 8.0 * NB * NB * NB / 6.0, 4.0 * sizeof(T) * (double)NB * NB);
-        }
-        (void)hipEventRecord(e_linv, ps);
         (void)hipStreamWaitEvent(us, e_panel, 0);
         if (nr <= 0) {
-            launch_laswp<T>(c, us, Ar, Ai, ld, 0, k0, 0, 0, panel_lists(w, k0), NB / PB);
-            (void)hipStreamWaitEvent(us, e_linv, 0);
+            swap_left(k0);
             break;
         }
         // columns of panel K+1 first, then hand panel K+1 to the panel stream
-        launch_laswp<T>(c, us, Ar, Ai, ld, k0 + NB, k0 + 2 * NB, 0, 0, panel_lists(w, k0), NB / PB);
-        (void)hipStreamWaitEvent(us, e_linv, 0);
-        update_columns<T>(c, us, Ar, Ai, Lir, Lii, k0, k0 + NB, NB, w, false);
+        update_columns<T>(c, us, Ar, Ai, k0, k0 + NB, NB, w, false);
         (void)hipEventRecord(e_next, us);
         (void)hipStreamWaitEvent(ps, e_next, 0);
-        // the rest of the update is enqueued before panel K+1's ~40 launches,
-        // so a host that enqueues slowly (under a profiler, say) does not
-        // hold the update stream back
-        launch_laswp<T>(c, us, Ar, Ai, ld, 0, k0, k0 + 2 * NB, n, panel_lists(w, k0), NB / PB);
+        // the rest of the update is enqueued before panel K+1's launches, so a
+        // host that enqueues slowly (under a profiler, say) does not hold the
+        // update stream back
+        swap_left(k0);
         if (nr > NB)
-            update_columns<T>(c, us, Ar, Ai, Lir, Lii, k0, k0 + 2 * NB, nr - NB, w, ps != us && c->gemm_plan[sizeof(T) == 4 ? 0 : 1].cap > 0);
+            update_columns<T>(c, us, Ar, Ai, k0, k0 + 2 * NB, nr - NB, w, ps != us && c->gemm_plan[sizeof(T) == 4 ? 0 : 1].cap > 0);
         factor_panel<T>(c, ps, Ar, Ai, k0 + NB, w);
     }
-    // U^{-1} of all diagonal blocks in one launch (FP32; the FP64 solves
-    // substitute with the diagonal blocks themselves)
+    // the inverses of all diagonal blocks (FP32; the FP64 solves substitute with
+    // the diagonal blocks themselves)
     if constexpr (sizeof(T) == 4) {
         const int kt = kt_mark(c, KS_TRSM, us);
-        invert_diag_blocks<T>(us, NB, nb, Ar, Ai, ld, Uir, Uii, false);
-        kt_close(c, kt, 8.0 * (double)n * NB * NB / 6.0, 4.0 * sizeof(T) * (double)n * NB);
-    }
-    if (us != c->stream) {  // the context stream continues after the last update
-        (void)hipEventRecord(e_start, us);
-        (void)hipStreamWaitEvent(c->stream, e_start, 0);
+        invert_blocks(us, nb, Ar, Ai, ld, Lir, Lii, Uir, Uii, w.utr, w.uti);
+        kt_close(c, kt, 16.0 * (double)n * NB * NB / 6.0, 8.0 * sizeof(T) * (double)n * NB);
     }
 }
 
@@ -1305,17 +1595,18 @@ int factor_prec(bem_ctx* c, T* Ar, T* Ai, void*& inv, size_t& inv_bytes) {
     // diagonal blocks, compact columns, U12 buffers
     const int nsets0 = (n + 255) / 256;
     const size_t ncnt = 2 * (size_t)nsets0 + 64;
-    const size_t nint = 64 + ncnt + 2 * (NB / PB) * PLS + 2 * (size_t)nsets0 * PB;
+    const size_t nint = 64 + ncnt + (NB / PB) * PLS + 2 * NETS + 2 * (size_t)nsets0 * PB;
     const size_t bytes = nint * sizeof(int) + 256 + 4 * (size_t)nsets0 * PB * PB * sizeof(T) +
-                         6 * (size_t)PB * PB * sizeof(T) + 4 * (size_t)NB * n * sizeof(T) +
-                         2 * (size_t)(NB / 2) * (NB / 2) * sizeof(T) + 4 * (size_t)PB * n * sizeof(T) + 256;
+                         6 * (size_t)PB * PB * sizeof(T) + 4 * (size_t)PB * n * sizeof(T) +
+                         (with_inv ? 2 * (size_t)NB * n * sizeof(T) : 0) + 256;
     void* scr = nullptr;
     if (int rc = ctx_scratch(c, bytes, &scr)) return rc;
     LuWork<T> w;
     w.info = static_cast<int*>(scr);
     w.cnt = w.info + 64;
     w.pl = w.cnt + ncnt;
-    w.cid = w.pl + 2 * (NB / PB) * PLS;
+    w.net = w.pl + (NB / PB) * PLS;
+    w.cid = w.net + 2 * NETS;
     char* p = reinterpret_cast<char*>(w.info + nint);
     p += (256 - reinterpret_cast<uintptr_t>(p) % 256) % 256;
     w.cvr = reinterpret_cast<T*>(p);
@@ -1325,15 +1616,11 @@ int factor_prec(bem_ctx* c, T* Ar, T* Ai, void*& inv, size_t& inv_bytes) {
     w.sui = w.sur + PB * PB;
     w.cpr = w.sui + PB * PB;
     w.cpi = w.cpr + 2 * (size_t)PB * n;
-    w.ubr = w.cpi + 2 * (size_t)PB * n;
-    w.ubi = w.ubr + (size_t)NB * n;
-    w.utr = w.ubi + (size_t)NB * n;
+    w.utr = w.cpi + 2 * (size_t)PB * n;
     w.uti = w.utr + (size_t)NB * n;
-    w.tr = w.uti + (size_t)NB * n;
-    w.ti = w.tr + (size_t)(NB / 2) * (NB / 2);
     BEM_HIP(c, hipMemsetAsync(w.info, 0, (64 + ncnt) * sizeof(int), c->stream));
-    // the doubling writes only the diagonal and lower blocks of each L11^{-1}
-    if (with_inv) BEM_HIP(c, hipMemsetAsync(Lir, 0, 2 * (size_t)n * NB * sizeof(T), c->stream));
+    // the triangles beside the inverses stay zero
+    if (with_inv) BEM_HIP(c, hipMemsetAsync(Lir, 0, 4 * (size_t)n * NB * sizeof(T), c->stream));
     factor<T>(c, Ar, Ai, Lir, Lii, Uir, Uii, w);
     return 0;
 }
