@@ -1,5 +1,5 @@
 // abi.cpp -- implementation of include/bem_abi.h: context, mesh upload,
-// device buffers, argument checking, host<->device layout conversion.
+// device buffers, argument checking.
 // The numerical work is in kernels/*.hip.
 #include <algorithm>
 #include <cmath>
@@ -541,17 +541,8 @@ int bem_assemble(bem_ctx* c, double ker, double kei, double kir, double kii, dou
 int bem_get_Z(bem_ctx* c, double* Z, int row_major) {
     if (!c || !Z) return BEM_ERR_ARG;
     if (!c->has_Z64) return bem_fail(c, BEM_ERR_STATE, "get_Z: no FP64 Z on the device");
-    const int n = c->n, ld = c->npad;
-    std::vector<double> re((size_t)n * ld), im((size_t)n * ld);
-    BEM_HIP(c, hipMemcpy(re.data(), c->Zr, re.size() * sizeof(double), hipMemcpyDeviceToHost));
-    BEM_HIP(c, hipMemcpy(im.data(), c->Zi, im.size() * sizeof(double), hipMemcpyDeviceToHost));
-    for (int i = 0; i < n; i++)
-        for (int j = 0; j < n; j++) {
-            const size_t o = row_major ? (size_t)i * n + j : (size_t)j * n + i;
-            Z[2 * o] = re[(size_t)i * ld + j];
-            Z[2 * o + 1] = im[(size_t)i * ld + j];
-        }
-    return 0;
+    (void)hipSetDevice(c->device);
+    return planes_download(c, c->Zr, c->Zi, c->npad, c->n, c->n, row_major != 0, 1.0, Z);
 }
 
 int bem_get_Z_entries(bem_ctx* c, const int* rows, const int* cols, int count, double* out) {
@@ -592,17 +583,9 @@ int bem_assemble_LK(bem_ctx* c, double kr, double ki, double* L, double* K) {
     if (int rc = bem_assemble(c, kr, ki, kr, ki, 1.0, 1.0, BEM_ASM_Z64)) return rc;
     // with equal wavenumbers and eta = 1: Z_TL = 2 L, Z_BL = 2 K
     const int N = c->rwg.N, ld = c->npad;
-    std::vector<double> re((size_t)c->n * ld), im((size_t)c->n * ld);
-    BEM_HIP(c, hipMemcpy(re.data(), c->Zr, re.size() * sizeof(double), hipMemcpyDeviceToHost));
-    BEM_HIP(c, hipMemcpy(im.data(), c->Zi, im.size() * sizeof(double), hipMemcpyDeviceToHost));
-    for (int i = 0; i < N; i++)
-        for (int j = 0; j < N; j++) {
-            const size_t o = (size_t)i * N + j;
-            L[2 * o] = 0.5 * re[(size_t)i * ld + j];
-            L[2 * o + 1] = 0.5 * im[(size_t)i * ld + j];
-            K[2 * o] = 0.5 * re[(size_t)(N + i) * ld + j];
-            K[2 * o + 1] = 0.5 * im[(size_t)(N + i) * ld + j];
-        }
+    const size_t half = (size_t)N * ld;
+    if (int rc = planes_download(c, c->Zr, c->Zi, ld, N, N, true, 0.5, L)) return rc;
+    if (int rc = planes_download(c, c->Zr + half, c->Zi + half, ld, N, N, true, 0.5, K)) return rc;
     c->has_Z64 = false;  // the matrix on the device is not a PMCHWT system
     c->asm_valid = false;
     return 0;
@@ -613,20 +596,7 @@ int bem_set_Z(bem_ctx* c, const double* Z, int n, int row_major) {
     (void)hipSetDevice(c->device);
     if (int rc = set_size(c, n)) return rc;
     if (int rc = ensure_z64(c)) return rc;
-    const int ld = c->npad;
-    std::vector<double> re((size_t)ld * ld, 0.0), im((size_t)ld * ld, 0.0);
-    for (int i = 0; i < ld; i++)
-        for (int j = 0; j < ld; j++) {
-            if (i < n && j < n) {
-                const size_t o = row_major ? (size_t)i * n + j : (size_t)j * n + i;
-                re[(size_t)i * ld + j] = Z[2 * o];
-                im[(size_t)i * ld + j] = Z[2 * o + 1];
-            } else if (i == j) {
-                re[(size_t)i * ld + j] = 1.0;
-            }
-        }
-    BEM_HIP(c, hipMemcpy(c->Zr, re.data(), re.size() * sizeof(double), hipMemcpyHostToDevice));
-    BEM_HIP(c, hipMemcpy(c->Zi, im.data(), im.size() * sizeof(double), hipMemcpyHostToDevice));
+    if (int rc = planes_upload(c, Z, n, n, row_major != 0, c->Zr, c->Zi, c->npad, c->npad, true)) return rc;
     c->has_Z64 = true;
     c->has_Z32 = false;
     if (c->factored >= 0) c->factors_stale = true;  // kept for bem_solve_gmres
@@ -676,16 +646,8 @@ int bem_get_pivots(const bem_ctx* c, int* ipiv) {
 int bem_get_lu(bem_ctx* c, double* LU) {
     if (!c || !LU) return BEM_ERR_ARG;
     if (c->lu_avail != BEM_F64) return bem_fail(c, BEM_ERR_STATE, "get_lu: no FP64 factorisation");
-    const int n = c->n, ld = c->npad;
-    std::vector<double> re((size_t)n * ld), im((size_t)n * ld);
-    BEM_HIP(c, hipMemcpy(re.data(), c->Vr, re.size() * sizeof(double), hipMemcpyDeviceToHost));
-    BEM_HIP(c, hipMemcpy(im.data(), c->Vi, im.size() * sizeof(double), hipMemcpyDeviceToHost));
-    for (int i = 0; i < n; i++)
-        for (int j = 0; j < n; j++) {
-            LU[2 * ((size_t)i * n + j)] = re[(size_t)i * ld + j];
-            LU[2 * ((size_t)i * n + j) + 1] = im[(size_t)i * ld + j];
-        }
-    return 0;
+    (void)hipSetDevice(c->device);
+    return planes_download(c, c->Vr, c->Vi, c->npad, c->n, c->n, true, 1.0, LU);
 }
 
 int bem_set_lu(bem_ctx* c, const double* LU, const int* ipiv, int n) {
@@ -704,23 +666,12 @@ int bem_set_lu(bem_ctx* c, const double* LU, const int* ipiv, int n) {
         if (int rc = dalloc(c, c->ipiv, ld, "pivots")) return rc;
         if (int rc = dalloc(c, c->perm, ld, "permutation")) return rc;
     }
-    std::vector<double> re(nn, 0.0), im(nn, 0.0);
-    for (int i = 0; i < ld; i++)
-        for (int j = 0; j < ld; j++) {
-            if (i < n && j < n) {
-                re[(size_t)i * ld + j] = LU[2 * ((size_t)i * n + j)];
-                im[(size_t)i * ld + j] = LU[2 * ((size_t)i * n + j) + 1];
-            } else if (i == j) {
-                re[(size_t)i * ld + j] = 1.0;
-            }
-        }
     std::vector<int> ip(ld), perm(ld);
     for (int i = 0; i < ld; i++) ip[i] = i < n ? ipiv[i] - 1 : i;
     for (int i = 0; i < ld; i++) perm[i] = i;
     for (int i = 0; i < ld; i++)
         if (ip[i] != i) std::swap(perm[i], perm[ip[i]]);
-    BEM_HIP(c, hipMemcpy(c->Vr, re.data(), nn * sizeof(double), hipMemcpyHostToDevice));
-    BEM_HIP(c, hipMemcpy(c->Vi, im.data(), nn * sizeof(double), hipMemcpyHostToDevice));
+    if (int rc = planes_upload(c, LU, n, n, true, c->Vr, c->Vi, ld, ld, true)) return rc;
     BEM_HIP(c, hipMemcpy(c->ipiv, ip.data(), ld * sizeof(int), hipMemcpyHostToDevice));
     BEM_HIP(c, hipMemcpy(c->perm, perm.data(), ld * sizeof(int), hipMemcpyHostToDevice));
     c->factored = BEM_F64;
@@ -737,15 +688,7 @@ static int load_rhs(bem_ctx* c, const double* B, int& nrhs, const char* who) {
     if (B) {
         if (nrhs < 1) return bem_fail(c, BEM_ERR_ARG, std::string(who) + ": nrhs must be positive");
         if (int rc = ctx_ensure_rhs(c, nrhs)) return rc;
-        const int ld = c->ldr;
-        std::vector<double> re((size_t)c->npad * ld, 0.0), im((size_t)c->npad * ld, 0.0);
-        for (int j = 0; j < nrhs; j++)
-            for (int i = 0; i < n; i++) {
-                re[(size_t)i * ld + j] = B[2 * ((size_t)j * n + i)];
-                im[(size_t)i * ld + j] = B[2 * ((size_t)j * n + i) + 1];
-            }
-        BEM_HIP(c, hipMemcpy(c->Br, re.data(), re.size() * sizeof(double), hipMemcpyHostToDevice));
-        BEM_HIP(c, hipMemcpy(c->Bi, im.data(), im.size() * sizeof(double), hipMemcpyHostToDevice));
+        if (int rc = planes_upload(c, B, n, nrhs, false, c->Br, c->Bi, c->npad, c->ldr, false)) return rc;
         c->has_B = true;
         c->rhs_planewave = false;
     } else {
@@ -757,16 +700,7 @@ static int load_rhs(bem_ctx* c, const double* B, int& nrhs, const char* who) {
 
 // The device solutions into X (column-major n x nrhs complex).
 static int store_solution(bem_ctx* c, int nrhs, double* X) {
-    const int n = c->n, ld = c->ldr;
-    std::vector<double> re((size_t)n * ld), im((size_t)n * ld);
-    BEM_HIP(c, hipMemcpy(re.data(), c->Xr, re.size() * sizeof(double), hipMemcpyDeviceToHost));
-    BEM_HIP(c, hipMemcpy(im.data(), c->Xi, im.size() * sizeof(double), hipMemcpyDeviceToHost));
-    for (int j = 0; j < nrhs; j++)
-        for (int i = 0; i < n; i++) {
-            X[2 * ((size_t)j * n + i)] = re[(size_t)i * ld + j];
-            X[2 * ((size_t)j * n + i) + 1] = im[(size_t)i * ld + j];
-        }
-    return 0;
+    return planes_download(c, c->Xr, c->Xi, c->ldr, c->n, nrhs, false, 1.0, X);
 }
 
 int bem_solve(bem_ctx* c, const double* B, int nrhs, double* X, double ir_tol, int ir_max, bem_solve_stats* st) {
@@ -918,15 +852,7 @@ int bem_rhs_planewave(bem_ctx* c, double kr, double ki, double eta, const double
     c->has_B = true;
     c->rhs_planewave = true;
     if (B_out) {
-        const int n = c->n, ld = c->ldr;
-        std::vector<double> re((size_t)n * ld), im((size_t)n * ld);
-        BEM_HIP(c, hipMemcpy(re.data(), c->Br, re.size() * sizeof(double), hipMemcpyDeviceToHost));
-        BEM_HIP(c, hipMemcpy(im.data(), c->Bi, im.size() * sizeof(double), hipMemcpyDeviceToHost));
-        for (int j = 0; j < nrhs; j++)
-            for (int i = 0; i < n; i++) {
-                B_out[2 * ((size_t)j * n + i)] = re[(size_t)i * ld + j];
-                B_out[2 * ((size_t)j * n + i) + 1] = im[(size_t)i * ld + j];
-            }
+        if (int rc = planes_download(c, c->Br, c->Bi, c->ldr, c->n, nrhs, false, 1.0, B_out)) return rc;
     }
     return 0;
 }

@@ -212,6 +212,13 @@ int bem_fail(bem_ctx* c, int code, const std::string& msg);
 
 // Device scratch of at least `bytes` (reallocated when too small).
 int ctx_scratch(bem_ctx* c, size_t bytes, void** out);
+// A host matrix of rows x cols interleaved complex values (row- or column-major) into
+// planar FP64 (prows x ld), padded with zeros, or with the identity; and planes
+// (times scale) into a host matrix.  Through at most 32 MiB of the context's scratch.
+int planes_upload(bem_ctx* c, const double* src, int rows, int cols, bool row_major, double* Pr, double* Pi, int prows,
+                  int ld, bool identity);
+int planes_download(bem_ctx* c, const double* Pr, const double* Pi, int ld, int rows, int cols, bool row_major,
+                    double scale, double* dst);
 
 // Launchers (kernels/*.hip).  All enqueue on c->stream and return 0 or < 0.
 int asm_launch(bem_ctx* c, const AsmParams& p, bool want64, bool want32);
