@@ -106,8 +106,6 @@ struct GemmPlan {
     int occ[kMaxCfgs] = {1, 1, 1, 1, 1};     // resident blocks per CU of each configuration
     bool occ_known = false;                  // cus and occ queried from the device
     long cap = 0;                            // grid of capped launches; 0: from occ and cus
-    int sk_cfg = -1;                         // split-K products: configuration timed fastest for
-    int sk_shape[4] = {0, 0, 0, 0};          //   this (M, N, K, role)
     bool trialed = false;                    // trailing-update tile chosen by whole trial factorisations
     double trial_ms[kMaxCfgs] = {};          // their times per configuration (0: not run): FP32 over `nt`,
                                              //   FP64 over `large`
@@ -212,6 +210,14 @@ int bem_fail(bem_ctx* c, int code, const std::string& msg);
 
 // Device scratch of at least `bytes` (reallocated when too small).
 int ctx_scratch(bem_ctx* c, size_t bytes, void** out);
+// O = B - Z X, or Z X without B, for the FP64 matrix and blocks of ncol vectors (npad x
+// ncol, planar; ncol a multiple of 16).
+int z_product(bem_ctx* c, int ncol, const double* Xr, const double* Xi, const double* Br, const double* Bi, double* Or,
+              double* Oi);
+// out[j] = sum over the rows i < n of |A[i][j]|^2, j < ncol, in a fixed order; part: work
+// area of col_norm2_work() values.
+size_t col_norm2_work(int n, int ncol);
+void col_norm2(hipStream_t s, int n, int ncol, const double* Ar, const double* Ai, long ld, double* part, double* out);
 // A host matrix of rows x cols interleaved complex values (row- or column-major) into
 // planar FP64 (prows x ld), padded with zeros, or with the identity; and planes
 // (times scale) into a host matrix.  Through at most 32 MiB of the context's scratch.

@@ -30,6 +30,7 @@
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef double v4d __attribute__((ext_vector_type(4)));
+typedef double v2d __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ v4f mfma16x16x4(float a, float b, v4f c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -138,9 +139,6 @@ __device__ __forceinline__ void vec_split<double>(const double2& v, double* o) {
 
 // ROLE 1 only names the instantiation (the LU trailing updates, so a
 // profiler lists them apart from the other products of the same tile).
-// ROLE 2 selects the 3M form in FP64: the refinement residual, whose
-// rounding (a few eps of |Z||X|) only has to stay far below the FP32
-// factors' error, takes three real products instead of four.
 template <typename T, int CFG, int ROLE = 0>
 __global__ __launch_bounds__(256, (GemmCfg<T, CFG>::MINB)) void k_cgemm(int M, int N, int K, const T* __restrict__ Ar,
                                                const T* __restrict__ Ai, long lda, const T* __restrict__ Br,
@@ -155,7 +153,7 @@ __global__ __launch_bounds__(256, (GemmCfg<T, CFG>::MINB)) void k_cgemm(int M, i
     constexpr int AV = (AVT + 255) / 256, BV = (BVT + 255) / 256;  // per thread
     typedef typename C::vec_t vec_t;
     typedef typename C::acc_t acc_t;
-    constexpr bool M3 = sizeof(T) == 4 || ROLE == 2;  // 3M form (FP32 always; FP64 for ROLE 2)
+    constexpr bool M3 = sizeof(T) == 4;  // 3M form
     constexpr int NACC = M3 ? 3 : 2;
 
     __shared__ T sA[2][2][BK][SA];
@@ -333,14 +331,6 @@ inline void cgemm_cfg(hipStream_t s, int M, int N, int K, const T* Ar, const T* 
     if (role == 1)
         hipLaunchKernelGGL((k_cgemm<T, CFG, 1>), dim3((unsigned)grid), dim3(256), 0, s, M, N, K, Ar, Ai, lda, Br, Bi,
                            ldb, Cr, Ci, ldc, mode, nb, sa, sb, sc);
-    else if constexpr (sizeof(T) == 8 && CFG != 0) {  // the 128 x 64 tile would spill in the 3M form
-        if (role == 2)
-            hipLaunchKernelGGL((k_cgemm<T, CFG, 2>), dim3((unsigned)grid), dim3(256), 0, s, M, N, K, Ar, Ai, lda, Br,
-                               Bi, ldb, Cr, Ci, ldc, mode, nb, sa, sb, sc);
-        else
-            hipLaunchKernelGGL((k_cgemm<T, CFG, 0>), dim3((unsigned)grid), dim3(256), 0, s, M, N, K, Ar, Ai, lda, Br,
-                               Bi, ldb, Cr, Ci, ldc, mode, nb, sa, sb, sc);
-    }
     else
         hipLaunchKernelGGL((k_cgemm<T, CFG, 0>), dim3((unsigned)grid), dim3(256), 0, s, M, N, K, Ar, Ai, lda, Br, Bi,
                            ldb, Cr, Ci, ldc, mode, nb, sa, sb, sc);
@@ -437,135 +427,6 @@ inline void cgemm_ctx(bem_ctx* c, int M, int N, int K, const T* Ar, const T* Ai,
     const double mnk = (double)M * N * K;
     const double bytes = 2.0 * sizeof(T) * ((double)M * K + (double)K * N + (mode == 1 ? 1.0 : 2.0) * M * N);
     kt_close(c, k, (sizeof(T) == 4 ? 6.0 : 8.0) * mnk, bytes);
-}
-
-// Sum of S split-K partial products (planes of M x N at P + 2 s M N, imaginary
-// plane M N further) into C: C -= sum (mode 0) or C = sum (mode 1), summed in
-// split order so results do not depend on scheduling.
-template <typename T>
-__global__ __launch_bounds__(256) void k_splitk_sum(long count, int N, int S, const T* __restrict__ P,
-                                                    T* __restrict__ Cr, T* __restrict__ Ci, long ldc, int mode) {
-    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= count) return;
-    T vr = T(0), vi = T(0);
-    for (int s = 0; s < S; s++) {
-        vr += P[2 * s * count + idx];
-        vi += P[(2 * s + 1) * count + idx];
-    }
-    const long o = (idx / N) * ldc + idx % N;
-    if (mode == 0) {
-        Cr[o] -= vr;
-        Ci[o] -= vi;
-    } else {
-        Cr[o] = vr;
-        Ci[o] = vi;
-    }
-}
-
-// Splits for a product whose output tiles leave the device's block slots
-// unevenly used (few tiles, long K): the smallest S in {1, 2, 4, 8, 16} whose
-// last round of blocks is at least 90 % full (else the fullest), with every
-// K slice a multiple of 16 and at least 512 long.
-template <typename T>
-inline int gemm_splits(bem_ctx* c, int cfg, int M, int N, int K) {
-    const GemmPlan& p = c->gemm_plan[sizeof(T) == 4 ? 0 : 1];
-    const long tiles = gemm_blocks<T>(cfg, M, N);
-    const long slots = (long)p.cus * (p.occ[cfg] > 0 ? p.occ[cfg] : 1);
-    int best = 1;
-    double best_eff = 0.0;
-    for (int S = 1; S <= 16; S *= 2) {
-        if (S > 1 && (K % (16 * S) != 0 || K / S < 512)) break;
-        const long blocks = tiles * S;
-        const double eff = (double)blocks / (double)(slots * ((blocks + slots - 1) / slots));
-        if (eff > best_eff + 1e-9) {
-            best = S;
-            best_eff = eff;
-        }
-        if (eff >= 0.9) break;
-    }
-    return best;
-}
-
-// One split-K product on configuration cfg with S splits: S batched partial
-// products into P (2 S M N values), summed into C by k_splitk_sum.
-template <typename T>
-inline void splitk_launch(bem_ctx* c, int cfg, int S, int M, int N, int K, const T* Ar, const T* Ai, long lda,
-                          const T* Br, const T* Bi, long ldb, T* P, T* Cr, T* Ci, long ldc, int mode, int role) {
-    if (S == 1) {
-        cgemm_any<T>(cfg, c->stream, M, N, K, Ar, Ai, lda, Br, Bi, ldb, Cr, Ci, ldc, mode, 1, 0, 0, 0, 0, role);
-        return;
-    }
-    const long count = (long)M * N;
-    const int Ks = K / S;
-    cgemm_any<T>(cfg, c->stream, M, N, Ks, Ar, Ai, lda, Br, Bi, ldb, P, P + count, N, 1, S, (long)Ks, (long)Ks * ldb,
-                 2 * count, 0, role);
-    hipLaunchKernelGGL(k_splitk_sum<T>, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, c->stream, count, N, S,
-                       (const T*)P, Cr, Ci, ldc, mode);
-}
-
-// C = C - A B (mode 0) or C = A B (mode 1) for products with few output tiles
-// and a long K (the refinement residual), with K split over S batched
-// products into the context's partial buffer, then summed in split order
-// (k_splitk_sum).  The configuration is chosen once per shape by timing
-// each one (with its own S) into a scratch output; the choice changes speed
-// only.
-template <typename T>
-inline int cgemm_splitk_ctx(bem_ctx* c, int M, int N, int K, const T* Ar, const T* Ai, long lda, const T* Br,
-                            const T* Bi, long ldb, T* Cr, T* Ci, long ldc, int mode, int role = 0) {
-    if (M <= 0 || N <= 0 || K <= 0) return 0;
-    gemm_plan_occupancy(c, sizeof(T) == 4);
-    GemmPlan& plan = c->gemm_plan[sizeof(T) == 4 ? 0 : 1];
-    const long count = (long)M * N;
-    int Smax = 1;
-    for (int cfg = 0; cfg < kGemmCfgs; cfg++) Smax = std::max(Smax, gemm_splits<T>(c, cfg, M, N, K));
-    const size_t bytes = (2 * (size_t)Smax + 2) * count * sizeof(T);  // partials + a scratch output
-    if (c->part_bytes < bytes) {
-        if (c->part) (void)hipFree(c->part);
-        c->part = nullptr;
-        c->part_bytes = 0;
-        if (hipMalloc(&c->part, bytes) != hipSuccess) return bem_fail(c, BEM_ERR_NOMEM, "split-K partial products");
-        c->part_bytes = bytes;
-    }
-    T* P = static_cast<T*>(c->part);
-    if (plan.sk_cfg < 0 || plan.sk_shape[0] != M || plan.sk_shape[1] != N || plan.sk_shape[2] != K ||
-        plan.sk_shape[3] != role) {
-        T* Xr = P + 2 * (size_t)Smax * count;  // scratch output, ld N
-        hipEvent_t e0 = nullptr, e1 = nullptr;
-        if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
-            if (e0) (void)hipEventDestroy(e0);
-            return bem_fail(c, BEM_ERR_HIP, "split-K tuning: events");
-        }
-        float best_ms = 0.0f;
-        int best = gemm_choose<T>(c, M, N);
-        for (int cfg = 0; cfg < kGemmCfgs; cfg++) {
-            const int S = gemm_splits<T>(c, cfg, M, N, K);
-            (void)hipEventRecord(e0, c->stream);
-            splitk_launch<T>(c, cfg, S, M, N, K, Ar, Ai, lda, Br, Bi, ldb, P, Xr, Xr + count, N, 1, role);
-            (void)hipEventRecord(e1, c->stream);
-            if (hipEventSynchronize(e1) != hipSuccess) break;
-            float ms = 0.0f;
-            (void)hipEventElapsedTime(&ms, e0, e1);
-            if (ms > 0.0f && (best_ms == 0.0f || ms < best_ms)) {
-                best_ms = ms;
-                best = cfg;
-            }
-        }
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
-        plan.sk_cfg = best;
-        plan.sk_shape[0] = M;
-        plan.sk_shape[1] = N;
-        plan.sk_shape[2] = K;
-        plan.sk_shape[3] = role;
-    }
-    const int cfg = plan.sk_cfg;
-    const int S = gemm_splits<T>(c, cfg, M, N, K);
-    const double fl = (sizeof(T) == 4 || (role == 2 && cfg != 0) ? 6.0 : 8.0) * (double)M * N * K;
-    const double b = 2.0 * sizeof(T) * ((double)M * K + (double)K * N + (2.0 * S + (mode == 1 ? 1.0 : 2.0)) * count);
-    const int k = kt_mark(c, sizeof(T) == 4 ? KS_GEMM32 : KS_GEMM64, c->stream);
-    splitk_launch<T>(c, cfg, S, M, N, K, Ar, Ai, lda, Br, Bi, ldb, P, Cr, Ci, ldc, mode, role);
-    kt_close(c, k, fl, b);
-    return 0;
 }
 
 // ---------------------------------------------------------------------------

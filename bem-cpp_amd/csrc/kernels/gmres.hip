@@ -7,8 +7,7 @@
 // of the exterior-only matrix A_ext = [[eta L_ext, -K_ext], [K_ext,
 // L_ext/eta]] as preconditioner, python/bem_core.py:1071-1101).  Here every
 // right-hand side runs its own Krylov process in lock step with the others:
-// one matvec per iteration is one FP64 complex GEMM Z V (n x n x nrhs, 3M
-// form, split K), one preconditioner application is one multi-RHS solve with
+// one matvec per iteration is one FP64 product Z V (zmul.hip), one preconditioner application is one multi-RHS solve with
 // the factors on the device (FP32 factors on the matrix cores, or FP64), or
 // the block-Jacobi / RAS preconditioner of precond.hip, or none.
 // The factors may belong to an earlier matrix: with the factors of Z at
@@ -118,25 +117,6 @@ __global__ __launch_bounds__(256) void k_gs_update(long count, int ncol, int m, 
     wi[o] = ai;
 }
 
-// out[j] = sum_k |w[k][j]|^2 over k < n, one block per column, fixed order.
-__global__ __launch_bounds__(256) void k_colnorm2_ld(int n, int ncol, const double* __restrict__ wr,
-                                                     const double* __restrict__ wi, double* __restrict__ out) {
-    __shared__ double red[256];
-    const int j = blockIdx.x;
-    double s = 0.0;
-    for (int k = threadIdx.x; k < n; k += 256) {
-        const double a = wr[(long)k * ncol + j], b = wi[(long)k * ncol + j];
-        s += a * a + b * b;
-    }
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[j] = red[0];
-}
-
 // dst[k][j] = src[k][j] * s[j] (s real per column)
 __global__ __launch_bounds__(256) void k_scale_cols(long count, int ncol, const double* __restrict__ sr,
                                                     const double* __restrict__ si, const double* __restrict__ s,
@@ -164,7 +144,7 @@ int gmres_solve_launch(bem_ctx* c, int nrhs, double tol, int restart, int max_it
     // each), Gram-Schmidt partials and products, column scales, preconditioner work
     const size_t vec = 2 * (size_t)cnt;  // doubles per planar block vector
     const size_t nP = 2 * (size_t)(m + 1) * nchunk * ncol, nH = 2 * (size_t)(m + 1) * ncol;
-    const size_t doubles = vec * (2 * (size_t)m + 3) + nP + 2 * nH + 2 * (size_t)ncol;
+    const size_t doubles = vec * (2 * (size_t)m + 3) + nP + 2 * nH + 2 * (size_t)ncol + col_norm2_work(nphys, ncol);
     const size_t pwork = precond == BEM_PRECOND_LU ? lu_precond_work_bytes(c)
                          : precond == BEM_PRECOND_BLOCK ? bj_work_bytes(c)
                                                         : 0;
@@ -180,8 +160,8 @@ int gmres_solve_launch(bem_ctx* c, int nrhs, double tol, int restart, int max_it
     double* H = P + nP;                     // Gram-Schmidt products (two passes)
     double* H2 = H + nH;
     double* cs = H2 + nH;                   // column scales
-    double* nrm = cs + ncol;                // column norms
-    char* pw = reinterpret_cast<char*>(nrm + ncol);
+    double* nrm = cs + ncol;                // column norms, then their partial sums
+    char* pw = reinterpret_cast<char*>(nrm + ncol + col_norm2_work(nphys, ncol));
     pw += (256 - reinterpret_cast<uintptr_t>(pw) % 256) % 256;
     void* work = pw;
     auto re = [&](double* v) { return v; };
@@ -192,18 +172,13 @@ int gmres_solve_launch(bem_ctx* c, int nrhs, double tol, int restart, int max_it
 
     std::vector<double> hn2(ncol), bn2(ncol), rn2(ncol), scale(ncol);
     auto colnorm2 = [&](const double* vr, const double* vi, std::vector<double>& out) -> int {
-        hipLaunchKernelGGL(k_colnorm2_ld, dim3(ncol), dim3(256), 0, s, nphys, ncol, vr, vi, nrm);
+        col_norm2(s, nphys, ncol, vr, vi, ncol, nrm + ncol, nrm);
         BEM_HIP(c, hipMemcpyAsync(out.data(), nrm, ncol * sizeof(double), hipMemcpyDeviceToHost, s));
         BEM_HIP(c, hipStreamSynchronize(s));
         return 0;
     };
-    // r = B - Z X (FP64, 3M form, split K)
-    auto residual = [&]() -> int {
-        BEM_HIP(c, hipMemcpyAsync(re(r), c->Br, cnt * sizeof(double), hipMemcpyDeviceToDevice, s));
-        BEM_HIP(c, hipMemcpyAsync(im(r), c->Bi, cnt * sizeof(double), hipMemcpyDeviceToDevice, s));
-        return cgemm_splitk_ctx<double>(c, n, ncol, n, c->Zr, c->Zi, n, c->Xr, c->Xi, ncol, re(r), im(r), ncol, 0,
-                                        2);
-    };
+    // r = B - Z X
+    auto residual = [&]() -> int { return z_product(c, ncol, c->Xr, c->Xi, c->Br, c->Bi, re(r), im(r)); };
     auto max_rel = [&](const std::vector<double>& r2) {
         double mx = 0.0;
         for (int j = 0; j < nrhs; j++) mx = std::max(mx, bn2[j] > 0 ? std::sqrt(r2[j] / bn2[j]) : 0.0);
@@ -275,9 +250,7 @@ int gmres_solve_launch(bem_ctx* c, int nrhs, double tol, int restart, int max_it
             else
                 BEM_HIP(c, hipMemcpyAsync(Zk(it), Vk(it), vec * sizeof(double), hipMemcpyDeviceToDevice, s));
             if (prc) return prc;
-            if (int rc = cgemm_splitk_ctx<double>(c, n, ncol, n, c->Zr, c->Zi, n, re(Zk(it)), im(Zk(it)), ncol, re(w),
-                                                  im(w), ncol, 1, 2))
-                return rc;
+            if (int rc = z_product(c, ncol, re(Zk(it)), im(Zk(it)), nullptr, nullptr, re(w), im(w))) return rc;
             // classical Gram-Schmidt, twice
             gs_products(it + 1, H);
             gs_products(it + 1, H2);
