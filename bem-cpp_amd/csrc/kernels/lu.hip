@@ -30,6 +30,7 @@
 #include <vector>
 
 #include "../bem_internal.h"
+#include "cmul.h"
 #include "gemm.h"
 #include "gemm_nt.h"
 #include "trsm.h"
@@ -1261,18 +1262,17 @@ __global__ __launch_bounds__(512) void k_u12_strip(T* __restrict__ Ar, T* __rest
     }
 }
 
-// Inverses of the 32 x 32 diagonal triangles of every 256 x 256 diagonal block
-// (block p at F + p NB (ldf + 1)) into the diagonals of the zeroed blocks Li, Ui
-// (block p at p NB NB, ld NB): blockIdx.x = triangle, blockIdx.y = 0 unit lower, 1
-// upper.  One wave each, the triangle staged in LDS, lane j forms column j by
+// Inverses of the 32 x 32 diagonal triangles of the factors at F into the diagonals of
+// the blocks L, U (block p at p IB IB, ld IB), with their zeros: blockIdx.x = triangle,
+// blockIdx.y = 0 unit lower, 1 upper.  One wave each, the triangle staged in LDS, lane j forms column j by
 // substitution in registers.
 template <typename T>
 __global__ __launch_bounds__(64) void k_inv_tri32(const T* __restrict__ Fr, const T* __restrict__ Fi, long ldf,
                                                   T* __restrict__ Lr, T* __restrict__ Li, T* __restrict__ Ur,
                                                   T* __restrict__ Ui) {
     __shared__ T sr[PB][PB + 1], si[PB][PB + 1];
-    const int lane = threadIdx.x, p = blockIdx.x / (NB / PB), d = blockIdx.x % (NB / PB);
-    const long f = (long)(p * NB + d * PB) * (ldf + 1), o = (long)p * NB * NB + (long)d * PB * (NB + 1);
+    const int lane = threadIdx.x, p = blockIdx.x / (IB / PB), d = blockIdx.x % (IB / PB);
+    const long f = (long)blockIdx.x * PB * (ldf + 1), o = (long)p * IB * IB + (long)d * PB * (IB + 1);
 #pragma unroll
     for (int u = 0; u < PB * PB / 64; u++) {
         const int e = lane + 64 * u, r = e / PB, q = e % PB;
@@ -1313,80 +1313,40 @@ __global__ __launch_bounds__(64) void k_inv_tri32(const T* __restrict__ Fr, cons
 #pragma unroll
     for (int v = 0; v < PB; v++) {
         const int row = lower ? v : PB - 1 - v;
-        outr[o + (long)row * NB + j] = xr[v];
-        outi[o + (long)row * NB + j] = xi[v];
+        outr[o + (long)row * IB + j] = xr[v];
+        outi[o + (long)row * IB + j] = xi[v];
     }
 }
 
-// One product of the doubling of the block inverses: every pair of h x h diagonal
-// inverses (h = 16 KQ) of every 256 x 256 block is joined,
+// One product of joining the diagonal inverses of all IB x IB blocks in pairs of h rows:
 //   lower [X11 0; X21 X22]  with X21 = -X22 (L21 X11),
 //   upper [X11 X12; 0 X22]  with X12 = -X11 (U12 X22)
-// (blockIdx.z = 0, 1; blockIdx.y = pair of all blocks; stage 0: W = the inner
-// product, 1: the outer one).  FP32 in the 3M form, no LDS and no barrier: a
-// wave owns one 16 x 16 tile over the whole K and issues every operand load before
-// the first product.
-template <int KQ>
-__global__ __launch_bounds__(256) void k_tri_join(int stage, const float* __restrict__ Fr,
-                                                  const float* __restrict__ Fi, long ldf, float* Lr, float* Li,
-                                                  float* Ur, float* Ui, float* Wr, float* Wi) {
-    constexpr int h = 16 * KQ, pairs = NB / (2 * h), nt = h / 16;
-    const int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (tile >= nt * nt) return;
+// (blockIdx.z = 0, 1; blockIdx.y = pair of all blocks; stage 0: the inner product W, to the
+// unused triangle of the block, 1: the outer one).  The sums run over the triangles
+// only, so that no value beside them is read; the 32 x 32 triangles at the start are
+// stored with their zeros.
+__global__ __launch_bounds__(256, 2) void k_tri_join(int stage, int h, const float* __restrict__ Fr,
+                                                     const float* __restrict__ Fi, long ldf, float* Lr, float* Li,
+                                                     float* Ur, float* Ui) {
+    constexpr int NT = 2;
+    __shared__ __align__(16) float red[4 * 2 * 16 * 16 * NT];
     const bool lower = blockIdx.z == 0;
-    const int p = blockIdx.y / pairs, d = (blockIdx.y % pairs) * 2 * h;
-    const long fo = (long)(p * NB + d) * (ldf + 1), xo = (long)p * NB * NB + (long)d * (NB + 1);
-    const long wo = ((long)blockIdx.z * gridDim.y + blockIdx.y) * h * h;
-    float* Xr = lower ? Lr : Ur;
-    float* Xi = lower ? Li : Ui;
-    const long x11 = xo, x22 = xo + (long)h * (NB + 1), x21 = xo + (long)h * NB, x12 = xo + h;
-    const float *ar, *ai, *br, *bi;
-    float *cr, *ci;
-    long lda, ldb, ldc;
+    const int nct = h / (16 * NT), m0 = blockIdx.x / nct * 16, n0 = blockIdx.x % nct * 16 * NT;
+    const int np = IB / (2 * h), blk = blockIdx.y / np, d = blockIdx.y % np * 2 * h;
+    const long f = ((long)blk * IB + d) * (ldf + 1), x = (long)blk * IB * IB + (long)d * (IB + 1);
+    float* Xr = (lower ? Lr : Ur) + x;
+    float* Xi = (lower ? Li : Ui) + x;
+    const long x22 = (long)h * (IB + 1), x21 = (long)h * IB, x12 = h;
+    const long o = lower ? x21 : x12, w = lower ? x12 : x21;
     if (stage == 0) {
-        const long f = lower ? fo + (long)h * ldf : fo + h;
-        const long b = lower ? x11 : x22;
-        ar = Fr + f, ai = Fi + f, lda = ldf;
-        br = Xr + b, bi = Xi + b, ldb = NB;
-        cr = Wr + wo, ci = Wi + wo, ldc = h;
+        const long a = f + (lower ? (long)h * ldf : h), b = lower ? 0 : x22;
+        cmul_tile<NT>(m0, n0, lower ? n0 : 0, lower ? h : n0 + 16 * NT, Fr + a, Fi + a, ldf, Xr + b, Xi + b, IB, Xr + w,
+                      Xi + w, IB, 1, red);
     } else {
-        const long a = lower ? x22 : x11, o = lower ? x21 : x12;
-        ar = Xr + a, ai = Xi + a, lda = NB;
-        br = Wr + wo, bi = Wi + wo, ldb = h;
-        cr = Xr + o, ci = Xi + o, ldc = NB;
+        const long a = lower ? x22 : 0;
+        cmul_tile<NT>(m0, n0, lower ? 0 : m0, lower ? m0 + 16 : h, Xr + a, Xi + a, IB, Xr + w, Xi + w, IB, Xr + o,
+                      Xi + o, IB, 3, red);
     }
-    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    const int m0 = tile / nt * 16, n0 = tile % nt * 16;
-    v4f a0[KQ], a1[KQ];
-    float b0[KQ][4], b1[KQ][4];
-    const long oa = (long)(m0 + r) * lda + 4 * g;
-#pragma unroll
-    for (int q = 0; q < KQ; q++) {
-        a0[q] = *reinterpret_cast<const v4f*>(ar + oa + 16 * q);
-        a1[q] = *reinterpret_cast<const v4f*>(ai + oa + 16 * q);
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const long ob = (long)(16 * q + 4 * g + e) * ldb + n0 + r;
-            b0[q][e] = br[ob];
-            b1[q][e] = bi[ob];
-        }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    v4f t1 = v4f{0.f, 0.f, 0.f, 0.f}, t2 = t1, t3 = t1;
-#pragma unroll
-    for (int q = 0; q < KQ; q++) {
-        const v4f a2 = a0[q] + a1[q];
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            t1 = mfma16x16x4(b0[q][e], a0[q][e], t1);
-            t2 = mfma16x16x4(b1[q][e], a1[q][e], t2);
-            t3 = mfma16x16x4(b0[q][e] + b1[q][e], a2[e], t3);
-        }
-    }
-    const v4f pr = t1 - t2, pi = t3 - t1 - t2;
-    const long oc = (long)(m0 + r) * ldc + n0 + 4 * g;
-    *reinterpret_cast<v4f*>(cr + oc) = stage == 0 ? pr : -pr;
-    *reinterpret_cast<v4f*>(ci + oc) = stage == 0 ? pi : -pi;
 }
 
 // Work buffers of one factorisation (device).
@@ -1400,7 +1360,7 @@ struct LuWork {
     T* d11;          // factored 32 x 32 diagonal block (2 planes), two sets by step parity
     T *cpr, *cpi;    // compact copies (n x 32 per plane) of the columns being factored, two sets by step parity
     T *sur, *sui;    // U12 of the next 32 columns (32 x 32)
-    T *utr, *uti;    // n x 256 transpose of U12 (FP32 trailing update), then the products of the inverses
+    T *utr, *uti;    // n x 256 transpose of U12 (FP32 trailing update)
     int* net;        // net row interchanges of an outer panel, two sets
 };
 
@@ -1411,22 +1371,17 @@ int* panel_net(const LuWork<T>& w, int k0) {
     return w.net + ((k0 / NB) & 1) * NETS;
 }
 
-// L^{-1} and U^{-1} of the NB x NB diagonal blocks of the FP32 factors at F into
-// the blocks at L and U (zeroed), all blocks in each launch: the 32 x 32 diagonal
-// triangles by substitution, then joined in pairs three times.  For the solves;
-// the factorisation itself does not use them.
-void invert_blocks(hipStream_t s, int nb, const float* Fr, const float* Fi, long ldf, float* Lr, float* Li, float* Ur,
-                   float* Ui, float* Wr, float* Wi) {
-    hipLaunchKernelGGL(k_inv_tri32<float>, dim3(nb * (NB / PB), 2), dim3(64), 0, s, Fr, Fi, ldf, Lr, Li, Ur, Ui);
-    for (int stage = 0; stage < 2; stage++)
-        hipLaunchKernelGGL(k_tri_join<2>, dim3(1, 4 * nb, 2), dim3(256), 0, s, stage, Fr, Fi, ldf, Lr, Li, Ur, Ui, Wr,
-                           Wi);
-    for (int stage = 0; stage < 2; stage++)
-        hipLaunchKernelGGL(k_tri_join<4>, dim3(4, 2 * nb, 2), dim3(256), 0, s, stage, Fr, Fi, ldf, Lr, Li, Ur, Ui, Wr,
-                           Wi);
-    for (int stage = 0; stage < 2; stage++)
-        hipLaunchKernelGGL(k_tri_join<8>, dim3(16, nb, 2), dim3(256), 0, s, stage, Fr, Fi, ldf, Lr, Li, Ur, Ui, Wr,
-                           Wi);
+// L^{-1} and U^{-1} of the IB x IB diagonal blocks of the n x n FP32 factors at F into the
+// blocks at L and U (ld IB, block b at b IB IB), all blocks in each launch: the 32 x 32
+// diagonal triangles by substitution, then joined in pairs.  For the solves; the
+// factorisation itself does not use them.
+void invert_blocks(hipStream_t s, int n, const float* Fr, const float* Fi, long ldf, float* Lr, float* Li, float* Ur,
+                   float* Ui) {
+    hipLaunchKernelGGL(k_inv_tri32<float>, dim3(n / PB, 2), dim3(64), 0, s, Fr, Fi, ldf, Lr, Li, Ur, Ui);
+    for (int h = PB; h < IB; h *= 2)
+        for (int stage = 0; stage < 2; stage++)
+            hipLaunchKernelGGL(k_tri_join, dim3(h / 16 * (h / 32), n / (2 * h), 2), dim3(256), 0, s, stage, h, Fr, Fi,
+                               ldf, Lr, Li, Ur, Ui);
 }
 
 // Factors the outer panel of columns k0 .. k0+NB-1 (rows k0 .. n-1) on stream
@@ -1563,8 +1518,8 @@ void factor(bem_ctx* c, T* Ar, T* Ai, T* Lir, T* Lii, T* Uir, T* Uii, const LuWo
     // the diagonal blocks themselves)
     if constexpr (sizeof(T) == 4) {
         const int kt = kt_mark(c, KS_TRSM, us);
-        invert_blocks(us, nb, Ar, Ai, ld, Lir, Lii, Uir, Uii, w.utr, w.uti);
-        kt_close(c, kt, 16.0 * (double)n * NB * NB / 6.0, 8.0 * sizeof(T) * (double)n * NB);
+        invert_blocks(us, n, Ar, Ai, ld, Lir, Lii, Uir, Uii);
+        kt_close(c, kt, 16.0 * (double)n * IB * IB / 6.0, 8.0 * sizeof(T) * (double)n * IB);
     }
 }
 
@@ -1579,7 +1534,7 @@ int factor_prec(bem_ctx* c, T* Ar, T* Ai, void*& inv, size_t& inv_bytes) {
     const int n = c->npad;
     // diagonal-block inverses (FP32 only): L and U, npad x NB per plane each
     constexpr bool with_inv = sizeof(T) == 4;
-    const size_t ib = 4 * (size_t)n * NB * sizeof(T);
+    const size_t ib = 4 * (size_t)n * IB * sizeof(T);
     if (with_inv && inv_bytes < ib) {
         if (inv) (void)hipFree(inv);
         inv = nullptr;
@@ -1588,9 +1543,9 @@ int factor_prec(bem_ctx* c, T* Ar, T* Ai, void*& inv, size_t& inv_bytes) {
         inv_bytes = ib;
     }
     T* Lir = with_inv ? static_cast<T*>(inv) : nullptr;
-    T* Lii = with_inv ? Lir + (size_t)n * NB : nullptr;
-    T* Uir = with_inv ? Lii + (size_t)n * NB : nullptr;
-    T* Uii = with_inv ? Uir + (size_t)n * NB : nullptr;
+    T* Lii = with_inv ? Lir + (size_t)n * IB : nullptr;
+    T* Uir = with_inv ? Lii + (size_t)n * IB : nullptr;
+    T* Uii = with_inv ? Uir + (size_t)n * IB : nullptr;
     // work: info, counters, row-pair list, candidate ids, candidate values,
     // diagonal blocks, compact columns, U12 buffers
     const int nsets0 = (n + 255) / 256;
@@ -1619,8 +1574,6 @@ int factor_prec(bem_ctx* c, T* Ar, T* Ai, void*& inv, size_t& inv_bytes) {
     w.utr = w.cpi + 2 * (size_t)PB * n;
     w.uti = w.utr + (size_t)NB * n;
     BEM_HIP(c, hipMemsetAsync(w.info, 0, (64 + ncnt) * sizeof(int), c->stream));
-    // the triangles beside the inverses stay zero
-    if (with_inv) BEM_HIP(c, hipMemsetAsync(Lir, 0, 4 * (size_t)n * NB * sizeof(T), c->stream));
     factor<T>(c, Ar, Ai, Lir, Lii, Uir, Uii, w);
     return 0;
 }

@@ -1,5 +1,6 @@
-"""The FP64 residual of the refinement at the edges of its kernels: one to several groups
-of one to five column tiles, split and unsplit sums, rows and columns of padding."""
+"""The FP32 solves and the FP64 residual of the refinement at the edges of their kernels:
+one to several groups of one to five column tiles, one- and two-level solves, split and
+unsplit sums, rows and columns of padding."""
 import numpy as np
 import pytest
 
@@ -9,7 +10,7 @@ EPS = 2.3e-16
 
 
 @pytest.mark.parametrize("n,nrhs", [(1, 1), (250, 1), (257, 17), (300, 48), (700, 64), (513, 65), (1030, 129),
-                                    (260, 209), (770, 1100)])
+                                    (260, 209), (770, 1100), (8200, 17)])
 def test_refinement_residual(bem, n, nrhs):
     print(f"residual n={n} nrhs={nrhs}", flush=True)
     rs = np.random.RandomState(n + nrhs)
