@@ -233,11 +233,10 @@ __device__ __forceinline__ void half_pair(const Mom& m, double kr, double ki, do
     K.i = cc * km[1];
 }
 
-// Writes the 9 half-pair values of pair (t, s) to their slots; `corr` (self
-// pairs only) holds the symmetrised static part per wavenumber and half pair.
+// Writes the 9 half-pair values of pair (t, s) to their slots.
 __device__ __forceinline__ void write_record(double* __restrict__ H, int ntile, const int* __restrict__ hrwg,
                                              const Mom* mom, const AsmParams& p, const double* __restrict__ hc,
-                                             const double* __restrict__ hp, int t, int s, const C2* corr) {
+                                             const double* __restrict__ hp, int t, int s) {
 #pragma unroll 1
     for (int a = 0; a < 3; a++) {
         const double ca = hc[t * 3 + a];
@@ -251,13 +250,7 @@ __device__ __forceinline__ void write_record(double* __restrict__ H, int ntile, 
             const double pb[3] = {hp[(s * 3 + b) * 3], hp[(s * 3 + b) * 3 + 1], hp[(s * 3 + b) * 3 + 2]};
             C2 L[2], K[2];
 #pragma unroll
-            for (int kk = 0; kk < 2; kk++) {
-                half_pair(mom[kk], p.kr[kk], p.ki[kk], ca, pa, cb, pb, L[kk], K[kk]);
-                if (corr) {
-                    L[kk].r += corr[kk * 9 + a * 3 + b].r;
-                    L[kk].i += corr[kk * 9 + a * 3 + b].i;
-                }
-            }
+            for (int kk = 0; kk < 2; kk++) half_pair(mom[kk], p.kr[kk], p.ki[kk], ca, pa, cb, pb, L[kk], K[kk]);
             store_slot(H, slot, dup,
                        make_double2(p.eta[0] * L[0].r + p.eta[1] * L[1].r, p.eta[0] * L[0].i + p.eta[1] * L[1].i),
                        make_double2(L[0].r / p.eta[0] + L[1].r / p.eta[1], L[0].i / p.eta[0] + L[1].i / p.eta[1]),
@@ -272,12 +265,10 @@ __device__ __forceinline__ void cmac(double acc[2], const double a[2], double x,
     acc[1] = fma(a[0], y, fma(a[1], x, acc[1]));
 }
 
-// Writes the 9 half-pair values of pair (t, s) combined with q (RecCoef);
-// `sv` (self pairs, moments of G only) holds the static parts vec_ab (9
-// values) and S_P (sv[9]), which enter U and V with c_a c_b / (4 pi).
+// Writes the 9 half-pair values of pair (t, s) combined with q (RecCoef).
 __device__ __forceinline__ void write_record_coef(double* __restrict__ H, int ntile, const int* __restrict__ hrwg,
                                                   const Mom* mom, const RecCoef& q, const double* __restrict__ hc,
-                                                  const double* __restrict__ hp, int t, int s, const double* sv) {
+                                                  const double* __restrict__ hp, int t, int s) {
 #pragma unroll 1
     for (int a = 0; a < 3; a++) {
         const double ca = hc[t * 3 + a];
@@ -296,10 +287,6 @@ __device__ __forceinline__ void write_record_coef(double* __restrict__ H, int nt
                 double lm[2], km[2];
                 raw_parts(mom[w], pa, pb, lm, km);
                 double U[2] = {cc * lm[0], cc * lm[1]}, V[2] = {cc * mom[w].m0[0], cc * mom[w].m0[1]};
-                if (sv) {
-                    U[0] += cc * kInv4Pi * sv[a * 3 + b];
-                    V[0] += cc * kInv4Pi * sv[9];
-                }
                 cmac(P, q.aP[w], U[0], U[1]);
                 cmac(P, q.bP[w], V[0], V[1]);
                 cmac(Q, q.aQ[w], U[0], U[1]);
@@ -402,10 +389,10 @@ __global__ __launch_bounds__(256) void k_tripair_far(int T, const double4* __res
         mom_fold(mom[1], in1, P);
     }
     if (MODE == 0) {
-        write_record(H, ntile, hrwg, mom, p, hc, hp, t, s, nullptr);
+        write_record(H, ntile, hrwg, mom, p, hc, hp, t, s);
     } else {
 #pragma unroll 1
-        for (int j = 0; j < q.n; j++) write_record_coef(q.H[j], ntile, hrwg, mom, q.q[j], hc, hp, t, s, nullptr);
+        for (int j = 0; j < q.n; j++) write_record_coef(q.H[j], ntile, hrwg, mom, q.q[j], hc, hp, t, s);
     }
 }
 
@@ -504,134 +491,189 @@ __global__ __launch_bounds__(256) void k_graglia(int T, const double4* __restric
 //                                                 + (p_a.p_b) S_P) ]
 // with S_P = sum jw P, S_Pr = sum jw P r, S_V = sum jw V, S_rV = sum jw r.V.
 // ---------------------------------------------------------------------------
+// One lane per test point and wavenumber: NearLanes<NQ> = 2 P lanes of a wave take a pair
+// (P >= NQ a power of two), lane i + P kk the inner sums of test point i for wavenumber
+// kk; the moments are summed across the P lanes, which then take half pairs i, i + P, ..
+// each.  With a thread per pair, NQ^2 pairs of FP64 sincos and exponential followed one
+// another in a few workgroups: 99 us for the 2176 pairs at 2N = 240 (94 us at 4608;
+// 13 points at 960: 212 us), now 12 us (13 points: 21).
+template <int NQ>
+struct NearLanes {
+    static constexpr int P = NQ <= 1 ? 1 : NQ <= 2 ? 2 : NQ <= 4 ? 4 : NQ <= 8 ? 8 : NQ <= 16 ? 16 : 32;
+    static_assert(NQ <= 32, "a pair's lanes lie in one wave");
+};
+
+template <int P>
+__device__ __forceinline__ double lanes_sum(double v) {
+#pragma unroll
+    for (int w = 1; w < P; w *= 2) v += __shfl_xor(v, w);
+    return v;
+}
+
 template <int NQ, int MODE>
-__global__ __launch_bounds__(128) void k_tripair_near(int T, int n_near, const int2* __restrict__ pairs,
+__global__ __launch_bounds__(256) void k_tripair_near(int T, int n_near, const int2* __restrict__ pairs,
                                                       const double4* __restrict__ qp,
                                                       const double* __restrict__ hc,
                                                       const double* __restrict__ hp,
                                                       const double4* __restrict__ pv,
                                                       const int* __restrict__ hrwg, int ntile, AsmParams p,
                                                       RecCoefSet q, double* __restrict__ H) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= n_near) return;
+    constexpr int P = NearLanes<NQ>::P;
+    const int idx = (blockIdx.x * 256 + threadIdx.x) / (2 * P);
+    if (idx >= n_near) return;  // whole groups of lanes; shuffles stay inside a group
+    const int sub = threadIdx.x % (2 * P), i = sub % P, kk = sub / P;
     const int t = pairs[idx].x, s = pairs[idx].y;
     const bool self = t == s;
+    const double kr = p.kr[kk], ki = p.ki[kk];
     // In MODE 2 the R = 0 value of a self pair depends on the coefficient
     // set, so such a pair forms its moments once per set.
     const int nmom = (MODE == 2 && self) ? q.n : 1;
 #pragma unroll 1
     for (int js = 0; js < nmom; js++) {
-        Mom mom[2];
-        mom_zero(mom[0]);
-        mom_zero(mom[1]);
-#pragma unroll 1
-        for (int i = 0; i < NQ; i++) {
-            const double4 P = qp[t * NQ + i];
-            Inner in[2];
-            inner_zero(in[0]);
-            inner_zero(in[1]);
+        Mom mom;
+        mom_zero(mom);
+        if (i < NQ) {
+            const double4 X = qp[t * NQ + i];
+            Inner in;
+            inner_zero(in);
 #pragma unroll 1
             for (int j = 0; j < NQ; j++) {
                 const double4 Q = qp[s * NQ + j];
-                const double dx = P.x - Q.x, dy = P.y - Q.y, dz = P.z - Q.z;
+                const double dx = X.x - Q.x, dy = X.y - Q.y, dz = X.z - Q.z;
                 const double r2 = dx * dx + dy * dy + dz * dz;
                 const double R = sqrt(r2);
-#pragma unroll
-                for (int kk = 0; kk < 2; kk++) {
-                    const double kr = p.kr[kk], ki = p.ki[kk];
-                    double Gr, Gi, gr = 0.0, gi = 0.0;
-                    if (self && R < 1e-12) {
-                        if (MODE == 2) {
-                            Gr = q.q[js].r0[kk][0];
-                            Gi = q.q[js].r0[kk][1];
-                        } else {
-                            Gr = 0.0;
-                            Gi = kr * kInv4Pi;
-                        }
+                double Gr, Gi, gr = 0.0, gi = 0.0;
+                if (self && R < 1e-12) {
+                    if (MODE == 2) {
+                        Gr = q.q[js].r0[kk][0];
+                        Gi = q.q[js].r0[kk][1];
                     } else {
-                        double sn, cs;
-                        sincos(kr * R, &sn, &cs);
-                        const double amp = exp(-ki * R) * kInv4Pi / R;
-                        Gr = amp * cs;
-                        Gi = amp * sn;
-                        const bool with_g = !self && R > 1e-6;
-                        if (MODE == 2) {  // dG/dk = iR G (the static 1/(4 pi R) has none), dg/dk = -k G
-                            if (with_g) {
-                                gr = -(kr * Gr - ki * Gi);
-                                gi = -(kr * Gi + ki * Gr);
-                            }
-                            const double t0 = -R * Gi;
-                            Gi = R * Gr;
-                            Gr = t0;
-                        } else {
-                            if (with_g) {
-                                const double ar = (-ki - 1.0 / R) / R, ai = kr / R;
-                                gr = Gr * ar - Gi * ai;
-                                gi = Gr * ai + Gi * ar;
-                            }
-                            if (self) Gr -= kInv4Pi / R;
-                        }
+                        Gr = 0.0;
+                        Gi = kr * kInv4Pi;
                     }
-                    inner_add(in[kk], Q.w, Gr, Gi, gr, gi, Q);
+                } else {
+                    double sn, cs;
+                    sincos(kr * R, &sn, &cs);
+                    const double amp = exp(-ki * R) * kInv4Pi / R;
+                    Gr = amp * cs;
+                    Gi = amp * sn;
+                    const bool with_g = !self && R > 1e-6;
+                    if (MODE == 2) {  // dG/dk = iR G (the static 1/(4 pi R) has none), dg/dk = -k G
+                        if (with_g) {
+                            gr = -(kr * Gr - ki * Gi);
+                            gi = -(kr * Gi + ki * Gr);
+                        }
+                        const double t0 = -R * Gi;
+                        Gi = R * Gr;
+                        Gr = t0;
+                    } else {
+                        if (with_g) {
+                            const double ar = (-ki - 1.0 / R) / R, ai = kr / R;
+                            gr = Gr * ar - Gi * ai;
+                            gi = Gr * ai + Gi * ar;
+                        }
+                        if (self) Gr -= kInv4Pi / R;
+                    }
                 }
+                inner_add(in, Q.w, Gr, Gi, gr, gi, Q);
             }
-            mom_fold(mom[0], in[0], P);
-            mom_fold(mom[1], in[1], P);
+            mom_fold(mom, in, X);
         }
-        if (!self || MODE == 2) {
-            if (MODE == 0) {
-                write_record(H, ntile, hrwg, mom, p, hc, hp, t, s, nullptr);
-            } else {
-                const int j0 = nmom > 1 ? js : 0, j1 = nmom > 1 ? js + 1 : q.n;
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            mom.m0[c] = lanes_sum<P>(mom.m0[c]);
+            mom.mrs[c] = lanes_sum<P>(mom.mrs[c]);
+#pragma unroll
+            for (int e = 0; e < 3; e++) {
+                mom.mr[e][c] = lanes_sum<P>(mom.mr[e][c]);
+                mom.ms[e][c] = lanes_sum<P>(mom.ms[e][c]);
+                mom.nx[e][c] = lanes_sum<P>(mom.nx[e][c]);
+                mom.nd[e][c] = lanes_sum<P>(mom.nd[e][c]);
+            }
+        }
+        // static part of self pairs
+        double SP = 0.0, SPV[3] = {0, 0, 0}, SrV = 0.0;  // SPV = S_Pr + S_V
+        if (self && MODE != 2) {
+            if (i < NQ) {
+                const double4 x = qp[t * NQ + i];
+                const double4 w = pv[t * NQ + i];  // (P, Vx, Vy, Vz)
+                SP = x.w * w.x;
+                SPV[0] = x.w * w.x * x.x + x.w * w.y;
+                SPV[1] = x.w * w.x * x.y + x.w * w.z;
+                SPV[2] = x.w * w.x * x.z + x.w * w.w;
+                SrV = x.w * (x.x * w.y + x.y * w.z + x.z * w.w);
+            }
+            SP = lanes_sum<P>(SP);
+            SrV = lanes_sum<P>(SrV);
+#pragma unroll
+            for (int e = 0; e < 3; e++) SPV[e] = lanes_sum<P>(SPV[e]);
+        }
 #pragma unroll 1
-                for (int j = j0; j < j1; j++)
-                    write_record_coef(q.H[j], ntile, hrwg, mom, q.q[j], hc, hp, t, s, nullptr);
-            }
-            continue;
-        }
-        double SP = 0.0, SPr[3] = {0, 0, 0}, SV[3] = {0, 0, 0}, SrV = 0.0;
-        for (int iq = 0; iq < NQ; iq++) {
-            const double4 x = qp[t * NQ + iq];
-            const double4 w = pv[t * NQ + iq];  // (P, Vx, Vy, Vz)
-            SP += x.w * w.x;
-            SPr[0] += x.w * w.x * x.x;
-            SPr[1] += x.w * w.x * x.y;
-            SPr[2] += x.w * w.x * x.z;
-            SV[0] += x.w * w.y;
-            SV[1] += x.w * w.z;
-            SV[2] += x.w * w.w;
-            SrV += x.w * (x.x * w.y + x.y * w.z + x.z * w.w);
-        }
-        C2 corr[18];
-        double sv[10];
-        sv[9] = SP;
-        for (int a = 0; a < 3; a++)
-            for (int b = 0; b < 3; b++) {
-                const double ca = hc[t * 3 + a], cb = hc[t * 3 + b];
-                const double* pa = hp + (t * 3 + a) * 3;
-                const double* pb = hp + (t * 3 + b) * 3;
+        for (int ab = i; ab < 9; ab += P) {
+            const int a = ab / 3, b = ab % 3;
+            long long dup;
+            const long long slot = half_pair_slot(hrwg, hc, t, a, s, b, ntile, &dup);
+            if (slot < 0) continue;  // the same for both wavenumbers
+            const double ca = hc[t * 3 + a], cb = hc[s * 3 + b], cc = ca * cb;
+            const double pa[3] = {hp[(t * 3 + a) * 3], hp[(t * 3 + a) * 3 + 1], hp[(t * 3 + a) * 3 + 2]};
+            const double pb[3] = {hp[(s * 3 + b) * 3], hp[(s * 3 + b) * 3 + 1], hp[(s * 3 + b) * 3 + 2]};
+            double vec = 0.0;  // static part, real
+            if (self && MODE != 2) {
                 double sym = 0.0, papb = 0.0;
+#pragma unroll
                 for (int e = 0; e < 3; e++) {
-                    sym += (pa[e] + pb[e]) * (SPr[e] + SV[e]);
+                    sym += (pa[e] + pb[e]) * SPV[e];
                     papb += pa[e] * pb[e];
                 }
-                const double vec = SrV - 0.5 * sym + papb * SP;  // real
-                sv[a * 3 + b] = vec;
-                for (int kk = 0; kk < 2; kk++) {
-                    const double kr = p.kr[kk], ki = p.ki[kk], k2 = kr * kr + ki * ki;
-                    // -(4i/k) SP + ik vec, i/k = (ki + i kr)/|k|^2, ik = -ki + i kr
-                    const double re = -4.0 * ki / k2 * SP - ki * vec;
-                    const double im = -4.0 * kr / k2 * SP + kr * vec;
-                    const double f = ca * cb * kInv4Pi;
-                    corr[kk * 9 + a * 3 + b].r = f * re;
-                    corr[kk * 9 + a * 3 + b].i = f * im;
-                }
+                vec = SrV - 0.5 * sym + papb * SP;
             }
-        if (MODE == 0) {
-            write_record(H, ntile, hrwg, mom, p, hc, hp, t, t, corr);
-        } else {
+            const int j0 = nmom > 1 ? js : 0, j1 = MODE == 0 ? 1 : nmom > 1 ? js + 1 : q.n;
 #pragma unroll 1
-            for (int j = 0; j < q.n; j++) write_record_coef(q.H[j], ntile, hrwg, mom, q.q[j], hc, hp, t, t, sv);
+            for (int j = j0; j < j1; j++) {
+                double o[6];  // this wavenumber's share of the slot: P, Q, K
+                if (MODE == 0) {
+                    C2 L, K;
+                    half_pair(mom, kr, ki, ca, pa, cb, pb, L, K);
+                    if (self) {
+                        // -(4i/k) SP + ik vec, i/k = (ki + i kr)/|k|^2, ik = -ki + i kr
+                        const double k2 = kr * kr + ki * ki, f = cc * kInv4Pi;
+                        L.r += f * (-4.0 * ki / k2 * SP - ki * vec);
+                        L.i += f * (-4.0 * kr / k2 * SP + kr * vec);
+                    }
+                    o[0] = p.eta[kk] * L.r;
+                    o[1] = p.eta[kk] * L.i;
+                    o[2] = L.r / p.eta[kk];
+                    o[3] = L.i / p.eta[kk];
+                    o[4] = K.r;
+                    o[5] = K.i;
+                } else {
+                    const RecCoef& u = q.q[j];
+                    double lm[2], km[2];
+                    raw_parts(mom, pa, pb, lm, km);
+                    double U[2] = {cc * lm[0], cc * lm[1]}, V[2] = {cc * mom.m0[0], cc * mom.m0[1]};
+                    if (self && MODE != 2) {
+                        U[0] += cc * kInv4Pi * vec;
+                        V[0] += cc * kInv4Pi * SP;
+                    }
+                    double A[2] = {0.0, 0.0}, B[2] = {0.0, 0.0}, K[2] = {0.0, 0.0};
+                    cmac(A, u.aP[kk], U[0], U[1]);
+                    cmac(A, u.bP[kk], V[0], V[1]);
+                    cmac(B, u.aQ[kk], U[0], U[1]);
+                    cmac(B, u.bQ[kk], V[0], V[1]);
+                    cmac(K, u.cK[kk], cc * km[0], cc * km[1]);
+                    o[0] = A[0];
+                    o[1] = A[1];
+                    o[2] = B[0];
+                    o[3] = B[1];
+                    o[4] = K[0];
+                    o[5] = K[1];
+                }
+#pragma unroll
+                for (int e = 0; e < 6; e++) o[e] += __shfl_xor(o[e], P);
+                if (kk == 0)
+                    store_slot(MODE == 0 ? H : q.H[j], slot, dup, make_double2(o[0], o[1]), make_double2(o[2], o[3]),
+                               make_double2(o[4], o[5]));
+            }
         }
     }
 }
@@ -852,8 +894,9 @@ void launch_records(bem_ctx* c, const AsmParams& p, const RecCoefSet& q, bool lo
     kt_close(c, kt, npair * NQ * NQ, npair * kRec * 8.0);  // unit: triangle point pairs
     kt = kt_mark(c, KS_TRIPAIR_NEAR);
     if (d.n_near > 0)
-        hipLaunchKernelGGL((k_tripair_near<NQ, MODE>), dim3((d.n_near + 127) / 128), dim3(128), 0, c->stream, T,
-                           d.n_near, d.near, d.qp, d.hc, d.hp, d.pv, d.hrwg, ntile, p, q, c->H);
+        hipLaunchKernelGGL((k_tripair_near<NQ, MODE>),
+                           dim3((unsigned)(((long)d.n_near * 2 * NearLanes<NQ>::P + 255) / 256)), dim3(256), 0,
+                           c->stream, T, d.n_near, d.near, d.qp, d.hc, d.hp, d.pv, d.hrwg, ntile, p, q, c->H);
     kt_close(c, kt, (double)d.n_near * NQ * NQ, (double)d.n_near * kRec * 8.0);
 }
 
