@@ -158,40 +158,40 @@ __device__ __forceinline__ void inner_zero(Inner& s) {
     for (int e = 0; e < 3; e++) s.b[e][0] = s.b[e][1] = s.c[e][0] = s.c[e][1] = 0.0;
 }
 
-__device__ __forceinline__ void inner_add(Inner& s, double w, double Gr, double Gi, double gr, double gi,
-                                          const double4& q) {
-    const double wGr = w * Gr, wGi = w * Gi, wgr = w * gr, wgi = w * gi;
-    s.a[0] += wGr;
-    s.a[1] += wGi;
-    s.d[0] += wgr;
-    s.d[1] += wgi;
-    s.b[0][0] = fma(wGr, q.x, s.b[0][0]); s.b[0][1] = fma(wGi, q.x, s.b[0][1]);
-    s.b[1][0] = fma(wGr, q.y, s.b[1][0]); s.b[1][1] = fma(wGi, q.y, s.b[1][1]);
-    s.b[2][0] = fma(wGr, q.z, s.b[2][0]); s.b[2][1] = fma(wGi, q.z, s.b[2][1]);
-    s.c[0][0] = fma(wgr, q.x, s.c[0][0]); s.c[0][1] = fma(wgi, q.x, s.c[0][1]);
-    s.c[1][0] = fma(wgr, q.y, s.c[1][0]); s.c[1][1] = fma(wgi, q.y, s.c[1][1]);
-    s.c[2][0] = fma(wgr, q.z, s.c[2][0]); s.c[2][1] = fma(wgi, q.z, s.c[2][1]);
+// q: w_j and w_j r_j.
+__device__ __forceinline__ void inner_add(Inner& s, double Gr, double Gi, double gr, double gi, const double4& q) {
+    s.a[0] = fma(Gr, q.w, s.a[0]);
+    s.a[1] = fma(Gi, q.w, s.a[1]);
+    s.d[0] = fma(gr, q.w, s.d[0]);
+    s.d[1] = fma(gi, q.w, s.d[1]);
+    s.b[0][0] = fma(Gr, q.x, s.b[0][0]); s.b[0][1] = fma(Gi, q.x, s.b[0][1]);
+    s.b[1][0] = fma(Gr, q.y, s.b[1][0]); s.b[1][1] = fma(Gi, q.y, s.b[1][1]);
+    s.b[2][0] = fma(Gr, q.z, s.b[2][0]); s.b[2][1] = fma(Gi, q.z, s.b[2][1]);
+    s.c[0][0] = fma(gr, q.x, s.c[0][0]); s.c[0][1] = fma(gi, q.x, s.c[0][1]);
+    s.c[1][0] = fma(gr, q.y, s.c[1][0]); s.c[1][1] = fma(gi, q.y, s.c[1][1]);
+    s.c[2][0] = fma(gr, q.z, s.c[2][0]); s.c[2][1] = fma(gi, q.z, s.c[2][1]);
+}
+__device__ __forceinline__ double4 weighted(const double4& q) {
+    return make_double4(q.w * q.x, q.w * q.y, q.w * q.z, q.w);
 }
 
 // Folds the inner sums of test point p (weight p.w) into the moments.
 __device__ __forceinline__ void mom_fold(Mom& m, const Inner& s, const double4& p) {
     const double w = p.w;
-    const double r[3] = {p.x, p.y, p.z};
+    const double r[3] = {w * p.x, w * p.y, w * p.z};
 #pragma unroll
     for (int c = 0; c < 2; c++) {
         m.m0[c] = fma(w, s.a[c], m.m0[c]);
-        double dotb = 0.0;
 #pragma unroll
         for (int e = 0; e < 3; e++) {
-            m.mr[e][c] = fma(w * r[e], s.a[c], m.mr[e][c]);
+            m.mr[e][c] = fma(r[e], s.a[c], m.mr[e][c]);
             m.ms[e][c] = fma(w, s.b[e][c], m.ms[e][c]);
-            dotb = fma(r[e], s.b[e][c], dotb);
-            m.nd[e][c] = fma(w, r[e] * s.d[c] - s.c[e][c], m.nd[e][c]);
+            m.mrs[c] = fma(r[e], s.b[e][c], m.mrs[c]);
+            m.nd[e][c] = fma(r[e], s.d[c], fma(-w, s.c[e][c], m.nd[e][c]));
         }
-        m.mrs[c] = fma(w, dotb, m.mrs[c]);
-        m.nx[0][c] = fma(w, r[1] * s.c[2][c] - r[2] * s.c[1][c], m.nx[0][c]);
-        m.nx[1][c] = fma(w, r[2] * s.c[0][c] - r[0] * s.c[2][c], m.nx[1][c]);
-        m.nx[2][c] = fma(w, r[0] * s.c[1][c] - r[1] * s.c[0][c], m.nx[2][c]);
+        m.nx[0][c] = fma(r[1], s.c[2][c], fma(-r[2], s.c[1][c], m.nx[0][c]));
+        m.nx[1][c] = fma(r[2], s.c[0][c], fma(-r[0], s.c[2][c], m.nx[1][c]));
+        m.nx[2][c] = fma(r[0], s.c[1][c], fma(-r[1], s.c[0][c], m.nx[2][c]));
     }
 }
 
@@ -237,6 +237,7 @@ __device__ __forceinline__ void half_pair(const Mom& m, double kr, double ki, do
 __device__ __forceinline__ void write_record(double* __restrict__ H, int ntile, const int* __restrict__ hrwg,
                                              const Mom* mom, const AsmParams& p, const double* __restrict__ hc,
                                              const double* __restrict__ hp, int t, int s) {
+    const double ie[2] = {1.0 / p.eta[0], 1.0 / p.eta[1]};
 #pragma unroll 1
     for (int a = 0; a < 3; a++) {
         const double ca = hc[t * 3 + a];
@@ -253,7 +254,7 @@ __device__ __forceinline__ void write_record(double* __restrict__ H, int ntile, 
             for (int kk = 0; kk < 2; kk++) half_pair(mom[kk], p.kr[kk], p.ki[kk], ca, pa, cb, pb, L[kk], K[kk]);
             store_slot(H, slot, dup,
                        make_double2(p.eta[0] * L[0].r + p.eta[1] * L[1].r, p.eta[0] * L[0].i + p.eta[1] * L[1].i),
-                       make_double2(L[0].r / p.eta[0] + L[1].r / p.eta[1], L[0].i / p.eta[0] + L[1].i / p.eta[1]),
+                       make_double2(ie[0] * L[0].r + ie[1] * L[1].r, ie[0] * L[0].i + ie[1] * L[1].i),
                        make_double2(K[0].r + K[1].r, K[0].i + K[1].i));
         }
     }
@@ -309,20 +310,27 @@ __device__ __forceinline__ bool touching(const int4& a, const int4& b) {
 // ---------------------------------------------------------------------------
 // MODE 0: forward records; 1: RecCoef records of the moments of G, g;
 // 2: RecCoef records of the moments of dG/dk = iR G and dg/dk = -k G.
+// Bound by VALU issue, most of it FP64 (8 cycles an instruction and wave here): some
+// 70 FP64 and 80 FP32 instructions per point pair and, per triangle pair, 9 records.
+// The source functions w, w r come ready from LDS, the folds are plain FMAs, and the loop
+// over j stays rolled, so that two waves fit a SIMD: unrolled (290 registers, one
+// wave) it took 731 us at 2N = 4608 and 9.5 ms at 18432, now 466 us and 6.5 ms; three
+// waves spill (18.6 ms with the gather instead of 11.0).
 template <int NQ, bool LOSSY, int MODE>
-__global__ __launch_bounds__(256) void k_tripair_far(int T, const double4* __restrict__ qp,
+__global__ __launch_bounds__(256, 2) void k_tripair_far(int T, const double4* __restrict__ qp,
                                                      const int4* __restrict__ tv, const double* __restrict__ hc,
                                                      const double* __restrict__ hp, const int* __restrict__ hrwg,
                                                      int ntile, AsmParams p, RecCoefSet q,
                                                      double* __restrict__ H) {
     const int bt = blockIdx.y, bs = blockIdx.x;
     if (bt > bs) return;
-    __shared__ double4 sT[16 * NQ], sS[16 * NQ];
+    __shared__ double4 sT[16 * NQ], sS[16 * NQ], sW[16 * NQ];
     __shared__ int4 vT[16], vS[16];
     for (int i = threadIdx.x; i < 16 * NQ; i += 256) {
         const int t = bt * 16 + i / NQ, s = bs * 16 + i / NQ;
         sT[i] = t < T ? qp[t * NQ + i % NQ] : make_double4(0, 0, 0, 0);
         sS[i] = s < T ? qp[s * NQ + i % NQ] : make_double4(0, 0, 0, 0);
+        sW[i] = weighted(sS[i]);
     }
     if (threadIdx.x < 16) {
         const int t = bt * 16 + threadIdx.x, s = bs * 16 + threadIdx.x;
@@ -348,9 +356,9 @@ __global__ __launch_bounds__(256) void k_tripair_far(int T, const double4* __res
         Inner in0, in1;
         inner_zero(in0);
         inner_zero(in1);
-#pragma unroll
+#pragma unroll 1
         for (int j = 0; j < NQ; j++) {
-            const double4 Q = sS[tj * NQ + j];
+            const double4 Q = sS[tj * NQ + j], W = sW[tj * NQ + j];
             const double dx = P.x - Q.x, dy = P.y - Q.y, dz = P.z - Q.z;
             const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
             double y = (double)__builtin_amdgcn_rsqf((float)r2);
@@ -365,10 +373,10 @@ __global__ __launch_bounds__(256) void k_tripair_far(int T, const double4* __res
                 const float Gr = a0 * cs, Gi = a0 * sn;
                 if (MODE == 2) {
                     const float Rf = (float)R;
-                    inner_add(in0, Q.w, -Rf * Gi, Rf * Gr, -(krf0 * Gr - kif0 * Gi), -(krf0 * Gi + kif0 * Gr), Q);
+                    inner_add(in0, -Rf * Gi, Rf * Gr, -(krf0 * Gr - kif0 * Gi), -(krf0 * Gi + kif0 * Gr), W);
                 } else {
                     const float ar = (-kif0 - invR) * invR, ai = krf0 * invR;
-                    inner_add(in0, Q.w, Gr, Gi, Gr * ar - Gi * ai, Gr * ai + Gi * ar, Q);
+                    inner_add(in0, Gr, Gi, Gr * ar - Gi * ai, Gr * ai + Gi * ar, W);
                 }
             }
             {  // interior wavenumber
@@ -378,10 +386,10 @@ __global__ __launch_bounds__(256) void k_tripair_far(int T, const double4* __res
                 const float Gr = a1 * cs, Gi = a1 * sn;
                 if (MODE == 2) {
                     const float Rf = (float)R;
-                    inner_add(in1, Q.w, -Rf * Gi, Rf * Gr, -(krf1 * Gr - kif1 * Gi), -(krf1 * Gi + kif1 * Gr), Q);
+                    inner_add(in1, -Rf * Gi, Rf * Gr, -(krf1 * Gr - kif1 * Gi), -(krf1 * Gi + kif1 * Gr), W);
                 } else {
                     const float ar = (-kif1 - invR) * invR, ai = krf1 * invR;
-                    inner_add(in1, Q.w, Gr, Gi, Gr * ar - Gi * ai, Gr * ai + Gi * ar, Q);
+                    inner_add(in1, Gr, Gi, Gr * ar - Gi * ai, Gr * ai + Gi * ar, W);
                 }
             }
         }
@@ -524,7 +532,7 @@ __global__ __launch_bounds__(256) void k_tripair_near(int T, int n_near, const i
     const int sub = threadIdx.x % (2 * P), i = sub % P, kk = sub / P;
     const int t = pairs[idx].x, s = pairs[idx].y;
     const bool self = t == s;
-    const double kr = p.kr[kk], ki = p.ki[kk];
+    const double kr = p.kr[kk], ki = p.ki[kk], ie = 1.0 / p.eta[kk];
     // In MODE 2 the R = 0 value of a self pair depends on the coefficient
     // set, so such a pair forms its moments once per set.
     const int nmom = (MODE == 2 && self) ? q.n : 1;
@@ -575,7 +583,7 @@ __global__ __launch_bounds__(256) void k_tripair_near(int T, int n_near, const i
                         if (self) Gr -= kInv4Pi / R;
                     }
                 }
-                inner_add(in, Q.w, Gr, Gi, gr, gi, Q);
+                inner_add(in, Gr, Gi, gr, gi, weighted(Q));
             }
             mom_fold(mom, in, X);
         }
@@ -642,8 +650,8 @@ __global__ __launch_bounds__(256) void k_tripair_near(int T, int n_near, const i
                     }
                     o[0] = p.eta[kk] * L.r;
                     o[1] = p.eta[kk] * L.i;
-                    o[2] = L.r / p.eta[kk];
-                    o[3] = L.i / p.eta[kk];
+                    o[2] = ie * L.r;
+                    o[3] = ie * L.i;
                     o[4] = K.r;
                     o[5] = K.i;
                 } else {
