@@ -77,9 +77,9 @@ __global__ __launch_bounds__(256) void k_bj_gather(BjView v, int N, int ld, cons
 // (k_bj_panel, then k_bj_inner for the other 48 columns of the panel), then
 // the rest of the matrix takes one rank-64 product (k_bj_rows, k_bj_update).
 //
-// What bounds it: the panels' serial chain of pivot steps (98 us per 16
-// columns at 1107 unknowns, blocks side by side), then the rank-64 FP64
-// products (175 us each).  26 blocks of up to 1107 unknowns: 15 ms, where one
+// What bounds it: the rank-64 FP64 products (186 us each) and the panels' serial
+// chain of pivot steps (45 us per 16 columns at 1107 unknowns, blocks side by
+// side).  27 blocks of up to 1107 unknowns: 8.3 ms, where one
 // workgroup sweeping its whole block from memory at every pivot step (the
 // earlier form) took 1600 ms, n2^2 complex values moved per step.
 // ---------------------------------------------------------------------------
@@ -94,6 +94,74 @@ __device__ __forceinline__ unsigned bj_key(double r, double i) {
     return m >= 0.0 ? (unsigned)((unsigned long long)__double_as_longlong(m) >> 32) + 1u : 1u;
 }
 extern "C" __device__ unsigned __ockl_wfred_max_u32(unsigned);
+
+// Columns of unrolled elimination steps; the registers rotate by so many after them.
+// (All 16 steps unrolled, each row read ahead whole and with two selects per value
+// for the pivot row, spilled: 98 us per panel of 1107 rows, 45 now.)
+constexpr int BJ_S = 4;
+
+// Entries BJ_S .. to the front, the first BJ_S to the end.
+__device__ __forceinline__ void bj_rotate(double (&x)[BJ_W]) {
+    double h[BJ_S];
+#pragma unroll
+    for (int c = 0; c < BJ_S; c++) h[c] = x[c];
+#pragma unroll
+    for (int c = 0; c < BJ_W - BJ_S; c++) x[c] = x[c + BJ_S];
+#pragma unroll
+    for (int c = 0; c < BJ_S; c++) x[BJ_W - BJ_S + c] = h[c];
+}
+
+// The BJ_W columns of rows i0 .. i0+63 from / to memory (rows n2 and beyond: some other
+// row, nothing), row i0 + lane in the lane's registers.  Four lanes take 64 bytes of a row
+// side by side and the wave's part of LDS turns them (a lane read its own row, 16
+// bytes of 64 lines per load).  The LDS operations of a wave
+// stay in order, so the buffer needs no barrier.
+struct alignas(16) BjStage {
+    double x[64][BJ_W / 2 + 2];
+};
+__device__ __forceinline__ void bj_load_rows(const double* __restrict__ a, int ld, int i0, int n2, BjStage& st,
+                                             double (&x)[BJ_W]) {
+    const int lane = threadIdx.x & 63, r = lane / 4, c = 2 * (lane % 4);
+    v2d v[2][4];
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int i = min(i0 + 16 * u + r, n2 - 1);
+            v[h][u] = *reinterpret_cast<const v2d*>(a + (long)i * ld + 8 * h + c);
+        }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) *reinterpret_cast<v2d*>(&st.x[16 * u + r][c]) = v[h][u];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const v2d y = *reinterpret_cast<const v2d*>(&st.x[lane][2 * k]);
+            x[8 * h + 2 * k] = y[0];
+            x[8 * h + 2 * k + 1] = y[1];
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+__device__ __forceinline__ void bj_store_rows(double* __restrict__ a, int ld, int i0, int n2, BjStage& st,
+                                              const double (&x)[BJ_W]) {
+    const int lane = threadIdx.x & 63, r = lane / 4, c = 2 * (lane % 4);
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            *reinterpret_cast<v2d*>(&st.x[lane][2 * k]) = v2d{x[8 * h + 2 * k], x[8 * h + 2 * k + 1]};
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int i = i0 + 16 * u + r;
+            if (i < n2)
+                *reinterpret_cast<v2d*>(a + (long)i * ld + 8 * h + c) = *reinterpret_cast<const v2d*>(&st.x[16 * u + r][c]);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
 
 // Elimination of columns c0 .. c0+15 of every block, one workgroup each.
 // RPT > 0: the panel's rows in registers, rows t + BJ_T r, r < RPT (n2 <= RPT
@@ -111,6 +179,7 @@ __global__ __launch_bounds__(BJ_T) void k_bj_panel(BjView v, int ld, int c0, int
     __shared__ unsigned long long kb[NW];
     __shared__ double row_r[BJ_W], row_i[BJ_W];
     __shared__ int prows[BJ_W];
+    __shared__ BjStage stage[RPT > 0 ? NW : 1];
     const int b = blockIdx.x, t = threadIdx.x, wave = t >> 6;
     const int n2 = 2 * v.Be[b];
     if (c0 >= n2) return;
@@ -125,120 +194,143 @@ __global__ __launch_bounds__(BJ_T) void k_bj_panel(BjView v, int ld, int c0, int
         for (int q = 0; q < R; q++) {
             const int i = t + BJ_T * q;
             used[q] = i < n2 ? st[i] : 0;
-#pragma unroll
-            for (int c = 0; c < BJ_W; c++) {
-                xr[q][c] = i < n2 ? ar[(long)i * ld + c] : 0.0;  // columns beyond n2 are zero (ld is a multiple of 64)
-                xi[q][c] = i < n2 ? ai[(long)i * ld + c] : 0.0;
-            }
+            bj_load_rows(ar, ld, i - (t & 63), n2, stage[wave], xr[q]);
+            bj_load_rows(ai, ld, i - (t & 63), n2, stage[wave], xi[q]);
         }
     }
+#pragma unroll 1
+    for (int s = 0; s < BJ_W; s += BJ_S) {
+        // register c holds column (c + s) % BJ_W of the panel
 #pragma unroll
-    for (int j = 0; j < BJ_W; j++) {
-        if (j < w) {  // the same for the whole workgroup; a break would keep the loop from unrolling
-        unsigned key = 0;
-        int best = 0x7fffffff;
+        for (int j = 0; j < BJ_S; j++) {
+            if (s + j < w) {  // the same for the whole workgroup; a break would keep the loop from unrolling
+                unsigned key = 0;
+                int best = 0x7fffffff;
+                if constexpr (RPT > 0) {
+#pragma unroll
+                    for (int q = 0; q < R; q++) {
+                        const unsigned k = used[q] < 0 ? bj_key(xr[q][j], xi[q][j]) : 0u;
+                        if (k > key) {
+                            key = k;
+                            best = t + BJ_T * q;
+                        }
+                    }
+                } else {
+                    for (int i = t; i < n2; i += BJ_T) {
+                        const unsigned k =
+                            st[i] < 0 ? bj_key(ar[(long)i * ld + s + j], ai[(long)i * ld + s + j]) : 0u;
+                        if (k > key) {
+                            key = k;
+                            best = i;
+                        }
+                    }
+                }
+                const unsigned wk = __ockl_wfred_max_u32(key);
+                const int lane = __ffsll((long long)__ballot(key == wk)) - 1;
+                if ((t & 63) == lane) kb[wave] = ((unsigned long long)wk << 32) | (0xffffffffu - (unsigned)best);
+                __syncthreads();
+                unsigned long long kbest = kb[0];
+#pragma unroll
+                for (int q = 1; q < NW; q++) kbest = max(kbest, kb[q]);
+                const int p = (int)(0xffffffffu - (unsigned)kbest);  // some row is unused: n2 pivots over n2 steps
+                if (p % BJ_T == t) {
+                    if constexpr (RPT > 0) {
+#pragma unroll
+                        for (int q = 0; q < R; q++)
+                            if (p == t + BJ_T * q) {
+                                used[q] = c0 + s + j;
+#pragma unroll
+                                for (int c = 0; c < BJ_W; c++) {
+                                    row_r[c] = xr[q][c];
+                                    row_i[c] = xi[q][c];
+                                    xr[q][c] = xi[q][c] = 0.0;
+                                }
+                            }
+                    } else {
+#pragma unroll
+                        for (int c = 0; c < BJ_W; c++) {
+                            const long o = (long)p * ld + (c + s) % BJ_W;
+                            row_r[c] = ar[o];
+                            row_i[c] = ai[o];
+                            ar[o] = ai[o] = 0.0;
+                        }
+                    }
+                    st[p] = c0 + s + j;
+                    prows[s + j] = p;
+                }
+                __syncthreads();
+                double dr = row_r[j], di = row_i[j];
+                if (dr * dr + di * di < 1e-60) {
+                    dr = 1e-15;
+                    di = 0.0;
+                }
+                const double inv = 1.0 / (dr * dr + di * di), qr = dr * inv, qi = -di * inv;  // 1 / pivot
+                // row i: a_ic -= g u_c (c != j), a_ij = -g, g = a_ij / pivot; the pivot
+                // row, cleared above, the same with g = -1 / pivot: a_pc = u_c / pivot,
+                // a_pj = 1 / pivot
+                auto eliminate = [&](int i0, double (&yr)[R][BJ_W], double (&yi)[R][BJ_W]) {
+                    double gr[R], gi[R];
+#pragma unroll
+                    for (int q = 0; q < R; q++) {
+                        const bool piv = i0 + BJ_T * q == p;
+                        const double fr = yr[q][j], fi = yi[q][j];
+                        gr[q] = piv ? -qr : fr * qr - fi * qi;
+                        gi[q] = piv ? -qi : fr * qi + fi * qr;
+                    }
+#pragma unroll
+                    for (int c = 0; c < BJ_W; c++) {
+                        if (c != j) {
+                            const double ur = row_r[c], ui = row_i[c];
+#pragma unroll
+                            for (int q = 0; q < R; q++) {
+                                yr[q][c] = fma(gi[q], ui, fma(-gr[q], ur, yr[q][c]));
+                                yi[q][c] = fma(-gi[q], ur, fma(-gr[q], ui, yi[q][c]));
+                            }
+                        }
+                        // (more of the row read ahead does not fit in the registers)
+                        if (c % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                    }
+#pragma unroll
+                    for (int q = 0; q < R; q++) {
+                        yr[q][j] = -gr[q];
+                        yi[q][j] = -gi[q];
+                    }
+                };
+                if constexpr (RPT > 0) {
+                    eliminate(t, xr, xi);
+                } else {
+                    for (int i = t; i < n2; i += BJ_T) {
+#pragma unroll
+                        for (int c = 0; c < BJ_W; c++) {
+                            xr[0][c] = ar[(long)i * ld + (c + s) % BJ_W];
+                            xi[0][c] = ai[(long)i * ld + (c + s) % BJ_W];
+                        }
+                        eliminate(i, xr, xi);
+#pragma unroll
+                        for (int c = 0; c < BJ_W; c++) {
+                            ar[(long)i * ld + (c + s) % BJ_W] = xr[0][c];
+                            ai[(long)i * ld + (c + s) % BJ_W] = xi[0][c];
+                        }
+                    }
+                }
+                // (a thread reads the row before it reaches the next step's first
+                // barrier, the keys before this step's second)
+            }
+        }
         if constexpr (RPT > 0) {
 #pragma unroll
             for (int q = 0; q < R; q++) {
-                const unsigned k = used[q] < 0 ? bj_key(xr[q][j], xi[q][j]) : 0u;
-                if (k > key) {
-                    key = k;
-                    best = t + BJ_T * q;
-                }
+                bj_rotate(xr[q]);
+                bj_rotate(xi[q]);
             }
-        } else {
-            for (int i = t; i < n2; i += BJ_T) {
-                const unsigned k = st[i] < 0 ? bj_key(ar[(long)i * ld + j], ai[(long)i * ld + j]) : 0u;
-                if (k > key) {
-                    key = k;
-                    best = i;
-                }
-            }
-        }
-        const unsigned wk = __ockl_wfred_max_u32(key);
-        const int lane = __ffsll((long long)__ballot(key == wk)) - 1;
-        if ((t & 63) == lane) kb[wave] = ((unsigned long long)wk << 32) | (0xffffffffu - (unsigned)best);
-        __syncthreads();
-        unsigned long long kbest = kb[0];
-#pragma unroll
-        for (int q = 1; q < NW; q++) kbest = max(kbest, kb[q]);
-        const int p = (int)(0xffffffffu - (unsigned)kbest);  // some row is unused: n2 pivots over n2 steps
-        if (p % BJ_T == t) {
-            if constexpr (RPT > 0) {
-#pragma unroll
-                for (int q = 0; q < R; q++)
-                    if (p == t + BJ_T * q) {
-                        used[q] = c0 + j;
-#pragma unroll
-                        for (int c = 0; c < BJ_W; c++) {
-                            row_r[c] = xr[q][c];
-                            row_i[c] = xi[q][c];
-                        }
-                    }
-            } else {
-                for (int c = 0; c < BJ_W; c++) {
-                    row_r[c] = ar[(long)p * ld + c];
-                    row_i[c] = ai[(long)p * ld + c];
-                }
-            }
-            st[p] = c0 + j;
-            prows[j] = p;
-        }
-        __syncthreads();
-        double dr = row_r[j], di = row_i[j];
-        if (hypot(dr, di) < 1e-30) {
-            dr = 1e-15;
-            di = 0.0;
-        }
-        const double inv = 1.0 / (dr * dr + di * di), qr = dr * inv, qi = -di * inv;  // 1 / pivot
-        // row i: a_ic -= g u_c (c != j), a_ij = -g, g = a_ij / pivot; the pivot
-        // row: a_pc = u_c / pivot, a_pj = 1 / pivot
-        auto eliminate = [&](int i, double (&yr)[BJ_W], double (&yi)[BJ_W]) {
-            const bool piv = i == p;
-            const double fr = yr[j], fi = yi[j];
-            const double gr = piv ? -qr : fr * qr - fi * qi, gi = piv ? -qi : fr * qi + fi * qr;
-#pragma unroll
-            for (int c = 0; c < BJ_W; c++) {
-                if (c == j) continue;
-                const double ur = row_r[c], ui = row_i[c];
-                const double br = piv ? 0.0 : yr[c], bi = piv ? 0.0 : yi[c];
-                yr[c] = br - (gr * ur - gi * ui);
-                yi[c] = bi - (gr * ui + gi * ur);
-            }
-            yr[j] = -gr;
-            yi[j] = -gi;
-        };
-        if constexpr (RPT > 0) {
-#pragma unroll
-            for (int q = 0; q < R; q++) eliminate(t + BJ_T * q, xr[q], xi[q]);
-        } else {
-            for (int i = t; i < n2; i += BJ_T) {
-#pragma unroll
-                for (int c = 0; c < BJ_W; c++) {
-                    xr[0][c] = ar[(long)i * ld + c];
-                    xi[0][c] = ai[(long)i * ld + c];
-                }
-                eliminate(i, xr[0], xi[0]);
-#pragma unroll
-                for (int c = 0; c < BJ_W; c++) {
-                    ar[(long)i * ld + c] = xr[0][c];
-                    ai[(long)i * ld + c] = xi[0][c];
-                }
-            }
-        }
-        __syncthreads();  // the row and the keys are read before the next step writes them
         }
     }
     if constexpr (RPT > 0) {
 #pragma unroll
         for (int q = 0; q < R; q++) {
             const int i = t + BJ_T * q;
-            if (i >= n2) continue;
-#pragma unroll
-            for (int c = 0; c < BJ_W; c++) {
-                ar[(long)i * ld + c] = xr[q][c];
-                ai[(long)i * ld + c] = xi[q][c];
-            }
+            bj_store_rows(ar, ld, i - (t & 63), n2, stage[wave], xr[q]);
+            bj_store_rows(ai, ld, i - (t & 63), n2, stage[wave], xi[q]);
         }
     }
     if (t < w) prow[v.poff[b] + c0 + t] = prows[t];
