@@ -668,7 +668,7 @@ int rhs_launch(bem_ctx* c, double kr, double ki, double eta, const double* khat,
     }
     void* s = nullptr;
     if (int rc = ctx_scratch(c, prm.size() * sizeof(double), &s)) return rc;
-    BEM_HIP(c, hipMemcpyAsync(s, prm.data(), prm.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    if (int rc = ctx_put(c, s, prm.data(), prm.size() * sizeof(double))) return rc;
     const DevMesh& d = c->dm;
     const long cnt = (long)c->npad * c->ldr;
     const int kt = kt_mark(c, KS_RHS);
@@ -827,9 +827,9 @@ int mueller_launch(bem_ctx* c, double kr, double ki, double eta, const double* R
     char* work = reinterpret_cast<char*>(dM + 16 * (size_t)ntheta);
     work += (256 - reinterpret_cast<uintptr_t>(work) % 256) % 256;
     hipStream_t s = c->stream;
-    BEM_HIP(c, hipMemcpyAsync(drh, rh.data(), rh.size() * 8, hipMemcpyHostToDevice, s));
-    BEM_HIP(c, hipMemcpyAsync(dgeo, geo.data(), geo.size() * 8, hipMemcpyHostToDevice, s));
-    BEM_HIP(c, hipMemcpyAsync(dw, w, (size_t)n_orient * 8, hipMemcpyHostToDevice, s));
+    if (int rc = ctx_put(c, drh, rh.data(), rh.size() * 8)) return rc;
+    if (int rc = ctx_put(c, dgeo, geo.data(), geo.size() * 8)) return rc;
+    if (int rc = ctx_put(c, dw, w, (size_t)n_orient * 8)) return rc;
     // device solution: column c is call c; J rows 0..N-1, M rows N..2N-1
     const int N = c->rwg.N;
     const long ld = c->ldr;
@@ -839,10 +839,8 @@ int mueller_launch(bem_ctx* c, double kr, double ki, double eta, const double* R
                        kr, ki, mirror, dMo);
     hipLaunchKernelGGL(k_mueller_avg, dim3((16 * ntheta + 255) / 256), dim3(256), 0, s, n_orient, ntheta, dMo, dw, dM);
     BEM_HIP(c, hipGetLastError());
-    BEM_HIP(c, hipMemcpyAsync(M_avg, dM, 16 * (size_t)ntheta * 8, hipMemcpyDeviceToHost, s));
-    if (M_orient) BEM_HIP(c, hipMemcpyAsync(M_orient, dMo, mob, hipMemcpyDeviceToHost, s));
-    BEM_HIP(c, hipStreamSynchronize(s));
-    return 0;
+    const size_t avg = 16 * (size_t)ntheta * 8;
+    return M_orient ? ctx_fetch(c, {{M_avg, dM, avg}, {M_orient, dMo, mob}}) : ctx_fetch(c, {{M_avg, dM, avg}});
 }
 
 int ff_adjoint_launch(bem_ctx* c, const double* dL_dM, double* gr, double* gi, double* explicit_dk) {

@@ -89,6 +89,7 @@ __global__ __launch_bounds__(256) void k_gs_final(int m, int ncol, int nchunk, c
     if (idx >= m * ncol) return;
     const int i = idx / ncol, j = idx % ncol;
     double sr = 0.0, si = 0.0;
+#pragma unroll 8
     for (int ch = 0; ch < nchunk; ch++) {
         const long p = ((long)i * nchunk + ch) * ncol + j;
         sr += Pr[p];
@@ -144,7 +145,7 @@ int gmres_solve_launch(bem_ctx* c, int nrhs, double tol, int restart, int max_it
     // each), Gram-Schmidt partials and products, column scales, preconditioner work
     const size_t vec = 2 * (size_t)cnt;  // doubles per planar block vector
     const size_t nP = 2 * (size_t)(m + 1) * nchunk * ncol, nH = 2 * (size_t)(m + 1) * ncol;
-    const size_t doubles = vec * (2 * (size_t)m + 3) + nP + 2 * nH + 2 * (size_t)ncol + col_norm2_work(nphys, ncol);
+    const size_t doubles = vec * (2 * (size_t)m + 3) + nP + 2 * nH + 3 * (size_t)ncol + col_norm2_work(nphys, ncol);
     const size_t pwork = precond == BEM_PRECOND_LU ? lu_precond_work_bytes(c)
                          : precond == BEM_PRECOND_BLOCK ? bj_work_bytes(c)
                                                         : 0;
@@ -157,9 +158,10 @@ int gmres_solve_launch(bem_ctx* c, int nrhs, double tol, int restart, int max_it
     double* w = Zb + vec * m;               // one vector
     double* r = w + vec;                    // one vector
     double* P = r + vec;                    // partials
-    double* H = P + nP;                     // Gram-Schmidt products (two passes)
-    double* H2 = H + nH;
-    double* cs = H2 + nH;                   // column scales
+    // both passes' Gram-Schmidt products (k vectors: real, imaginary) and then the
+    // norms, side by side for one transfer
+    double* H = P + nP;
+    double* cs = H + 2 * nH + ncol;         // column scales
     double* nrm = cs + ncol;                // column norms, then their partial sums
     char* pw = reinterpret_cast<char*>(nrm + ncol + col_norm2_work(nphys, ncol));
     pw += (256 - reinterpret_cast<uintptr_t>(pw) % 256) % 256;
@@ -170,12 +172,10 @@ int gmres_solve_launch(bem_ctx* c, int nrhs, double tol, int restart, int max_it
     auto Zk = [&](int k) { return Zb + vec * k; };
     const dim3 g1((unsigned)((cnt + 255) / 256));
 
-    std::vector<double> hn2(ncol), bn2(ncol), rn2(ncol), scale(ncol);
+    std::vector<double> bn2(ncol), rn2(ncol), scale(ncol);
     auto colnorm2 = [&](const double* vr, const double* vi, std::vector<double>& out) -> int {
         col_norm2(s, nphys, ncol, vr, vi, ncol, nrm + ncol, nrm);
-        BEM_HIP(c, hipMemcpyAsync(out.data(), nrm, ncol * sizeof(double), hipMemcpyDeviceToHost, s));
-        BEM_HIP(c, hipStreamSynchronize(s));
-        return 0;
+        return ctx_fetch(c, {{out.data(), nrm, ncol * sizeof(double)}});
     };
     // r = B - Z X
     auto residual = [&]() -> int { return z_product(c, ncol, c->Xr, c->Xi, c->Br, c->Bi, re(r), im(r)); };
@@ -186,7 +186,7 @@ int gmres_solve_launch(bem_ctx* c, int nrhs, double tol, int restart, int max_it
     };
     // v_dst = src * scale[j] per column
     auto scale_into = [&](double* src, double* dst) -> int {
-        BEM_HIP(c, hipMemcpyAsync(cs, scale.data(), ncol * sizeof(double), hipMemcpyHostToDevice, s));
+        if (int rc = ctx_put(c, cs, scale.data(), ncol * sizeof(double))) return rc;
         hipLaunchKernelGGL(k_scale_cols, g1, dim3(256), 0, s, cnt, ncol, re(src), im(src), cs, re(dst), im(dst));
         return 0;
     };
@@ -195,9 +195,9 @@ int gmres_solve_launch(bem_ctx* c, int nrhs, double tol, int restart, int max_it
         hipLaunchKernelGGL(k_gs_partial, dim3(nchunk, k), dim3(256), 0, s, n, ncol, re(V), im(V), (long)vec, re(w),
                            im(w), P, P + nP / 2, nchunk);
         hipLaunchKernelGGL(k_gs_final, dim3((k * ncol + 255) / 256), dim3(256), 0, s, k, ncol, nchunk, P, P + nP / 2,
-                           Hbuf, Hbuf + nH / 2);
+                           Hbuf, Hbuf + (size_t)k * ncol);
         hipLaunchKernelGGL(k_gs_update, g1, dim3(256), 0, s, cnt, ncol, k, re(V), im(V), (long)vec, Hbuf,
-                           Hbuf + nH / 2, re(w), im(w));
+                           Hbuf + (size_t)k * ncol, re(w), im(w));
     };
 
     BEM_HIP(c, hipMemsetAsync(c->Xr, 0, cnt * sizeof(double), s));
@@ -209,8 +209,7 @@ int gmres_solve_launch(bem_ctx* c, int nrhs, double tol, int restart, int max_it
     // host Hessenberg data per right-hand side: column-major (m + 1) x m
     std::vector<cd> Hh((size_t)(m + 1) * m * ncol), g((size_t)(m + 1) * ncol), sn((size_t)m * ncol);
     std::vector<double> cn((size_t)m * ncol);
-    std::vector<cd> hcol((size_t)(m + 1) * ncol);
-    std::vector<double> hbr((size_t)(m + 1) * ncol), hbi((size_t)(m + 1) * ncol);
+    std::vector<double> hb((4 * (size_t)(m + 1) + 1) * ncol);
     std::vector<int> mj(ncol), active(ncol);
     bool first = true, checked = false;
     while (total < max_iter) {
@@ -252,16 +251,12 @@ int gmres_solve_launch(bem_ctx* c, int nrhs, double tol, int restart, int max_it
             if (prc) return prc;
             if (int rc = z_product(c, ncol, re(Zk(it)), im(Zk(it)), nullptr, nullptr, re(w), im(w))) return rc;
             // classical Gram-Schmidt, twice
+            const size_t hk = (size_t)(it + 1) * ncol;
             gs_products(it + 1, H);
-            gs_products(it + 1, H2);
-            BEM_HIP(c, hipMemcpyAsync(hbr.data(), H, (size_t)(it + 1) * ncol * sizeof(double), hipMemcpyDeviceToHost,
-                                      s));
-            BEM_HIP(c, hipMemcpyAsync(hbi.data(), H + nH / 2, (size_t)(it + 1) * ncol * sizeof(double),
-                                      hipMemcpyDeviceToHost, s));
-            std::vector<double> h2r((size_t)(it + 1) * ncol), h2i((size_t)(it + 1) * ncol);
-            BEM_HIP(c, hipMemcpyAsync(h2r.data(), H2, h2r.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-            BEM_HIP(c, hipMemcpyAsync(h2i.data(), H2 + nH / 2, h2i.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-            if (int rc = colnorm2(re(w), im(w), hn2)) return rc;
+            gs_products(it + 1, H + 2 * hk);
+            col_norm2(s, nphys, ncol, re(w), im(w), ncol, nrm + ncol, H + 4 * hk);
+            if (int rc = ctx_fetch(c, {{hb.data(), H, (4 * hk + ncol) * sizeof(double)}})) return rc;
+            const double *h1r = hb.data(), *h1i = h1r + hk, *h2r = h1i + hk, *h2i = h2r + hk, *hn2 = h2i + hk;
             int still = 0;
             for (int j = 0; j < ncol; j++) {
                 if (!active[j]) {
@@ -270,8 +265,8 @@ int gmres_solve_launch(bem_ctx* c, int nrhs, double tol, int restart, int max_it
                 }
                 cd* Hj = &Hh[(size_t)j * (m + 1) * m + (size_t)it * (m + 1)];  // column it
                 for (int i = 0; i <= it; i++)
-                    Hj[i] = cd(hbr[(size_t)i * ncol + j] + h2r[(size_t)i * ncol + j],
-                               hbi[(size_t)i * ncol + j] + h2i[(size_t)i * ncol + j]);
+                    Hj[i] = cd(h1r[(size_t)i * ncol + j] + h2r[(size_t)i * ncol + j],
+                               h1i[(size_t)i * ncol + j] + h2i[(size_t)i * ncol + j]);
                 const double hnext = std::sqrt(hn2[j]);
                 // earlier rotations, then a new one that zeroes h_{it+1,it}
                 for (int i = 0; i < it; i++) {

@@ -1753,14 +1753,13 @@ int lu_factor_launch(bem_ctx* c, int precision) {
     void* scr = nullptr;
     if (int e = ctx_scratch(c, 256, &scr)) return e;
     int info = 0;
-    BEM_HIP(c, hipMemcpyAsync(&info, scr, sizeof(int), hipMemcpyDeviceToHost, s));
     // swap sequence -> row permutation (row i of P Z is row perm[i] of Z)
     std::vector<int> ip(n), perm(n);
-    BEM_HIP(c, hipMemcpyAsync(ip.data(), c->ipiv, n * sizeof(int), hipMemcpyDeviceToHost, s));
-    BEM_HIP(c, hipStreamSynchronize(s));
+    if (int e = ctx_fetch(c, {{&info, scr, sizeof(int)}, {ip.data(), c->ipiv, n * sizeof(int)}})) return e;
     for (int i = 0; i < n; i++) perm[i] = i;
     for (int i = 0; i < n; i++)
         if (ip[i] != i) std::swap(perm[i], perm[ip[i]]);
-    BEM_HIP(c, hipMemcpy(c->perm, perm.data(), n * sizeof(int), hipMemcpyHostToDevice));
+    if (int e = ctx_put(c, c->perm, perm.data(), n * sizeof(int))) return e;
+    if (n * sizeof(int) > kPinBytes / 2) BEM_HIP(c, hipStreamSynchronize(s));
     return info > c->n ? 0 : info;  // a zero pivot inside the identity padding cannot occur
 }

@@ -332,12 +332,11 @@ int lu_solve_launch(bem_ctx* c, int nrhs, double tol, int maxit, int* iters, dou
             hipLaunchKernelGGL(k_accumulate<double>, g1, dim3(256), 0, s, cnt, Yr, Yi, c->Xr, c->Xi, assign);
         }
     };
-    auto residual = [&]() -> int {  // R = B - Z X, returns max relative residual in *res
+    auto residual = [&](bool first) -> int {  // R = B - Z X and its norms, with B's at first
         if (int rc = z_product(c, ncol, c->Xr, c->Xi, c->Br, c->Bi, Rr, Ri)) return rc;
         col_norm2(s, c->n, nrhs, Rr, Ri, (long)ldr, npt, nr2);
-        BEM_HIP(c, hipMemcpyAsync(r2.data(), nr2, nrhs * sizeof(double), hipMemcpyDeviceToHost, s));
-        BEM_HIP(c, hipStreamSynchronize(s));
-        return 0;
+        const size_t nb = nrhs * sizeof(double);
+        return first ? ctx_fetch(c, {{r2.data(), nr2, nb}, {b2.data(), nb2, nb}}) : ctx_fetch(c, {{r2.data(), nr2, nb}});
     };
 
     // plain solve
@@ -352,8 +351,7 @@ int lu_solve_launch(bem_ctx* c, int nrhs, double tol, int maxit, int* iters, dou
     if (can_refine && (maxit > 0 || f32)) {
         BEM_HIP(c, hipEventRecord(e[2], s));
         col_norm2(s, c->n, nrhs, c->Br, c->Bi, (long)ldr, npt, nb2);
-        BEM_HIP(c, hipMemcpyAsync(b2.data(), nb2, nrhs * sizeof(double), hipMemcpyDeviceToHost, s));
-        if (int e2 = residual()) return e2;
+        if (int e2 = residual(true)) return e2;
         *res0 = *res = max_ratio(r2, b2, nrhs);
         int it = 0;
         float ts_loop = 0.0f;  // triangular solves inside the sweeps
@@ -362,7 +360,7 @@ int lu_solve_launch(bem_ctx* c, int nrhs, double tol, int maxit, int* iters, dou
             BEM_HIP(c, hipEventRecord(e[0], s));
             solve_into_X(Rr, Ri, 0);
             BEM_HIP(c, hipEventRecord(e[1], s));
-            if (int e2 = residual()) return e2;
+            if (int e2 = residual(false)) return e2;
             BEM_HIP(c, hipEventElapsedTime(&t0, e[0], e[1]));
             ts_loop += t0;
             *res = max_ratio(r2, b2, nrhs);
