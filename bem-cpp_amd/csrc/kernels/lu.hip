@@ -61,48 +61,22 @@ struct Vec16<double> {
 template <typename T>
 using Nat16 = T __attribute__((ext_vector_type(16 / sizeof(T))));
 
-// PB consecutive values at p (16-byte aligned) <-> registers.
-template <typename T>
-__device__ __forceinline__ void load_row(const T* __restrict__ p, T (&x)[PB]) {
-    using V = typename Vec16<T>::type;
-    constexpr int E = 16 / sizeof(T);
-#pragma unroll
-    for (int q = 0; q < PB; q += E) {
-        const V a = *reinterpret_cast<const V*>(p + q);
-        __builtin_memcpy(&x[q], &a, 16);
-    }
-}
-template <typename T>
-__device__ __forceinline__ void store_row(T* __restrict__ p, const T (&x)[PB]) {
-    using V = typename Vec16<T>::type;
-    constexpr int E = 16 / sizeof(T);
-#pragma unroll
-    for (int q = 0; q < PB; q += E) {
-        V a;
-        __builtin_memcpy(&a, &x[q], 16);
-        *reinterpret_cast<V*>(p + q) = a;
-    }
-}
-
 // 1 / d for the pivot scaling: the hardware reciprocal in FP32 (1 ulp), an
 // IEEE division in FP64.
 __device__ __forceinline__ float recip(float d) { return __builtin_amdgcn_rcpf(d); }
 __device__ __forceinline__ double recip(double d) { return 1.0 / d; }
 
 // Order-preserving 32-bit key of a non-negative magnitude, with the row in its
-// low bits (r of R rows per thread, then the lane; ties: lowest), so the wave's
-// maximum names its row; 0 is "no candidate".  That leaves 17 mantissa bits of a
-// float and 14 of a double (one less for two rows per thread): rows closer than
-// that in magnitude tie.  (The sign of a NaN is masked.)
+// low bits (the lane; ties: lowest), so the wave's maximum names its row; 0 is "no
+// candidate".  That leaves 17 mantissa bits of a float and 14 of a double: rows
+// closer than that in magnitude tie.  (The sign of a NaN is masked.)
 __device__ __forceinline__ unsigned mag_bits(float m) { return __float_as_uint(m); }
 __device__ __forceinline__ unsigned mag_bits(double m) {
     return (unsigned)((unsigned long long)__double_as_longlong(m) >> 32);
 }
-template <int R, typename T>
-__device__ __forceinline__ unsigned mag_key(T m, int r, int lane) {
-    static_assert(R <= 2, "one bit for the row");
-    constexpr unsigned low = 64 * R;  // values of the row part
-    return (mag_bits(m) & 0x7fffffffu & ~(low - 1)) + low + 64 * (R - 1 - r) + (unsigned)(63 - lane);
+template <typename T>
+__device__ __forceinline__ unsigned mag_key(T m, int lane) {
+    return (mag_bits(m) & 0x7fffffc0u) + 64u + (unsigned)(63 - lane);
 }
 
 // Maximum over the wave, in a scalar register (DPP within rows of 16, then
@@ -131,44 +105,139 @@ __device__ __forceinline__ double from_lane(double v, int l) {
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-constexpr int EW = 4;  // columns of an elimination window
-
-// Columns EW .. PB-1 to the front, columns 0 .. EW-1 to the end.
+constexpr int EW = 4;        // columns of an elimination window
+constexpr int NG = PB / EW;  // windows of a row
 template <typename T>
-__device__ __forceinline__ void rotate_row(T (&x)[PB]) {
-    T h[EW];
+using Grp = T __attribute__((ext_vector_type(EW)));  // a row's entries of a window
+
+template <typename T>
+__device__ __forceinline__ void load_groups(const T* __restrict__ p, Grp<T> (&x)[NG]) {
+    constexpr int E = 16 / sizeof(T);
 #pragma unroll
-    for (int c = 0; c < EW; c++) h[c] = x[c];
+    for (int g = 0; g < NG; g++)
 #pragma unroll
-    for (int c = 0; c < PB - EW; c++) x[c] = x[c + EW];
+        for (int c = 0; c < EW; c += E) {
+            const Nat16<T> a = *reinterpret_cast<const Nat16<T>*>(p + g * EW + c);
 #pragma unroll
-    for (int c = 0; c < EW; c++) x[PB - EW + c] = h[c];
+            for (int e = 0; e < E; e++) x[g][c + e] = a[e];
+        }
+}
+template <typename T>
+__device__ __forceinline__ void store_group(T* p, const Grp<T>& x, int from = 0) {
+    constexpr int E = 16 / sizeof(T);
+#pragma unroll
+    for (int c = 0; c < EW; c += E)
+        if (c + E - 1 >= from) {
+            Nat16<T> a;
+#pragma unroll
+            for (int e = 0; e < E; e++) a[e] = x[c + e];
+            *reinterpret_cast<Nat16<T>*>(p + c) = a;
+        }
 }
 
-// Exchange area of the register-resident elimination (4 waves).
-template <typename T>
+// Exchange area of the register-resident elimination (W waves).
+template <typename T, int W>
 struct ElimLds {
-    alignas(16) T win[2][4][2][EW];   // [step parity][wave][plane]: the wave's best row, window columns
-    alignas(16) unsigned key[2][4];   // its key
-    alignas(16) T raw[EW][2][PB];     // the window's pivot rows before the window's updates right of it
-    alignas(16) T u[4][EW][2][PB];    // the same as rows of U, one copy per wave
-    alignas(16) int oid[PB];          // chosen rows in pivot order
+    alignas(16) T win[2][W][2][EW];  // [step parity][wave][plane]: the wave's best row, window columns
+    alignas(16) unsigned key[2][W];  // its key
+    alignas(16) T raw[EW][2][PB];    // the window's pivot rows before the window's updates right of it
+    alignas(16) T u[sizeof(T) == 8 ? W : 1][EW][2][PB];  // FP64: the same as rows of U, one copy per wave
+    alignas(16) int oid[PB];         // chosen rows in pivot order
     int osrc[PB];
-    alignas(16) int sw[2][PB];        // root_swaps
+    alignas(16) int sw[2][PB];       // root_swaps
     int last;
     int zmin;  // first zero pivot of the root (1-based)
 };
 
-// Partial pivoting over the block's rows, R rows per thread in registers (row
-// t + 256 r; rows at nrows and beyond take no part; nrows >= PB), with
-// implicit row interchanges: rows stay with their thread and a chosen row is
-// only marked.  Step jc: the largest |x_jc|^2 among the rows not chosen yet (by
-// mag_key; ties: lowest r, wave, lane) becomes pivot jc, and the remaining rows
-// are eliminated (multiplier stored in x_jc).  An all-zero column chooses the
-// lowest open row and eliminates nothing.
-// Afterwards mine[r] is the pivot number of row r (its thread holds that row of
-// L11 \ U11), -1 for rows not chosen; oid/osrc list the chosen rows in pivot
-// order.
+// Group G of the row takes the window's EW pivots and moves to G - 1, from G = 1 on:
+// with the window at the end, the row has rotated by one group then.  Groups beyond
+// ng only move.  (vr, vi): lane l's values of the window's pivot rows in column EW + l.
+// Per element and pivot the four multiply-adds are those of the column-by-column
+// elimination, in its order.
+// FP32: v_mfma_f32_4x4x1 with one block's A operand broadcast to all 16 is a rank-1
+// update of four columns with a row per lane, and that block is group G's lanes of vr
+// and vi as they lie.
+template <int G>
+__device__ __forceinline__ void window_update(Grp<float> (&xr)[NG], Grp<float> (&xi)[NG], const float (&lr)[EW],
+                                              const float (&li)[EW], const float (&vr)[EW], const float (&vi)[EW],
+                                              int ng) {
+    if constexpr (G < NG) {
+        if (G <= ng) {
+            v4f a = xr[G], b = xi[G];
+#pragma unroll
+            for (int q = 0; q < EW; q++) {
+                const float nl = -lr[q];
+                a = __builtin_amdgcn_mfma_f32_4x4x1f32(vr[q], nl, a, 4, G - 1, 0);
+                b = __builtin_amdgcn_mfma_f32_4x4x1f32(vi[q], nl, b, 4, G - 1, 0);
+                a = __builtin_amdgcn_mfma_f32_4x4x1f32(vi[q], li[q], a, 4, G - 1, 0);
+                b = __builtin_amdgcn_mfma_f32_4x4x1f32(-vr[q], li[q], b, 4, G - 1, 0);
+            }
+            xr[G - 1] = a;
+            xi[G - 1] = b;
+        } else {
+            xr[G - 1] = xr[G];
+            xi[G - 1] = xi[G];
+        }
+        window_update<G + 1>(xr, xi, lr, li, vr, vi, ng);
+    }
+}
+// FP64 has no such form: the values come from LDS (u, the wave's copy), two columns
+// read ahead; the scheduling barriers keep more from being hoisted, which would not
+// fit in the registers.
+struct WindowCols {
+    v2d r[EW], i[EW];
+};
+__device__ __forceinline__ void window_read(const double (*u)[2][PB], int c, WindowCols& w) {
+#pragma unroll
+    for (int q = 0; q < EW; q++) {
+        w.r[q] = *reinterpret_cast<const v2d*>(&u[q][0][c]);
+        w.i[q] = *reinterpret_cast<const v2d*>(&u[q][1][c]);
+    }
+}
+template <int G>
+__device__ __forceinline__ void window_update(Grp<double> (&xr)[NG], Grp<double> (&xi)[NG], const double (&lr)[EW],
+                                              const double (&li)[EW], const double (*u)[2][PB], WindowCols& cur,
+                                              int ng) {
+    if constexpr (G < NG) {
+        if (G <= ng) {
+            WindowCols nxt;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                if (h == 0)
+                    window_read(u, G * EW + 2, nxt);
+                else if (G + 1 < NG)
+                    window_read(u, (G + 1) * EW, cur);  // (unused beyond group ng)
+                __builtin_amdgcn_sched_barrier(0);
+                const WindowCols now = h ? nxt : cur;
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    double a = xr[G][2 * h + e], b = xi[G][2 * h + e];
+#pragma unroll
+                    for (int q = 0; q < EW; q++) {
+                        a = fmadd(li[q], double(now.i[q][e]), fmadd(-lr[q], double(now.r[q][e]), a));
+                        b = fmadd(-li[q], double(now.r[q][e]), fmadd(-lr[q], double(now.i[q][e]), b));
+                    }
+                    xr[G - 1][2 * h + e] = a;
+                    xi[G - 1][2 * h + e] = b;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+            xr[G - 1] = xr[G];
+            xi[G - 1] = xi[G];
+        }
+        window_update<G + 1>(xr, xi, lr, li, u, cur, ng);
+    }
+}
+
+// Partial pivoting over the block's rows, one per thread in registers (rows at
+// nrows and beyond take no part; nrows >= PB), with implicit row interchanges: rows
+// stay with their thread and a chosen row is only marked.  Step jc: the largest
+// |x_jc|^2 among the rows not chosen yet (by mag_key; ties: lowest wave, lane)
+// becomes pivot jc, and the remaining rows are eliminated (multiplier stored in
+// x_jc).  An all-zero column chooses the lowest open row and eliminates nothing.
+// Afterwards mine is the pivot number of the thread's row (the thread holds that row
+// of L11 \ U11), -1 for rows not chosen; oid/osrc list the chosen rows in pivot order.
 //
 // The chain of 32 steps is bound by the exchange between the waves and by
 // instruction fetch, so:
@@ -177,83 +246,63 @@ struct ElimLds {
 //   is also all that is updated within the window.  The columns right of it take
 //   the window's EW pivots at once: their rows go to LDS, each wave solves them
 //   against the window's unit triangle, one column per lane, and updates its
-//   rows.  Per element the operations and their order are those of the
-//   column-by-column elimination.
-// - the windows are a loop, not unrolled code: the row registers rotate by EW
-//   columns after each window, so the window is always columns 0 .. EW-1 of the
-//   registers and the eighth rotation brings every column home.  (Unrolled, the
-//   32 steps are 40 KB of code per call site.)
-// 3840 rows: 72.7 us before, 58.7 now (with the root's parallel swaps and sets
-// of 512 rows); one level of 256 rows 27.7 and 24.5.
-template <typename T, int R>
-__device__ __forceinline__ void elim_rows(ElimLds<T>& L, T (&xr)[R][PB], T (&xi)[R][PB], const int (&id)[R],
-                                          const int (&src)[R], int nrows, int (&mine)[R]) {
-    using V = typename Vec16<T>::type;
-    constexpr int E = 16 / sizeof(T);
+//   rows (window_update).
+// - the windows are a loop, not unrolled code: the row registers rotate by a
+//   group after each window, so the window is always group 0 and the eighth
+//   rotation brings every column home.  (Unrolled, the 32 steps are 40 KB of code.)
+// One level of 256 rows takes 22.1 us (FP64 31.3), of 512 31.0, alone; with the
+// products of window_update as multiply-adds on operands from LDS and the rows rotated
+// by copies it took 24.5 (31.5), and 35.8 with two rows per thread of 4 waves.
+template <typename T, int W>
+__device__ __forceinline__ void elim_rows(ElimLds<T, W>& L, Grp<T> (&xr)[NG], Grp<T> (&xi)[NG], int id, int src,
+                                          int nrows, int& mine) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    bool valid[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        valid[r] = t + 256 * r < nrows;
-        mine[r] = -1;
-    }
+    const bool valid = t < nrows;
+    // Of 8 waves, one without rows only keeps the barriers (and its key, 0): 256 rows
+    // 23.4 us instead of 27.0.  (With 4 waves the branches cost full sets 1.3 us.)
+    const bool active = W == 4 || __builtin_amdgcn_readfirstlane(wave) * 64 < nrows;
+    if (!active && lane < 2) L.key[lane][wave] = 0u;
+    mine = -1;
 #pragma unroll 1
-    for (int w = 0; w < PB / EW; w++) {
-        const int s = w * EW, ng = PB / EW - 1 - w;  // first column; groups of EW columns right of the window
-        T lr[R][EW], li[R][EW];  // the window's multipliers (0: row not eliminated)
+    for (int w = 0; w < NG; w++) {
+        const int s = w * EW, ng = NG - 1 - w;  // first column; groups right of the window
+        T lr[EW], li[EW];                       // the window's multipliers (0: row not eliminated)
+        Grp<T> hr = xr[0], hi = xi[0];          // the window
 #pragma unroll
         for (int q = 0; q < EW; q++) {
             const int par = q & 1;
-            unsigned key = 0u;
-            int rb = 0;
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const unsigned k = valid[r] && mine[r] < 0 ? mag_key<R>(mag2(xr[r][q], xi[r][q]), r, lane) : 0u;
-                if (k > key) {
-                    key = k;
-                    rb = r;
+            unsigned key = 0u, wk = 0u;
+            if (active) {
+                key = valid && mine < 0 ? mag_key(mag2(T(hr[q]), T(hi[q])), lane) : 0u;
+                wk = wave_max(key);
+                if (key == wk) {  // one lane, or a wave without candidates
+                    store_group<T>(L.win[par][wave][0], hr, q);
+                    store_group<T>(L.win[par][wave][1], hi, q);
+                    L.key[par][wave] = wk;
                 }
-            }
-            const unsigned wk = wave_max(key);
-            T wr[EW], wi[EW];
-#pragma unroll
-            for (int c = 0; c < EW; c++) {
-                wr[c] = xr[0][c];
-                wi[c] = xi[0][c];
-#pragma unroll
-                for (int r = 1; r < R; r++) {
-                    wr[c] = rb == r ? xr[r][c] : wr[c];
-                    wi[c] = rb == r ? xi[r][c] : wi[c];
-                }
-            }
-            if (key == wk) {  // one lane, or a wave without candidates
-#pragma unroll
-                for (int c = 0; c < EW; c += E)
-                    if (c + E - 1 >= q) {
-                        V a, d;
-                        __builtin_memcpy(&a, &wr[c], 16);
-                        __builtin_memcpy(&d, &wi[c], 16);
-                        *reinterpret_cast<V*>(&L.win[par][wave][0][c]) = a;
-                        *reinterpret_cast<V*>(&L.win[par][wave][1][c]) = d;
-                    }
-                L.key[par][wave] = wk;
             }
             __syncthreads();
-            // lane l reads wave l % 4's entry; the maximum over four lanes then
+            if (!active) continue;
+            // lane l reads wave l % W's entry; the maximum over W lanes then
             // names the wave whose window the scalar registers take (one LDS
             // latency instead of the keys' and then the window's)
-            const unsigned kw = L.key[par][lane & 3] | 63u;  // without the lane: ties go to the lower wave
+            const unsigned kw = L.key[par][lane & (W - 1)] | 63u;  // without the lane: ties go to the lower wave
             T cr[EW], ci[EW];
+            constexpr int E = 16 / sizeof(T);
 #pragma unroll
             for (int c = 0; c < EW; c += E)
                 if (c + E - 1 >= q) {
-                    const V a = *reinterpret_cast<const V*>(&L.win[par][lane & 3][0][c]);
-                    const V d = *reinterpret_cast<const V*>(&L.win[par][lane & 3][1][c]);
-                    __builtin_memcpy(&cr[c], &a, 16);
-                    __builtin_memcpy(&ci[c], &d, 16);
+                    const Nat16<T> a = *reinterpret_cast<const Nat16<T>*>(&L.win[par][lane & (W - 1)][0][c]);
+                    const Nat16<T> d = *reinterpret_cast<const Nat16<T>*>(&L.win[par][lane & (W - 1)][1][c]);
+#pragma unroll
+                    for (int e = 0; e < E; e++) {
+                        cr[c + e] = a[e];
+                        ci[c + e] = d[e];
+                    }
                 }
             unsigned best = max_dpp<0xb1, 0xf>(kw);  // quad_perm [1, 0, 3, 2], then [2, 3, 0, 1]
             best = max_dpp<0x4e, 0xf>(best);
+            if constexpr (W == 8) best = max_dpp<0x141, 0xf>(best);  // row_half_mirror
             const int wv = __ffsll((long long)__ballot(kw == best)) - 1;
             T ur[EW], ui[EW];
 #pragma unroll
@@ -266,113 +315,77 @@ __device__ __forceinline__ void elim_rows(ElimLds<T>& L, T (&xr)[R][PB], T (&xi)
             const T d = ur[q] * ur[q] + ui[q] * ui[q];
             const T inv = d > T(0) ? recip(d) : T(0);
             const T qr = ur[q] * inv, qi = -ui[q] * inv;
+            if (won) mine = s + q;
+            // branch-free update: rows that are not eliminated use multiplier 0
+            const bool upd = valid && mine < 0 && d > T(0);
+            const T a = hr[q] * qr - hi[q] * qi, b = hr[q] * qi + hi[q] * qr;
+            lr[q] = upd ? a : T(0);
+            li[q] = upd ? b : T(0);
+            hr[q] = upd ? a : T(hr[q]);
+            hi[q] = upd ? b : T(hi[q]);
+            const T nlr = -lr[q], nli = -li[q];
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                if (won && rb == r) mine[r] = s + q;
-                // branch-free update: rows that are not eliminated use multiplier 0
-                const bool upd = valid[r] && mine[r] < 0 && d > T(0);
-                const T a = xr[r][q] * qr - xi[r][q] * qi, b = xr[r][q] * qi + xi[r][q] * qr;
-                lr[r][q] = upd ? a : T(0);
-                li[r][q] = upd ? b : T(0);
-                xr[r][q] = upd ? a : xr[r][q];
-                xi[r][q] = upd ? b : xi[r][q];
-                const T nlr = -lr[r][q], nli = -li[r][q];
-#pragma unroll
-                for (int c = q + 1; c < EW; c++) {
-                    xr[r][c] = fmadd(nlr, ur[c], xr[r][c]);
-                    xr[r][c] = fmadd(li[r][q], ui[c], xr[r][c]);
-                    xi[r][c] = fmadd(nlr, ui[c], xi[r][c]);
-                    xi[r][c] = fmadd(nli, ur[c], xi[r][c]);
-                }
+            for (int c = q + 1; c < EW; c++) {
+                hr[c] = fmadd(li[q], ui[c], fmadd(nlr, ur[c], T(hr[c])));
+                hi[c] = fmadd(nli, ur[c], fmadd(nlr, ui[c], T(hi[c])));
             }
         }
-        if (ng > 0) {
-            // the window's pivot rows (window columns final, the others without
-            // the window's updates)
+        // the window's pivot rows (window columns final, the others without the
+        // window's updates); the last window has no others, the rows only rotate
+        if (ng > 0 && mine >= s) {
+            T *pr = L.raw[mine - s][0], *pi = L.raw[mine - s][1];
+            store_group<T>(pr, hr);
+            store_group<T>(pi, hi);
 #pragma unroll
-            for (int r = 0; r < R; r++)
-                if (mine[r] >= s) {
-#pragma unroll
-                    for (int g = 0; g < PB / EW; g++)
-                        if (g <= ng) {
-#pragma unroll
-                            for (int c = g * EW; c < (g + 1) * EW; c += E) {
-                                V a, d;
-                                __builtin_memcpy(&a, &xr[r][c], 16);
-                                __builtin_memcpy(&d, &xi[r][c], 16);
-                                *reinterpret_cast<V*>(&L.raw[mine[r] - s][0][c]) = a;
-                                *reinterpret_cast<V*>(&L.raw[mine[r] - s][1][c]) = d;
-                            }
-                        }
+            for (int g = 1; g < NG; g++)
+                if (g <= ng) {
+                    store_group<T>(pr + g * EW, xr[g]);
+                    store_group<T>(pi + g * EW, xi[g]);
                 }
-            __syncthreads();
+        }
+        __syncthreads();
+        if (!active) continue;
+        // lane l solves column EW + l against the window's unit triangle
+        // (beyond the groups left, some value)
+        const int cl = EW + min(lane, PB - EW - 1);
+        T vr[EW], vi[EW];
+#pragma unroll
+        for (int q = 0; q < EW; q++) {
+            vr[q] = L.raw[q][0][cl];
+            vi[q] = L.raw[q][1][cl];
+        }
+#pragma unroll
+        for (int q = 0; q < EW; q++)
+#pragma unroll
+            for (int k = 0; k < q; k++) {
+                const T mr = L.raw[q][0][k], mi = L.raw[q][1][k];
+                vr[q] = fmadd(-mr, vr[k], vr[q]);
+                vr[q] = fmadd(mi, vi[k], vr[q]);
+                vi[q] = fmadd(-mr, vi[k], vi[q]);
+                vi[q] = fmadd(-mi, vr[k], vi[q]);
+            }
+        if constexpr (sizeof(T) == 4) {
+            window_update<1>(xr, xi, lr, li, vr, vi, ng);
+        } else {
             if (lane < ng * EW) {
-                T vr[EW], vi[EW];
 #pragma unroll
                 for (int q = 0; q < EW; q++) {
-                    vr[q] = L.raw[q][0][EW + lane];
-                    vi[q] = L.raw[q][1][EW + lane];
-                }
-#pragma unroll
-                for (int q = 0; q < EW; q++) {
-#pragma unroll
-                    for (int k = 0; k < q; k++) {
-                        const T mr = L.raw[q][0][k], mi = L.raw[q][1][k];
-                        vr[q] = fmadd(-mr, vr[k], vr[q]);
-                        vr[q] = fmadd(mi, vi[k], vr[q]);
-                        vi[q] = fmadd(-mr, vi[k], vi[q]);
-                        vi[q] = fmadd(-mi, vr[k], vi[q]);
-                    }
                     L.u[wave][q][0][EW + lane] = vr[q];
                     L.u[wave][q][1][EW + lane] = vi[q];
                 }
             }
             __builtin_amdgcn_wave_barrier();  // the wave's own copy: LDS operations of a wave stay in order
-            // the scheduling barriers keep the reads of later columns from being
-            // hoisted (they would not fit in the registers)
-#pragma unroll
-            for (int g = 1; g < PB / EW; g++)
-                if (g <= ng) {
-#pragma unroll
-                    for (int c0 = g * EW; c0 < (g + 1) * EW; c0 += E) {
-                        T ur[EW][E], ui[EW][E];
-#pragma unroll
-                        for (int q = 0; q < EW; q++) {
-                            const V a = *reinterpret_cast<const V*>(&L.u[wave][q][0][c0]);
-                            const V d = *reinterpret_cast<const V*>(&L.u[wave][q][1][c0]);
-                            __builtin_memcpy(ur[q], &a, 16);
-                            __builtin_memcpy(ui[q], &d, 16);
-                        }
-#pragma unroll
-                        for (int q = 0; q < EW; q++)
-#pragma unroll
-                            for (int r = 0; r < R; r++) {
-                                const T nlr = -lr[r][q], nli = -li[r][q];
-#pragma unroll
-                                for (int e = 0; e < E; e++) {
-                                    const int c = c0 + e;
-                                    xr[r][c] = fmadd(nlr, ur[q][e], xr[r][c]);
-                                    xr[r][c] = fmadd(li[r][q], ui[q][e], xr[r][c]);
-                                    xi[r][c] = fmadd(nlr, ui[q][e], xi[r][c]);
-                                    xi[r][c] = fmadd(nli, ur[q][e], xi[r][c]);
-                                }
-                            }
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                }
+            WindowCols cur;
+            window_read(L.u[wave], EW, cur);
+            window_update<1>(xr, xi, lr, li, L.u[wave], cur, ng);
         }
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            rotate_row(xr[r]);
-            rotate_row(xi[r]);
-        }
+        xr[NG - 1] = hr;
+        xi[NG - 1] = hi;
     }
-#pragma unroll
-    for (int r = 0; r < R; r++)
-        if (mine[r] >= 0) {
-            L.oid[mine[r]] = id[r];
-            L.osrc[mine[r]] = src[r];
-        }
+    if (mine >= 0) {
+        L.oid[mine] = id;
+        L.osrc[mine] = src;
+    }
     __syncthreads();
 }
 
@@ -427,7 +440,7 @@ __device__ void root_swaps(const int* __restrict__ oid, int* __restrict__ y, int
 
 // What the columns of the panel beyond the next 32 still need from the step at
 // columns jp: the rank-32 update of the columns [c0, c0 + ncol), rows from jp +
-// 32 on (16 x 16 tiles, four per workgroup), and U12 of the next 32 columns put
+// 32 on (16 x 16 tiles, one per wave), and U12 of the next 32 columns put
 // in place (one workgroup).  It rides in the launch of the next tournament,
 // whose few workgroups leave the device idle, instead of on a stream of its own
 // with an event each way.
@@ -437,11 +450,11 @@ struct FarUpdate {
 
 // One 16 x 16 tile of C -= L21 U12 per wave with K = 32, operands straight from
 // memory to the matrix cores, every load issued before the first product.
-template <typename T>
+template <typename T, int W>
 __device__ __forceinline__ void far_update(T* __restrict__ Ar, T* __restrict__ Ai, long ld, int n, FarUpdate f,
                                            int block, const T* __restrict__ Ur, const T* __restrict__ Ui) {
     if (block == f.blocks - 1) {
-        for (int e = threadIdx.x; e < PB * PB; e += 256) {
+        for (int e = threadIdx.x; e < PB * PB; e += 64 * W) {
             const long o = (long)(f.jp + e / PB) * ld + f.jp + PB + e % PB;
             Ar[o] = Ur[e];
             Ai[o] = Ui[e];
@@ -449,7 +462,7 @@ __device__ __forceinline__ void far_update(T* __restrict__ Ar, T* __restrict__ A
         return;
     }
     const int i0 = f.jp + PB, nct = f.ncol / 16, ntiles = (n - i0) / 16 * nct;
-    const int tile = block * 4 + (threadIdx.x >> 6);
+    const int tile = block * W + (threadIdx.x >> 6);
     if (tile >= ntiles) return;
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const int m0 = i0 + tile / nct * 16, n0 = f.c0 + tile % nct * 16;
@@ -509,7 +522,7 @@ __device__ __forceinline__ void far_update(T* __restrict__ Ar, T* __restrict__ A
 
 // ---------------------------------------------------------------------------
 // Pivot tournament for columns j0..j0+31 over rows j0..n-1, one launch; row i
-// of the columns at S + i lds.  Sets of CH = 256 R rows (R per thread) choose 32
+// of the columns at S + i lds.  Sets of CH = 64 W rows (one per thread) choose 32
 // candidates each, groups of G = CH / 32 sets merge.
 // Candidate sets of level L live at set index off[L] + i; a set is 32 ids and
 // the 32 x 32 original values per plane.  cnt: one arrival counter per group
@@ -518,51 +531,38 @@ __device__ __forceinline__ void far_update(T* __restrict__ Ar, T* __restrict__ A
 // plane) and the first zero pivot into *info.  The last f.blocks workgroups do
 // the previous step's far update instead (A, U; other columns than S's).
 // ---------------------------------------------------------------------------
-template <typename T, int R>
-__global__ __launch_bounds__(256) void k_tslu(const T* __restrict__ Sr, const T* __restrict__ Si, long lds, int j0,
+template <typename T, int W>
+__global__ __launch_bounds__(64 * W, sizeof(T) == 4 ? 2 : 1) void k_tslu(const T* __restrict__ Sr, const T* __restrict__ Si, long lds, int j0,
                                               int n, int* __restrict__ cid, T* __restrict__ cvr, T* __restrict__ cvi,
                                               int* __restrict__ cnt, int* __restrict__ ipiv, int* __restrict__ pl,
                                               T* __restrict__ d11r, T* __restrict__ d11i, int* __restrict__ info,
                                               T* __restrict__ Ar, T* __restrict__ Ai, long ld, FarUpdate f,
                                               const T* __restrict__ Ur, const T* __restrict__ Ui) {
     __builtin_amdgcn_s_setprio(3);  // latency-bound: win issue slots over co-resident GEMM waves
-    constexpr int CH = 256 * R, G = CH / PB;
+    constexpr int CH = 64 * W, G = CH / PB;
     if (blockIdx.x >= gridDim.x - f.blocks) {
-        far_update<T>(Ar, Ai, ld, n, f, blockIdx.x - (gridDim.x - f.blocks), Ur, Ui);
+        far_update<T, W>(Ar, Ai, ld, n, f, blockIdx.x - (gridDim.x - f.blocks), Ur, Ui);
         return;
     }
-    __shared__ ElimLds<T> L;
+    __shared__ ElimLds<T, W> L;
     const int t = threadIdx.x;
     // level 0: rows j0 + b*CH .. (n - j0 is a multiple of PB, so every set is full)
     const int r0 = j0 + blockIdx.x * CH;
     int nrows = min(CH, n - r0);
-    T xr[R][PB], xi[R][PB];
-    int id[R], src[R], mine[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int i = t + 256 * r;
-        id[r] = src[r] = r0 + i;
-        if (i < nrows) {
-            load_row(Sr + (long)(r0 + i) * lds, xr[r]);
-            load_row(Si + (long)(r0 + i) * lds, xi[r]);
-        }
+    Grp<T> xr[NG], xi[NG];
+    int id = r0 + t, src = r0 + t, mine;
+    if (t < nrows) {
+        load_groups(Sr + (long)(r0 + t) * lds, xr);
+        load_groups(Si + (long)(r0 + t) * lds, xi);
     }
     int level_sets = (n - j0 + CH - 1) / CH;  // sets at this level
     int set = blockIdx.x, off = 0, cnt_off = 0;
     bool from_matrix = true;
     for (;;) {
-        if (R > 1 && nrows <= 256) {  // a merge that needs one row per thread
-#pragma unroll
-            for (int r = 1; r < R; r++) mine[r] = -1;
-            elim_rows<T, 1>(L, reinterpret_cast<T(&)[1][PB]>(xr), reinterpret_cast<T(&)[1][PB]>(xi),
-                            reinterpret_cast<const int(&)[1]>(id), reinterpret_cast<const int(&)[1]>(src), nrows,
-                            reinterpret_cast<int(&)[1]>(mine));
-        } else {
-            elim_rows<T, R>(L, xr, xi, id, src, nrows, mine);
-        }
+        elim_rows<T, W>(L, xr, xi, id, src, nrows, mine);
         if (level_sets <= 1) break;
         // candidate set = original values of the chosen rows
-        for (int e = t; e < PB * PB; e += 256) {
+        for (int e = t; e < PB * PB; e += 64 * W) {
             const int r = e / PB, c = e % PB;
             const long o = ((long)(off + set) * PB + r) * PB + c;
             if (from_matrix) {
@@ -591,16 +591,12 @@ __global__ __launch_bounds__(256) void k_tslu(const T* __restrict__ Sr, const T*
         __threadfence();
         const int s0 = off + grp * G;
         nrows = gsize * PB;
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            const int i = t + 256 * r;
-            id[r] = -1;
-            src[r] = s0 * PB + i;
-            if (i < nrows) {
-                load_row(cvr + ((long)s0 * PB + i) * PB, xr[r]);
-                load_row(cvi + ((long)s0 * PB + i) * PB, xi[r]);
-                id[r] = cid[s0 * PB + i];
-            }
+        id = -1;
+        src = s0 * PB + t;
+        if (t < nrows) {
+            load_groups(cvr + ((long)s0 * PB + t) * PB, xr);
+            load_groups(cvi + ((long)s0 * PB + t) * PB, xi);
+            id = cid[s0 * PB + t];
         }
         from_matrix = false;
         cnt_off += (level_sets + G - 1) / G;
@@ -611,20 +607,21 @@ __global__ __launch_bounds__(256) void k_tslu(const T* __restrict__ Sr, const T*
     // root: the factored diagonal block, swaps, row-pair list, zero pivot
     if (t == 0) L.zmin = 0x7fffffff;
     __syncthreads();
+    if (mine >= 0) {
+        T dr = T(0), di = T(0);
 #pragma unroll
-    for (int r = 0; r < R; r++)
-        if (mine[r] >= 0) {
-            store_row(d11r + mine[r] * PB, xr[r]);
-            store_row(d11i + mine[r] * PB, xi[r]);
-            T dr = T(0), di = T(0);
+        for (int g = 0; g < NG; g++) {
+            store_group<T>(d11r + mine * PB + g * EW, xr[g]);
+            store_group<T>(d11i + mine * PB + g * EW, xi[g]);
 #pragma unroll
-            for (int c = 0; c < PB; c++)
-                if (c == mine[r]) {
-                    dr = xr[r][c];
-                    di = xi[r][c];
+            for (int c = 0; c < EW; c++)
+                if (g * EW + c == mine) {
+                    dr = xr[g][c];
+                    di = xi[g][c];
                 }
-            if (dr == T(0) && di == T(0)) atomicMin(&L.zmin, j0 + mine[r] + 1);
         }
+        if (dr == T(0) && di == T(0)) atomicMin(&L.zmin, j0 + mine + 1);
+    }
     __syncthreads();
     if (t == 0 && L.zmin != 0x7fffffff && *info == 0) *info = L.zmin;
     if (t < 64) root_swaps(L.oid, L.sw[0], L.sw[1], j0, ipiv, pl);
@@ -632,10 +629,10 @@ __global__ __launch_bounds__(256) void k_tslu(const T* __restrict__ Sr, const T*
 
 constexpr int kWideSetRows = 4096;
 
-// Levels of the tournament over m rows with sets of 256 r rows.
-int tslu_levels(int m, int r) {
+// Levels of the tournament over m rows with w waves per set.
+int tslu_levels(int m, int w) {
     int l = 1;
-    for (int sets = (m + 256 * r - 1) / (256 * r); sets > 1; sets = (sets + 8 * r - 1) / (8 * r)) l++;
+    for (int sets = (m + 64 * w - 1) / (64 * w); sets > 1; sets = (sets + 2 * w - 1) / (2 * w)) l++;
     return l;
 }
 
@@ -1392,12 +1389,11 @@ void invert_blocks(hipStream_t s, int n, const float* Fr, const float* Fi, long 
 // stream, behind an event each way, and the next 32 columns' swaps, panel solve
 // and update as three launches a step took 115 us at 3840 rows; now 75.)  The
 // swaps of the steps end as one net list for the columns outside the panel.
-// The FP32 tournament takes sets of 512 rows where they save a level: a set costs
-// 29 us of elimination instead of 19 for 256 rows, a level of merges ~23 (3840
-// rows: 58.7 against 73.1 us, 12288 rows, which save none: 91.9 against 80.6).
-// Up to kWideSetRows only: with two rows per thread the kernel does not start
-// beside the trailing update until a whole CU is free.  In FP64 two rows per
-// thread do not fit the registers.
+// The FP32 tournament takes sets of 512 rows (8 waves) where they save a level: 3840
+// rows 54.9 us against 65.0 (59.2 with two rows per thread of 4 waves); 1920 rows, where
+// they save none, 51.8 against 44.5.
+// Up to kWideSetRows only: 8 waves start beside the trailing update later than 4, when
+// two of its workgroups on a CU have ended.  In FP64 8 waves do not fit the registers.
 template <typename T>
 void factor_panel(bem_ctx* c, hipStream_t s, T* Ar, T* Ai, int k0, const LuWork<T>& w) {
     const int n = c->npad;
@@ -1407,6 +1403,7 @@ void factor_panel(bem_ctx* c, hipStream_t s, T* Ar, T* Ai, int k0, const LuWork<
     hipLaunchKernelGGL(k_compact<T>, dim3(first), dim3(256), 0, s, Ar, Ai, ld, k0, n, w.cpr, w.cpi);
     kt_close(c, kt, 0.0, 4.0 * sizeof(T) * (double)(n - k0) * PB);
     FarUpdate far{0, 0, 0, 0};
+    int far_tiles = -1;  // -1: nothing left to do
     for (int j0 = k0; j0 < k1; j0 += PB) {
         const int m = n - j0, par = ((j0 - k0) / PB) & 1;
         T *Sr = w.cpr + par * cp, *Si = w.cpi + par * cp;
@@ -1414,14 +1411,16 @@ void factor_panel(bem_ctx* c, hipStream_t s, T* Ar, T* Ai, int k0, const LuWork<
         T *d11r = w.d11 + par * 2 * PB * PB, *d11i = d11r + PB * PB;
         int* pl = w.pl + ((j0 - k0) / PB) * PLS;
         kt = kt_mark(c, KS_TSLU, s);
-        auto tslu = k_tslu<T, 1>;
-        int set = 256;
+        auto tslu = k_tslu<T, 4>;
+        int waves = 4;
         if constexpr (sizeof(T) == 4)
-            if (m <= kWideSetRows && tslu_levels(m, 2) < tslu_levels(m, 1)) {
-                tslu = k_tslu<T, 2>;
-                set = 512;
+            if (m <= kWideSetRows && tslu_levels(m, 8) < tslu_levels(m, 4)) {
+                tslu = k_tslu<T, 8>;
+                waves = 8;
             }
-        hipLaunchKernelGGL(tslu, dim3((m + set - 1) / set + far.blocks), dim3(256), 0, s, Sr, Si, (long)PB, j0, n,
+        const int set = 64 * waves;
+        far.blocks = far_tiles < 0 ? 0 : (far_tiles + waves - 1) / waves + 1;
+        hipLaunchKernelGGL(tslu, dim3((m + set - 1) / set + far.blocks), dim3(set), 0, s, Sr, Si, (long)PB, j0, n,
                            w.cid, w.cvr, w.cvi, w.cnt, c->ipiv, pl, d11r, d11i, w.info, Ar, Ai, ld, far, w.sur, w.sui);
         kt_close(c, kt, (sizeof(T) == 4 ? 6.0 : 8.0) * far.ncol * (double)m * PB,
                  2.0 * sizeof(T) * (double)m * (PB + 2 * far.ncol));
@@ -1431,7 +1430,8 @@ void factor_panel(bem_ctx* c, hipStream_t s, T* Ar, T* Ai, int k0, const LuWork<
                            Sr, Si, k0, j0, n, next, pl, d11r, d11i, Dr, Di, w.sur, w.sui, panel_net(w, k0));
         kt_close(c, kt, (next ? 10.0 : 4.0) * (double)m * PB * PB, (next ? 8.0 : 4.0) * sizeof(T) * (double)m * PB);
         const int c0 = std::min(k1, j0 + 2 * PB), ncol = k1 - c0;  // columns beyond the next 32
-        far = FarUpdate{j0, c0, ncol, next ? ((m - PB) / 16 * (ncol / 16) + 3) / 4 + 1 : 0};
+        far = FarUpdate{j0, c0, ncol, 0};
+        far_tiles = next ? (m - PB) / 16 * (ncol / 16) : -1;
     }
 }
 
