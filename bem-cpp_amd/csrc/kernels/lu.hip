@@ -764,42 +764,66 @@ constexpr int NETS = 3 * NB + 64;  // ints per net list
 // Composes the NB / PB row-pair lists of a panel (list l at pl + l PLS, applied in
 // order) into net: the last list with a row as destination names its source, whose
 // content before that list is followed through the earlier lists.  One workgroup.
-__device__ void compose_lists(const int* __restrict__ pl, int k0, int* __restrict__ net, int2 (*list)[2 * PB],
-                              int* top, int* count) {
-    constexpr int NL = NB / PB;
-    const int t = threadIdx.x;
-    int np[NL];
-#pragma unroll
-    for (int l = 0; l < NL; l++) np[l] = pl[l * PLS];
-#pragma unroll
-    for (int u = 0; u < NL * 2 * PB / 256; u++) {
-        const int e = t + 256 * u, l = e / (2 * PB), k = e % (2 * PB);
-        list[l][k] = make_int2(pl[l * PLS + 1 + 2 * k], pl[l * PLS + 2 + 2 * k]);  // beyond np: not used
+// A list's pairs lie in a table of their own, kListSlots places probed in order from a
+// hash of the destination, so that a row is found in a list in one or two steps: the
+// chain is what bounds it (each entry going through all pairs of the lists, k_step of a
+// panel's last step took 60 - 80 us for a random matrix and 22 for an assembled one, now 17 and 9).
+constexpr int kListSlots = 128;  // twice the pairs of a list, so a probe always ends
+struct PairTable {
+    int *dst, *src;  // NB / PB tables; dst -1: empty
+    __device__ __forceinline__ static int first(int row) { return (int)((unsigned)row * 0x9e3779b1u >> 25); }
+    __device__ __forceinline__ void insert(int l, int row, int from) const {
+        int h = first(row);
+        while (atomicCAS(&dst[l * kListSlots + h], -1, row) != -1) h = (h + 1) % kListSlots;
+        src[l * kListSlots + h] = from;
     }
+    // the source of `row` in list l, -1 if it is no destination there
+    __device__ __forceinline__ int find(int l, int row) const {
+        for (int h = first(row);; h = (h + 1) % kListSlots) {
+            const int d = dst[l * kListSlots + h];
+            if (d == row) return src[l * kListSlots + h];
+            if (d == -1) return -1;
+        }
+    }
+};
+__device__ void compose_lists(const int* __restrict__ pl, int k0, int* __restrict__ net, PairTable tab, int* top,
+                              int* count) {
+    constexpr int NL = NB / PB, PER = NL * 2 * PB / 256;
+    const int t = threadIdx.x;
+    static_assert(kListSlots == 128 && kListSlots >= 4 * PB, "the hash gives 7 bits; half of the places stay empty");
+    int2 pair[PER];
+    bool in[PER];
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+        const int e = t + 256 * u, l = e / (2 * PB), k = e % (2 * PB);
+        pair[u] = make_int2(pl[l * PLS + 1 + 2 * k], pl[l * PLS + 2 + 2 * k]);  // beyond the count: not used
+        in[u] = k < pl[l * PLS];
+    }
+    for (int e = t; e < NL * kListSlots; e += 256) tab.dst[e] = -1;
     top[t] = k0 + t;
     if (t == 0) *count = 0;
     __syncthreads();
-#pragma unroll 1
-    for (int u = 0; u < NL * 2 * PB / 256; u++) {
-        const int e = t + 256 * u, l = __builtin_amdgcn_readfirstlane(e / (2 * PB)), k = e % (2 * PB);
-        if (k >= np[l]) continue;
-        const int2 p = list[l][k];
+#pragma unroll
+    for (int u = 0; u < PER; u++)
+        if (in[u]) tab.insert((t + 256 * u) / (2 * PB), pair[u].x, pair[u].y);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+        const int l = (t + 256 * u) / (2 * PB), dst = pair[u].x;
+        if (!in[u]) continue;
         bool last = true;
-        for (int m = l + 1; m < NL; m++)
-            for (int q = 0; q < np[m]; q++) last = last && list[m][q].x != p.x;
+        for (int m = l + 1; m < NL && last; m++) last = tab.find(m, dst) < 0;
         if (!last) continue;
-        int src = p.y;
+        int src = pair[u].y;
         for (int m = l - 1; m >= 0; m--) {
-            int from = src;
-            for (int q = 0; q < np[m]; q++)
-                if (list[m][q].x == src) from = list[m][q].y;
-            src = from;
+            const int from = tab.find(m, src);
+            src = from < 0 ? src : from;
         }
-        if (p.x < k0 + NB) {
-            top[p.x - k0] = src;
-        } else if (src != p.x) {
+        if (dst < k0 + NB) {
+            top[dst - k0] = src;
+        } else if (src != dst) {
             const int i = atomicAdd(count, 1);
-            net[NB + 1 + 2 * i] = p.x;
+            net[NB + 1 + 2 * i] = dst;
             net[NB + 2 + 2 * i] = src;
         }
     }
@@ -847,8 +871,9 @@ __global__ __launch_bounds__(256) void k_step(T* __restrict__ Ar, T* __restrict_
     const int nrow = max(1, (n - j0 - PB) / PB), strip = (int)blockIdx.x - nrow;  // strip >= 0: other columns
     const int r0 = j0 + PB + blockIdx.x * PB;
     if (strip == NB / PB - 1 && !with_next) {  // beside the panel's last step
-        compose_lists(pl - (NB / PB - 1) * PLS, k0, net, reinterpret_cast<int2(*)[2 * PB]>(ur),
-                      reinterpret_cast<int*>(ui), map);
+        static_assert(sizeof(ur) >= NB / PB * kListSlots * sizeof(int), "a table's half fits");
+        compose_lists(pl - (NB / PB - 1) * PLS, k0, net, PairTable{reinterpret_cast<int*>(ur), reinterpret_cast<int*>(ui)},
+                      reinterpret_cast<int*>(lr), map);
         return;
     }
     const int np = pl[0];
