@@ -21,11 +21,11 @@
 //        and the rank-32 update of the next 32 columns on the matrix cores; the
 //        update of the panel's other columns rides in the next tournament's
 //        launch
-//   then L11^{-1} of the 256 x 256 diagonal block (by doubling: eight 32 x 32
-//   inverses in LDS, then three levels of batched GEMMs), U12 = L11^{-1} A12
-//   and the rank-256 trailing update A22 -= L21 U12 as matrix-core GEMMs
-//   (gemm.h; 3M form in FP32).  The inverses of all L and U diagonal blocks
-//   are kept for the GEMM-based multi-RHS solves.
+//   then the panel's net row interchanges in the other columns, U12 = L11^{-1} A12 by
+//   blocked substitution (k_u12_strip) and the rank-256 trailing update A22 -= L21 U12
+//   as matrix-core GEMMs (gemm_nt.h in FP32, 3M form; gemm.h).  The inverses of all
+//   256 x 256 L and U diagonal blocks are formed after the last panel for the
+//   GEMM-based multi-RHS solves (FP32 only).
 #include <cstdlib>
 #include <vector>
 
@@ -842,8 +842,8 @@ __device__ void compose_lists(const int* __restrict__ pl, int k0, int* __restric
 // S + 32 i, a compact copy) and L21 goes to the matrix; the columns J' are read
 // from the matrix and go, updated, to the compact copy D that the next
 // tournament and step read.  U12 of J' goes to U (32 x 32), not over the rows
-// other workgroups still read.  The other columns of the panel follow on
-// another stream.
+// other workgroups still read.  The other columns of the panel follow in the
+// next tournament's launch.
 //
 // Waves 0 and 1 form L21 (one row per quad of lanes), waves 2 and 3 U12 (one
 // column per quad) at the same time, then each wave multiplies one 16 x 16 tile
