@@ -1344,7 +1344,11 @@ __global__ __launch_bounds__(64) void k_inv_tri32(const T* __restrict__ Fr, cons
 //   lower [X11 0; X21 X22]  with X21 = -X22 (L21 X11),
 //   upper [X11 X12; 0 X22]  with X12 = -X11 (U12 X22)
 // (blockIdx.z = 0, 1; blockIdx.y = pair of all blocks; stage 0: the inner product W, to the
-// unused triangle of the block, 1: the outer one).  The sums run over the triangles
+// unused triangle of the block, 1: the outer one).  The upper ones then take one step of
+// correction, 2: W <- W + U11 X12, 3: X12 <- X12 - X11 W, since U X = I has to hold to
+// the rounding of |U||X|: the products alone leave |U11||X11||W|, which on meshes with
+// triangles of very different sizes made the first solve's residual 3 - 30 times as
+// large as with inverses by substitution (7200 edges: 1e-2, 6 sweeps instead of 3).  The sums run over the triangles
 // only, so that no value beside them is read; the 32 x 32 triangles at the start are
 // stored with their zeros.
 __global__ __launch_bounds__(256, 2) void k_tri_join(int stage, int h, const float* __restrict__ Fr,
@@ -1352,7 +1356,7 @@ __global__ __launch_bounds__(256, 2) void k_tri_join(int stage, int h, const flo
                                                      float* Ur, float* Ui) {
     constexpr int NT = 2;
     __shared__ __align__(16) float red[4 * 2 * 16 * 16 * NT];
-    const bool lower = blockIdx.z == 0;
+    const bool lower = stage < 2 && blockIdx.z == 0;
     const int nct = h / (16 * NT), m0 = blockIdx.x / nct * 16, n0 = blockIdx.x % nct * 16 * NT;
     const int np = IB / (2 * h), blk = blockIdx.y / np, d = blockIdx.y % np * 2 * h;
     const long f = ((long)blk * IB + d) * (ldf + 1), x = (long)blk * IB * IB + (long)d * (IB + 1);
@@ -1364,6 +1368,10 @@ __global__ __launch_bounds__(256, 2) void k_tri_join(int stage, int h, const flo
         const long a = f + (lower ? (long)h * ldf : h), b = lower ? 0 : x22;
         cmul_tile<NT>(m0, n0, lower ? n0 : 0, lower ? h : n0 + 16 * NT, Fr + a, Fi + a, ldf, Xr + b, Xi + b, IB, Xr + w,
                       Xi + w, IB, 1, red);
+    } else if (stage == 2) {
+        cmul_tile<NT, true>(m0, n0, m0, h, Fr + f, Fi + f, ldf, Xr + o, Xi + o, IB, Xr + w, Xi + w, IB, 4, red);
+    } else if (stage == 3) {
+        cmul_tile<NT>(m0, n0, m0, h, Xr, Xi, IB, Xr + w, Xi + w, IB, Xr + o, Xi + o, IB, 0, red);
     } else {
         const long a = lower ? x22 : 0;
         cmul_tile<NT>(m0, n0, lower ? 0 : m0, lower ? m0 + 16 : h, Xr + a, Xi + a, IB, Xr + w, Xi + w, IB, Xr + o,
@@ -1401,8 +1409,8 @@ void invert_blocks(hipStream_t s, int n, const float* Fr, const float* Fi, long 
                    float* Ui) {
     hipLaunchKernelGGL(k_inv_tri32<float>, dim3(n / PB, 2), dim3(64), 0, s, Fr, Fi, ldf, Lr, Li, Ur, Ui);
     for (int h = PB; h < IB; h *= 2)
-        for (int stage = 0; stage < 2; stage++)
-            hipLaunchKernelGGL(k_tri_join, dim3(h / 16 * (h / 32), n / (2 * h), 2), dim3(256), 0, s, stage, h, Fr, Fi,
+        for (int stage = 0; stage < 4; stage++)
+            hipLaunchKernelGGL(k_tri_join, dim3(h / 16 * (h / 32), n / (2 * h), stage < 2 ? 2 : 1), dim3(256), 0, s, stage, h, Fr, Fi,
                                ldf, Lr, Li, Ur, Ui);
 }
 
