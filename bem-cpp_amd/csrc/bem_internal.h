@@ -236,10 +236,11 @@ int ctx_fetch(bem_ctx* c, std::initializer_list<Fetch> list);
 // ncol, planar; ncol a multiple of 16).
 int z_product(bem_ctx* c, int ncol, const double* Xr, const double* Xi, const double* Br, const double* Bi, double* Or,
               double* Oi);
-// out[j] = sum over the rows i < n of |A[i][j]|^2, j < ncol, in a fixed order; part: work
-// area of col_norm2_work() values.
+// out[j] = sum over the rows i < n of |scale A[i][j]|^2, j < ncol, in a fixed order; part:
+// work area of col_norm2_work() values.
 size_t col_norm2_work(int n, int ncol);
-void col_norm2(hipStream_t s, int n, int ncol, const double* Ar, const double* Ai, long ld, double* part, double* out);
+void col_norm2(hipStream_t s, int n, int ncol, const double* Ar, const double* Ai, long ld, double* part, double* out,
+               double scale = 1.0);
 // A host matrix of rows x cols interleaved complex values (row- or column-major) into
 // planar FP64 (prows x ld), padded with zeros, or with the identity; and planes
 // (times scale) into a host matrix.  Through at most 32 MiB of the context's scratch.

@@ -179,9 +179,13 @@ int gmres_solve_launch(bem_ctx* c, int nrhs, double tol, int restart, int max_it
     };
     // r = B - Z X
     auto residual = [&]() -> int { return z_product(c, ncol, c->Xr, c->Xi, c->Br, c->Bi, re(r), im(r)); };
-    auto max_rel = [&](const std::vector<double>& r2) {
+    auto max_rel = [&](const std::vector<double>& r2) {  // NaN if any is
         double mx = 0.0;
-        for (int j = 0; j < nrhs; j++) mx = std::max(mx, bn2[j] > 0 ? std::sqrt(r2[j] / bn2[j]) : 0.0);
+        for (int j = 0; j < nrhs; j++) {
+            const double v = bn2[j] == 0.0 ? 0.0 : std::sqrt(r2[j] / bn2[j]);
+            if (std::isnan(v)) return v;
+            mx = std::max(mx, v);
+        }
         return mx;
     };
     // v_dst = src * scale[j] per column

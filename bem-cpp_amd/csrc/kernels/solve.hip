@@ -11,6 +11,9 @@
 // Mixed precision (factors in FP32): X_0 = 0, R_0 = B, and per sweep
 //   D = solve32(fp32(P R));  X += D;  R = B - Z X   (with the FP64 Z: zmul.hip)
 // until max_j ||R_j|| / ||B_j|| <= tol.  Norm reductions use a fixed order.
+#include <algorithm>
+#include <cmath>
+
 #include "../bem_internal.h"
 #include "cmul.h"
 #include "gemm.h"
@@ -237,13 +240,16 @@ void lu_apply64(bem_ctx* c, const double* Fr, const double* Fi, double* Yr, doub
     }
 }
 
-double max_ratio(const std::vector<double>& r2, const std::vector<double>& b2, int nrhs) {
-    double m = 0.0;
-    for (int j = 0; j < nrhs; j++) {
-        const double v = b2[j] > 0 ? std::sqrt(r2[j] / b2[j]) : std::sqrt(r2[j]);
-        m = std::max(m, v);
-    }
-    return m;
+// |r| / |b| of one column from the squares (|r| itself for b = 0).
+double ratio(double r2, double b2) { return b2 == 0.0 ? std::sqrt(r2) : std::sqrt(r2 / b2); }
+
+constexpr double kTiny = 0x1p-540;  // the squares of all doubles times this, and their sums, are finite
+
+// The same where a square is not finite, from the squares of the columns times kTiny.
+double ratio_scaled(double r2, double b2, double r2s, double b2s) {
+    const double r = std::isfinite(r2) ? kTiny * std::sqrt(r2) : std::sqrt(r2s);
+    const double b = std::isfinite(b2) ? kTiny * std::sqrt(b2) : std::sqrt(b2s);
+    return r / b;
 }
 
 }  // namespace
@@ -332,11 +338,31 @@ int lu_solve_launch(bem_ctx* c, int nrhs, double tol, int maxit, int* iters, dou
             hipLaunchKernelGGL(k_accumulate<double>, g1, dim3(256), 0, s, cnt, Yr, Yi, c->Xr, c->Xi, assign);
         }
     };
-    auto residual = [&](bool first) -> int {  // R = B - Z X and its norms, with B's at first
+    auto residual = [&](bool first) -> int {  // R = B - Z X and *res, with B's norms at first
         if (int rc = z_product(c, ncol, c->Xr, c->Xi, c->Br, c->Bi, Rr, Ri)) return rc;
         col_norm2(s, c->n, nrhs, Rr, Ri, (long)ldr, npt, nr2);
         const size_t nb = nrhs * sizeof(double);
-        return first ? ctx_fetch(c, {{r2.data(), nr2, nb}, {b2.data(), nb2, nb}}) : ctx_fetch(c, {{r2.data(), nr2, nb}});
+        if (int rc = first ? ctx_fetch(c, {{r2.data(), nr2, nb}, {b2.data(), nb2, nb}})
+                           : ctx_fetch(c, {{r2.data(), nr2, nb}}))
+            return rc;
+        auto finite = [&](int j) { return std::isfinite(r2[j]) && std::isfinite(b2[j]); };
+        int bad = 0;
+        while (bad < nrhs && finite(bad)) bad++;
+        std::vector<double> r2s, b2s;
+        if (bad < nrhs) {  // values above 1e154, or no numbers at all
+            r2s.resize(nrhs);
+            b2s.resize(nrhs);
+            col_norm2(s, c->n, nrhs, Rr, Ri, (long)ldr, npt, nr2, kTiny);
+            col_norm2(s, c->n, nrhs, c->Br, c->Bi, (long)ldr, npt, nb2, kTiny);
+            if (int rc = ctx_fetch(c, {{r2s.data(), nr2, nb}, {b2s.data(), nb2, nb}})) return rc;
+        }
+        *res = 0.0;
+        for (int j = 0; j < nrhs; j++) {
+            const double v = finite(j) ? ratio(r2[j], b2[j]) : ratio_scaled(r2[j], b2[j], r2s[j], b2s[j]);
+            if (!(v <= *res)) *res = v;
+            if (std::isnan(v)) break;  // (std::max would drop it, and a solution of NaN would count as converged)
+        }
+        return 0;
     };
 
     // plain solve
@@ -352,7 +378,7 @@ int lu_solve_launch(bem_ctx* c, int nrhs, double tol, int maxit, int* iters, dou
         BEM_HIP(c, hipEventRecord(e[2], s));
         col_norm2(s, c->n, nrhs, c->Br, c->Bi, (long)ldr, npt, nb2);
         if (int e2 = residual(true)) return e2;
-        *res0 = *res = max_ratio(r2, b2, nrhs);
+        *res0 = *res;
         int it = 0;
         float ts_loop = 0.0f;  // triangular solves inside the sweeps
         while (it < maxit && *res > tol) {
@@ -363,7 +389,6 @@ int lu_solve_launch(bem_ctx* c, int nrhs, double tol, int maxit, int* iters, dou
             if (int e2 = residual(false)) return e2;
             BEM_HIP(c, hipEventElapsedTime(&t0, e[0], e[1]));
             ts_loop += t0;
-            *res = max_ratio(r2, b2, nrhs);
             it++;
         }
         *iters = it;
@@ -373,7 +398,7 @@ int lu_solve_launch(bem_ctx* c, int nrhs, double tol, int maxit, int* iters, dou
         BEM_HIP(c, hipEventElapsedTime(&tall, e[2], e[3]));
         ts += ts_loop;          // all triangular solves
         ti = tall - ts_loop;    // residual GEMMs, norms, updates
-        if (maxit > 0 && *res > tol) rc = BEM_ERR_NOCONV;
+        if (maxit > 0 && !(*res <= tol)) rc = BEM_ERR_NOCONV;  // a residual of NaN, too
     }
     BEM_HIP(c, hipGetLastError());
     for (auto& x : e) (void)hipEventDestroy(x);

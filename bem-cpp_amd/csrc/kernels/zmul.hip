@@ -170,12 +170,12 @@ void zmul_launch(hipStream_t s, int nt, int M, int N, int c0, int ngrp, int S, c
     hipLaunchKernelGGL(k, grid, dim3(256), 0, s, M, N, c0, ngrp, Ks, nblk, Ar, Ai, Xr, Xi, P);
 }
 
-// part[b][j] = sum of |A[i][j]|^2 over the rows i of block b (kNormRows of them), j <
+// part[b][j] = sum of |scale A[i][j]|^2 over the rows i of block b (kNormRows of them), j <
 // ncol.  cw columns (a power of two, at most 64) side by side, the rows in 256 / cw
 // lanes, summed in a fixed order.
 constexpr int kNormRows = 128;
 __global__ __launch_bounds__(256) void k_colnorm2_part(int n, int ncol, int cw, const double* __restrict__ Ar,
-                                                       const double* __restrict__ Ai, long ld,
+                                                       const double* __restrict__ Ai, long ld, double scale,
                                                        double* __restrict__ part) {
     __shared__ double red[256];
     const int tx = threadIdx.x % cw, ty = threadIdx.x / cw, lanes = 256 / cw;
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(256) void k_colnorm2_part(int n, int ncol, int cw, 
     if (j < ncol)
 #pragma unroll 8
         for (int i = r0 + ty; i < r1; i += lanes) {
-            const double a = Ar[(long)i * ld + j], b = Ai[(long)i * ld + j];
+            const double a = scale * Ar[(long)i * ld + j], b = scale * Ai[(long)i * ld + j];
             s += a * a + b * b;
         }
     red[threadIdx.x] = s;
@@ -240,10 +240,11 @@ int z_product(bem_ctx* c, int N, const double* Xr, const double* Xi, const doubl
 
 size_t col_norm2_work(int n, int ncol) { return (size_t)norm_blocks(n) * ncol; }
 
-void col_norm2(hipStream_t s, int n, int ncol, const double* Ar, const double* Ai, long ld, double* part, double* out) {
+void col_norm2(hipStream_t s, int n, int ncol, const double* Ar, const double* Ai, long ld, double* part, double* out,
+               double scale) {
     int cw = 1;
     while (cw < ncol && cw < 64) cw *= 2;
     hipLaunchKernelGGL(k_colnorm2_part, dim3(norm_blocks(n), (ncol + cw - 1) / cw), dim3(256), 0, s, n, ncol, cw, Ar,
-                       Ai, ld, part);
+                       Ai, ld, scale, part);
     hipLaunchKernelGGL(k_colnorm2_sum, dim3(ncol), dim3(64), 0, s, norm_blocks(n), ncol, (const double*)part, out);
 }
