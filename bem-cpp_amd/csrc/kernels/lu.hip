@@ -42,7 +42,7 @@ constexpr int PB = 32;   // inner panel width (pivot block)
 
 template <typename T>
 __device__ __forceinline__ T mag2(T r, T i) {
-    return r * r + i * i;
+    return fmadd(r, r, i * i);
 }
 
 // 16-byte vector type of T (4 floats or 2 doubles).
@@ -66,15 +66,6 @@ using Nat16 = T __attribute__((ext_vector_type(16 / sizeof(T))));
 __device__ __forceinline__ float recip(float d) { return __builtin_amdgcn_rcpf(d); }
 __device__ __forceinline__ double recip(double d) { return 1.0 / d; }
 
-// Order-preserving 32-bit key of a non-negative magnitude; 0 is "no candidate".  A double
-// keeps 20 mantissa bits: rows closer than that in magnitude tie.  (The sign of a NaN is
-// masked.)  The row is found by a ballot: with the lane in the key's low bits instead (2N =
-// 3840 10.14 ms, now 10.23) 17 (14) mantissa bits are left, and a zero ties with a small entry.
-__device__ __forceinline__ unsigned mag_key(float m) { return (__float_as_uint(m) & 0x7fffffffu) + 1u; }
-__device__ __forceinline__ unsigned mag_key(double m) {
-    return ((unsigned)((unsigned long long)__double_as_longlong(m) >> 32) & 0x7fffffffu) + 1u;
-}
-
 // Maximum over the wave, in a scalar register (DPP within rows of 16, then
 // across the rows).
 template <int CTRL, int ROWS>
@@ -89,6 +80,76 @@ __device__ __forceinline__ unsigned wave_max(unsigned v) {
     v = max_dpp<0x142, 0xa>(v);  // row_bcast 15, 31
     v = max_dpp<0x143, 0xc>(v);
     return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// Order-preserving 32-bit keys of |r + i i|; 0 is "no candidate".  The row is found by a
+// ballot: with the lane in the key's low bits instead (2N = 3840 10.14 ms, now 10.23) 17 (14)
+// mantissa bits are left, and a zero ties with a small entry.
+// FP64: sign (that of a NaN masked), exponent and 20 mantissa bits of |x|^2; rows closer
+// than that tie.
+// FP32: all of |2^e x|^2 with the exponent counted from 2^-253, so that the keys of e = 0,
+// 63 (for squares below the range) and -64 (above) compare with each other.
+__device__ __forceinline__ unsigned mag_key(double r, double i) {
+    return ((unsigned)((unsigned long long)__double_as_longlong(mag2(r, i)) >> 32) & 0x7fffffffu) + 1u;
+}
+template <int E>
+__device__ __forceinline__ unsigned mag_key(float r, float i) {
+    if constexpr (E != 0) {
+        r = ldexpf(r, E);
+        i = ldexpf(i, E);
+    }
+    return (__float_as_uint(mag2(r, i)) & 0x7fffffffu) + ((126u - 2 * E) << 23) + 1u;
+}
+
+// FP32 values whose squares and their reciprocals are normal numbers: those within these
+// bounds.  The tournament computes with the squares; where a pivot turns out to lie outside,
+// the factorisation is done again with WIDE set, which scales such values by powers of two
+// first (in every tournament that costs 7 % at 2N = 3840, 10.2 -> 10.8 ms).
+constexpr float kSquareMin = 0x1p-62f, kSquareMax = 0x1p62f;
+
+// The largest key of the wave's open rows into wk, and the lane that has it (ties: the
+// lowest; a wave without open rows: lane 0, key 0).
+template <bool WIDE>
+__device__ __forceinline__ int best_lane(bool open, double r, double i, unsigned& wk) {
+    const unsigned key = open ? mag_key(r, i) : 0u;
+    wk = wave_max(key);
+    return __ffsll((long long)__ballot(key == wk)) - 1;
+}
+template <bool WIDE>
+__device__ __forceinline__ int best_lane(bool open, float r, float i, unsigned& wk) {
+    constexpr unsigned kLow = ((27u + 126u) << 23) + 1u, kHigh = ((254u + 126u) << 23) + 1u;  // 2^-100, 2^127
+    unsigned key = open ? mag_key<0>(r, i) : 0u;
+    wk = wave_max(key);
+    if constexpr (WIDE) {
+        if (wk - 1u < kLow - 1u) {
+            key = open ? mag_key<63>(r, i) : 0u;
+            wk = wave_max(key);
+        } else if (wk >= kHigh) {
+            key = open ? mag_key<-64>(r, i) : 0u;
+            wk = wave_max(key);
+        }
+    }
+    return __ffsll((long long)__ballot(key == wk)) - 1;
+}
+
+// l = x / u by the reciprocal of u (the rows scale by it, as zgetf2 does), 0 for u = 0;
+// returns whether u is not 0.  WIDE: x and u by the power of two that brings u to [1/2, 1)
+// first; otherwise rounded the same.
+template <bool WIDE, typename T>
+__device__ __forceinline__ bool scale_row(T xr, T xi, T ur, T ui, T& lr, T& li) {
+    if constexpr (WIDE) {
+        const int e = -__builtin_amdgcn_frexp_expf(fmaxf(fabsf(ur), fabsf(ui)));
+        xr = ldexpf(xr, e);
+        xi = ldexpf(xi, e);
+        ur = ldexpf(ur, e);
+        ui = ldexpf(ui, e);
+    }
+    const T d = mag2(ur, ui);
+    const T inv = d > T(0) ? recip(d) : T(0);
+    const T qr = ur * inv, qi = -ui * inv;
+    lr = fmadd(xr, qr, -(xi * qi));
+    li = fmadd(xr, qi, xi * qr);
+    return d > T(0);
 }
 
 // v of lane l (l the same for the whole wave) as a scalar.
@@ -249,7 +310,7 @@ __device__ __forceinline__ void window_update(Grp<double> (&xr)[NG], Grp<double>
 // One level of 256 rows takes 22.1 us (FP64 31.3), of 512 31.0, alone; with the
 // products of window_update as multiply-adds on operands from LDS and the rows rotated
 // by copies it took 24.5 (31.5), and 35.8 with two rows per thread of 4 waves.
-template <typename T, int W>
+template <typename T, int W, bool WIDE>
 __device__ __forceinline__ void elim_rows(ElimLds<T, W>& L, Grp<T> (&xr)[NG], Grp<T> (&xi)[NG], int id, int src,
                                           int nrows, int& mine) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -269,9 +330,8 @@ __device__ __forceinline__ void elim_rows(ElimLds<T, W>& L, Grp<T> (&xr)[NG], Gr
             const int par = q & 1;
             int wl = 0;  // the wave's best lane (ties: the lowest)
             if (active) {
-                const unsigned key = valid && mine < 0 ? mag_key(mag2(T(hr[q]), T(hi[q]))) : 0u;
-                const unsigned wk = wave_max(key);
-                wl = __ffsll((long long)__ballot(key == wk)) - 1;
+                unsigned wk;
+                wl = best_lane<WIDE>(valid && mine < 0, T(hr[q]), T(hi[q]), wk);
                 if (lane == wl) {
                     store_group<T>(L.win[par][wave][0], hr, q);
                     store_group<T>(L.win[par][wave][1], hi, q);
@@ -308,14 +368,11 @@ __device__ __forceinline__ void elim_rows(ElimLds<T, W>& L, Grp<T> (&xr)[NG], Gr
                 ui[c] = from_lane(ci[c], wv);
             }
             const bool won = wave == wv && lane == wl;
-            // reciprocal of the pivot (the rows scale by it, as zgetf2 does)
-            const T d = ur[q] * ur[q] + ui[q] * ui[q];
-            const T inv = d > T(0) ? recip(d) : T(0);
-            const T qr = ur[q] * inv, qi = -ui[q] * inv;
+            T a, b;
+            const bool nonzero = scale_row<WIDE>(T(hr[q]), T(hi[q]), ur[q], ui[q], a, b);
             if (won) mine = s + q;
             // branch-free update: rows that are not eliminated use multiplier 0
-            const bool upd = valid && mine < 0 && d > T(0);
-            const T a = hr[q] * qr - hi[q] * qi, b = hr[q] * qi + hi[q] * qr;
+            const bool upd = valid && mine < 0 && nonzero;
             lr[q] = upd ? a : T(0);
             li[q] = upd ? b : T(0);
             hr[q] = upd ? a : T(hr[q]);
@@ -525,10 +582,11 @@ __device__ __forceinline__ void far_update(T* __restrict__ Ar, T* __restrict__ A
 // the 32 x 32 original values per plane.  cnt: one arrival counter per group
 // per level (zero on entry; reset by the merging block).  The root writes
 // ipiv, the row-pair list pl, the factored diagonal block d11 (32 x 32 per
-// plane) and the first zero pivot into *info.  The last f.blocks workgroups do
+// plane), the first zero pivot into *info and whether a pivot asks for WIDE into
+// info[1].  The last f.blocks workgroups do
 // the previous step's far update instead (A, U; other columns than S's).
 // ---------------------------------------------------------------------------
-template <typename T, int W>
+template <typename T, int W, bool WIDE = false>
 __global__ __launch_bounds__(64 * W, sizeof(T) == 4 ? 2 : 1) void k_tslu(const T* __restrict__ Sr, const T* __restrict__ Si, long lds, int j0,
                                               int n, int* __restrict__ cid, T* __restrict__ cvr, T* __restrict__ cvi,
                                               int* __restrict__ cnt, int* __restrict__ ipiv, int* __restrict__ pl,
@@ -556,7 +614,7 @@ __global__ __launch_bounds__(64 * W, sizeof(T) == 4 ? 2 : 1) void k_tslu(const T
     int set = blockIdx.x, off = 0, cnt_off = 0;
     bool from_matrix = true;
     for (;;) {
-        elim_rows<T, W>(L, xr, xi, id, src, nrows, mine);
+        elim_rows<T, W, WIDE>(L, xr, xi, id, src, nrows, mine);
         if (level_sets <= 1) break;
         // candidate set = original values of the chosen rows
         for (int e = t; e < PB * PB; e += 64 * W) {
@@ -618,6 +676,10 @@ __global__ __launch_bounds__(64 * W, sizeof(T) == 4 ? 2 : 1) void k_tslu(const T
                 }
         }
         if (dr == T(0) && di == T(0)) atomicMin(&L.zmin, j0 + mine + 1);
+        if constexpr (sizeof(T) == 4 && !WIDE) {
+            const float m = fmaxf(fabsf(dr), fabsf(di));
+            if (m < kSquareMin || m > kSquareMax) info[1] = 1;
+        }
     }
     __syncthreads();
     if (t == 0 && L.zmin != 0x7fffffff && *info == 0) *info = L.zmin;
@@ -1379,7 +1441,7 @@ __global__ __launch_bounds__(256, 2) void k_tri_join(int stage, int h, const flo
 // Work buffers of one factorisation (device).
 template <typename T>
 struct LuWork {
-    int* info;       // first zero pivot (1-based), 0 if none
+    int* info;       // first zero pivot (1-based), 0 if none; whether a pivot lies outside kSquareMin .. kSquareMax
     int* cnt;        // tournament arrival counters
     int* cid;        // candidate row ids
     T *cvr, *cvi;    // candidate values
@@ -1425,7 +1487,7 @@ void invert_blocks(hipStream_t s, int n, const float* Fr, const float* Fi, long 
 // Up to kWideSetRows only: 8 waves start beside the trailing update later than 4, when
 // two of its workgroups on a CU have ended.  In FP64 8 waves do not fit the registers.
 template <typename T>
-void factor_panel(bem_ctx* c, hipStream_t s, T* Ar, T* Ai, int k0, const LuWork<T>& w) {
+void factor_panel(bem_ctx* c, hipStream_t s, T* Ar, T* Ai, int k0, const LuWork<T>& w, bool wide) {
     const int n = c->npad;
     const long ld = n, cp = (long)n * PB;
     const int k1 = k0 + NB, first = ((n - k0) * (PB * (int)sizeof(T) / 16) + 255) / 256;
@@ -1443,11 +1505,10 @@ void factor_panel(bem_ctx* c, hipStream_t s, T* Ar, T* Ai, int k0, const LuWork<
         kt = kt_mark(c, KS_TSLU, s);
         auto tslu = k_tslu<T, 4>;
         int waves = 4;
-        if constexpr (sizeof(T) == 4)
-            if (m <= kWideSetRows && tslu_levels(m, 8) < tslu_levels(m, 4)) {
-                tslu = k_tslu<T, 8>;
-                waves = 8;
-            }
+        if constexpr (sizeof(T) == 4) {
+            if (m <= kWideSetRows && tslu_levels(m, 8) < tslu_levels(m, 4)) waves = 8;
+            tslu = waves == 8 ? (wide ? k_tslu<T, 8, true> : k_tslu<T, 8>) : wide ? k_tslu<T, 4, true> : k_tslu<T, 4>;
+        }
         const int set = 64 * waves;
         far.blocks = far_tiles < 0 ? 0 : (far_tiles + waves - 1) / waves + 1;
         hipLaunchKernelGGL(tslu, dim3((m + set - 1) / set + far.blocks), dim3(set), 0, s, Sr, Si, (long)PB, j0, n,
@@ -1510,7 +1571,7 @@ void update_columns(bem_ctx* c, hipStream_t us, T* Ar, T* Ai, int k0, int c0, in
 // Stream layout (c->lu_streams): 0 = everything on the context stream (no
 // overlap); 1 = panel stream and context stream over all CUs.
 template <typename T>
-void factor(bem_ctx* c, T* Ar, T* Ai, T* Lir, T* Lii, T* Uir, T* Uii, const LuWork<T>& w) {
+void factor(bem_ctx* c, T* Ar, T* Ai, T* Lir, T* Lii, T* Uir, T* Uii, const LuWork<T>& w, bool wide) {
     const int n = c->npad, nb = n / NB;
     const long ld = n;
     hipStream_t us = c->stream, ps = c->stream2;
@@ -1524,7 +1585,7 @@ void factor(bem_ctx* c, T* Ar, T* Ai, T* Lir, T* Lii, T* Uir, T* Uii, const LuWo
         hipLaunchKernelGGL(k_swap_net<T>, dim3(k0 / 16), dim3(256), 0, us, Ar, Ai, ld, k0, 0, panel_net(w, k0));
         kt_close(c, kt, 0.0, 4.0 * sizeof(T) * (double)k0 * 2 * NB);
     };
-    factor_panel<T>(c, ps, Ar, Ai, 0, w);
+    factor_panel<T>(c, ps, Ar, Ai, 0, w, wide);
     for (int K = 0; K < nb; K++) {
         const int k0 = K * NB;
         const int nr = n - (k0 + NB);
@@ -1547,7 +1608,7 @@ void factor(bem_ctx* c, T* Ar, T* Ai, T* Lir, T* Lii, T* Uir, T* Uii, const LuWo
         if (nr > NB)
             update_columns<T>(c, us, Ar, Ai, k0, k0 + 2 * NB, nr - NB, w, ps != us && c->gemm_plan[sizeof(T) == 4 ? 0 : 1].cap > 0);
         (void)hipEventRecord(e_rest, us);
-        factor_panel<T>(c, ps, Ar, Ai, k0 + NB, w);
+        factor_panel<T>(c, ps, Ar, Ai, k0 + NB, w, wide);
     }
     // the inverses of all diagonal blocks (FP32; the FP64 solves substitute with
     // the diagonal blocks themselves)
@@ -1565,7 +1626,7 @@ __global__ void k_convert(const double* __restrict__ a, T* __restrict__ b, size_
 }
 
 template <typename T>
-int factor_prec(bem_ctx* c, T* Ar, T* Ai, void*& inv, size_t& inv_bytes) {
+int factor_prec(bem_ctx* c, T* Ar, T* Ai, void*& inv, size_t& inv_bytes, bool wide = false) {
     const int n = c->npad;
     // diagonal-block inverses (FP32 only): L and U, npad x NB per plane each
     constexpr bool with_inv = sizeof(T) == 4;
@@ -1609,7 +1670,7 @@ int factor_prec(bem_ctx* c, T* Ar, T* Ai, void*& inv, size_t& inv_bytes) {
     w.utr = w.cpi + 2 * (size_t)PB * n;
     w.uti = w.utr + (size_t)NB * n;
     BEM_HIP(c, hipMemsetAsync(w.info, 0, (64 + ncnt) * sizeof(int), c->stream));
-    factor<T>(c, Ar, Ai, Lir, Lii, Uir, Uii, w);
+    factor<T>(c, Ar, Ai, Lir, Lii, Uir, Uii, w, wide);
     return 0;
 }
 
@@ -1784,17 +1845,25 @@ int lu_factor_launch(bem_ctx* c, int precision) {
         rc = factor_prec<float>(c, c->Wr, c->Wi, c->inv32, c->inv32_bytes);
     }
     if (rc) return rc;
-    BEM_HIP(c, hipGetLastError());
-    void* scr = nullptr;
-    if (int e = ctx_scratch(c, 256, &scr)) return e;
-    int info = 0;
+    int info[2] = {0, 0};
     // swap sequence -> row permutation (row i of P Z is row perm[i] of Z)
     std::vector<int> ip(n), perm(n);
-    if (int e = ctx_fetch(c, {{&info, scr, sizeof(int)}, {ip.data(), c->ipiv, n * sizeof(int)}})) return e;
+    auto fetch = [&]() -> int {
+        BEM_HIP(c, hipGetLastError());
+        void* scr = nullptr;
+        if (int e = ctx_scratch(c, 256, &scr)) return e;
+        return ctx_fetch(c, {{info, scr, sizeof(info)}, {ip.data(), c->ipiv, n * sizeof(int)}});
+    };
+    if ((rc = fetch())) return rc;
+    if (info[1] && c->has_Z64) {  // FP32 pivots whose squares leave the range
+        if ((rc = load_working_copy<float>(c, c->Wr, c->Wi))) return rc;
+        if ((rc = factor_prec<float>(c, c->Wr, c->Wi, c->inv32, c->inv32_bytes, true))) return rc;
+        if ((rc = fetch())) return rc;
+    }
     for (int i = 0; i < n; i++) perm[i] = i;
     for (int i = 0; i < n; i++)
         if (ip[i] != i) std::swap(perm[i], perm[ip[i]]);
     if (int e = ctx_put(c, c->perm, perm.data(), n * sizeof(int))) return e;
     if (n * sizeof(int) > kPinBytes / 2) BEM_HIP(c, hipStreamSynchronize(s));
-    return info > c->n ? 0 : info;  // a zero pivot inside the identity padding cannot occur
+    return info[0] > c->n ? 0 : info[0];  // a zero pivot inside the identity padding cannot occur
 }

@@ -7,11 +7,23 @@
 __device__ __forceinline__ float fmadd(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fmadd(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
+// a / b.  In FP32 with b brought to [1/2, 1) by a power of two: the square of a divisor
+// below 5e-20 or above 1.8e19 leaves the range (that of a double below 1e-154).
 template <typename T>
 __device__ __forceinline__ void cdiv(T ar, T ai, T br, T bi, T& qr, T& qi) {
+    int e = 0;
+    if constexpr (sizeof(T) == 4) {
+        e = -__builtin_amdgcn_frexp_expf(fmaxf(fabsf(br), fabsf(bi)));
+        br = ldexpf(br, e);
+        bi = ldexpf(bi, e);
+    }
     const T d = br * br + bi * bi;
     qr = (ar * br + ai * bi) / d;
     qi = (ai * br - ar * bi) / d;
+    if constexpr (sizeof(T) == 4) {
+        qr = ldexpf(qr, e);
+        qi = ldexpf(qi, e);
+    }
 }
 
 // Value of lane l (uniform) of the wave, broadcast through the scalar unit.
