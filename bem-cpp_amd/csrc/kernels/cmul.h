@@ -22,9 +22,8 @@
 
 #include "gemm.h"
 
-// Rows of the diagonal blocks that the FP32 solves apply as inverses.  Larger ones would
-// shorten their chain but cost accuracy: the first solve's residual is 3 - 30 times
-// as large with 1024 rows, and 2N = 6042 needs a third sweep.
+// Rows of the diagonal blocks that the FP32 solves apply as inverses: the padded size is a
+// multiple of 256 and of nothing larger.
 constexpr int IB = 256;
 
 typedef float v2f __attribute__((ext_vector_type(2)));
@@ -57,10 +56,8 @@ __device__ __forceinline__ void cmul_store(float* __restrict__ p, int r, const f
 }
 
 // The workgroup's tile at (m0, n0) over k = [k0, k1) (multiples of 16).  mode 0: C -= A B,
-// 4: C += A B,
-// 1: C = A B, 3: C = -A B.  C may not overlap A or B.  UPPER:
-// A's values left of its diagonal are taken as zero.  red: 4 x 2 x 16 x 16 NT floats of LDS.
-template <int NT, bool UPPER = false>
+// 1: C = A B, 3: C = -A B.  C may not overlap A or B.  red: 4 x 2 x 16 x 16 NT floats of LDS.
+template <int NT>
 __device__ __forceinline__ void cmul_tile(int m0, int n0, int k0, int k1, const float* __restrict__ Ar,
                                           const float* __restrict__ Ai, long lda, const float* __restrict__ Br,
                                           const float* __restrict__ Bi, long ldb, float* __restrict__ Cr,
@@ -79,11 +76,6 @@ __device__ __forceinline__ void cmul_tile(int m0, int n0, int k0, int k1, const 
     auto load = [&](Step& s, int k) {
         s.a[0] = *reinterpret_cast<const v4f*>(ar + k);
         s.a[1] = *reinterpret_cast<const v4f*>(ai + k);
-        if constexpr (UPPER) {
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                if (k + 4 * g + e < m0 + r) s.a[0][e] = s.a[1][e] = 0.f;
-        }
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             cmul_load<NT>(br + (long)(k + e) * ldb, r, s.b[0][e]);
@@ -94,7 +86,7 @@ __device__ __forceinline__ void cmul_tile(int m0, int n0, int k0, int k1, const 
     const int row = threadIdx.x / 16, c = threadIdx.x % 16;
     const long o = (long)(m0 + row) * ldc + n0;
     float old[2][NT] = {};
-    if (mode == 0 || mode == 4) {
+    if (mode == 0) {
         cmul_load<NT>(Cr + o, c, old[0]);
         cmul_load<NT>(Ci + o, c, old[1]);
     }
@@ -155,7 +147,7 @@ __device__ __forceinline__ void cmul_tile(int m0, int n0, int k0, int k1, const 
             for (int t = 0; t < NT; t++) v[t] += u[t];
         }
 #pragma unroll
-        for (int t = 0; t < NT; t++) v[t] = mode == 0 ? old[p][t] - v[t] : mode == 4 ? old[p][t] + v[t] : mode == 1 ? v[t] : -v[t];
+        for (int t = 0; t < NT; t++) v[t] = mode == 0 ? old[p][t] - v[t] : mode == 1 ? v[t] : -v[t];
         cmul_store<NT>((p ? Ci : Cr) + o, c, v);
     }
 }

@@ -1404,12 +1404,9 @@ __global__ __launch_bounds__(64) void k_inv_tri32(const T* __restrict__ Fr, cons
 //   upper [X11 X12; 0 X22]  with X12 = -X11 (U12 X22)
 // (blockIdx.z = 0, 1; blockIdx.y = pair of all blocks; stage 0: the inner product W, to the
 // unused triangle of the block, 1: the outer one).  The upper ones then take one step of
-// correction, 2: W <- W + U11 X12, 3: X12 <- X12 - X11 W, since U X = I has to hold to
-// the rounding of |U||X|: the products alone leave |U11||X11||W|, which on meshes with
-// triangles of very different sizes made the first solve's residual 3 - 30 times as
-// large as with inverses by substitution (7200 edges: 1e-2, 6 sweeps instead of 3).  The sums run over the triangles
-// only, so that no value beside them is read; the 32 x 32 triangles at the start are
-// stored with their zeros.
+// correction: W <- U12 X22 + U11 X12 (k_tri_residual), 2: X12 <- X12 - X11 W.  The sums
+// run over the triangles only, so that no value beside them is read; the 32 x 32 triangles
+// at the start are stored with their zeros.
 __global__ __launch_bounds__(256, 2) void k_tri_join(int stage, int h, const float* __restrict__ Fr,
                                                      const float* __restrict__ Fi, long ldf, float* Lr, float* Li,
                                                      float* Ur, float* Ui) {
@@ -1427,14 +1424,75 @@ __global__ __launch_bounds__(256, 2) void k_tri_join(int stage, int h, const flo
         const long a = f + (lower ? (long)h * ldf : h), b = lower ? 0 : x22;
         cmul_tile<NT>(m0, n0, lower ? n0 : 0, lower ? h : n0 + 16 * NT, Fr + a, Fi + a, ldf, Xr + b, Xi + b, IB, Xr + w,
                       Xi + w, IB, 1, red);
-    } else if (stage == 2) {
-        cmul_tile<NT, true>(m0, n0, m0, h, Fr + f, Fi + f, ldf, Xr + o, Xi + o, IB, Xr + w, Xi + w, IB, 4, red);
-    } else if (stage == 3) {
-        cmul_tile<NT>(m0, n0, m0, h, Xr, Xi, IB, Xr + w, Xi + w, IB, Xr + o, Xi + o, IB, 0, red);
-    } else {
+    } else if (stage == 1) {
         const long a = lower ? x22 : 0;
         cmul_tile<NT>(m0, n0, lower ? 0 : m0, lower ? m0 + 16 : h, Xr + a, Xi + a, IB, Xr + w, Xi + w, IB, Xr + o,
                       Xi + o, IB, 3, red);
+    } else {
+        cmul_tile<NT>(m0, n0, m0, h, Xr, Xi, IB, Xr + w, Xi + w, IB, Xr + o, Xi + o, IB, 0, red);
+    }
+}
+
+// The residual of a join of upper triangles (h, blockIdx.y as in k_tri_join): W = U12 X22 +
+// U11 X12, to the unused triangle of the block, with products and sums in FP64, so that the
+// corrected X12 is good to its own rounding given X11 and X22: U X = I has to hold to the
+// rounding of |U||X|, as by substitution.  The joined products alone leave |U11||X11||W|,
+// which on meshes with triangles of very different sizes made the first solve's residual
+// 3 - 30 times as large (7200 edges: 1e-2, 6 sweeps instead of 3).  With W in FP32 X12 keeps
+// cond(U11) roundings (an ellipsoid of 10440 unknowns: 2e-2 before and 4e-5 after the
+// first sweep, 4 sweeps; now 1e-2, 3e-6 and 3, by substitution 2e-2, 3e-5 and 3).
+// A workgroup takes 16 x 32 values, its waves a quarter of k each, as in cmul_tile.
+__global__ __launch_bounds__(256, 2) void k_tri_residual(int h, const float* __restrict__ Fr,
+                                                         const float* __restrict__ Fi, long ldf, float* Ur,
+                                                         float* Ui) {
+    constexpr int NT = 2;
+    __shared__ double red[4][2][16][16 * NT];
+    const int nct = h / (16 * NT), m0 = blockIdx.x / nct * 16, n0 = blockIdx.x % nct * 16 * NT;
+    const int np = IB / (2 * h), blk = blockIdx.y / np, d = blockIdx.y % np * 2 * h;
+    const long f = ((long)blk * IB + d) * (ldf + 1), x = (long)blk * IB * IB + (long)d * (IB + 1);
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    v4d re[NT], im[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) re[t] = im[t] = v4d{};
+    // U11 X12 over k = m0 .. h, then U12 X22 over k = h .. h + n0 + 16 NT (columns of U, rows of X)
+    const int n1 = (h - m0) / 16, ns = n1 + n0 / 16 + NT;
+    const float* ar = Fr + f + (long)(m0 + r) * ldf;
+    const float* ai = Fi + f + (long)(m0 + r) * ldf;
+    const float* br = Ur + x + h + n0 + r;
+    const float* bi = Ui + x + h + n0 + r;
+    for (int q = wave; q < ns; q += 4) {
+        const int k = (q < n1 ? m0 + 16 * q : h + 16 * (q - n1)) + 4 * g;
+        float a0[4], a1[4];
+        load_row4<float>(ar + k, a0);
+        load_row4<float>(ai + k, a1);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const bool in = k + e >= m0 + r;  // left of the diagonal lies L
+            const double p = in ? a0[e] : 0.f, s = in ? a1[e] : 0.f;
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                const double b0 = br[(long)(k + e) * IB + 16 * t], b1 = bi[(long)(k + e) * IB + 16 * t];
+                re[t] = mfma16x16x4(p, b0, re[t]);
+                re[t] = mfma16x16x4(s, -b1, re[t]);
+                im[t] = mfma16x16x4(p, b1, im[t]);
+                im[t] = mfma16x16x4(s, b0, im[t]);
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            red[wave][0][g + 4 * q][16 * t + r] = re[t][q];
+            red[wave][1][g + 4 * q][16 * t + r] = im[t][q];
+        }
+    __syncthreads();
+    for (int e = threadIdx.x; e < 16 * 16 * NT; e += 256) {
+        const int row = e / (16 * NT), col = e % (16 * NT);
+        const long o = x + (long)(h + m0 + row) * IB + n0 + col;
+        Ur[o] = (float)(((red[0][0][row][col] + red[1][0][row][col]) + red[2][0][row][col]) + red[3][0][row][col]);
+        Ui[o] = (float)(((red[0][1][row][col] + red[1][1][row][col]) + red[2][1][row][col]) + red[3][1][row][col]);
     }
 }
 
@@ -1467,10 +1525,15 @@ int* panel_net(const LuWork<T>& w, int k0) {
 void invert_blocks(hipStream_t s, int n, const float* Fr, const float* Fi, long ldf, float* Lr, float* Li, float* Ur,
                    float* Ui) {
     hipLaunchKernelGGL(k_inv_tri32<float>, dim3(n / PB, 2), dim3(64), 0, s, Fr, Fi, ldf, Lr, Li, Ur, Ui);
-    for (int h = PB; h < IB; h *= 2)
-        for (int stage = 0; stage < 4; stage++)
-            hipLaunchKernelGGL(k_tri_join, dim3(h / 16 * (h / 32), n / (2 * h), stage < 2 ? 2 : 1), dim3(256), 0, s, stage, h, Fr, Fi,
-                               ldf, Lr, Li, Ur, Ui);
+    for (int h = PB; h < IB; h *= 2) {
+        const unsigned tiles = h / 16 * (h / 32), pairs = n / (2 * h);
+        for (int stage = 0; stage < 3; stage++) {
+            if (stage == 2)
+                hipLaunchKernelGGL(k_tri_residual, dim3(tiles, pairs), dim3(256), 0, s, h, Fr, Fi, ldf, Ur, Ui);
+            hipLaunchKernelGGL(k_tri_join, dim3(tiles, pairs, stage < 2 ? 2 : 1), dim3(256), 0, s, stage, h, Fr, Fi, ldf, Lr,
+                               Li, Ur, Ui);
+        }
+    }
 }
 
 // Factors the outer panel of columns k0 .. k0+NB-1 (rows k0 .. n-1) on stream
