@@ -88,12 +88,37 @@ constexpr int BJ_O = 64;   // outer panel
 constexpr int BJ_T = 512;  // threads of k_bj_panel (256 threads with twice the rows each measured the same)
 constexpr int BJ_MAXR = 3; // rows per thread it can hold in registers (64 registers each)
 
-// 32-bit order-preserving key of |z|^2 (20 mantissa bits); 0: no candidate.
-__device__ __forceinline__ unsigned bj_key(double r, double i) {
-    const double m = r * r + i * i;
-    return m >= 0.0 ? (unsigned)((unsigned long long)__double_as_longlong(m) >> 32) + 1u : 1u;
-}
+// |z|^2, 0 for a NaN: a column always has a pivot.
+__device__ __forceinline__ double bj_mag(double r, double i) { return fmax(r * r + i * i, 0.0); }
+
 extern "C" __device__ unsigned __ockl_wfred_max_u32(unsigned);
+// Maximum over the eight lanes of each row half (DPP).
+__device__ __forceinline__ unsigned bj_max8(unsigned v) {
+    v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0xb1, 0xf, 0xf, false));  // quad_perm [1, 0, 3, 2]
+    v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x4e, 0xf, 0xf, false));  // [2, 3, 0, 1]
+    return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, false));  // row_half_mirror
+}
+
+// A lane's candidate: the upper word of its |z|^2 plus one (0: none), the lower word, its row.
+struct BjCand {
+    unsigned hi, lo, row;
+};
+// The first lane with the largest candidate (ties: the lowest row) of the wave, or of its
+// first eight lanes: by the upper word, which mostly decides, then the lower, then the row.
+template <bool EIGHT>
+__device__ __forceinline__ int bj_best_lane(const BjCand& k) {
+    auto top = [](unsigned v) { return EIGHT ? bj_max8(v) : __ockl_wfred_max_u32(v); };
+    constexpr unsigned long long kLanes = EIGHT ? 0xffull : ~0ull;
+    unsigned long long mask = __ballot(k.hi == top(k.hi)) & kLanes;
+    if (__popcll(mask) > 1) {
+        const int lane = threadIdx.x & 63;
+        const unsigned lo = (mask >> lane) & 1ull ? k.lo : 0u;
+        mask &= __ballot(lo == top(lo));
+        const unsigned low = (mask >> lane) & 1ull ? ~k.row : 0u;
+        mask &= __ballot(low == top(low));
+    }
+    return __ffsll((long long)mask) - 1;
+}
 
 // Columns of unrolled elimination steps; the registers rotate by so many after them.
 // (All 16 steps unrolled, each row read ahead whole and with two selects per value
@@ -166,9 +191,9 @@ __device__ __forceinline__ void bj_store_rows(double* __restrict__ a, int ld, in
 // Elimination of columns c0 .. c0+15 of every block, one workgroup each.
 // RPT > 0: the panel's rows in registers, rows t + BJ_T r, r < RPT (n2 <= RPT
 // BJ_T); RPT == 0: the panel stays in memory (any n2).  step[row] is the
-// column a row is the pivot of (-1: none yet).  The pivot is the largest |a|
-// (to 2^-20; ties: the lowest row of the lowest thread) of the unused rows; a
-// pivot below 1e-30 in modulus is replaced by 1e-15 (precond.cu:842-859).
+// column a row is the pivot of (-1: none yet).  The pivot is the largest |a|^2
+// (ties: the lowest row) of the unused rows; a pivot below 1e-30 in modulus is
+// replaced by 1e-15 (precond.cu:842-859).
 // At the end the pivot rows' entries in the outer panel's 64 columns (from k0)
 // go to Bin (16 x 64 per plane and block).
 template <int RPT>
@@ -176,7 +201,7 @@ __global__ __launch_bounds__(BJ_T) void k_bj_panel(BjView v, int ld, int c0, int
                                                    double* __restrict__ Ai, int* __restrict__ step,
                                                    int* __restrict__ prow, double* __restrict__ Bin) {
     constexpr int NW = BJ_T / 64, R = RPT > 0 ? RPT : 1;
-    __shared__ unsigned long long kb[NW];
+    __shared__ BjCand kb[NW];  // the waves' candidates
     __shared__ double row_r[BJ_W], row_i[BJ_W];
     __shared__ int prows[BJ_W];
     __shared__ BjStage stage[RPT > 0 ? NW : 1];
@@ -204,35 +229,34 @@ __global__ __launch_bounds__(BJ_T) void k_bj_panel(BjView v, int ld, int c0, int
 #pragma unroll
         for (int j = 0; j < BJ_S; j++) {
             if (s + j < w) {  // the same for the whole workgroup; a break would keep the loop from unrolling
-                unsigned key = 0;
+                double big = -1.0;
                 int best = 0x7fffffff;
                 if constexpr (RPT > 0) {
 #pragma unroll
                     for (int q = 0; q < R; q++) {
-                        const unsigned k = used[q] < 0 ? bj_key(xr[q][j], xi[q][j]) : 0u;
-                        if (k > key) {
-                            key = k;
+                        const double m = used[q] < 0 ? bj_mag(xr[q][j], xi[q][j]) : -1.0;
+                        if (m > big) {
+                            big = m;
                             best = t + BJ_T * q;
                         }
                     }
                 } else {
                     for (int i = t; i < n2; i += BJ_T) {
-                        const unsigned k =
-                            st[i] < 0 ? bj_key(ar[(long)i * ld + s + j], ai[(long)i * ld + s + j]) : 0u;
-                        if (k > key) {
-                            key = k;
+                        const double m = st[i] < 0 ? bj_mag(ar[(long)i * ld + s + j], ai[(long)i * ld + s + j]) : -1.0;
+                        if (m > big) {
+                            big = m;
                             best = i;
                         }
                     }
                 }
-                const unsigned wk = __ockl_wfred_max_u32(key);
-                const int lane = __ffsll((long long)__ballot(key == wk)) - 1;
-                if ((t & 63) == lane) kb[wave] = ((unsigned long long)wk << 32) | (0xffffffffu - (unsigned)best);
+                const unsigned long long u = (unsigned long long)__double_as_longlong(big);
+                const BjCand mine{big >= 0.0 ? (unsigned)(u >> 32) + 1u : 0u, (unsigned)u, (unsigned)best};
+                if ((t & 63) == bj_best_lane<false>(mine)) kb[wave] = mine;
                 __syncthreads();
-                unsigned long long kbest = kb[0];
-#pragma unroll
-                for (int q = 1; q < NW; q++) kbest = max(kbest, kb[q]);
-                const int p = (int)(0xffffffffu - (unsigned)kbest);  // some row is unused: n2 pivots over n2 steps
+                const BjCand all = kb[t & (NW - 1)];
+                static_assert(NW == 8, "a wave's first eight lanes hold every wave's candidate");
+                // some row is unused: n2 pivots over n2 steps
+                const int p = __builtin_amdgcn_readlane((int)all.row, bj_best_lane<true>(all));
                 if (p % BJ_T == t) {
                     if constexpr (RPT > 0) {
 #pragma unroll
