@@ -53,14 +53,15 @@ def test_matrix(bem, how):
     assert st["converged"] == 0 and not st["residual"] <= 1e-10, st
 
 
-def test_squares_beyond_the_range(bem):
-    print("right-hand sides of 1e200 and 1, FP64", flush=True)
+@pytest.mark.parametrize("middle", [1.0, 2.0**600])
+def test_squares_beyond_the_range(bem, middle):
+    print(f"right-hand sides of 1e198, {middle:.0e} and 1e198, FP64", flush=True)
     Z, B = _system(3)
     with bem.Context(0) as ctx:
         ctx.set_Z(Z)
         assert ctx.factor("fp64") == 0
         ref, _ = ctx.solve(B, ir_tol=1e-13, ir_max=5)
-        s = np.array([2.0**660, 1.0, 2.0**660])
+        s = np.array([2.0**660, middle, 2.0**660])
         X, st = ctx.solve(B * s, ir_tol=1e-13, ir_max=5)
     # powers of two: the same solutions, bit for bit
     assert st["converged"] == 1 and 0.0 < st["residual"] <= 1e-13

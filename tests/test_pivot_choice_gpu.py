@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 
 def _shared_out(n, gap, seed):
-    """Column j < 32 has the values 1 - gap * rank, turned by multiples of 90
+    """Column j < 32 has the values 1.5 + gap * (8 - rank), turned by multiples of 90
     degrees, in the rows r = j mod 32; the other columns are random."""
     rs = np.random.RandomState(seed)
     Z = rs.randn(n, n) + 1j * rs.randn(n, n)
@@ -18,7 +18,7 @@ def _shared_out(n, gap, seed):
     for j in range(32):
         rows = np.arange(j, n, 32)
         rank = rs.permutation(len(rows))
-        Z[rows, j] = (1 - gap * rank) * 1j ** rs.randint(4, size=len(rows))
+        Z[rows, j] = (1.5 + gap * (8 - rank)) * 1j ** rs.randint(4, size=len(rows))
         want.append(rows[rank == 0][0])
     return Z, np.array(want)
 
