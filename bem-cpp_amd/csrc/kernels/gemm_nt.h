@@ -220,15 +220,6 @@ typedef NtCfg<64, 64, 32, 32, 16, 2> NtCfg1;
 typedef NtCfg<128, 64, 64, 32, 16, 1> NtCfg2;
 typedef NtCfg<64, 64, 32, 32, 32, 2> NtCfg3;
 
-// Whether configuration cfg takes the product (shape and alignment).
-inline bool cupdate_nt_fits(int cfg, int M, int N, int K, const float* Ar, const float* Ai, long lda,
-                            const float* Btr, const float* Bti, long ldb, const float* Cr, const float* Ci, long ldc) {
-    const int bm = cfg == 2 ? 128 : 64, bn = 64, bk = cfg == 3 ? 32 : 16;
-    auto al = [](const float* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-    return M > 0 && N > 0 && M % bm == 0 && N % bn == 0 && K % bk == 0 && lda % 4 == 0 && ldb % 4 == 0 &&
-           ldc % 4 == 0 && al(Ar) && al(Ai) && al(Btr) && al(Bti) && al(Cr) && al(Ci);
-}
-
 template <class C>
 inline void cupdate_nt_cfg(hipStream_t s, int M, int N, int K, const float* Ar, const float* Ai, long lda,
                            const float* Btr, const float* Bti, long ldb, float* Cr, float* Ci, long ldc, long cap) {
@@ -239,8 +230,8 @@ inline void cupdate_nt_cfg(hipStream_t s, int M, int N, int K, const float* Ar, 
                        Cr, Ci, ldc);
 }
 
-// C -= A Bt^T with configuration cfg (cupdate_nt_fits must hold); cap > 0
-// limits the grid (rounded to a multiple of 8 blocks) and the blocks loop.
+// C -= A Bt^T with configuration cfg: M a multiple of 128, N of 64, K of 32, rows of 16-byte
+// pieces; cap > 0 limits the grid (rounded to a multiple of 8 blocks) and the blocks loop.
 inline void cupdate_nt(int cfg, hipStream_t s, int M, int N, int K, const float* Ar, const float* Ai, long lda,
                        const float* Btr, const float* Bti, long ldb, float* Cr, float* Ci, long ldc, long cap = 0) {
     switch (cfg) {

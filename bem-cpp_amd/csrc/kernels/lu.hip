@@ -1606,20 +1606,17 @@ void update_columns(bem_ctx* c, hipStream_t us, T* Ar, T* Ai, int k0, int c0, in
     int kt = kt_mark(c, KS_TRSM, us);
     hipLaunchKernelGGL(k_u12_strip<T>, dim3(nc / 16), dim3(512), 0, us, Ar, Ai, ld, k0, c0, panel_net(w, k0), utr, uti);
     kt_close(c, kt, 4.0 * (double)NB * NB * nc, (sizeof(T) == 4 ? 8.0 : 6.0) * sizeof(T) * (double)NB * nc);
-    if constexpr (sizeof(T) == 4) {
-        // FP32: the trailing update on the k-contiguous kernel, when the shape fits it
+    if constexpr (sizeof(T) == 4) {  // on the k-contiguous kernel; nr and nc are multiples of 256
         const GemmPlan& plan = c->gemm_plan[0];
-        if (cupdate_nt_fits(plan.nt, nr, nc, NB, Ar + o21, Ai + o21, ld, utr, uti, NB, Ar + o22, Ai + o22, ld)) {
-            kt = kt_mark(c, KS_UPDATE32, us);
-            cupdate_nt(plan.nt, us, nr, nc, NB, Ar + o21, Ai + o21, ld, utr, uti, NB, Ar + o22, Ai + o22, ld,
-                       headroom ? gemm_headroom_cap(plan, plan.large) : 0);
-            kt_close(c, kt, 6.0 * (double)nr * nc * NB,
-                     2.0 * sizeof(T) * ((double)nr * NB + (double)NB * nc + 2.0 * nr * nc));
-            return;
-        }
+        kt = kt_mark(c, KS_UPDATE32, us);
+        cupdate_nt(plan.nt, us, nr, nc, NB, Ar + o21, Ai + o21, ld, utr, uti, NB, Ar + o22, Ai + o22, ld,
+                   headroom ? plan.cap : 0);
+        kt_close(c, kt, 6.0 * (double)nr * nc * NB,
+                 2.0 * sizeof(T) * ((double)nr * NB + (double)NB * nc + 2.0 * nr * nc));
+    } else {
+        cgemm_ctx<T>(c, nr, nc, NB, Ar + o21, Ai + o21, ld, Ar + o12, Ai + o12, ld, Ar + o22, Ai + o22, ld, 0, us,
+                     GEMM_UPDATE | (headroom ? GEMM_HEADROOM : 0));
     }
-    cgemm_ctx<T>(c, nr, nc, NB, Ar + o21, Ai + o21, ld, Ar + o12, Ai + o12, ld, Ar + o22, Ai + o22, ld, 0, us,
-                 GEMM_UPDATE | (headroom ? GEMM_HEADROOM : 0));
 }
 
 // Blocked right-looking factorisation of the padded npad x npad matrix with

@@ -1,9 +1,11 @@
-// tune.hip -- autotuner for the GEMM tile shapes of the factorisation and the
-// solves.  The reference leaves these choices to cuSOLVER; here the LU
-// trailing updates (m x m x 256 products) and the GEMM-based triangular solves
-// and refinement residuals (n x nrhs products) run on the configurations of
-// kernels/gemm.h, and this routine times every configuration at the shapes of
-// the context's system and keeps the fastest per shape class.
+// tune.hip -- the plans of the GEMM tile shapes.  The reference leaves these
+// choices to cuSOLVER; here FP64 trailing updates (m x m x 256 products), longer
+// FP64 updates of the solves (n x nrhs x 256) and the adjoint's outer product run on
+// the configurations of kernels/gemm.h, and this routine times every configuration at
+// those shapes and keeps the fastest.  The FP32 trailing update runs on k_cupdate_nt
+// (gemm_nt.h), whose configuration whole factorisations choose (lu.hip); its plans
+// are kept here, too.  bem_autotune times and reports the FP32 tiles of gemm.h beside
+// the FP64 ones; no factorisation or solve takes them.
 //
 // Every configuration accumulates K in the same order (slices of 16, four
 // MFMA steps of 4), so the choice changes speed only, not results.
@@ -251,23 +253,25 @@ void plan_save(int device, int prec, int npad, int ldr, const GemmPlan& p) {
     if (std::rename(tmp.c_str(), path.c_str()) != 0) (void)std::remove(tmp.c_str());
 }
 
+// The plan of this process or of the plan file; prec: bytes of a real number.
+bool plan_known(bem_ctx* c, int prec, int npad, int ldr, GemmPlan& plan) {
+    const auto key = std::make_tuple(c->device, prec, npad, ldr);
+    std::lock_guard<std::mutex> lk(g_mu);
+    auto it = g_cache.find(key);
+    if (it != g_cache.end()) {
+        plan = it->second;  // carries npad
+        return true;
+    }
+    if (!plan_load(c->device, prec, npad, ldr, plan)) return false;
+    gemm_plan_occupancy(c, prec == 4);
+    g_cache[key] = plan;
+    return true;
+}
+
 template <typename T>
 int tune_precision(bem_ctx* c, int npad, int ldr, double* rates_large, double* rates_skinny) {
     GemmPlan& plan = c->gemm_plan[sizeof(T) == 4 ? 0 : 1];
-    const auto key = std::make_tuple(c->device, (int)sizeof(T), npad, ldr);
-    {
-        std::lock_guard<std::mutex> lk(g_mu);
-        auto it = g_cache.find(key);
-        if (it != g_cache.end() && !rates_large) {
-            plan = it->second;  // carries npad
-            return 0;
-        }
-        if (!rates_large && plan_load(c->device, (int)sizeof(T), npad, ldr, plan)) {
-            gemm_plan_occupancy(c, sizeof(T) == 4);
-            g_cache[key] = plan;
-            return 0;
-        }
-    }
+    if (!rates_large && plan_known(c, sizeof(T), npad, ldr, plan)) return 0;
     // trailing update (capped so the timing stays short) and GEMM-solve shapes
     const Shape large{std::min(npad, 8192), std::min(npad, 8192), 256};
     const Shape skinny{npad, ldr, 256};
@@ -301,7 +305,7 @@ int tune_precision(bem_ctx* c, int npad, int ldr, double* rates_large, double* r
             rates_skinny[i] = rs[i];
         }
     std::lock_guard<std::mutex> lk(g_mu);
-    g_cache[key] = plan;
+    g_cache[std::make_tuple(c->device, (int)sizeof(T), npad, ldr)] = plan;
     plan_save(c->device, (int)sizeof(T), npad, ldr, plan);
     return 0;
 }
@@ -362,8 +366,10 @@ int gemm_set_plan(bem_ctx* c, int prec, int large, int skinny, long cap) {
     return 0;
 }
 
-// Tunes the precision about to be factored once per (device, size) unless the
-// environment sets BEM_AUTOTUNE=0 (then the defaults of GemmPlan stay).
+// The plan of the precision about to be factored, once per (device, size): FP64 times its
+// tiles; FP32 has none to time (its factorisation and solves run on k_cupdate_nt, chosen by
+// whole factorisations, and on k_cmul) and takes a known plan or the default.  The
+// environment can set BEM_AUTOTUNE=0: then the defaults of GemmPlan stay and no trials run.
 int gemm_ensure_tuned(bem_ctx* c, bool f32) {
     GemmPlan& plan = c->gemm_plan[f32 ? 0 : 1];
     if (plan.tuned && plan.npad == c->npad) return 0;
@@ -376,8 +382,13 @@ int gemm_ensure_tuned(bem_ctx* c, bool f32) {
         return 0;
     }
     const int ldr = round_up(std::max(c->ldr > 0 ? c->ldr : 128, 1), 16);
-    return f32 ? tune_precision<float>(c, c->npad, ldr, nullptr, nullptr)
-               : tune_precision<double>(c, c->npad, ldr, nullptr, nullptr);
+    if (!f32) return tune_precision<double>(c, c->npad, ldr, nullptr, nullptr);
+    if (plan_known(c, 4, c->npad, ldr, plan)) return 0;
+    plan = GemmPlan(0, 2);
+    gemm_plan_occupancy(c, true);
+    plan.tuned = true;
+    plan.npad = c->npad;
+    return 0;
 }
 
 namespace {

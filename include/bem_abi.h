@@ -86,11 +86,11 @@ int bem_timings(const bem_ctx* ctx, double* out, int n);
  * 13 LU trailing-update GEMM FP64.  Returns the number of classes. */
 int bem_kernel_stats(bem_ctx* ctx, int mode, double* out, int n);
 
-/* Times the GEMM tile configurations of the factorisation and the solves at
- * the current system size with nrhs right-hand sides and keeps the fastest
- * (no counterpart in the reference, which leaves tiling to cuSOLVER; the
- * factorisation also tunes itself on its first call for a size unless
- * BEM_AUTOTUNE=0).  out (nullable, nout doubles) receives the measured TFLOP/s: FP32
+/* Times the GEMM tile configurations at the current system size with nrhs
+ * right-hand sides and keeps the fastest (no counterpart in the reference, which
+ * leaves tiling to cuSOLVER).  FP64 factorisations and solves take them, and time
+ * them on the first factorisation of a size unless BEM_AUTOTUNE=0; the FP32 ones
+ * are for comparison only, FP32 runs on kernels of its own (bem_gemm_plan_get).  out (nullable, nout doubles) receives the measured TFLOP/s: FP32
  * trailing-update shape per configuration, FP32 solve shape, FP64
  * trailing-update shape, FP64 solve shape (5 configurations each), then the
  * chosen (large, skinny) configuration per precision.  Returns the number of
@@ -99,7 +99,7 @@ int bem_autotune(bem_ctx* ctx, int nrhs, double* out, int nout);
 
 /* Fixes the GEMM plan of one precision (prec 0 FP32, 1 FP64) instead of the
  * autotuner's: configuration `large` for products with enough tiles to fill
- * the device, `skinny` for the others; cap > 0 runs the trailing updates that
+ * the device, `skinny` for the others (FP64; FP32 has no product on them); cap > 0 runs the trailing updates that
  * overlap the panel factorisation on a persistent grid of cap blocks (0: one
  * block per tile).  No counterpart in the reference; for experiments and
  * tests.  Requires a system size; returns 0 or < 0. */
