@@ -220,10 +220,10 @@ int ctx_scratch(bem_ctx* c, size_t bytes, void** out);
 // Small transfers between the caller's memory and the device on the context stream,
 // through page-locked staging: from pageable memory every copy waits for the device
 // (15-20 us each; an iteration of GMRES had six: 38 iterations at n = 4608 took 13.5 ms
-// and take 10.4, the pipeline at 2N = 240 0.93 and 0.82).  Larger ones take the
-// pageable path.  ctx_put may return before the copy has run, src is free again then
-// up to kPinBytes / 2 and otherwise once the stream is synchronised; ctx_fetch
-// synchronises the stream and fills every dst.
+// and take 10.4, the pipeline at 2N = 240 0.93 and 0.82).  Larger ones, and all where
+// no page-locked memory is to be had, take the pageable path.  ctx_put may return before
+// the copy has run, but src is free again; ctx_fetch synchronises the stream and fills
+// every dst.
 constexpr size_t kPinBytes = (size_t)1 << 20;
 struct Fetch {
     void* dst;

@@ -1887,7 +1887,6 @@ int factor_trials(bem_ctx* c, T* Ar, T* Ai, void*& inv, size_t& inv_bytes, bool*
 
 int lu_factor_launch(bem_ctx* c, int precision) {
     const int n = c->npad;
-    hipStream_t s = c->stream;
     int rc = gemm_ensure_tuned(c, precision != BEM_F64);
     if (rc) return rc;
     if ((rc = lu_setup_streams(c))) return rc;
@@ -1924,6 +1923,5 @@ int lu_factor_launch(bem_ctx* c, int precision) {
     for (int i = 0; i < n; i++)
         if (ip[i] != i) std::swap(perm[i], perm[ip[i]]);
     if (int e = ctx_put(c, c->perm, perm.data(), n * sizeof(int))) return e;
-    if (n * sizeof(int) > kPinBytes / 2) BEM_HIP(c, hipStreamSynchronize(s));
     return info[0] > c->n ? 0 : info[0];  // a zero pivot inside the identity padding cannot occur
 }
