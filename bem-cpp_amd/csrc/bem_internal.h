@@ -103,10 +103,7 @@ struct GemmPlan {
     long fill = 512;
     bool tuned = false;
     int npad = 0;                            // system size the plan was tuned for
-    int cus = 256;                           // compute units of the device
-    int occ[kMaxCfgs] = {1, 1, 1, 1, 1};     // resident blocks per CU of each configuration
-    bool occ_known = false;                  // cus and occ queried from the device
-    long cap = 0;                            // grid of capped launches; 0: from occ and cus
+    long cap = 0;                            // grid of the trailing updates beside a panel; 0: one block per tile
     bool trialed = false;                    // trailing-update tile chosen by whole trial factorisations
     double trial_ms[kMaxCfgs] = {};          // their times per configuration (0: not run): FP32 over `nt`,
                                              //   FP64 over `large`
@@ -129,6 +126,7 @@ struct BlockJacobi {
 
 struct bem_ctx {
     int device = 0;
+    int cus = 256;  // its compute units
     GemmPlan gemm_plan[2] = {GemmPlan(0, 2), GemmPlan(1, 2)};  // [0] FP32 3M, [1] FP64 (defaults before tuning)
     KernelTimer kt;
     hipStream_t stream = nullptr;
@@ -295,14 +293,12 @@ int adjoint_launch(bem_ctx* c, const double* dL_dM, double* grad);
 int gemm_autotune_launch(bem_ctx* c, int npad, int nrhs, double* out, int nout);
 int gemm_ensure_tuned(bem_ctx* c, bool f32);
 // Sets the plan of one precision (0 FP32, 1 FP64) to the given configurations
-// and grid cap of the capped trailing updates (0: one block short of full
-// occupancy per CU), replacing the autotuner's choice.
+// and grid cap of the trailing updates beside a panel (0: none), replacing the
+// autotuner's choice.
 int gemm_set_plan(bem_ctx* c, int prec, int large, int skinny, long cap);
 // Stores the context's plan of one precision in the per-process cache of
 // tuned plans (after the factorisation trials changed it).
 void gemm_cache_store(bem_ctx* c, bool f32);
-// Fills cus and occ of the plan of one precision from the device (no timing).
-void gemm_plan_occupancy(bem_ctx* c, bool f32);
 // Chooses the factorisation stream layout (environment BEM_LU_STREAMS) and, once
 // a system is large enough to gain, a panel stream that runs beside the context
 // stream.

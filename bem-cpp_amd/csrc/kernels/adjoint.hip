@@ -249,7 +249,7 @@ int adjoint_launch(bem_ctx* c, const double* dL_dM, double* grad) {
     // 3. W = Lambda X^T (npad x npad, K = ldr, a multiple of 16)
     hipLaunchKernelGGL(k_transpose, dim3((ldr + 31) / 32, (npad + 31) / 32), dim3(256), 0, s, npad, ldr, Xsr, Xsi,
                        (long)ldr, XTr, XTi, (long)npad);
-    cgemm_ctx<double>(c, npad, npad, ldr, Lr, Li, ldr, XTr, XTi, npad, Wr, Wi, npad, 1);
+    cgemm_ctx(c, npad, npad, ldr, Lr, Li, ldr, XTr, XTi, npad, Wr, Wi, npad, 1);
 
     // 4. RHS term: sum lambda . dB/dka
     if (int e = rhs_dk_launch(c, dBr, dBi)) return e;

@@ -310,8 +310,7 @@ __device__ __forceinline__ bool touching(const int4& a, const int4& b) {
 // ---------------------------------------------------------------------------
 // MODE 0: forward records; 1: RecCoef records of the moments of G, g;
 // 2: RecCoef records of the moments of dG/dk = iR G and dg/dk = -k G.
-// Bound by VALU issue, most of it FP64 (8 cycles an instruction and wave here): some
-// 70 FP64 and 80 FP32 instructions per point pair and, per triangle pair, 9 records.
+// Bound by VALU issue, most of it FP64: some 70 FP64 and 80 FP32 instructions per point pair and, per triangle pair, 9 records.
 // The source functions w, w r come ready from LDS, the folds are plain FMAs, and the loop
 // over j stays rolled, so that two waves fit a SIMD: unrolled (290 registers, one
 // wave) it took 731 us at 2N = 4608 and 9.5 ms at 18432, now 466 us and 6.5 ms; three

@@ -1,10 +1,7 @@
 // gemm.h -- complex GEMM on CDNA4 matrix cores, planar operands.
 //
-//   C = C - A B   (mode 0)     C = A B   (mode 1)     C = C + A B   (mode 2)
-//   C = -A B      (mode 3)
+//   C = C - A B   (mode 0)     C = A B   (mode 1)
 //
-// A batch of independent products of one shape runs in one launch
-// (blockIdx.z), operand z at the base pointers plus z times the batch strides.
 // A is M x K, B is K x N, C is M x N; every matrix is stored as two planes
 // (real, imaginary) in row-major order with its own leading dimension.
 //
@@ -44,7 +41,8 @@ __device__ __forceinline__ v4d mfma16x16x4(double a, double b, v4d c) {
 // register allocation must allow (two per CU let one block's prologue and C
 // update overlap another's MFMA stream).  Which configuration a launch uses
 // is decided by the context's plan (gemm_plan in bem_ctx), set by the
-// autotuner from measured times at the context's shapes.
+// autotuner from measured times at the context's shapes.  FP64 products run
+// here; the FP32 tiles are for the autotuner's report only.
 template <typename T, int CFG>
 struct GemmCfg;
 template <>
@@ -106,8 +104,7 @@ struct GemmCfg<double, 3> {
     static constexpr int VEC = 2;
 };
 // 32 x 32 (one 16 x 16 MFMA tile per wave): products too small to give the
-// device one block per CU with the other tiles (the block-inverse products
-// and the late updates of the solves, the L11^{-1} doubling).
+// device one block per CU with the other tiles.
 template <>
 struct GemmCfg<float, 4> {
     static constexpr int BM = 32, BN = 32, BK = 16, WM = 16, WN = 16, PAD = 16, MINB = 4;
@@ -143,8 +140,7 @@ template <typename T, int CFG, int ROLE = 0>
 __global__ __launch_bounds__(256, (GemmCfg<T, CFG>::MINB)) void k_cgemm(int M, int N, int K, const T* __restrict__ Ar,
                                                const T* __restrict__ Ai, long lda, const T* __restrict__ Br,
                                                const T* __restrict__ Bi, long ldb, T* __restrict__ Cr,
-                                               T* __restrict__ Ci, long ldc, int mode, int nz, long sa, long sb,
-                                               long sc) {
+                                               T* __restrict__ Ci, long ldc, int mode) {
     typedef GemmCfg<T, CFG> C;
     constexpr int BM = C::BM, BN = C::BN, BK = C::BK, WM = C::WM, WN = C::WN, VEC = C::VEC;
     constexpr int TM = WM / 16, TN = WN / 16;
@@ -159,22 +155,16 @@ __global__ __launch_bounds__(256, (GemmCfg<T, CFG>::MINB)) void k_cgemm(int M, i
     __shared__ T sA[2][2][BK][SA];
     __shared__ T sB[2][2][BK][SB];
 
-    mode &= 3;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm0 = (wave >> 1) * WM, wn0 = (wave & 1) * WN;
     const int ntx = (N + BN - 1) / BN, nty = (M + BM - 1) / BM;
-    const int ntiles = ntx * nty * nz;
+    const int ntiles = ntx * nty;
     const int nk = K / BK;
 
-    // Tiles in row-major order over (z, row, column); a grid smaller than the
-    // tile count makes every block loop (persistent launch).
+    // Tiles in row-major order; a grid smaller than the tile count makes every
+    // block loop (persistent launch).
     for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int bz = tile / (ntx * nty), rem = tile - bz * (ntx * nty);
-        const int row0 = (rem / ntx) * BM, col0 = (rem % ntx) * BN;
-        const T* __restrict__ ar_ = Ar + bz * sa;
-        const T* __restrict__ ai_ = Ai + bz * sa;
-        const T* __restrict__ br_ = Br + bz * sb;
-        const T* __restrict__ bi_ = Bi + bz * sb;
+        const int row0 = (tile / ntx) * BM, col0 = (tile % ntx) * BN;
 
         vec_t ga[2][AV], gb[2][BV];
         auto load = [&](int k0) {
@@ -184,8 +174,8 @@ __global__ __launch_bounds__(256, (GemmCfg<T, CFG>::MINB)) void k_cgemm(int M, i
                 const int r = v / (BK / VEC), kv = (v % (BK / VEC)) * VEC;
                 const bool ok = (AVT % 256 == 0 || v < AVT) && row0 + r < M;
                 const long o = (long)(row0 + r) * lda + k0 + kv;
-                ga[0][u] = ok ? *reinterpret_cast<const vec_t*>(ar_ + o) : vec_t{};
-                ga[1][u] = ok ? *reinterpret_cast<const vec_t*>(ai_ + o) : vec_t{};
+                ga[0][u] = ok ? *reinterpret_cast<const vec_t*>(Ar + o) : vec_t{};
+                ga[1][u] = ok ? *reinterpret_cast<const vec_t*>(Ai + o) : vec_t{};
             }
 #pragma unroll
             for (int u = 0; u < BV; u++) {
@@ -193,8 +183,8 @@ __global__ __launch_bounds__(256, (GemmCfg<T, CFG>::MINB)) void k_cgemm(int M, i
                 const int kr = v / (BN / VEC), nv = (v % (BN / VEC)) * VEC;
                 const bool ok = (BVT % 256 == 0 || v < BVT) && col0 + nv < N;
                 const long o = (long)(k0 + kr) * ldb + col0 + nv;
-                gb[0][u] = ok ? *reinterpret_cast<const vec_t*>(br_ + o) : vec_t{};
-                gb[1][u] = ok ? *reinterpret_cast<const vec_t*>(bi_ + o) : vec_t{};
+                gb[0][u] = ok ? *reinterpret_cast<const vec_t*>(Br + o) : vec_t{};
+                gb[1][u] = ok ? *reinterpret_cast<const vec_t*>(Bi + o) : vec_t{};
             }
         };
         auto store = [&](int buf) {
@@ -279,8 +269,6 @@ __global__ __launch_bounds__(256, (GemmCfg<T, CFG>::MINB)) void k_cgemm(int M, i
             __syncthreads();  // also ends the reads of this tile before the next tile's first store
         }
 
-        T* __restrict__ cr_ = Cr + bz * sc;
-        T* __restrict__ ci_ = Ci + bz * sc;
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -300,17 +288,11 @@ __global__ __launch_bounds__(256, (GemmCfg<T, CFG>::MINB)) void k_cgemm(int M, i
                     }
                     const long o = (long)row * ldc + col;
                     if (mode == 0) {
-                        cr_[o] -= vr;
-                        ci_[o] -= vi;
-                    } else if (mode == 1) {
-                        cr_[o] = vr;
-                        ci_[o] = vi;
-                    } else if (mode == 3) {
-                        cr_[o] = -vr;
-                        ci_[o] = -vi;
+                        Cr[o] -= vr;
+                        Ci[o] -= vi;
                     } else {
-                        cr_[o] += vr;
-                        ci_[o] += vi;
+                        Cr[o] = vr;
+                        Ci[o] = vi;
                     }
                 }
             }
@@ -319,66 +301,31 @@ __global__ __launch_bounds__(256, (GemmCfg<T, CFG>::MINB)) void k_cgemm(int M, i
 
 // Host launcher of configuration cfg.  K must be a multiple of BK; N a
 // multiple of the vector width (4 floats / 2 doubles) and every leading
-// dimension a multiple of it.  nb products with batch strides sa, sb, sc.
-// cap > 0 limits the grid to cap blocks, which then loop over the tiles.
+// dimension a multiple of it.  cap > 0 limits the grid to cap blocks, which
+// then loop over the tiles.
 template <typename T, int CFG>
 inline void cgemm_cfg(hipStream_t s, int M, int N, int K, const T* Ar, const T* Ai, long lda, const T* Br,
-                      const T* Bi, long ldb, T* Cr, T* Ci, long ldc, int mode, int nb, long sa, long sb, long sc,
-                      long cap, int role) {
+                      const T* Bi, long ldb, T* Cr, T* Ci, long ldc, int mode, long cap, int role) {
     typedef GemmCfg<T, CFG> C;
-    const long tiles = (long)((N + C::BN - 1) / C::BN) * ((M + C::BM - 1) / C::BM) * nb;
+    const long tiles = (long)((N + C::BN - 1) / C::BN) * ((M + C::BM - 1) / C::BM);
     const long grid = cap > 0 && cap < tiles ? cap : tiles;
-    if (role == 1)
-        hipLaunchKernelGGL((k_cgemm<T, CFG, 1>), dim3((unsigned)grid), dim3(256), 0, s, M, N, K, Ar, Ai, lda, Br, Bi,
-                           ldb, Cr, Ci, ldc, mode, nb, sa, sb, sc);
-    else
-        hipLaunchKernelGGL((k_cgemm<T, CFG, 0>), dim3((unsigned)grid), dim3(256), 0, s, M, N, K, Ar, Ai, lda, Br, Bi,
-                           ldb, Cr, Ci, ldc, mode, nb, sa, sb, sc);
+    auto k = role == 1 ? k_cgemm<T, CFG, sizeof(T) == 8 ? 1 : 0> : k_cgemm<T, CFG, 0>;
+    hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(256), 0, s, M, N, K, Ar, Ai, lda, Br, Bi, ldb, Cr, Ci, ldc, mode);
 }
 
 template <typename T>
 inline void cgemm_any(int cfg, hipStream_t s, int M, int N, int K, const T* Ar, const T* Ai, long lda, const T* Br,
-                      const T* Bi, long ldb, T* Cr, T* Ci, long ldc, int mode, int nb = 1, long sa = 0, long sb = 0,
-                      long sc = 0, long cap = 0, int role = 0) {
-    if (M <= 0 || N <= 0 || K <= 0 || nb <= 0) return;
+                      const T* Bi, long ldb, T* Cr, T* Ci, long ldc, int mode, long cap = 0, int role = 0) {
+    if (M <= 0 || N <= 0 || K <= 0) return;
     switch (cfg) {
-        case 1: cgemm_cfg<T, 1>(s, M, N, K, Ar, Ai, lda, Br, Bi, ldb, Cr, Ci, ldc, mode, nb, sa, sb, sc, cap, role); break;
-        case 2: cgemm_cfg<T, 2>(s, M, N, K, Ar, Ai, lda, Br, Bi, ldb, Cr, Ci, ldc, mode, nb, sa, sb, sc, cap, role); break;
-        case 3: cgemm_cfg<T, 3>(s, M, N, K, Ar, Ai, lda, Br, Bi, ldb, Cr, Ci, ldc, mode, nb, sa, sb, sc, cap, role); break;
-        case 4: cgemm_cfg<T, 4>(s, M, N, K, Ar, Ai, lda, Br, Bi, ldb, Cr, Ci, ldc, mode, nb, sa, sb, sc, cap, role); break;
-        default: cgemm_cfg<T, 0>(s, M, N, K, Ar, Ai, lda, Br, Bi, ldb, Cr, Ci, ldc, mode, nb, sa, sb, sc, cap, role); break;
+        case 1: cgemm_cfg<T, 1>(s, M, N, K, Ar, Ai, lda, Br, Bi, ldb, Cr, Ci, ldc, mode, cap, role); break;
+        case 2: cgemm_cfg<T, 2>(s, M, N, K, Ar, Ai, lda, Br, Bi, ldb, Cr, Ci, ldc, mode, cap, role); break;
+        case 3: cgemm_cfg<T, 3>(s, M, N, K, Ar, Ai, lda, Br, Bi, ldb, Cr, Ci, ldc, mode, cap, role); break;
+        case 4: cgemm_cfg<T, 4>(s, M, N, K, Ar, Ai, lda, Br, Bi, ldb, Cr, Ci, ldc, mode, cap, role); break;
+        default: cgemm_cfg<T, 0>(s, M, N, K, Ar, Ai, lda, Br, Bi, ldb, Cr, Ci, ldc, mode, cap, role); break;
     }
 }
-
-// Blocks of configuration cfg that fit on one CU (registers, LDS, waves).
-template <typename T, int CFG>
-inline int cgemm_occ_cfg() {
-    int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, reinterpret_cast<const void*>(k_cgemm<T, CFG>), 256, 0) !=
-        hipSuccess)
-        return 1;
-    return nb > 0 ? nb : 1;
-}
-template <typename T>
-inline int cgemm_occupancy(int cfg) {
-    switch (cfg) {
-        case 1: return cgemm_occ_cfg<T, 1>();
-        case 2: return cgemm_occ_cfg<T, 2>();
-        case 3: return cgemm_occ_cfg<T, 3>();
-        case 4: return cgemm_occ_cfg<T, 4>();
-        default: return cgemm_occ_cfg<T, 0>();
-    }
-}
-static_assert(kGemmCfgs <= GemmPlan::kMaxCfgs, "GemmPlan holds one occupancy per configuration");
-
-// Grid cap that leaves one block of the configuration free on every CU: a
-// trailing update launched this way never takes all of a CU's LDS, so the
-// panel kernels running beside it on the other stream find room at once.
-inline long gemm_headroom_cap(const GemmPlan& p, int cfg) {
-    if (p.cap > 0) return p.cap;
-    const int per_cu = p.occ[cfg] > 1 ? p.occ[cfg] - 1 : 1;
-    return (long)p.cus * per_cu;
-}
+static_assert(kGemmCfgs <= GemmPlan::kMaxCfgs, "GemmPlan holds one trial time per configuration");
 
 // Blocks of configuration cfg for an M x N product.
 template <typename T>
@@ -397,36 +344,26 @@ inline long gemm_blocks(int cfg, int M, int N) {
 // The plan's configuration for an M x N product: the large-product tile when
 // it still gives at least `fill` blocks, else the skinny-product tile while
 // that gives one block per CU, else the 32 x 32 tile.
-template <typename T>
 inline int gemm_choose(const bem_ctx* c, int M, int N) {
-    const GemmPlan& p = c->gemm_plan[sizeof(T) == 4 ? 0 : 1];
-    if (gemm_blocks<T>(p.large, M, N) >= p.fill) return p.large;
-    return gemm_blocks<T>(p.skinny, M, N) >= p.cus ? p.skinny : kGemmSmall;
+    const GemmPlan& p = c->gemm_plan[1];
+    if (gemm_blocks<double>(p.large, M, N) >= p.fill) return p.large;
+    return gemm_blocks<double>(p.skinny, M, N) >= c->cus ? p.skinny : kGemmSmall;
 }
 
-// Launch flags of cgemm_ctx: GEMM_HEADROOM caps the grid as
-// gemm_headroom_cap does (an update running beside the panel stream);
-// GEMM_UPDATE: an LU trailing update (its own kernel symbol and timing class).
-constexpr int GEMM_HEADROOM = 1, GEMM_UPDATE = 4;
-
-// GEMM with optional per-launch timing, on stream s (default: the context
-// stream), tile configuration from the context's plan.  Counted work: 3M
-// form 6 M N K real flops (FP32), 4M form 8 M N K (FP64); bytes = operands
-// read once plus C read and written.
-template <typename T>
-inline void cgemm_ctx(bem_ctx* c, int M, int N, int K, const T* Ar, const T* Ai, long lda, const T* Br, const T* Bi,
-                      long ldb, T* Cr, T* Ci, long ldc, int mode, hipStream_t s = nullptr, int flags = 0) {
+// FP64 GEMM with optional per-launch timing, on stream s (default: the context
+// stream), tile configuration from the context's plan; update: an LU trailing
+// update (its own kernel symbol and timing class); cap as in cgemm_cfg.
+// Counted work: 8 M N K real flops; bytes = operands read once plus C read and
+// written.
+inline void cgemm_ctx(bem_ctx* c, int M, int N, int K, const double* Ar, const double* Ai, long lda, const double* Br,
+                      const double* Bi, long ldb, double* Cr, double* Ci, long ldc, int mode, hipStream_t s = nullptr,
+                      bool update = false, long cap = 0) {
     if (M <= 0 || N <= 0 || K <= 0) return;
     if (!s) s = c->stream;
-    const bool upd = flags & GEMM_UPDATE;
-    const int k = kt_mark(c, sizeof(T) == 4 ? (upd ? KS_UPDATE32 : KS_GEMM32) : (upd ? KS_UPDATE64 : KS_GEMM64), s);
-    const GemmPlan& plan = c->gemm_plan[sizeof(T) == 4 ? 0 : 1];
-    const int cfg = gemm_choose<T>(c, M, N);
-    const long cap = (flags & GEMM_HEADROOM) ? gemm_headroom_cap(plan, cfg) : 0;
-    cgemm_any<T>(cfg, s, M, N, K, Ar, Ai, lda, Br, Bi, ldb, Cr, Ci, ldc, mode, 1, 0, 0, 0, cap, upd ? 1 : 0);
-    const double mnk = (double)M * N * K;
-    const double bytes = 2.0 * sizeof(T) * ((double)M * K + (double)K * N + (mode == 1 ? 1.0 : 2.0) * M * N);
-    kt_close(c, k, (sizeof(T) == 4 ? 6.0 : 8.0) * mnk, bytes);
+    const int k = kt_mark(c, update ? KS_UPDATE64 : KS_GEMM64, s);
+    cgemm_any<double>(gemm_choose(c, M, N), s, M, N, K, Ar, Ai, lda, Br, Bi, ldb, Cr, Ci, ldc, mode, cap, update ? 1 : 0);
+    kt_close(c, k, 8.0 * M * N * (double)K,
+             16.0 * ((double)M * K + (double)K * N + (mode == 1 ? 1.0 : 2.0) * M * N));
 }
 
 // Four consecutive values of a row, by 16-byte loads.

@@ -1503,7 +1503,7 @@ struct LuWork {
     int* cnt;        // tournament arrival counters
     int* cid;        // candidate row ids
     T *cvr, *cvi;    // candidate values
-    int* pl;         // row-pair lists of the 8 steps of an outer panel (PLS ints each), two sets
+    int* pl;         // row-pair lists of the 8 steps of an outer panel (PLS ints each)
     T* d11;          // factored 32 x 32 diagonal block (2 planes), two sets by step parity
     T *cpr, *cpi;    // compact copies (n x 32 per plane) of the columns being factored, two sets by step parity
     T *sur, *sui;    // U12 of the next 32 columns (32 x 32)
@@ -1590,10 +1590,11 @@ void factor_panel(bem_ctx* c, hipStream_t s, T* Ar, T* Ai, int k0, const LuWork<
 }
 
 // The swaps of outer panel k0, U12 = L11^{-1} A12 and A22 -= L21 U12 for the
-// columns [c0, c0 + nc) right of the panel, on stream us.
+// columns [c0, c0 + nc) right of the panel, on stream us; cap > 0: the update on that many
+// workgroups.
 template <typename T>
 void update_columns(bem_ctx* c, hipStream_t us, T* Ar, T* Ai, int k0, int c0, int nc, const LuWork<T>& w,
-                    bool headroom) {
+                    long cap) {
     const int n = c->npad;
     const long ld = n;
     const int nr = n - (k0 + NB);
@@ -1610,12 +1611,12 @@ void update_columns(bem_ctx* c, hipStream_t us, T* Ar, T* Ai, int k0, int c0, in
         const GemmPlan& plan = c->gemm_plan[0];
         kt = kt_mark(c, KS_UPDATE32, us);
         cupdate_nt(plan.nt, us, nr, nc, NB, Ar + o21, Ai + o21, ld, utr, uti, NB, Ar + o22, Ai + o22, ld,
-                   headroom ? plan.cap : 0);
+                   cap);
         kt_close(c, kt, 6.0 * (double)nr * nc * NB,
                  2.0 * sizeof(T) * ((double)nr * NB + (double)NB * nc + 2.0 * nr * nc));
     } else {
-        cgemm_ctx<T>(c, nr, nc, NB, Ar + o21, Ai + o21, ld, Ar + o12, Ai + o12, ld, Ar + o22, Ai + o22, ld, 0, us,
-                     GEMM_UPDATE | (headroom ? GEMM_HEADROOM : 0));
+        cgemm_ctx(c, nr, nc, NB, Ar + o21, Ai + o21, ld, Ar + o12, Ai + o12, ld, Ar + o22, Ai + o22, ld, 0, us, true,
+                  cap);
     }
 }
 
@@ -1658,7 +1659,7 @@ void factor(bem_ctx* c, T* Ar, T* Ai, T* Lir, T* Lii, T* Uir, T* Uii, const LuWo
         // columns of panel K+1 first, on the panel stream, once the update of panel K-1
         // has left them
         if (K > 0) (void)hipStreamWaitEvent(ps, e_rest, 0);
-        update_columns<T>(c, ps, Ar, Ai, k0, k0 + NB, NB, w, false);
+        update_columns<T>(c, ps, Ar, Ai, k0, k0 + NB, NB, w, 0);
         (void)hipEventRecord(e_next, ps);
         (void)hipStreamWaitEvent(us, e_next, 0);
         // the rest of the update is enqueued before panel K+1's launches, so a
@@ -1666,7 +1667,8 @@ void factor(bem_ctx* c, T* Ar, T* Ai, T* Lir, T* Lii, T* Uir, T* Uii, const LuWo
         // update stream back
         swap_left(k0);
         if (nr > NB)
-            update_columns<T>(c, us, Ar, Ai, k0, k0 + 2 * NB, nr - NB, w, ps != us && c->gemm_plan[sizeof(T) == 4 ? 0 : 1].cap > 0);
+            update_columns<T>(c, us, Ar, Ai, k0, k0 + 2 * NB, nr - NB, w,
+                              ps != us ? c->gemm_plan[sizeof(T) == 4 ? 0 : 1].cap : 0);
         (void)hipEventRecord(e_rest, us);
         factor_panel<T>(c, ps, Ar, Ai, k0 + NB, w, wide);
     }

@@ -122,7 +122,8 @@ __device__ __forceinline__ int bj_best_lane(const BjCand& k) {
 
 // Columns of unrolled elimination steps; the registers rotate by so many after them.
 // (All 16 steps unrolled, each row read ahead whole and with two selects per value
-// for the pivot row, spilled: 98 us per panel of 1107 rows, 45 now.)
+// for the pivot row, took 98 us per panel of 1107 rows, 45 now.  With three rows per
+// thread, those rows' included, the kernel takes all 256 registers and spills eight.)
 constexpr int BJ_S = 4;
 
 // Entries BJ_S .. to the front, the first BJ_S to the end.

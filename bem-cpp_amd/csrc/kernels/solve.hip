@@ -59,8 +59,7 @@ void cmul(bem_ctx* c, int M, int N, int K, int tri, const float* Ar, const float
     if (M <= 0) return;
     const int kt = kt_mark(c, KS_GEMM32, c->stream);
     const int tiles = N / 16, rows = M / 16;
-    constexpr int kCus = 256;
-    auto cost = [&](int nt, int ngrp) { return ngrp ? (2 * nt + 1) * (((long)rows * ngrp + kCus - 1) / kCus) : 0L; };
+    auto cost = [&](int nt, int ngrp) { return ngrp ? (2 * nt + 1) * (((long)rows * ngrp + c->cus - 1) / c->cus) : 0L; };
     int G = tiles;
     long least = cost(1, tiles);
     for (int g = tiles - 1; g * kCmulTiles >= tiles && g > 0; g--) {
@@ -219,7 +218,7 @@ void lu_apply64(bem_ctx* c, const double* Fr, const double* Fi, double* Yr, doub
         if (rows <= kShortRows)
             cgemm_short_ctx(c, rows, ncol, ar, ai, ld, br, bi, ncol, cr, ci, ncol);
         else
-            cgemm_ctx<double>(c, rows, ncol, NB, ar, ai, ld, br, bi, ncol, cr, ci, ncol, 0);
+            cgemm_ctx(c, rows, ncol, NB, ar, ai, ld, br, bi, ncol, cr, ci, ncol, 0);
     };
     for (int I = 0; I < nb; I++) {
         const long y = (long)I * NB * ncol, dg = (long)I * NB * (ld + 1);

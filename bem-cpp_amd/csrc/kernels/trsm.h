@@ -32,9 +32,6 @@ __device__ __forceinline__ double wave_bcast(double v, int l) {
     const int lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
-__device__ __forceinline__ float wave_bcast(float v, int l) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
 
 // Solves T X = B by substitution for one 256 x 256 triangular block T (unit
 // lower: forward; non-unit upper: backward) and the columns of B, CW columns
@@ -166,12 +163,10 @@ __global__ __launch_bounds__(256) void k_trsm_rhs(const T* __restrict__ Tr, cons
 }
 
 // T X = B for the 256 x 256 triangle at (Tr, Ti) and ncols columns (a
-// multiple of 8) on stream s.  Few columns (the solves' right-hand sides, the
-// 256 columns of the next panel): 2 columns and 16-row slabs per block, so the
-// latency-bound chain of steps is as short as it gets; many columns (the rest
-// of a panel's U12): 8 columns and 8-row slabs, where throughput counts
-// (measured on MI355X, FP64: 48 / 61 us lower / upper at 128 columns, 274 /
-// 322 us at 9216).
+// multiple of 8) on stream s.  Up to 512 right-hand sides: 2 columns and 16-row
+// slabs per block, so the latency-bound chain of steps is as short as it gets
+// (lower / upper 48 / 61 us at 128 columns); more: 8 columns and 8-row slabs, where
+// throughput counts (274 / 322 us at 9216).
 template <typename T>
 inline void trsm_rhs(hipStream_t s, bool lower, const T* Tr, const T* Ti, long ldt, const T* Br, const T* Bi,
                      long ldb, T* Xr, T* Xi, long ldx, int ncols) {

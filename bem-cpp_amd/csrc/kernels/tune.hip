@@ -45,9 +45,8 @@ struct Shape {
 };
 
 // Best configuration and its rate (TFLOP/s) for one shape; rates[cfg] filled.
-// With a plan, every configuration runs under its headroom grid cap.
 template <typename T>
-int time_configs(hipStream_t s, const Shape& sh, T* buf, double* rates, const GemmPlan* capped) {
+int time_configs(hipStream_t s, const Shape& sh, T* buf, double* rates) {
     T* Ar = buf;
     T* Ai = Ar + (size_t)sh.M * sh.K;
     T* Br = Ai + (size_t)sh.M * sh.K;
@@ -64,8 +63,7 @@ int time_configs(hipStream_t s, const Shape& sh, T* buf, double* rates, const Ge
     int best = 0;
     for (int cfg = 0; cfg < kGemmCfgs; cfg++) {
         auto run = [&]() {
-            cgemm_any<T>(cfg, s, sh.M, sh.N, sh.K, Ar, Ai, sh.K, Br, Bi, sh.N, Cr, Ci, sh.N, 0, 1, 0, 0, 0,
-                         capped ? gemm_headroom_cap(*capped, cfg) : 0);
+            cgemm_any<T>(cfg, s, sh.M, sh.N, sh.K, Ar, Ai, sh.K, Br, Bi, sh.N, Cr, Ci, sh.N, 0);
         };
         run();  // warm-up (code load, caches)
         const int reps = 3;
@@ -263,7 +261,6 @@ bool plan_known(bem_ctx* c, int prec, int npad, int ldr, GemmPlan& plan) {
         return true;
     }
     if (!plan_load(c->device, prec, npad, ldr, plan)) return false;
-    gemm_plan_occupancy(c, prec == 4);
     g_cache[key] = plan;
     return true;
 }
@@ -282,10 +279,9 @@ int tune_precision(bem_ctx* c, int npad, int ldr, double* rates_large, double* r
     if (hipMalloc(&buf, elems * sizeof(T)) != hipSuccess) return bem_fail(c, BEM_ERR_NOMEM, "autotune buffers");
     hipLaunchKernelGGL(k_fill_tune<T>, dim3((unsigned)((elems + 255) / 256)), dim3(256), 0, c->stream, buf,
                        (long)elems, 7u);
-    gemm_plan_occupancy(c, sizeof(T) == 4);
     double rl[kGemmCfgs] = {0}, rs[kGemmCfgs] = {0};
-    const int bl = time_configs<T>(c->stream, large, buf, rl, nullptr);
-    const int bs = time_configs<T>(c->stream, skinny, buf, rs, nullptr);
+    const int bl = time_configs<T>(c->stream, large, buf, rl);
+    const int bs = time_configs<T>(c->stream, skinny, buf, rs);
     const hipError_t e = hipStreamSynchronize(c->stream);
     (void)hipFree(buf);
     if (e != hipSuccess || bl < 0 || bs < 0)
@@ -296,7 +292,7 @@ int tune_precision(bem_ctx* c, int npad, int ldr, double* rates_large, double* r
     plan.cap = 0;
     plan.trialed = false;  // the first factorisation of this size times whole trials
     for (double& t : plan.trial_ms) t = 0.0;
-    plan.fill = 2L * plan.cus;  // fewer blocks of the large tile than two per CU: use the skinny tile
+    plan.fill = 2L * c->cus;  // fewer blocks of the large tile than two per CU: use the skinny tile
     plan.tuned = true;
     plan.npad = npad;
     if (rates_large)
@@ -333,14 +329,6 @@ int gemm_autotune_launch(bem_ctx* c, int npad, int nrhs, double* out, int nout) 
     return 0;
 }
 
-void gemm_plan_occupancy(bem_ctx* c, bool f32) {
-    GemmPlan& plan = c->gemm_plan[f32 ? 0 : 1];
-    if (plan.occ_known) return;
-    (void)hipDeviceGetAttribute(&plan.cus, hipDeviceAttributeMultiprocessorCount, c->device);
-    for (int i = 0; i < kGemmCfgs; i++) plan.occ[i] = f32 ? cgemm_occupancy<float>(i) : cgemm_occupancy<double>(i);
-    plan.occ_known = true;
-}
-
 void gemm_cache_store(bem_ctx* c, bool f32) {
     const GemmPlan& plan = c->gemm_plan[f32 ? 0 : 1];
     const int ldr = round_up(std::max(c->ldr > 0 ? c->ldr : 128, 1), 16);
@@ -355,7 +343,6 @@ int gemm_set_plan(bem_ctx* c, int prec, int large, int skinny, long cap) {
         return bem_fail(c, BEM_ERR_ARG, "gemm_plan: bad configuration");
     if (c->npad <= 0) return bem_fail(c, BEM_ERR_STATE, "gemm_plan: no system size yet (set a mesh or a matrix)");
     GemmPlan& plan = c->gemm_plan[prec];
-    gemm_plan_occupancy(c, prec == 0);
     plan.large = large;
     plan.skinny = skinny;
     plan.cap = cap;
@@ -375,7 +362,6 @@ int gemm_ensure_tuned(bem_ctx* c, bool f32) {
     if (plan.tuned && plan.npad == c->npad) return 0;
     const char* env = std::getenv("BEM_AUTOTUNE");
     if (env && env[0] == '0') {
-        gemm_plan_occupancy(c, f32);
         plan.tuned = true;
         plan.trialed = true;
         plan.npad = c->npad;
@@ -385,7 +371,6 @@ int gemm_ensure_tuned(bem_ctx* c, bool f32) {
     if (!f32) return tune_precision<double>(c, c->npad, ldr, nullptr, nullptr);
     if (plan_known(c, 4, c->npad, ldr, plan)) return 0;
     plan = GemmPlan(0, 2);
-    gemm_plan_occupancy(c, true);
     plan.tuned = true;
     plan.npad = c->npad;
     return 0;

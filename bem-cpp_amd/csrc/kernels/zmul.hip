@@ -143,14 +143,14 @@ __global__ __launch_bounds__(256) void k_zmul_sum(long count, int S, const doubl
 constexpr int kTiles = 5;
 
 // Splits of A's columns: the fewest of 1, 2, 4, 8, 16 that load the compute units evenly
-// (95 % of the last one's blocks), else the most even.  At least 16 columns each; 32 for
-// the long step.
+// (95 % of the last one's blocks), else the most even.  A split is a multiple of 32 columns,
+// two of the long steps.
 int zmul_splits(int cus, int M, int N) {
     const int tiles = N / 16, grps = (tiles + kTiles - 1) / kTiles;
     const long rows = (long)(M / 64) * grps;
     int best = 1;
     double best_eff = 0.0;
-    for (int S = 1; S <= 16 && M / S >= 16 && M % (32 * S) == 0; S *= 2) {
+    for (int S = 1; S <= 16 && M % (32 * S) == 0; S *= 2) {
         const long blocks = rows * S;
         const double eff = (double)blocks / (double)(cus * ((blocks + cus - 1) / cus));
         if (eff > best_eff + 1e-9) {
@@ -214,9 +214,7 @@ int z_product(bem_ctx* c, int N, const double* Xr, const double* Xi, const doubl
               double* Oi) {
     const int M = c->npad;
     const long count = (long)M * N;
-    int cus = 0;
-    BEM_HIP(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
-    const int S = zmul_splits(std::max(1, cus), M, N);
+    const int S = zmul_splits(c->cus, M, N);
     const size_t bytes = 2 * (size_t)S * count * sizeof(double);
     if (c->part_bytes < bytes) {
         if (c->part) (void)hipFree(c->part);

@@ -406,7 +406,7 @@ def main():
         ach = kflops / (kms * 1e-3) / 1e12
         tile = plan32["update"] if plan32 else "?"
         roof = {"kernel": f"k_cupdate_nt (3M complex GEMM C -= A Bt^T, both operands k-contiguous, LU trailing "
-                          f"updates, {tile} tile; k_cgemm<float, cfg, 1> for the last updates below 64 rows)",
+                          f"updates, {tile} tile)",
                 "bound": "mfma",
                 "achieved": ach, "peak": PEAK_TFLOPS["gemm_fp32_3m"], "unit": "TFLOP/s",
                 "frac": ach / PEAK_TFLOPS["gemm_fp32_3m"], "traffic": measured_traffic(args.workload, dom),
