@@ -208,6 +208,7 @@ class Context:
         if not self._h:
             raise RuntimeError(f"bem_create({device}) failed: no usable GPU")
         self.N = 0
+        self._n = 0  # size of the system on the device
 
     def close(self):
         if getattr(self, "_h", None):
@@ -231,12 +232,19 @@ class Context:
             raise BemError(rc, f"{what}: {self._L.bem_last_error(self._h).decode()}")
         return rc
 
+    def _rows(self, B):
+        """Shape of a block of vectors of the system on the device."""
+        if B.ndim != 2 or (self._n and B.shape[0] != self._n):
+            raise ValueError(f"vectors of {self._n} rows are needed, not {B.shape}")
+        return B.shape
+
     # -- mesh -------------------------------------------------------------
     def set_mesh(self, verts, tris, quad_order: int = 7):
         v = _cd(verts)
         t = np.ascontiguousarray(tris, dtype=np.int32)
         self._check(self._L.bem_set_mesh(self._h, _p(v), len(v), _pi(t), len(t), quad_order), "set_mesh")
         self.N = self._L.bem_num_rwg(self._h)
+        self._n = 2 * self.N
         return self.N
 
     def rwg(self):
@@ -253,9 +261,10 @@ class Context:
         k_ext, k_int = complex(k_ext), complex(k_int)
         self._check(self._L.bem_assemble(self._h, k_ext.real, k_ext.imag, k_int.real, k_int.imag, eta_ext, eta_int,
                                          flags), "assemble")
+        self._n = 2 * self.N
 
     def get_Z(self):
-        n = 2 * self.N
+        n = self._n
         Z = np.zeros((n, n), np.complex128)
         self._check(self._L.bem_get_Z(self._h, _p(Z), 1), "get_Z")
         return Z
@@ -289,12 +298,16 @@ class Context:
         L = np.zeros((self.N, self.N), np.complex128)
         K = np.zeros((self.N, self.N), np.complex128)
         self._check(self._L.bem_assemble_LK(self._h, k.real, k.imag, _p(L), _p(K)), "assemble_LK")
+        self._n = 2 * self.N
         return L, K
 
     # -- LU ---------------------------------------------------------------
     def set_Z(self, Z):
         Zc = np.ascontiguousarray(Z, dtype=np.complex128)
+        if Zc.ndim != 2 or Zc.shape[0] != Zc.shape[1]:
+            raise ValueError("set_Z: a square matrix is needed")
         self._check(self._L.bem_set_Z(self._h, _p(Zc), Zc.shape[0], 1), "set_Z")
+        self._n = Zc.shape[0]
 
     def factor(self, precision="fp32"):
         p = F32_3M if precision in ("fp32", F32_3M) else F64
@@ -314,6 +327,7 @@ class Context:
         LUc = np.ascontiguousarray(LU, dtype=np.complex128)
         ip = np.ascontiguousarray(ipiv, dtype=np.int32)
         self._check(self._L.bem_set_lu(self._h, _p(LUc), _pi(ip), LUc.shape[0]), "set_lu")
+        self._n = LUc.shape[0]
 
     def solve(self, B=None, ir_tol=1e-10, ir_max=10, return_X=True, n=None, nrhs=None, allow_noconv=False):
         """Solve Z X = B.  B: (n, nrhs) or (n,) array, or None for the device RHS."""
@@ -322,13 +336,13 @@ class Context:
             B = np.asarray(B, dtype=np.complex128)
             if B.ndim == 1:
                 B = B[:, None]
-            n, nrhs = B.shape
+            n, nrhs = self._rows(B)
             Bc = np.ascontiguousarray(B.T)
             bp = _p(Bc)
         else:
             bp = None
             if n is None:
-                n = 2 * self.N
+                n = self._n
         X = np.zeros((nrhs, n), np.complex128) if (return_X and nrhs) else None
         rc = self._L.bem_solve(self._h, bp, nrhs or 0, _p(X) if X is not None else None, ir_tol, ir_max,
                                ctypes.byref(st))
@@ -347,13 +361,13 @@ class Context:
             B = np.asarray(B, dtype=np.complex128)
             if B.ndim == 1:
                 B = B[:, None]
-            n, nrhs = B.shape
+            n, nrhs = self._rows(B)
             Bc = np.ascontiguousarray(B.T)
             bp = _p(Bc)
         else:
             bp = None
             if n is None:
-                n = 2 * self.N
+                n = self._n
         X = np.zeros((nrhs, n), np.complex128) if (return_X and nrhs) else None
         rc = self._L.bem_solve_gmres(self._h, bp, nrhs or 0, _p(X) if X is not None else None, tol, restart,
                                      max_iter, PRECONDS[precond], ctypes.byref(st))
@@ -376,7 +390,7 @@ class Context:
         one = R.ndim == 1
         if one:
             R = R[:, None]
-        n, nrhs = R.shape
+        n, nrhs = self._rows(R)
         Rc = np.ascontiguousarray(R.T)
         Zo = np.zeros((nrhs, n), np.complex128)
         self._check(self._L.bem_precond_apply(self._h, PRECONDS[precond], _p(Rc), nrhs, _p(Zo)), "precond_apply")
