@@ -78,8 +78,8 @@ __global__ __launch_bounds__(256) void k_bj_gather(BjView v, int N, int ld, cons
 // the rest of the matrix takes one rank-64 product (k_bj_rows, k_bj_update).
 //
 // What bounds it: the rank-64 FP64 products (186 us each) and the panels' serial
-// chain of pivot steps (45 us per 16 columns at 1107 unknowns, blocks side by
-// side).  27 blocks of up to 1107 unknowns: 8.3 ms, where one
+// chain of pivot steps (44 us per 16 columns at 1107 unknowns, blocks side by
+// side).  27 blocks of up to 1107 unknowns: 9.0 ms, where one
 // workgroup sweeping its whole block from memory at every pivot step (the
 // earlier form) took 1600 ms, n2^2 complex values moved per step.
 // ---------------------------------------------------------------------------
@@ -122,7 +122,7 @@ __device__ __forceinline__ int bj_best_lane(const BjCand& k) {
 
 // Columns of unrolled elimination steps; the registers rotate by so many after them.
 // (All 16 steps unrolled, each row read ahead whole and with two selects per value
-// for the pivot row, took 98 us per panel of 1107 rows, 45 now.  With three rows per
+// for the pivot row, took 98 us per panel of 1107 rows, 44 now.  With three rows per
 // thread, those rows' included, the kernel takes all 256 registers and spills eight.)
 constexpr int BJ_S = 4;
 
