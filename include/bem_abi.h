@@ -106,7 +106,7 @@ int bem_autotune(bem_ctx* ctx, int nrhs, double* out, int nout);
 int bem_gemm_plan(bem_ctx* ctx, int prec, int large, int skinny, long cap);
 
 /* The GEMM plan of one precision (prec 0 FP32, 1 FP64) as doubles: large,
- * skinny and panel configuration, grid cap, tuned (0/1), chosen by trial
+ * skinny and panel configuration (the last taken by no product), grid cap, tuned (0/1), chosen by trial
  * factorisations (0/1), then the trial factorisation time in ms of each
  * trailing-update configuration (5 values, 0 where none ran), then the
  * trailing update's configuration.  The FP32 trailing update runs on its own
